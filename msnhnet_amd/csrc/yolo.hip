@@ -919,6 +919,297 @@ __global__ __launch_bounds__(256) void yoloNmsScanKernel(const unsigned long lon
     }
 }
 
+// ---- all classes of an image by one workgroup, up to 1024 candidates --------------------------------------------------------------
+// What a detector's real scenes give: tens to some hundreds of candidates per image.  The launches above serve them badly -- a workgroup
+// per (class, image) of which all but a few are empty, one barrier per kept box (169 kept boxes of one class: 171 us), three further
+// launches from 257 members up (722 members: 105 us in all), records in no order behind a counter that has to be cleared first and
+// copied back.  Here the workgroup holds one candidate per lane:
+//   1. bitonic sort by (class, objectness, score, cell): partners less than a wavefront apart exchange registers, the others go through LDS;
+//   2. for every pair of 64-member chunks with a class in common, a word per member of the later one: which members of the earlier one would
+//      erase it (one wavefront per pair of chunks, lane = victim);
+//   3. the first wavefront walks the chunks: a member is out if one of its words meets a kept member of an earlier chunk, the rest of the
+//      chunk is resolved by fixed-point iteration on its own words (bit masks only, no barrier);
+//   4. the classes ordered by their best (score, cell), rows written where the reference's output has them -- straight into the caller's
+//      pinned memory when it passes such -- and the image's candidate counter reset for the next forward.
+// Bound by the instruction issue of the one CU in steps 1 and 2; 27 us for 338 candidates of one class and 64 us for 722, launch included,
+// where the launches above took 181 and 114 (trace) plus four copies and two stream hand-overs.
+constexpr int NMS_IMG = 1024;
+constexpr int NMS_IMG_LDS = (NMS_IMG / 64) * (NMS_IMG / 64 + 1) / 2 * 64 * 8;      // one word per member and chunk at or before its own
+
+// The value of lane ^ J, without LDS: quad permutes, mirrors of half rows (lane ^ 7) and rows (lane ^ 15), row and half-wave swaps.
+template <int J>
+__device__ __forceinline__ unsigned xorLane(unsigned v)
+{
+    const int x = static_cast<int>(v);
+    if (J == 1) return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);
+    if (J == 2) return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);
+    if (J == 4) return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xf, 0xf, false), 0x141, 0xf, 0xf, false);
+    if (J == 8) return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, false), 0x140, 0xf, 0xf, false);
+    if (J == 16)
+    {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (threadIdx.x & 16) ? r[0] : r[1];
+    }
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (threadIdx.x & 32) ? r[0] : r[1];
+}
+
+// iouAbove(kept, victim) for the lanes with `mine`, without a branch unless some lane's quotient stands next to the threshold.
+__device__ __forceinline__ bool iouAboveFlat(const float4 &k, float karea, const float4 &j, float jarea, float thr, bool mine)
+{
+#pragma clang fp contract(off)
+    const float ix2 = (k.z < j.z) ? k.z : j.z;
+    const float ix1 = (j.x < k.x) ? k.x : j.x;
+    const float iy2 = (k.w < j.w) ? k.w : j.w;
+    const float iy1 = (j.y < k.y) ? k.y : j.y;
+    const float iw = ix2 - ix1 + 1;
+    const float ih = iy2 - iy1 + 1;
+    const float inter = (iw < 0 ? 0 : iw) * (ih < 0 ? 0 : ih);
+    const float uni = jarea + karea - inter;
+    const float p = thr * uni;
+    const int plain = static_cast<int>(thr >= 0.f) & static_cast<int>(thr <= 1e3f) & static_cast<int>(uni > 1e-20f) & static_cast<int>(uni < 1e30f) & static_cast<int>(inter < 1e30f);
+    const int above = static_cast<int>(p > 1e-20f) & static_cast<int>(inter > p * 1.00001f);
+    const int below = static_cast<int>(inter == 0.f) | (static_cast<int>(p > 1e-20f) & static_cast<int>(inter < p * 0.99999f));
+    bool hit = (static_cast<int>(mine) & plain & above) != 0;
+    if (__any(static_cast<int>(mine) & ((plain & (above | below)) ^ 1))) hit = mine && 1.f * inter / uni > thr;
+    return hit;
+}
+
+struct NmsKey
+{
+    unsigned long long hi, lo;
+    unsigned ix;
+};
+
+__device__ __forceinline__ void nmsSortStep(NmsKey &e, const NmsKey &o, int j, int k2)
+{
+    const bool less = e.hi < o.hi || (e.hi == o.hi && (e.lo < o.lo || (e.lo == o.lo && e.ix > o.ix)));
+    const bool wantMax = ((threadIdx.x & j) == 0) == ((threadIdx.x & k2) == 0);
+    if (less == wantMax) e = o;
+}
+
+template <int J>
+__device__ __forceinline__ void nmsSortLanes(NmsKey &e, int k2)
+{
+    NmsKey o;
+    o.hi = (static_cast<unsigned long long>(xorLane<J>(static_cast<unsigned>(e.hi >> 32))) << 32) | xorLane<J>(static_cast<unsigned>(e.hi));
+    o.lo = (static_cast<unsigned long long>(xorLane<J>(static_cast<unsigned>(e.lo >> 32))) << 32) | xorLane<J>(static_cast<unsigned>(e.lo));
+    o.ix = xorLane<J>(e.ix);
+    nmsSortStep(e, o, J, k2);
+}
+
+__global__ __launch_bounds__(NMS_IMG) void yoloNmsImageKernel(const float *__restrict__ rows, int candCap, int *__restrict__ candCnt, float thr,
+                                                              float *__restrict__ outRows, int *__restrict__ outHdr)
+{
+#pragma clang fp contract(off)
+    constexpr int NW = NMS_IMG / 64;
+    __shared__ unsigned long long hiS[NMS_IMG], loS[NMS_IMG];      // sort exchange; afterwards hiS: the best key of a class segment
+    __shared__ unsigned ixS[NMS_IMG];                              // row of a sorted member
+    __shared__ float4 corner[NMS_IMG];                             // sorted members
+    __shared__ float area[NMS_IMG];
+    __shared__ int seg[NMS_IMG];                                   // class segment of a sorted member
+    __shared__ int segStart[NMS_IMG + 1], segOut[NMS_IMG];         // first kept member of a segment; where its rows go
+    __shared__ unsigned short keptPos[NMS_IMG];
+    __shared__ int heads[NW], nKept, bad;
+    extern __shared__ __attribute__((aligned(16))) unsigned long long erasedBy[];      // [c (c + 1) / 2 + rc][64], rc <= c
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int found = candCnt[b];
+    const int n = found < candCap ? found : candCap;
+    const float *r = rows + static_cast<size_t>(b) * candCap * 8;
+    int *hdr = outHdr + b * 4;
+    if (n == 0 || n > NMS_IMG)
+    {
+        __syncthreads();                                           // every lane has read the counter
+        if (tid == 0)
+        {
+            *reinterpret_cast<int4 *>(hdr) = make_int4(found, 0, n > NMS_IMG ? 1 : 0, 0);
+            candCnt[b] = 0;
+        }
+        return;
+    }
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    NmsKey e = {0ull, 0ull, static_cast<unsigned>(tid)};           // below every real key (class numbers are not negative)
+    if (tid < n)
+    {
+        const float4 q = *reinterpret_cast<const float4 *>(r + static_cast<size_t>(tid) * 8 + 4);    // objectness, class score, class, cell
+        const float score = q.x * q.y;
+        if (!(score == score) || !(q.x == q.x)) bad = 1;
+        e.hi = (static_cast<unsigned long long>(~static_cast<unsigned>(static_cast<int>(q.z))) << 32) | orderedBits(q.x);
+        e.lo = (static_cast<unsigned long long>(orderedBits(score)) << 32) | ~static_cast<unsigned>(q.w);
+    }
+    int S = 64;
+    while (S < n) S <<= 1;
+    for (int k2 = 2; k2 <= S; k2 <<= 1)
+    {
+        for (int j = k2 >> 1; j >= 64; j >>= 1)
+        {
+            __syncthreads();
+            if (tid < S) { hiS[tid] = e.hi; loS[tid] = e.lo; ixS[tid] = e.ix; }
+            __syncthreads();
+            if (tid < S) nmsSortStep(e, {hiS[tid ^ j], loS[tid ^ j], ixS[tid ^ j]}, j, k2);
+        }
+        if (tid >= S) continue;
+        if (k2 > 32) nmsSortLanes<32>(e, k2);
+        if (k2 > 16) nmsSortLanes<16>(e, k2);
+        if (k2 > 8) nmsSortLanes<8>(e, k2);
+        if (k2 > 4) nmsSortLanes<4>(e, k2);
+        if (k2 > 2) nmsSortLanes<2>(e, k2);
+        nmsSortLanes<1>(e, k2);
+    }
+    const unsigned long long hi = e.hi, lo = e.lo;
+    const int ix = static_cast<int>(e.ix);
+    __syncthreads();
+    if (bad)
+    {
+        if (tid == 0)
+        {
+            *reinterpret_cast<int4 *>(hdr) = make_int4(found, 0, 2, 0);
+            candCnt[b] = 0;
+        }
+        return;
+    }
+    hiS[tid] = hi;
+    ixS[tid] = ix;
+    if (tid < n)
+    {
+        const float4 q = *reinterpret_cast<const float4 *>(r + static_cast<size_t>(ix) * 8);
+        const float ax1 = q.x - q.z / 2.f, ax2 = q.x + q.z / 2.f, ay1 = q.y - q.w / 2.f, ay2 = q.y + q.w / 2.f;
+        corner[tid] = make_float4(ax1, ay1, ax2, ay2);
+        area[tid] = (ax2 - ax1 + 1) * (ay2 - ay1 + 1);
+    }
+    __syncthreads();
+    const bool head = tid < n && (tid == 0 || (hiS[tid - 1] >> 32) != (hi >> 32));
+    const unsigned long long headMask = __ballot(head);
+    if (lane == 0) heads[wave] = __popcll(headMask);
+    __syncthreads();
+    int before = 0, nSeg = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+    {
+        before += w < wave ? heads[w] : 0;
+        nSeg += heads[w];
+    }
+    const int mySeg = before + __popcll(headMask & ((2ull << lane) - 1ull)) - 1;       // (2 << 63 wraps to 0: every lane up to 63)
+    seg[tid] = mySeg;
+    unsigned long long *segTop = hiS;
+    segTop[tid] = 0ull;                                            // (the neighbour's key was read before the last barrier)
+    __syncthreads();
+    if (tid < n) atomicMax(&segTop[mySeg], lo);
+    const int W = (n + 63) / 64;
+    // Boxes more than a unit apart in x or y have no intersection (inter = 0, never above a threshold >= 0): most pairs, decided for the
+    // whole wavefront by four comparisons.  The margin of 2 instead of the "+ 1" of the extents keeps the skip on the safe side of any
+    // rounding; a comparison with a NaN corner is false, which does not skip.
+    const bool skipOk = thr >= 0.f;
+    for (int item = __builtin_amdgcn_readfirstlane(wave); item < W * (W + 1) / 2; item += NW)
+    {
+        int c = 0;
+        while ((c + 1) * (c + 2) / 2 <= item) ++c;
+        const int rc = item - c * (c + 1) / 2;
+        const int j = c * 64 + lane, jSafe = j < n ? j : n - 1;
+        const int i0 = rc * 64, iEnd = n - i0 < 64 ? n - i0 : 64;
+        unsigned long long word = 0ull;
+        if (seg[i0 + iEnd - 1] >= seg[c * 64])                     // (segments ascend: else no class in common)
+        {
+            const float4 jc = corner[jSafe];
+            const float ja = area[jSafe];
+            const int js = seg[jSafe];
+            const float jx1m = jc.x - 2.f, jy1m = jc.y - 2.f, jx2p = jc.z + 2.f, jy2p = jc.w + 2.f;
+            // every lane collects the members near its own victim as bits; what is left of them after the masks it tests exactly.  Member k's
+            // corners come out of lane k's registers: broadcast LDS reads of 16 bytes per lane kept the LDS busy for twice as long.
+            const float4 mc = corner[i0 + lane < n ? i0 + lane : n - 1];
+            const auto laneOf = [](float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); };
+            unsigned half[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+            {
+                unsigned bits = 0u;
+#pragma unroll 4
+                for (int k = 0; k < 32; ++k)
+                {
+                    const int m = h * 32 + k;                      // (past the end: masked below)
+                    const int apart = static_cast<int>(laneOf(mc.x, m) > jx2p) | static_cast<int>(jx1m > laneOf(mc.z, m)) | static_cast<int>(laneOf(mc.y, m) > jy2p) | static_cast<int>(jy1m > laneOf(mc.w, m));
+                    bits = (bits << 1) | static_cast<unsigned>(apart);
+                }
+                half[h] = ~__brev(bits);
+            }
+            unsigned long long todo = (static_cast<unsigned long long>(half[1]) << 32) | half[0];
+            if (!skipOk) todo = ~0ull;
+            if (iEnd < 64) todo &= (1ull << iEnd) - 1ull;
+            if (rc == c) todo &= (1ull << lane) - 1ull;            // a chunk's own: earlier members only
+            while (__any(todo != 0ull))
+            {
+                const int k = todo != 0ull ? __ffsll(static_cast<long long>(todo)) - 1 : 0;
+                const bool mine = todo != 0ull && seg[i0 + k] == js;
+                if (iouAboveFlat(corner[i0 + k], area[i0 + k], jc, ja, thr, mine)) word |= 1ull << k;
+                todo &= todo - 1ull;
+            }
+        }
+        erasedBy[item * 64 + lane] = word;
+    }
+    __syncthreads();
+    if (wave == 0)
+    {
+        unsigned long long aliveOf = 0ull;                         // lane c: the kept members of chunk c
+        int K = 0, lastSeg = -1;
+        for (int c = 0; c < W; ++c)
+        {
+            const unsigned long long *words = erasedBy + c * (c + 1) / 2 * 64 + lane;
+            unsigned long long hit = 0ull;
+            for (int rc = 0; rc < c; ++rc) hit |= words[rc * 64] & readLane64(aliveOf, rc);
+            const unsigned long long own = words[c * 64];
+            const int j = c * 64 + lane;
+            const unsigned long long cand = __ballot(j < n && hit == 0ull);
+            unsigned long long alive = cand;
+            for (;;)
+            {
+                const unsigned long long next = cand & ~__ballot((own & alive) != 0ull);
+                if (next == alive) break;                          // (the first t members are final after t rounds)
+                alive = next;
+            }
+            const int p = K + __popcll(alive & ((1ull << lane) - 1ull));
+            const int js = j < n ? seg[j] : -1;
+            const int leftSeg = __shfl_up(js, 1, 64);                // (every lane takes part)
+            if (js >= 0 && (lane == 0 ? lastSeg : leftSeg) != js) segStart[js] = p;
+            if ((alive >> lane) & 1ull) keptPos[p] = static_cast<unsigned short>(j);
+            if (lane == c) aliveOf = alive;
+            K += __popcll(alive);
+            lastSeg = __shfl(js, 63, 64);
+        }
+        if (lane == 0) nKept = K;
+    }
+    __syncthreads();
+    const int picks = nKept;
+    if (tid == 0) segStart[nSeg] = picks;
+    __syncthreads();
+    if (tid < nSeg)
+    {
+        const unsigned long long mine = segTop[tid];               // (score, cell) differ between any two members
+        int at = 0;
+#pragma unroll 4
+        for (int t = 0; t < nSeg; ++t)
+        {
+            const int kept = segStart[t + 1] - segStart[t];
+            at += segTop[t] > mine ? kept : 0;
+        }
+        segOut[tid] = at;
+    }
+    __syncthreads();
+    if (tid < picks)
+    {
+        const int at = keptPos[tid], s = seg[at];
+        const float4 *q = reinterpret_cast<const float4 *>(r + static_cast<size_t>(ixS[at]) * 8);
+        float4 *o = reinterpret_cast<float4 *>(outRows + (static_cast<size_t>(b) * NMS_IMG + segOut[s] + tid - segStart[s]) * 8);
+        o[0] = q[0];
+        o[1] = q[1];
+    }
+    if (tid == 0)
+    {
+        *reinterpret_cast<int4 *>(hdr) = make_int4(found, picks, 0, 0);
+        candCnt[b] = 0;
+    }
+}
+
 __global__ __launch_bounds__(256) void yoloGatherKernel(const float *__restrict__ decoded, long long decStride, const int *__restrict__ candIdx,
                                                         int candCap, const int *__restrict__ candCnt, float *__restrict__ rows, int per,
                                                         int batch)
@@ -1202,16 +1493,17 @@ int currentDevice(int *dev)
     return 0;
 }
 
-// (g_nmsMutex held) once per device: the LDS limits of the large-class kernels
+// (g_nmsMutex held) once per device: the kernels' LDS limits
 bool ensureNmsAttributes(NmsDeviceState &st)
 {
     if (st.attrsTried) return st.attrsOk;
     st.attrsTried = true;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(yoloNmsBigKernel), hipFuncAttributeMaxDynamicSharedMemorySize, NMS_BIG_LDS);
     if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(yoloNmsScanKernel), hipFuncAttributeMaxDynamicSharedMemorySize, NMS_SCAN_LDS);
+    if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(yoloNmsImageKernel), hipFuncAttributeMaxDynamicSharedMemorySize, NMS_IMG_LDS);
     if (e != hipSuccess)
     {
-        std::snprintf(st.error, sizeof(st.error), "yolo_nms: hipFuncSetAttribute for the large-class kernels: %s", hipGetErrorString(e));
+        std::snprintf(st.error, sizeof(st.error), "yolo_nms: hipFuncSetAttribute for the NMS kernels: %s", hipGetErrorString(e));
         (void)hipGetLastError();
     }
     st.attrsOk = e == hipSuccess;
@@ -1266,6 +1558,26 @@ extern "C" int msnh_hip_yolo_nms(int batch, int classes, const float *rows, int 
     }
     return launchYoloNms(batch, classes, rows, cand_cap, cand_cnt, nms_thresh, kept, kept_cap, kept_cnt, static_cast<int *>(workspace), workspace ? workspace_bytes : 0,
                          resolveStream(s));
+}
+
+extern "C" int msnh_hip_yolo_nms_images_cap(void) { return NMS_IMG; }
+
+extern "C" int msnh_hip_yolo_nms_images(int batch, const float *rows, int cand_cap, int *cand_cnt, float nms_thresh, float *out_rows, int *out_hdr,
+                                        msnh_stream_t s)
+{
+    MSNH_REQUIRE(batch > 0 && batch <= 65535 && cand_cap > 0 && cand_cap <= (1 << 24), "yolo_nms_images: bad geometry");
+    MSNH_REQUIRE(rows && cand_cnt && out_rows && out_hdr, "yolo_nms_images: NULL pointer");
+    MSNH_REQUIRE(reinterpret_cast<uintptr_t>(rows) % 16 == 0 && reinterpret_cast<uintptr_t>(out_rows) % 16 == 0 && reinterpret_cast<uintptr_t>(out_hdr) % 16 == 0,
+                 "yolo_nms_images: rows, out_rows and out_hdr must be 16-byte aligned");
+    int dev = -1;
+    if (int rc = currentDevice(&dev)) return rc;
+    {
+        std::lock_guard<std::mutex> lock(g_nmsMutex);
+        MSNH_REQUIRE(ensureNmsAttributes(g_nms[dev]), "%s", g_nms[dev].error);
+    }
+    hipLaunchKernelGGL(yoloNmsImageKernel, dim3(batch), dim3(NMS_IMG), NMS_IMG_LDS, resolveStream(s), rows, cand_cap, cand_cnt, nms_thresh, out_rows, out_hdr);
+    MSNH_LAUNCH_CHECK();
+    return 0;
 }
 
 extern "C" size_t msnh_hip_yolo_nms_static_max_bytes(void) { return kNmsScratchInts * sizeof(int); }

@@ -131,7 +131,14 @@ public:
     // YOLO post-processing buffers (only for networks ending in a yoloout layer)
     int  yoloCells = 0;                     // sum over heads of 3*H*W
     int  yoloClasses = 0;
-    DeviceBuffer yoloDecoded, yoloCandIdx, yoloCandCnt, yoloRows;
+    DeviceBuffer yoloDecoded, yoloCandIdx;
+    // candidate counts and rows, one set per copy-back slot: a forward writes the set of its own slot, so what an earlier forward left
+    // for the host or the NMS is read in place while the next one runs
+    DeviceBuffer yoloCandCnt[2], yoloRows[2];
+    int yoloSlot = 0;                       // the set that the launches issued now write
+    int   *candCnt() const { return yoloCandCnt[yoloSlot].as<int>(); }
+    float *candRows() const { return yoloRows[yoloSlot].as<float>(); }
+    void clearCandidates(msnh_stream_t s);  // the counts of the current set to zero: the start of every forward
 
     int addTensor(int n, int h, int w, int c, int dtype, const std::string &name, PlanTensor::Layout layout = PlanTensor::NHWC);
     PlanOp &addOp(PlanOp::Kind kind, int in0, int in1, int out, int layerIndex, const std::string &name);

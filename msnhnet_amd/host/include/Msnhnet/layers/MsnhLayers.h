@@ -337,10 +337,12 @@ public:
     ~YoloOutLayer() override;
     int lower(Plan &plan, int in, int layerIndex) override;
     void forwardGPU(NetworkState &netState) override;      // device candidate compaction + host sort / NMS
-    // The three stages of forwardGPU, separately, so that a caller can overlap the host stage of one batch with
+    // The stages of forwardGPU, separately, so that a caller can overlap the host stage of one batch with
     // the device work of the next (two copy-back slots):
+    bool nmsInForward();                                   // the next forward ends with the NMS itself (enqueueImageNms)
     void enqueueGather(msnh_stream_t s);                   // device: compact the candidate rows
-    void enqueueCopyBack(msnh_stream_t s, int slot);       // device -> pinned host, asynchronous
+    void enqueueImageNms(msnh_stream_t s, int slot);       // device: NMS of every image, kept boxes straight into the slot's pinned memory
+    void enqueueCopyBack(msnh_stream_t s, int slot, bool inForward);   // device -> pinned host, asynchronous (inForward: enqueueImageNms has done it)
     void finish(int slot);                                 // host: wait, sort, NMS -> finalOut
 
     static std::vector<YoloBox> nms(const std::vector<YoloBox> &bboxes, const float &nmsThresh, const bool &useSoftNms, const float &sigma = 0.3f);
@@ -368,6 +370,9 @@ public:
     // placement with the shorter time between results stays.
     static int deviceNms;
     static const int kDeviceNmsFew = 2048;
+    // Up to kImageNms candidates per image (msnh_hip_yolo_nms_images_cap) the NMS is the last launch of the forward itself: one workgroup
+    // per image takes about as long as the copies and stream hand-overs that a stream of its own would need.
+    static const int kImageNms = 1024;
     static const int kDeviceNmsCandidates = 6144;
     static const int kTrialBatches = 16;
 
@@ -392,14 +397,15 @@ private:
     std::vector<int> _yoloIndexes;
     std::vector<YoloInfo> _yoloLayersInfo;
     int _yoloAllInputNum = 0, _pixels = 0;
-    // devCnt / devRows: device-side snapshot of one forward's candidates, so the copy to the host can run on its own
-    // stream while the next forward already overwrites the plan's buffers
+    // The candidates themselves stay in the plan's set of this slot (Plan::yoloCandCnt / yoloRows) until the slot is fetched: the copy
+    // to the host runs on its own stream while the next forward writes the other set.
     struct Slot
     {
         PinnedBuffer cnt, rows, decoded, kept, keptCnt;
-        DeviceBuffer devCnt, devRows, devKept, devKeptCnt, devNmsWs;
+        PinnedBuffer imageHdr, imageRows;  // enqueueImageNms: {candidates, kept, flag, 0} and the kept rows of every image
+        DeviceBuffer devKept, devKeptCnt, devNmsWs;
         msnh_event_t event = nullptr, ready = nullptr;
-        bool pending = false, onDevice = false;
+        bool pending = false, onDevice = false, inForward = false;
         bool trial = false;                // part of a device trial of the automatic placement
         size_t rowsCopied = 0;             // row slots per image that the asynchronous copy brings to the host
         size_t quick = 0;                  // device NMS: records that the asynchronous copy brings to the host
@@ -417,6 +423,8 @@ private:
     bool _haveLastFinish = false, _lastFinishHost = false;
     void noteResult(const Slot &sl, bool pipelined);
     void prepareSlot(Slot &sl, bool deviceNmsBuffers);
+    void finishImages(const Slot &sl, const DeviceBuffer &devRows);
+    std::vector<YoloBox> hostNmsOfImage(const DeviceBuffer &devRows, int image, int candidates);
     Slot _slots[2];
 };
 }

@@ -11,6 +11,8 @@
 
 namespace Msnhnet
 {
+class YoloOutLayer;
+
 class MsnhNet_API NetBuilder
 {
 public:
@@ -63,6 +65,7 @@ public:
     void sync();
     std::vector<float> fetchClassify();
     std::vector<std::vector<YoloBox>> fetchYolo();
+    const std::vector<std::vector<YoloBox>> &fetchYoloResult();     // the same without the copy; valid until the next fetch
     float *deviceInputBuffer();               // the builder's own device input buffer (batch*C*H*W floats)
     // Letterboxes one 8-bit RGB image (HWC, host memory) on the device into slot `index` of the input batch: what
     // CVUtil::getPaddingZeroF32C3 + the float upload do in the reference (MsnhCVUtil.cpp:203-261); then
@@ -143,8 +146,12 @@ private:
     PinnedBuffer _imagePinned;
     PinnedBuffer _inputPinned, _outputPinned;
     msnh_stream_t _stream = nullptr;
-    msnh_graph_t  _graph = nullptr;
-    const float  *_graphInput = nullptr;
+    // The captured forward.  Detectors have one per copy-back slot and per place of the NMS (inside the forward or behind it), captured
+    // when first needed; [0][0] is the only one of a classifier.
+    msnh_graph_t  _graphs[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+    bool _countsClear[2] = {false, false};     // the slot's candidate counts are zero on the device (the NMS inside a forward leaves them so)
+    void dropGraphs();
+    void issueForward(YoloOutLayer *yout, bool inForward, msnh_stream_t s);
     int _nextSlot = 0, _inFlight = 0;          // copy-back slots of the detection post-processing
 };
 }

@@ -453,7 +453,7 @@ int msnhnet_fetch_classify(msnhnet_t net, float *out, long long cap, long long *
 
 int msnhnet_fetch_yolo(msnhnet_t net, int *counts, float *boxes, long long cap_boxes, long long *total)
 {
-    return guarded([&] { packBoxes(nb(net).fetchYolo(), counts, boxes, cap_boxes, total); });
+    return guarded([&] { packBoxes(nb(net).fetchYoloResult(), counts, boxes, cap_boxes, total); });
 }
 
 int msnhnet_profile_ops(msnhnet_t net, int kind, int reps, float *ms_total, int *launches, double *flops)

@@ -1417,7 +1417,23 @@ void YoloOutLayer::enqueueGather(msnh_stream_t s)
     Plan &pl = *plan;
     if (pl.sparseYolo) return;          // the heads' candidate-only decode already wrote the compact rows
     MSNH_DEV(msnh_hip_yolo_gather(_batch, _channel - 5, pl.yoloDecoded.as<float>(), static_cast<long long>(pl.yoloCells) * _channel,
-                                  pl.yoloCandIdx.as<int>(), pl.yoloCells, pl.yoloCandCnt.as<int>(), pl.yoloRows.as<float>(), s));
+                                  pl.yoloCandIdx.as<int>(), pl.yoloCells, pl.candCnt(), pl.candRows(), s));
+}
+
+bool YoloOutLayer::nmsInForward()
+{
+    if (plan == nullptr) MSNH_THROW("YoloOut: layer is not part of a planned network");
+    if (deviceNms == 0 || _useSoftNms || keepClassScores || !plan->sparseYolo || _lastMaxCandidates > kImageNms) return false;
+    prepareSlot(_slots[0], true);           // (not inside the capture of the forward: allocations)
+    prepareSlot(_slots[1], true);
+    return true;
+}
+
+void YoloOutLayer::enqueueImageNms(msnh_stream_t s, int slot)
+{
+    Plan &pl = *plan;
+    Slot &sl = _slots[slot & 1];
+    MSNH_DEV(msnh_hip_yolo_nms_images(_batch, pl.candRows(), pl.yoloCells, pl.candCnt(), _nmsThresh, sl.imageRows.as<float>(), sl.imageHdr.as<int>(), s));
 }
 
 // Everything a slot needs, at its full size, before the slot is first used.  An allocation or a free of device or pinned memory
@@ -1434,9 +1450,9 @@ void YoloOutLayer::prepareSlot(Slot &sl, bool deviceNmsBuffers)
     if (sl.event == nullptr) MSNH_DEV(msnh_hip_event_create(&sl.event));
     if (keepClassScores) return;
     if (sl.ready == nullptr) MSNH_DEV(msnh_hip_event_create(&sl.ready));
-    if (sl.devCnt.bytes() < cntBytes) sl.devCnt.alloc(cntBytes);
-    if (sl.devRows.bytes() < rowBytes) sl.devRows.alloc(rowBytes);
     if (!deviceNmsBuffers) return;
+    sl.imageHdr.reserve(sizeof(int) * 4 * static_cast<size_t>(_batch));
+    sl.imageRows.reserve(sizeof(float) * 8 * kImageNms * static_cast<size_t>(_batch));
     const size_t keptCntBytes = sizeof(int) * (1 + static_cast<size_t>(_batch));
     const size_t keptCap = cells * static_cast<size_t>(_batch);
     if (sl.devKeptCnt.bytes() < keptCntBytes) sl.devKeptCnt.alloc(keptCntBytes);
@@ -1447,12 +1463,21 @@ void YoloOutLayer::prepareSlot(Slot &sl, bool deviceNmsBuffers)
     if (sl.devNmsWs.bytes() < wsBytes) sl.devNmsWs.alloc(wsBytes);
 }
 
-void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
+void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot, bool inForward)
 {
     Plan &pl = *plan;
+    const DeviceBuffer &devCnt = pl.yoloCandCnt[slot & 1], &devRows = pl.yoloRows[slot & 1];
     Slot &sl = _slots[slot & 1];
     if (sl.pending) MSNH_THROW("YoloOut: the results of the previous forward in this slot were not fetched");
-    sl.onDevice = false;
+    sl.onDevice = sl.inForward = inForward;
+    sl.trial = false;
+    if (inForward)
+    {
+        // the forward's last launch leaves the boxes in pinned memory: nothing to copy
+        MSNH_DEV(msnh_hip_event_record(sl.event, s));
+        sl.pending = true;
+        return;
+    }
     const size_t cells = static_cast<size_t>(pl.yoloCells);
     const bool mayUseDevice = deviceNms != 0 && !_useSoftNms && !keepClassScores;
     prepareSlot(_slots[0], mayUseDevice);
@@ -1462,8 +1487,8 @@ void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
     if (keepClassScores)
     {
         // the decoded tensor is too large to snapshot: everything leaves on the forward's own stream
-        MSNH_DEV(msnh_hip_memcpy_d2h(sl.cnt.ptr(), pl.yoloCandCnt.ptr(), cntBytes, s));
-        MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.ptr(), pl.yoloRows.ptr(), rowBytes, s));
+        MSNH_DEV(msnh_hip_memcpy_d2h(sl.cnt.ptr(), devCnt.ptr(), cntBytes, s));
+        MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.ptr(), devRows.ptr(), rowBytes, s));
         const size_t bytes = sizeof(float) * cells * static_cast<size_t>(_channel) * static_cast<size_t>(_batch);
         sl.decoded.reserve(bytes);
         MSNH_DEV(msnh_hip_memcpy_d2h(sl.decoded.ptr(), pl.yoloDecoded.ptr(), bytes, s));
@@ -1472,7 +1497,7 @@ void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
         sl.rowsCopied = cells;
         return;
     }
-    // Snapshot on the device (microseconds), then cross PCIe on a second stream: the next forward does not wait for
+    // The candidates cross PCIe on a second stream: the next forward writes the other slot's set and does not wait for
     // the copy (several MiB: every cell has a row slot, the count is only known on the device).
     // copyOnForwardStream (the instances of a NetGroup): everything below goes onto the forward's own stream.  A process has four
     // hardware queues; three instances with a copy stream each are six busy streams, and a copy stream that shares a queue with
@@ -1481,11 +1506,12 @@ void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
     // other instances fill the gap.
     if (!copyOnForwardStream && _copyStream == nullptr) MSNH_DEV(msnh_hip_stream_create(&_copyStream));
     const msnh_stream_t cs = copyOnForwardStream ? s : _copyStream;
-    MSNH_DEV(msnh_hip_memcpy_d2d(sl.devCnt.ptr(), pl.yoloCandCnt.ptr(), cntBytes, s));
-    MSNH_DEV(msnh_hip_memcpy_d2d(sl.devRows.ptr(), pl.yoloRows.ptr(), rowBytes, s));
-    MSNH_DEV(msnh_hip_event_record(sl.ready, s));
-    if (!copyOnForwardStream) MSNH_DEV(msnh_hip_stream_wait_event(cs, sl.ready));
-    MSNH_DEV(msnh_hip_memcpy_d2h(sl.cnt.ptr(), sl.devCnt.ptr(), cntBytes, cs));
+    if (!copyOnForwardStream)
+    {
+        MSNH_DEV(msnh_hip_event_record(sl.ready, s));
+        MSNH_DEV(msnh_hip_stream_wait_event(cs, sl.ready));
+    }
+    MSNH_DEV(msnh_hip_memcpy_d2h(sl.cnt.ptr(), devCnt.ptr(), cntBytes, cs));
     // auto: few candidates (real detections) -> the device; thousands per image -> the device too unless a second forward is in flight
     // (the host's sort + NMS then runs beside that forward and costs the device nothing, whereas the device NMS takes about 0.1 ms of
     // device time per batch from it) and the host stage has kept up with the device so far
@@ -1499,7 +1525,7 @@ void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
     sl.onDevice = !_useSoftNms && (deviceNms == 2 || (deviceNms == 1 && autoDevice));
     if (sl.onDevice)
     {
-        // NMS on the snapshot, on the copy stream: it overlaps the next forward, and what crosses PCIe is the kept boxes.  The records
+        // NMS on the copy stream: it overlaps the next forward, and what crosses PCIe is the kept boxes.  The records
         // leave with the counters, as many as the previous result had and half as many again: a copy asked for in finish() would
         // queue behind whatever the device runs by then (the next forward), and the host would wait for that instead of working
         // beside it.  finish() fetches the rest only if there are more.
@@ -1508,7 +1534,7 @@ void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
         sl.quick = std::min(keptCap, std::max(kQuickRecords, _lastKept + _lastKept / 2 + 1024));
         MSNH_DEV(msnh_hip_fill_zero(sl.devKeptCnt.ptr(), keptCntBytes, cs));
         const size_t wsBytes = msnh_hip_yolo_nms_pair_workspace_bytes(_batch, _channel - 5, pl.yoloCells);
-        MSNH_DEV(msnh_hip_yolo_nms(_batch, _channel - 5, sl.devRows.as<float>(), pl.yoloCells, sl.devCnt.as<int>(), _nmsThresh, sl.devKept.as<float>(),
+        MSNH_DEV(msnh_hip_yolo_nms(_batch, _channel - 5, devRows.as<float>(), pl.yoloCells, devCnt.as<int>(), _nmsThresh, sl.devKept.as<float>(),
                                    static_cast<int>(keptCap), sl.devKeptCnt.as<int>(), sl.devNmsWs.ptr(), wsBytes, cs));
         MSNH_DEV(msnh_hip_memcpy_d2h(sl.keptCnt.ptr(), sl.devKeptCnt.ptr(), keptCntBytes, cs));
         MSNH_DEV(msnh_hip_memcpy_d2h(sl.kept.ptr(), sl.devKept.ptr(), sl.quick * kRecordBytes, cs));
@@ -1522,12 +1548,12 @@ void YoloOutLayer::enqueueCopyBack(msnh_stream_t s, int slot)
         if (const char *forced = std::getenv("MSNH_YOLO_ROWS_PREFIX")) guess = static_cast<size_t>(std::max(1L, std::atol(forced)));    // (tests)
         sl.rowsCopied = std::min(guess, cells);
         if (sl.rowsCopied == cells)
-            MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.ptr(), sl.devRows.ptr(), rowBytes, cs));
+            MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.ptr(), devRows.ptr(), rowBytes, cs));
         else
             for (int b = 0; b < _batch; ++b)
             {
                 const size_t off = static_cast<size_t>(b) * cells * 8;
-                MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.as<float>() + off, sl.devRows.as<float>() + off, sizeof(float) * 8 * sl.rowsCopied, cs));
+                MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.as<float>() + off, devRows.as<float>() + off, sizeof(float) * 8 * sl.rowsCopied, cs));
             }
     }
     MSNH_DEV(msnh_hip_event_record(sl.event, cs));
@@ -1589,6 +1615,48 @@ void YoloOutLayer::noteResult(const Slot &sl, bool pipelined)
     _lastFinishHost = !sl.onDevice;
 }
 
+// An image whose candidates the device did not suppress itself: its rows are still in the slot's set on the device.
+std::vector<YoloBox> YoloOutLayer::hostNmsOfImage(const DeviceBuffer &devRows, int image, int candidates)
+{
+    std::vector<float> rows(static_cast<size_t>(candidates) * 8);
+    if (_fetchStream == nullptr) MSNH_DEV(msnh_hip_stream_create(&_fetchStream));
+    MSNH_DEV(msnh_hip_memcpy_d2h(rows.data(), devRows.as<float>() + static_cast<size_t>(image) * static_cast<size_t>(plan->yoloCells) * 8, rows.size() * sizeof(float), _fetchStream));
+    MSNH_DEV(msnh_hip_stream_sync(_fetchStream));
+    return nmsSorted(boxesFromRows(rows.data(), candidates, nullptr), _nmsThresh);
+}
+
+// Results of enqueueImageNms: the rows are the kept boxes in output order.
+void YoloOutLayer::finishImages(const Slot &sl, const DeviceBuffer &devRows)
+{
+    const int *hdr = sl.imageHdr.as<int>();
+    batchHasBox.assign(static_cast<size_t>(_batch), false);
+    finalOut.resize(static_cast<size_t>(_batch));
+    _lastMaxCandidates = 0;
+    _lastKept = 0;
+    for (int b = 0; b < _batch; ++b, hdr += 4)
+    {
+        const int candidates = std::min(hdr[0], plan->yoloCells);
+        _lastMaxCandidates = std::max(_lastMaxCandidates, candidates);
+        batchHasBox[static_cast<size_t>(b)] = candidates > 0;
+        std::vector<YoloBox> &out = finalOut[static_cast<size_t>(b)];
+        if (hdr[2] != 0) out = hostNmsOfImage(devRows, b, candidates);        // more candidates than the kernel takes, or NaN scores
+        else
+        {
+            out.assign(static_cast<size_t>(hdr[1]), YoloBox());
+            const float *r = sl.imageRows.as<float>() + static_cast<size_t>(b) * kImageNms * 8;
+            for (YoloBox &q : out)
+            {
+                q.xywhBox = Box::XYWHBox(r[0], r[1], r[2], r[3]);
+                q.conf = r[4];
+                q.bestClsConf = r[5];
+                q.bestClsIdx = static_cast<int>(r[6]);
+                r += 8;
+            }
+        }
+        _lastKept += out.size();
+    }
+}
+
 void YoloOutLayer::finish(int slot)
 {
     Slot &sl = _slots[slot & 1];
@@ -1600,6 +1668,13 @@ void YoloOutLayer::finish(int slot)
     _lastSlot = slot & 1;
     lastOnDevice = sl.onDevice;
     noteResult(sl, _slots[(slot ^ 1) & 1].pending);
+    const DeviceBuffer &devRows = plan->yoloRows[slot & 1];
+    if (sl.inForward)
+    {
+        finishImages(sl, devRows);
+        if (std::getenv("MSNH_DEBUG_TIMING")) std::fprintf(stderr, "yoloout finish (NMS in the forward, %zu boxes): wait %.3f ms, host %.3f ms\n", _lastKept, dbgWait, TimeUtil::getElapsedTime(dbg0) - dbgWait);
+        return;
+    }
     const int cells = plan->yoloCells;
     const int per = _channel;
     const int *cnt = sl.cnt.as<int>();
@@ -1633,23 +1708,17 @@ void YoloOutLayer::finish(int slot)
         TaskPool::instance().parallelFor(_batch, [&](int b) {
             if (keptCnt[1 + b] == 0) finalOut[static_cast<size_t>(b)] = boxesFromKept(perImage[static_cast<size_t>(b)]);
         });
-        std::vector<float> hostRows;
         for (int b = 0; b < _batch; ++b)
         {
             batchHasBox[static_cast<size_t>(b)] = cnt[b] > 0;
-            if (keptCnt[1 + b] == 0) continue;
-            // the device left this image to the host (a class with very many candidates, or NaN scores): the snapshot still holds its rows
-            const int n = std::min(cnt[b], cells);
-            hostRows.resize(static_cast<size_t>(n) * 8);
-            MSNH_DEV(msnh_hip_memcpy_d2h(hostRows.data(), sl.devRows.as<float>() + static_cast<size_t>(b) * cells * 8, hostRows.size() * sizeof(float), _fetchStream));
-            MSNH_DEV(msnh_hip_stream_sync(_fetchStream));
-            finalOut[static_cast<size_t>(b)] = nmsSorted(boxesFromRows(hostRows.data(), n, nullptr), _nmsThresh);
+            // the device left this image to the host (a class with very many candidates, or NaN scores)
+            if (keptCnt[1 + b] != 0) finalOut[static_cast<size_t>(b)] = hostNmsOfImage(devRows, b, std::min(cnt[b], cells));
         }
         if (std::getenv("MSNH_DEBUG_TIMING")) std::fprintf(stderr, "yoloout finish (device NMS, %zu boxes): wait %.3f ms, host %.3f ms\n", total, dbgWait, TimeUtil::getElapsedTime(dbg0) - dbgWait);
         return;
     }
     {
-        // rows beyond the prefix that was copied ahead of time (the device snapshot of this slot is still intact)
+        // rows beyond the prefix that was copied ahead of time (the slot's set on the device is still intact)
         bool more = false;
         for (int b = 0; b < _batch; ++b)
         {
@@ -1657,7 +1726,7 @@ void YoloOutLayer::finish(int slot)
             if (n <= sl.rowsCopied) continue;
             if (_fetchStream == nullptr) MSNH_DEV(msnh_hip_stream_create(&_fetchStream));
             const size_t off = (static_cast<size_t>(b) * static_cast<size_t>(cells) + sl.rowsCopied) * 8;
-            MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.as<float>() + off, sl.devRows.as<float>() + off, sizeof(float) * 8 * (n - sl.rowsCopied), _fetchStream));
+            MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.as<float>() + off, devRows.as<float>() + off, sizeof(float) * 8 * (n - sl.rowsCopied), _fetchStream));
             more = true;
         }
         if (more) MSNH_DEV(msnh_hip_stream_sync(_fetchStream));
@@ -1748,7 +1817,7 @@ std::string YoloOutLayer::placementDetail() const
 void YoloOutLayer::forwardGPU(NetworkState &netState)
 {
     enqueueGather(netState.stream);
-    enqueueCopyBack(netState.stream, 0);
+    enqueueCopyBack(netState.stream, 0, false);
     finish(0);
 }
 

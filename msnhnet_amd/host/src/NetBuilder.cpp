@@ -66,7 +66,7 @@ void NetBuilder::setOnlyCpu(const bool &onlyCpu)
 
 void NetBuilder::clearLayers()
 {
-    if (_graph) { msnh_hip_graph_destroy(_graph); _graph = nullptr; }
+    dropGraphs();
     _net->plan.reset();
     for (BaseLayer *l : _net->layers) delete l;
     _net->layers.clear();
@@ -382,8 +382,11 @@ static void setupYoloBuffers(Plan &plan, int batch)
     const size_t cells = static_cast<size_t>(plan.yoloCells);
     plan.yoloDecoded.alloc(sizeof(float) * cells * per * static_cast<size_t>(batch));
     plan.yoloCandIdx.alloc(sizeof(int) * cells * static_cast<size_t>(batch));
-    plan.yoloCandCnt.alloc(sizeof(int) * static_cast<size_t>(std::max(batch, 64)));
-    plan.yoloRows.alloc(sizeof(float) * 8 * cells * static_cast<size_t>(batch));
+    for (int k = 0; k < 2; ++k)
+    {
+        plan.yoloCandCnt[k].alloc(sizeof(int) * static_cast<size_t>(std::max(batch, 64)));
+        plan.yoloRows[k].alloc(sizeof(float) * 8 * cells * static_cast<size_t>(batch));
+    }
     plan.findYoloHeads();
 }
 
@@ -396,7 +399,7 @@ void NetBuilder::finalizePlan()
     if (_inputDev.bytes() < inBytes) _inputDev.alloc(inBytes);
     _inputPinned.reserve(inBytes);
     _netState->gpuInput = _inputDev.as<float>();
-    if (_graph) { msnh_hip_graph_destroy(_graph); _graph = nullptr; }
+    dropGraphs();
     _nextSlot = 0;
     _inFlight = 0;
 
@@ -450,7 +453,7 @@ void NetBuilder::finalizePlan()
             host[i] = static_cast<float>(state >> 8) * (1.0f / 16777216.0f);
         }
         MSNH_DEV(msnh_hip_memcpy_h2d(_inputDev.ptr(), host, inBytes, _stream));
-        if (cal->yoloCandCnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(cal->yoloCandCnt.ptr(), cal->yoloCandCnt.bytes(), _stream));
+        cal->clearCandidates(_stream);
         cal->runCalibration(_stream);
         plan->applyCalibration(cal->amaxOfTensors());
     }
@@ -578,7 +581,8 @@ static std::vector<float> yoloLayerDump(Plan &plan, const YoloLayer *yl, const P
 void NetBuilder::runLayersEager()
 {
     Plan &plan = *_net->plan;
-    if (plan.yoloCandCnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(plan.yoloCandCnt.ptr(), plan.yoloCandCnt.bytes(), _stream));
+    plan.yoloSlot = 0;
+    plan.clearCandidates(_stream);
     _layerOutputs.assign(_net->layers.size(), std::vector<float>());
     msnh_event_t e0 = nullptr, e1 = nullptr;
     MSNH_DEV(msnh_hip_event_create(&e0));
@@ -625,25 +629,20 @@ void NetBuilder::enqueueForward(const float *deviceInput)
     {
         // the full decoded rows are only written for YoloBox::classesVal; the recorded launches carry the choice
         plan.yoloKeepDecoded = YoloOutLayer::keepClassScores;
-        if (_graph) { msnh_hip_graph_destroy(_graph); _graph = nullptr; }
+        dropGraphs();
     }
+    const int slot = yout ? _nextSlot : 0;
+    const bool inForward = yout && yout->nmsInForward();
+    plan.yoloSlot = slot;
+    if (inForward && !_countsClear[slot]) plan.clearCandidates(_stream);
     static const bool eager = std::getenv("MSNH_EAGER") != nullptr;
-    if (eager)
-    {
-        if (plan.yoloCandCnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(plan.yoloCandCnt.ptr(), plan.yoloCandCnt.bytes(), _stream));
-        plan.runAll(_stream);
-        if (yout) yout->enqueueGather(_stream);
-    }
-    else if (_graph == nullptr)
+    msnh_graph_t &graph = _graphs[slot][inForward ? 1 : 0];
+    if (eager) issueForward(yout, inForward, _stream);
+    else if (graph == nullptr)
     {
         // Record the whole forward once; later calls replay it with a single launch.
         MSNH_DEV(msnh_hip_graph_begin(_stream));
-        try
-        {
-            if (plan.yoloCandCnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(plan.yoloCandCnt.ptr(), plan.yoloCandCnt.bytes(), _stream));
-            plan.runAll(_stream);
-            if (yout) yout->enqueueGather(_stream);
-        }
+        try { issueForward(yout, inForward, _stream); }
         catch (...)
         {
             msnh_graph_t junk = nullptr;
@@ -651,16 +650,35 @@ void NetBuilder::enqueueForward(const float *deviceInput)
             if (junk) msnh_hip_graph_destroy(junk);
             throw;
         }
-        MSNH_DEV(msnh_hip_graph_end(_stream, &_graph));
+        MSNH_DEV(msnh_hip_graph_end(_stream, &graph));
     }
-    if (!eager) MSNH_DEV(msnh_hip_graph_launch(_graph, _stream));
+    if (!eager) MSNH_DEV(msnh_hip_graph_launch(graph, _stream));
     if (yout)
     {
+        _countsClear[slot] = inForward;
         // results leave the device right behind the forward, so the next forward can start while the host sorts
-        yout->enqueueCopyBack(_stream, _nextSlot);
+        yout->enqueueCopyBack(_stream, slot, inForward);
         _nextSlot ^= 1;
         ++_inFlight;
     }
+}
+
+// The launches of one forward, into a capture or straight onto the stream.
+void NetBuilder::issueForward(YoloOutLayer *yout, bool inForward, msnh_stream_t s)
+{
+    Plan &plan = *_net->plan;
+    if (!inForward) plan.clearCandidates(s);
+    plan.runAll(s);
+    if (yout) yout->enqueueGather(s);
+    if (inForward) yout->enqueueImageNms(s, plan.yoloSlot);
+}
+
+void NetBuilder::dropGraphs()
+{
+    for (auto &perSlot : _graphs)
+        for (msnh_graph_t &g : perSlot)
+            if (g) { msnh_hip_graph_destroy(g); g = nullptr; }
+    _countsClear[0] = _countsClear[1] = false;
 }
 
 void NetBuilder::sync() { MSNH_DEV(msnh_hip_stream_sync(_stream)); }
@@ -673,7 +691,9 @@ std::vector<float> NetBuilder::fetchClassify()
     return out;
 }
 
-std::vector<std::vector<YoloBox>> NetBuilder::fetchYolo()
+std::vector<std::vector<YoloBox>> NetBuilder::fetchYolo() { return fetchYoloResult(); }
+
+const std::vector<std::vector<YoloBox>> &NetBuilder::fetchYoloResult()
 {
     BaseLayer *last = _net->layers.back();
     if (last->type() != LayerType::YOLO_OUT) MSNH_THROW("not a yolo net");
@@ -920,12 +940,12 @@ std::string NetBuilder::profileEachOp(int reps, std::vector<double> *values)
         const PlanOp &op = plan.ops[i];
         if (op.dead || op.chainHead >= 0) continue;
         plan.run(i, i + 1, _stream);
-        const bool yolo = op.kind == PlanOp::YOLO_DECODE && plan.yoloCandCnt.ptr();
+        const bool yolo = op.kind == PlanOp::YOLO_DECODE;
         MSNH_DEV(msnh_hip_event_record(e0, _stream));
         for (int r = 0; r < reps; ++r)
         {
             // (a head appends to the candidate list: start every repetition from an empty one, as a forward does)
-            if (yolo) MSNH_DEV(msnh_hip_fill_zero(plan.yoloCandCnt.ptr(), plan.yoloCandCnt.bytes(), _stream));
+            if (yolo) plan.clearCandidates(_stream);
             plan.run(i, i + 1, _stream);
         }
         MSNH_DEV(msnh_hip_event_record(e1, _stream));

@@ -458,7 +458,7 @@ float Plan::fp16Headroom(msnh_stream_t s)
     struct WriteAll { bool &f; explicit WriteAll(bool &x) : f(x) { f = true; } ~WriteAll() { f = false; } } writeAll(_tailWriteAll);
     DeviceBuffer res(sizeof(float) * 2);
     MSNH_DEV(msnh_hip_fill_zero(res.ptr(), sizeof(float) * 2, s));
-    if (yoloCandCnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(yoloCandCnt.ptr(), yoloCandCnt.bytes(), s));
+    clearCandidates(s);
     for (PlanOp &op : ops)
     {
         if (op.dead) continue;
@@ -1418,16 +1418,16 @@ void Plan::launch(PlanOp &op, msnh_stream_t s)
             }
             MSNH_DEV(msnh_hip_yolo_decode_candidates_heads(in.dtype, in.n, op.classes, static_cast<int>(yoloHeadOps.size()), heads, op.yoloVersion,
                                                            yoloKeepDecoded ? yoloDecoded.as<float>() : nullptr, static_cast<long long>(yoloCells) * per,
-                                                           op.confThresh, yoloCandIdx.as<int>(), yoloCells, yoloCandCnt.as<int>(), yoloRows.as<float>(), s));
+                                                           op.confThresh, yoloCandIdx.as<int>(), yoloCells, candCnt(), candRows(), s));
         }
         else if (sparseYolo && cand)
             MSNH_DEV(msnh_hip_yolo_decode_candidates(in.dtype, in.n, in.h, in.w, op.classes, ptr(op.in0), ld(op.in0), mulOf(op.in0), op.anchors.data(),
                                                      op.ratio, op.yoloVersion, yoloKeepDecoded ? decoded : nullptr, static_cast<long long>(yoloCells) * per, op.confThresh,
-                                                     yoloCandIdx.as<int>(), yoloCells, op.cellBase, yoloCandCnt.as<int>(), yoloRows.as<float>(), s));
+                                                     yoloCandIdx.as<int>(), yoloCells, op.cellBase, candCnt(), candRows(), s));
         else
             MSNH_DEV(msnh_hip_yolo_decode(in.dtype, in.n, in.h, in.w, op.classes, ptr(op.in0), ld(op.in0), mulOf(op.in0), op.anchors.data(), op.ratio,
                                           op.yoloVersion, decoded, static_cast<long long>(yoloCells) * per, op.confThresh,
-                                          cand ? yoloCandIdx.as<int>() : nullptr, yoloCells, op.cellBase, cand ? yoloCandCnt.as<int>() : nullptr, s));
+                                          cand ? yoloCandIdx.as<int>() : nullptr, yoloCells, op.cellBase, cand ? candCnt() : nullptr, s));
         break;
     }
     }
@@ -1464,6 +1464,12 @@ void Plan::run(size_t opBegin, size_t opEnd, msnh_stream_t s)
 {
     for (size_t i = opBegin; i < opEnd && i < ops.size(); ++i)
         if (!ops[i].dead) launch(ops[i], s);
+}
+
+void Plan::clearCandidates(msnh_stream_t s)
+{
+    const DeviceBuffer &cnt = yoloCandCnt[yoloSlot];
+    if (cnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(cnt.ptr(), cnt.bytes(), s));
 }
 
 void Plan::exportTensor(int t, std::vector<float> &dst, msnh_stream_t s)

@@ -624,6 +624,43 @@ def test_yolo_nms():
         abi.check(abi.lib().msnh_hip_yolo_nms(5, cls, gu.ptr(rd), cells, gu.ptr(cd), nms_t, None, 7 * cells, gu.ptr(kcd), None, 0, None))
 
 
+@pytest.mark.parametrize("classes,spread", [(1, 120.0), (3, 300.0), (90, 60.0), (1, 1e4)])
+def test_yolo_nms_images(classes, spread):
+    """one-launch NMS per image against the host procedure, rows bit for bit and in output order: candidate counts around the chunk and
+    sort sizes, ties in both sort keys, infinite boxes; 1025 candidates and a NaN score are flagged; the counters come back zero"""
+    import gpuutil as gu
+    from msnhnet_amd import netapi
+    gu.init()
+    rng = np.random.default_rng(classes)
+    counts = [0, 1, 2, 63, 64, 65, 127, 129, 511, 722, 1000, 1023, 1024, 1025, 70]
+    cap = 1100
+    rows = np.zeros((len(counts), cap, 8), np.float32)
+    for b, n in enumerate(counts):
+        r = rows[b, :n]
+        r[:, :2] = rng.uniform(0, spread, (n, 2)); r[:, 2:4] = rng.uniform(5, 40, (n, 2))
+        r[:, 4] = rng.integers(9, 17, n) / 16.0; r[:, 5] = rng.integers(1, 9, n) / 8.0
+        r[:, 6] = rng.integers(0, classes, n); r[:, 7] = rng.permutation(4 * cap)[:n]
+        if n > 500:
+            r[3:6, 2] = np.inf
+    rows[14, 7, 5] = np.nan
+    rd, cd = gu.dev(rows), gu.dev(np.array(counts, np.int32))
+    out = torch.full((len(counts), abi.lib().msnh_hip_yolo_nms_images_cap(), 8), -7.0).cuda()
+    hdr = torch.full((len(counts), 4), -7, dtype=torch.int32).cuda()
+    gu.sync()
+    abi.check(abi.lib().msnh_hip_yolo_nms_images(len(counts), gu.ptr(rd), cap, gu.ptr(cd), 0.45, gu.ptr(out), gu.ptr(hdr), None))
+    gu.sync()
+    assert not cd.cpu().numpy().any()
+    for b, (n, h) in enumerate(zip(counts, hdr.cpu().numpy())):
+        assert h[0] == n and h[2] == (1 if n > 1024 else 2 if b == 14 else 0), (b, h)
+        if h[2]:
+            continue
+        want = netapi.boxes_from_candidates(rows[b, :n], 0.45)
+        assert h[1] == len(want), (n, h, len(want))
+        got = out[b].cpu().numpy()
+        assert np.array_equal(got[:h[1], :7], want, equal_nan=True), n
+        assert (got[h[1]:] == -7.0).all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_absmax(dtype):
     import gpuutil as gu
