@@ -88,7 +88,7 @@ def plan_hash(plan_text):
     import hashlib
     import re
     # (which of the GEMM-type kernels and which tile runs a layer is the per-layer search's choice and may differ between two runs)
-    lines = [re.sub(r"\[(igemm_splitk|igemm|pointwise)", "[gemm", re.sub(r" t\d+", "", l)) for l in plan_text.splitlines()[1:]]
+    lines = [re.sub(r"\[(igemm_fusedk|igemm_splitk|igemm|pointwise)", "[gemm", re.sub(r" t\d+", "", l)) for l in plan_text.splitlines()[1:]]
     return hashlib.sha256("\n".join(lines).encode()).hexdigest()[:16]
 
 

@@ -69,6 +69,11 @@ enum msnh_conv_algo
                                   for MSNH_CONV_WINOGRAD, no workspace */
     MSNH_CONV_IGEMM_TAIL = 11, /* not an algorithm of msnh_hip_conv2d: the label of a launch of msnh_hip_conv2d_tail (a convolution and the 1x1
                                   convolution that reads its result) */
+    MSNH_CONV_IGEMM_FUSEDK = 12, /* IGEMM with the K loop cut into slices on separate workgroups like IGEMM_SPLITK, but the slices of an output tile are
+                                  summed (in slice order) inside the launch, by the workgroup that finishes last, which also runs the
+                                  epilogue.  desc.tile = tile configuration + 256 * slices, both given (2..32 slices).  The workspace's
+                                  first 64 KiB must be zero before the first launch that uses it; every launch leaves them zero.
+                                  Same weight packing as IGEMM.  Never chosen by AUTO. */
     MSNH_CONV_MBCONV = 10      /* not an algorithm of msnh_hip_conv2d: the label of a launch of msnh_hip_mbconv (1x1 expand, 3x3 depthwise
                                   and 1x1 project convolution of an inverted-residual block as one) */
 };
@@ -139,7 +144,7 @@ typedef struct msnh_conv_desc
     float res_mul;
     float out_mul;
     int   algo;         /* msnh_conv_algo */
-    int   tile;         /* IGEMM only: 0 = library default, 1..msnh_hip_conv2d_tile_count() = forced tile configuration */
+    int   tile;         /* IGEMM only: 0 = library default, 1..msnh_hip_conv2d_tile_count() = forced tile configuration (IGEMM_FUSEDK: see there) */
     int   out_upsample; /* 0 or 1: y is [batch][out_h][out_w].  2 (MSNH_CONV_IGEMM only, no residual, out_c and out_ld multiples of 8): every
                            result pixel is written to the 2 x 2 pixels it maps to under nearest-neighbour upsampling, y is
                            [batch][2 out_h][2 out_w] -- the convolution in front of an UpSampleLayer (src/layers/MsnhUpSampleLayer.cpp:96-118,
@@ -173,7 +178,7 @@ size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo);
  *   STEM           : [k*k*in_c][out_c] float32 regardless of dtype
  * `packed` is host memory of msnh_hip_conv2d_packed_weight_elems() elements; upload it afterwards. */
 int msnh_hip_conv2d_pack_weights(const msnh_conv_desc *d, int algo, const float *oihw, void *packed);
-/* Scratch bytes `workspace` must provide for `algo` (0 for all but WINOGRAD). */
+/* Scratch bytes `workspace` must provide for `algo` (0 for all but WINOGRAD, IGEMM_SPLITK and IGEMM_FUSEDK). */
 size_t msnh_hip_conv2d_workspace_bytes(const msnh_conv_desc *d, int algo);
 /* x: NHWC d->dtype (STEM: NCHW float32); w: packed for the resolved algo; scale/shift: float32[out_c] or NULL;
  * residual: NHWC d->dtype with pixel stride res_ld, or NULL; y: NHWC d->out_dtype with pixel stride out_ld. */

@@ -17,6 +17,7 @@ int igemmTailTileFirst();
 int convIgemmWs(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                 const void *residual, void *y, hipStream_t st, bool dryRun, void *splitWs, size_t splitWsBytes);
 size_t igemmSplitKWorkspaceBytes(const msnh_conv_desc *d);
+size_t igemmFusedKWorkspaceBytes(const msnh_conv_desc *d);
 bool pointwiseOk(const msnh_conv_desc *d);
 int convPointwise(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift, const void *residual,
                   void *y, hipStream_t st);
@@ -355,7 +356,7 @@ int msnh_hip_conv2d_pack_layout_version(void) { return 1; }
 
 int msnh_hip_conv2d_tile_supported(const msnh_conv_desc *d, int tile)
 {
-    if (!d || validate(d) || tile < 0 || tile > igemmTileCount()) return 0;
+    if (!d || validate(d) || tile < 0 || (tile > igemmTileCount() && d->algo != MSNH_CONV_IGEMM_FUSEDK)) return 0;
     msnh_conv_desc t = *d;
     if (d->algo == MSNH_CONV_POINTWISE) return tile == 0 && pointwiseOk(d) ? 1 : 0;
     if (d->algo == MSNH_CONV_WINOGRAD_FUSED) return tile == 0 && winogradFusedOk(d) ? 1 : 0;
@@ -366,7 +367,7 @@ int msnh_hip_conv2d_tile_supported(const msnh_conv_desc *d, int tile)
         winogradGemmDesc(d, &t);
     }
     else if (!igemmOk(d)) return 0;
-    if (tile == 0 && d->algo != MSNH_CONV_IGEMM_SPLITK) return 1;
+    if (tile == 0 && d->algo != MSNH_CONV_IGEMM_SPLITK && d->algo != MSNH_CONV_IGEMM_FUSEDK) return 1;
     t.tile = tile;
     return convIgemm(&t, d, d, nullptr, nullptr, nullptr, &t, nullptr, true) == 0 ? 1 : 0;      // pointers unused in a dry run
 }
@@ -440,6 +441,7 @@ int msnh_hip_conv2d_pack_weights(const msnh_conv_desc *d, int algo, const float 
     case MSNH_CONV_DIRECT:
     case MSNH_CONV_IGEMM:
     case MSNH_CONV_IGEMM_SPLITK:
+    case MSNH_CONV_IGEMM_FUSEDK:
     case MSNH_CONV_POINTWISE:
         for (int oc = 0; oc < d->out_c; ++oc)
             for (int ci = 0; ci < cinG; ++ci)
@@ -477,6 +479,7 @@ size_t msnh_hip_conv2d_workspace_bytes(const msnh_conv_desc *d, int algo)
 {
     if (!d) return 0;
     if (algo == MSNH_CONV_IGEMM_SPLITK) return igemmSplitKWorkspaceBytes(d);
+    if (algo == MSNH_CONV_IGEMM_FUSEDK) return validate(d) == 0 && igemmOk(d) ? igemmFusedKWorkspaceBytes(d) : 0;
     return algo == MSNH_CONV_WINOGRAD ? winogradWorkspaceBytes(d) : 0;
 }
 
@@ -503,6 +506,7 @@ int msnh_hip_conv2d(const msnh_conv_desc *d, const void *x, const void *w, const
         MSNH_REQUIRE(d->out_upsample != 2 || reinterpret_cast<uintptr_t>(y) % 16 == 0, "conv2d: the upsampling epilogue needs a 16-byte aligned y");
         return convIgemm(d, x, w, scale, shift, residual, y, st, false);
     case MSNH_CONV_IGEMM_SPLITK:
+    case MSNH_CONV_IGEMM_FUSEDK:
         MSNH_REQUIRE(igemmOk(d), "conv2d: IGEMM needs (in_c/groups) and in_ld to be multiples of %d", d->dtype == MSNH_F16 ? 8 : 4);
         MSNH_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0, "conv2d: IGEMM needs 16-byte aligned x and w");
         return convIgemmWs(d, x, w, scale, shift, residual, y, st, false, workspace, workspace_bytes);

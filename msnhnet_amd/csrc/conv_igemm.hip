@@ -3,6 +3,34 @@
 
 namespace msnh {
 
+int igemmF16F16Part0(IgemmArgs &a, int groups, int tile, hipStream_t st);
+int igemmF16F16Part1(IgemmArgs &a, int groups, int tile, hipStream_t st);
+int igemmF16F16Part2(IgemmArgs &a, int groups, int tile, hipStream_t st);
+
+int igemmF16F16(IgemmArgs &a, int groups, int tile, hipStream_t st)
+{
+    return tile % kIgemmParts == 0 ? igemmF16F16Part0(a, groups, tile, st) : (tile % kIgemmParts == 1 ? igemmF16F16Part1(a, groups, tile, st) : igemmF16F16Part2(a, groups, tile, st));
+}
+
+int igemmF16F32Part0(IgemmArgs &a, int groups, int tile, hipStream_t st);
+int igemmF16F32Part1(IgemmArgs &a, int groups, int tile, hipStream_t st);
+int igemmF16F32Part2(IgemmArgs &a, int groups, int tile, hipStream_t st);
+
+int igemmF16F32(IgemmArgs &a, int groups, int tile, hipStream_t st)
+{
+    return tile % kIgemmParts == 0 ? igemmF16F32Part0(a, groups, tile, st) : (tile % kIgemmParts == 1 ? igemmF16F32Part1(a, groups, tile, st) : igemmF16F32Part2(a, groups, tile, st));
+}
+
+int igemmF32F32Part0(IgemmArgs &a, int groups, int tile, hipStream_t st);
+int igemmF32F32Part1(IgemmArgs &a, int groups, int tile, hipStream_t st);
+int igemmF32F32Part2(IgemmArgs &a, int groups, int tile, hipStream_t st);
+
+int igemmF32F32(IgemmArgs &a, int groups, int tile, hipStream_t st)
+{
+    return tile % kIgemmParts == 0 ? igemmF32F32Part0(a, groups, tile, st) : (tile % kIgemmParts == 1 ? igemmF32F32Part1(a, groups, tile, st) : igemmF32F32Part2(a, groups, tile, st));
+}
+
+
 // Default tile: BM follows the output-channel count so narrow layers do not waste MFMA rows; deep K
 // (>= 8 vectors per tap) moves 8 vectors per row per step, shallow K 4.
 int igemmHeuristicTile(const msnh_conv_desc *d)
@@ -27,7 +55,7 @@ size_t igemmSplitKWorkspaceBytes(const msnh_conv_desc *d)
 // tiles that carry a tail, 0 the first of them that takes the shape.
 static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                         const void *residual, void *y, hipStream_t st, bool dryRun, void *splitWs, size_t splitWsBytes,
-                        const msnh_conv_tail_desc *tail, const void *w2, const float *scale2, const float *shift2, void *z)
+                        const msnh_conv_tail_desc *tail, const void *w2, const float *scale2, const float *shift2, void *z, size_t *wsNeed = nullptr)
 {
     IgemmArgs a;
     a.tailOn = tail ? 1 : 0;
@@ -65,7 +93,7 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
     a.vecOk = (d->out_ld % 8 == 0) && ((d->out_c / d->groups) % 8 == 0 || d->groups == 1) &&
               (reinterpret_cast<uintptr_t>(y) % (8 * outEl) == 0) &&
               (!a.hasRes || (d->res_ld % 8 == 0 && reinterpret_cast<uintptr_t>(residual) % 16 == 0));
-    a.splitMax = 0; a.splitK = 1; a.ws = nullptr; a.wsLd = d->out_c;
+    a.splitMax = 0; a.splitK = 1; a.fusedK = 0; a.wsNeed = a.wsBytes = 0; a.ws = nullptr; a.wsLd = d->out_c;
     if (a.up2) MSNH_REQUIRE(d->algo != MSNH_CONV_IGEMM_SPLITK && !tail, "conv2d: the upsampling epilogue goes with the plain implicit GEMM");
     if (d->algo == MSNH_CONV_IGEMM_SPLITK)
     {
@@ -79,6 +107,15 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
         a.ws = static_cast<float *>(splitWs);
     }
     int tile = d->tile;
+    if (d->algo == MSNH_CONV_IGEMM_FUSEDK)
+    {
+        a.fusedK = d->tile >> 8;
+        tile = d->tile & 255;
+        MSNH_REQUIRE(!tail && tile >= 1 && tile <= kIgemmTiles && a.fusedK >= 2 && a.fusedK <= 32, "conv2d: IGEMM_FUSEDK takes desc.tile = tile + 256 * slices, 2 to 32 slices");
+        MSNH_REQUIRE(dryRun || reinterpret_cast<uintptr_t>(splitWs) % 16 == 0, "conv2d: the workspace must be 16-byte aligned");
+        a.ws = static_cast<float *>(splitWs);
+        a.wsBytes = splitWsBytes;
+    }
     if (tail)
     {
         MSNH_REQUIRE(d->dtype == MSNH_F16 && d->out_dtype == MSNH_F16 && d->groups == 1 && d->algo != MSNH_CONV_IGEMM_SPLITK, "conv2d_tail: float16, ungrouped, unsplit");
@@ -89,16 +126,26 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
         else a.vecOk = (d->out_ld % 8 == 0) && (d->out_c % 8 == 0) && (!d->has_residual || d->res_ld % 8 == 0);
     }
     if (tile <= 0 || tile > kIgemmTiles) tile = igemmHeuristicTile(d);
-    if (d->dtype == MSNH_F16)
-        return d->out_dtype == MSNH_F16 ? igemmF16F16(a, d->groups, tile, st) : igemmF16F32(a, d->groups, tile, st);
-    MSNH_REQUIRE(d->out_dtype == MSNH_F32, "igemm: float32 input needs float32 output");
-    return igemmF32F32(a, d->groups, tile, st);
+    MSNH_REQUIRE(d->dtype == MSNH_F16 || d->out_dtype == MSNH_F32, "igemm: float32 input needs float32 output");
+    const int rc = d->dtype != MSNH_F16 ? igemmF32F32(a, d->groups, tile, st)
+                                        : (d->out_dtype == MSNH_F16 ? igemmF16F16(a, d->groups, tile, st) : igemmF16F32(a, d->groups, tile, st));
+    if (wsNeed) *wsNeed = a.wsNeed;
+    return rc;
 }
 
 int convIgemmWs(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                 const void *residual, void *y, hipStream_t st, bool dryRun, void *splitWs, size_t splitWsBytes)
 {
     return convIgemmAny(d, x, w, scale, shift, residual, y, st, dryRun, splitWs, splitWsBytes, nullptr, nullptr, nullptr, nullptr, nullptr);
+}
+
+// Workspace of a sliced launch as desc.tile describes it; 0: the shape and tile do not take it.
+size_t igemmFusedKWorkspaceBytes(const msnh_conv_desc *d)
+{
+    size_t need = 0;
+    msnh_conv_desc t = *d;
+    t.algo = MSNH_CONV_IGEMM_FUSEDK;
+    return convIgemmAny(&t, d, d, nullptr, nullptr, nullptr, &t, nullptr, true, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, &need) == 0 ? need : 0;
 }
 
 int convIgemmTail(const msnh_conv_desc *d, const msnh_conv_tail_desc *tail, const void *x, const void *w, const float *scale, const float *shift,

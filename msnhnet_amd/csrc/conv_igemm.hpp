@@ -44,6 +44,8 @@ struct IgemmArgs
     int ragged;             // cinG is not a multiple of the tile's K step
     int splitMax;           // > 1: split-K requested, at most this many slices of the K loop (grid y)
     int splitK;             // slices actually used by the launch
+    int fusedK;             // > 1: that many slices, summed inside the launch (splitKCombine)
+    size_t wsNeed, wsBytes; // fusedK: workspace this launch needs / has
     float *ws;              // split-K: float32 partial sums [slice][pixel][out_c]
     int wsLd;               // = out_c of the whole convolution
     int buffersOk;          // both extents fit a buffer resource
@@ -254,6 +256,63 @@ template <int I, int N, typename F> __device__ __forceinline__ void staticFor(F 
 
 template <int BM, int TM, int NW = 4> constexpr size_t igemmEpilogueLds() { return (2 * BM + NW * 32 * (TM + 4)) * sizeof(float); }
 
+// Split-K with the sum inside the launch: the slices of an output tile are separate workgroups (grid.y); each parks its float32
+// accumulators in the workspace, and the one that arrives last (a counter per tile) adds all of them in slice order -- the result does
+// not depend on who that is -- and goes on to the ordinary epilogue.  Against a reduction launch behind the GEMM (splitKReduceKernel)
+// this saves that launch and its wait for the whole grid, and the partial sums travel as whole registers: 16 bytes per lane, 1 KiB per
+// wave instruction, no staging through LDS.
+// The slices of a tile may run on different XCDs, whose L2s are not coherent with each other: partial sums are stored and loaded at
+// device scope (sc1: past the L2), a slice's stores are complete (vmcnt) before it counts itself in, and nobody waits for anybody.
+// Bound by the few tiles a small image has: float32 3x3 256 -> 512 at 38x38, one image, 45 -> 38 us;
+// float32 1x1 512 -> 256 there 14 -> 8.4 us; float16 3x3 512 -> 1024 at 13x13 15.9 -> 12.2 us (against the best
+// split with its reduction launch, or the best unsplit tile).
+constexpr size_t kFusedKHead = 64 * 1024;          // counters at the start of the workspace, zero between launches
+constexpr int kCpolAgent = 16;                     // sc1
+
+template <int A, int B>
+__device__ __forceinline__ bool splitKCombine(const IgemmArgs &a, f32x16 (&acc)[A][B], int tileIdx, int nTiles, int wave, int nWaves, int lane, int *flag)
+{
+    constexpr int V = A * B * 4;                   // 16-byte vectors per lane
+    const size_t slot = static_cast<size_t>(nWaves) * V * 1024;
+    unsigned char *part = reinterpret_cast<unsigned char *>(a.ws) + kFusedKHead + static_cast<size_t>(tileIdx) * slot;
+    const size_t step = static_cast<size_t>(nTiles) * slot;        // from a slice to the next one's partial sums of the same tile
+    const int off = wave * V * 1024 + lane * 16;
+    {
+        const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + blockIdx.y * step, static_cast<unsigned>(slot));
+        staticFor<0, V>([&](auto vTag) {
+            constexpr int v = decltype(vTag)::value;
+            constexpr int ij = v / 4, q = v % 4;
+            const f32x16 &c = acc[ij / B][ij % B];
+            const f32x4 d = {c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, d), rs, off + v * 1024, 0, kCpolAgent);
+        });
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (wave == 0 && lane == 0)
+    {
+        int *count = reinterpret_cast<int *>(a.ws) + tileIdx;
+        const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = before == a.splitK - 1;
+        if (last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *flag = last ? 1 : 0;
+    }
+    __syncthreads();
+    if (*flag == 0) return false;
+    for (int s = 0; s < a.splitK; ++s)
+    {
+        const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + s * step, static_cast<unsigned>(slot));
+        staticFor<0, V>([&](auto vTag) {
+            constexpr int v = decltype(vTag)::value;
+            constexpr int ij = v / 4, q = v % 4;
+            const f32x4 d = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + v * 1024, 0, kCpolAgent));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[ij / B][ij % B][q * 4 + e] = s == 0 ? d[e] : acc[ij / B][ij % B][q * 4 + e] + d[e];
+        });
+    }
+    return true;
+}
+
 // ssReady / stageOwn (the K-split epilogue): the affines already stand at ssReady, published by a barrier the caller has passed, and this
 // wavefront stages in stageOwn (32 x (TM + 4) floats of its own) -- then the epilogue meets no workgroup barrier at all.
 template <typename T, typename TOut, int BM, int BN, int TM, int TN>
@@ -434,11 +493,11 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
 // its block (32 pixels x 68 floats) in the region it has just emptied -- the one its partner filled for it, which nobody else touches.
 // LDS: 32 x 68 floats per wavefront + the affines (igemmSwapLds).
 constexpr int kSwapRegion = 32 * (64 + 4);         // floats per wavefront: the staging block of a 64-channel wave tile, which holds the 2048 parked sums
-template <int NW, int BM> constexpr size_t igemmSwapLds() { return (static_cast<size_t>(NW) * kSwapRegion + 2 * BM) * sizeof(float); }
+template <int NW, int BM> constexpr size_t igemmSwapLds() { return (static_cast<size_t>(NW) * kSwapRegion + 2 * BM) * sizeof(float); }       // (fusedK: a flag behind it)
 
 template <typename T, typename TOut, int BM, int BN>
 __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&acc)[2][2], unsigned char *smemRaw, float chScale, float chShift,
-                                                  int m0, int p0, int wm, int wn, int kg, int wt, int wave, int lane, int g, int nWaves)
+                                                  int m0, int p0, int wm, int wn, int kg, int wt, int wave, int lane, int g, int nWaves, int tileIdx = 0, int nTiles = 0)
 {
     float *xch = reinterpret_cast<float *>(smemRaw);
     float *ss  = xch + nWaves * kSwapRegion;
@@ -466,6 +525,7 @@ __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&a
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (a.fusedK > 1 && !splitKCombine(a, mine, tileIdx, nTiles, wave, nWaves, lane, reinterpret_cast<int *>(ss + 2 * BM))) return;
     igemmEpilogue<T, TOut, BM, BN, 64, 32>(a, mine, smemRaw, chScale, chShift, m0, p0, wm, wn * 2 + kg, wave, lane, g, ss, stageOwn);
 }
 
@@ -840,6 +900,30 @@ void convIgemmKernel(IgemmArgs a)
     const int ldRow = tid / KV;
     const int ldVec = (tid % KV) ^ ((ldRow / SWDIV) % KV);   // the logical chunk this thread fetches
 
+    unsigned aOff[AROWS];
+#pragma unroll
+    for (int i = 0; i < AROWS; ++i)
+    {
+        const int m = m0 + ldRow + i * RPP;
+        aOff[i] = (m < a.coutG && ldRow + i * RPP < BM) ? (static_cast<unsigned>(m) * a.taps * a.cinG + ldVec * VEC) * ES : kOobOffset;
+    }
+
+    // split-K: this workgroup multiplies tile steps [itBegin, itBegin + nLocal) of the K loop
+    const int itBegin = a.splitK > 1 ? static_cast<int>(static_cast<long long>(blockIdx.y) * a.nIter / a.splitK) : 0;
+    const int nLocal  = a.splitK > 1 ? static_cast<int>(static_cast<long long>(blockIdx.y + 1) * a.nIter / a.splitK) - itBegin : a.nIter;
+    const unsigned waveLds = ldsBase + wave * 1024;
+    // The filters of the first tile step are asked for before the pixel rows are located: they come from far away (every launch reads
+    // its own), and the address arithmetic below runs while they travel.
+    const int tapFirst = itBegin / a.cChunks, chunkFirst = itBegin - tapFirst * a.cChunks;
+    {
+        const unsigned sA = (static_cast<unsigned>(tapFirst) * a.cinG + chunkFirst * BK) * ES;
+        const bool cut = a.ragged && (chunkFirst * BK + ldVec * VEC >= a.cinG);
+        staticFor<0, AROWS>([&](auto lTag) {
+            constexpr int l = decltype(lTag)::value;
+            dmaLoad16(rw, cut ? kOobOffset : aOff[l], sA, waveLds + l * RPP * ROWB);
+        });
+    }
+
     // Per-thread row state, fixed over the K loop: byte offset of the row's first tap (may be "negative", it wraps
     // back into range once a valid tap offset is added) and one bit per tap telling whether that tap lies inside
     // the image for this output pixel.
@@ -872,14 +956,6 @@ void convIgemmKernel(IgemmArgs a)
             if ((rowBits >> ki) & 1u) mask |= static_cast<unsigned long long>(colBits) << (ki * a.ksize);
         bMask[i] = ok ? mask : 0ull;
     }
-    unsigned aOff[AROWS];
-#pragma unroll
-    for (int i = 0; i < AROWS; ++i)
-    {
-        const int m = m0 + ldRow + i * RPP;
-        aOff[i] = (m < a.coutG && ldRow + i * RPP < BM) ? (static_cast<unsigned>(m) * a.taps * a.cinG + ldVec * VEC) * ES : kOobOffset;
-    }
-
     unsigned bVoff[BROWS];                       // B offsets of the tap being loaded
     auto setTap = [&](int tap) {
         const int ki = tap / a.ksize;
@@ -890,7 +966,6 @@ void convIgemmKernel(IgemmArgs a)
     };
     // Load l of a tile step (A rows first, then B rows) into the LDS stage at byte offset stageOff.  `cut` blanks
     // the lane: past the last channel of a ragged K chunk, or a step past the end of K.
-    const unsigned waveLds = ldsBase + wave * 1024;
     auto issueLoad = [&](auto lTag, unsigned sA, unsigned sB, bool cut, unsigned stageOff) {
         constexpr int l = decltype(lTag)::value;
         if constexpr (l < AROWS)
@@ -961,17 +1036,14 @@ void convIgemmKernel(IgemmArgs a)
     constexpr int AHEAD = NS >= 3 ? NS - 1 : 2;  // the loads issued during step `it` belong to step it + AHEAD
     constexpr int INFLIGHT = NS >= 3 ? (NS - 3) * NL + NPRE : 0;   // loads younger than step it+1's at the barrier
 
-    // split-K: this workgroup multiplies tile steps [itBegin, itBegin + nLocal) of the K loop
-    const int itBegin = a.splitK > 1 ? static_cast<int>(static_cast<long long>(blockIdx.y) * a.nIter / a.splitK) : 0;
-    const int nLocal  = a.splitK > 1 ? static_cast<int>(static_cast<long long>(blockIdx.y + 1) * a.nIter / a.splitK) - itBegin : a.nIter;
     const bool tailPrefetch = TAIL != 0 && a.hasRes && nLocal >= 2;
-    tapNext = itBegin / a.cChunks;
-    chunkNext = itBegin - tapNext * a.cChunks - 1;            // advance() steps onto the first tile step
+    tapNext = tapFirst;
+    chunkNext = chunkFirst - 1;                               // advance() steps onto the first tile step
     setTap(tapNext);
     staticFor<0, AHEAD>([&](auto stTag) {
         constexpr int st = decltype(stTag)::value;
         advance(nLocal <= st);
-        staticFor<0, NL>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, st * STAGE); });
+        staticFor<st == 0 ? AROWS : 0, NL>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, st * STAGE); });     // (step 0: the filters are on their way)
     });
     dmaWait<(AHEAD - 1) * NL>();                 // step 0 has landed
     __syncthreads();
@@ -1032,7 +1104,9 @@ void convIgemmKernel(IgemmArgs a)
         igemmTailEpilogue<BM, BN, WM, WN, STAGE>(a, acc, smemRaw, ldsBase, chScale, chShift, sc2, sh2, p0, wm, wn, wave, lane, tailPrefetch, tailPrefetch ? (nLocal & 1) : 0);
         return;
     }
-    if (a.splitK > 1)
+    const int nTilesP = (a.P + BN - 1) / BN;
+    const int nTiles = a.mTiles * nTilesP * static_cast<int>(gridDim.z), tileIdx = (g * nTilesP + pTile) * a.mTiles + mTile;
+    if (a.splitK > 1 && a.fusedK <= 1)
     {
         // raw float32 partial sums of this K slice; affine, activation and residual follow in the reduction pass
         IgemmArgs e = a;
@@ -1044,7 +1118,8 @@ void convIgemmKernel(IgemmArgs a)
         else igemmEpilogue<T, float, BM, BN, TM, TN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wm, wn, wave, lane, g);
         return;
     }
-    if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64);
+    if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles);
+    else if (a.fusedK > 1 && !splitKCombine(a, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + igemmEpilogueLds<BM, TM, NT / 64>()))) return;
     else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g);
 }
 
@@ -1113,6 +1188,7 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         smemEpi = TailLds<BM, BN, STAGE>::bytes();
     }
     else smemEpi = std::max(igemmEpilogueLds<BM, BM / WM, WM * WN * KG>(), KG == 2 ? igemmSwapLds<WM * WN * KG, BM>() : size_t(0));
+    if (a.fusedK > 1) smemEpi += 16;                  // the flag of splitKCombine
     const size_t smem = smemLoop > smemEpi ? smemLoop : smemEpi;
     a.mTiles = (a.coutG + BM - 1) / BM;
     const int tiles = a.mTiles * ((a.P + BN - 1) / BN);
@@ -1130,6 +1206,23 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         }
         a.splitK = want;
     }
+    if (a.fusedK > 1)
+    {
+        // A slice has at least two tile steps; more workgroups than the chip holds at once buy nothing.
+        const long long wgs = static_cast<long long>(tiles) * groups * a.fusedK;
+        a.wsNeed = kFusedKHead + static_cast<size_t>(wgs) * BM * BN * sizeof(float);
+        if (TAIL != 0 || a.nIter < 2 * a.fusedK || tiles * groups > static_cast<int>(kFusedKHead / sizeof(int)) || wgs > 2048)
+        {
+            setError("conv2d: that many slices do not apply to this shape and tile");
+            return 3;
+        }
+        if (!a.dryRun && (a.ws == nullptr || a.wsBytes < a.wsNeed))
+        {
+            setError("conv2d: the sliced implicit GEMM needs a workspace of msnh_hip_conv2d_workspace_bytes() bytes");
+            return 2;
+        }
+        a.splitK = a.fusedK;
+    }
     dim3 grid(igemmGridX(a, (a.P + BN - 1) / BN, sizeof(T), a.splitK == 1 && groups == 1), a.splitK, groups);
     if (a.dryRun) return 0;
     auto kern = convIgemmKernel<T, TOut, BM, BN, KV, WM, WN, NS, KG, TAIL>;
@@ -1141,7 +1234,7 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
     }
     hipLaunchKernelGGL(kern, grid, dim3(64 * WM * WN * KG), smem, st, a);
     MSNH_LAUNCH_CHECK();
-    if (a.splitK > 1)
+    if (a.splitK > 1 && a.fusedK <= 1)
     {
         const int outC = a.coutG * groups;
         const long long total = static_cast<long long>(a.P) * (outC / 4);
@@ -1161,117 +1254,132 @@ namespace msnh {
 // Tile configurations (BM x BN output tile, KV 16-byte vectors of K per step, WM x WN wavefront grid).
 // Index 0 is "choose for me"; the others can be forced through msnh_conv_desc::tile, which is how the host
 // library's per-layer search picks the fastest one at load time.
-constexpr int kIgemmTiles = 65;
-constexpr int kIgemmTailTileFirst = 64;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
+constexpr int kIgemmTiles = 68;
+constexpr int kIgemmTailTileFirst = 67;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
 
-template <typename T, typename TOut>
+// One translation unit instantiates every third configuration of one type pair (tile % kIgemmParts == PART), so that they compile in parallel.
+constexpr int kIgemmParts = 3;
+
+template <typename T, typename TOut, int PART>
 int igemmDispatch(IgemmArgs &a, int groups, int tile, hipStream_t st)
 {
     switch (tile)
     {
-    case 1:  return launchIgemm<T, TOut, 128, 128, 8, 2, 2>(a, groups, st);
-    case 2:  return launchIgemm<T, TOut, 128, 128, 4, 2, 2>(a, groups, st);
-    case 3:  return launchIgemm<T, TOut, 64, 256, 8, 1, 4>(a, groups, st);
-    case 4:  return launchIgemm<T, TOut, 64, 256, 4, 1, 4>(a, groups, st);
-    case 5:  return launchIgemm<T, TOut, 32, 256, 8, 1, 4>(a, groups, st);
-    case 6:  return launchIgemm<T, TOut, 64, 64, 4, 2, 2>(a, groups, st);
-    case 7:  return launchIgemm<T, TOut, 256, 128, 4, 2, 2>(a, groups, st);
-    case 8:  return launchIgemm<T, TOut, 128, 64, 8, 2, 2>(a, groups, st);
-    case 9:  return launchIgemm<T, TOut, 128, 64, 4, 2, 2>(a, groups, st);
-    case 10: return launchIgemm<T, TOut, 64, 128, 8, 1, 4>(a, groups, st);
-    case 11: return launchIgemm<T, TOut, 64, 128, 4, 1, 4>(a, groups, st);
-    case 12: return launchIgemm<T, TOut, 64, 64, 8, 2, 2>(a, groups, st);
-    case 13: return launchIgemm<T, TOut, 128, 256, 4, 2, 2>(a, groups, st);
+    case 1:  if constexpr (1 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2>(a, groups, st); else break;
+    case 2:  if constexpr (2 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 4, 2, 2>(a, groups, st); else break;
+    case 3:  if constexpr (3 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 8, 1, 4>(a, groups, st); else break;
+    case 4:  if constexpr (4 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 4, 1, 4>(a, groups, st); else break;
+    case 5:  if constexpr (5 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 256, 8, 1, 4>(a, groups, st); else break;
+    case 6:  if constexpr (6 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 4, 2, 2>(a, groups, st); else break;
+    case 7:  if constexpr (7 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 4, 2, 2>(a, groups, st); else break;
+    case 8:  if constexpr (8 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 2, 2>(a, groups, st); else break;
+    case 9:  if constexpr (9 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 4, 2, 2>(a, groups, st); else break;
+    case 10: if constexpr (10 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 1, 4>(a, groups, st); else break;
+    case 11: if constexpr (11 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 4, 1, 4>(a, groups, st); else break;
+    case 12: if constexpr (12 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 8, 2, 2>(a, groups, st); else break;
+    case 13: if constexpr (13 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 256, 4, 2, 2>(a, groups, st); else break;
     // 3x3 stride-1 pad-1 only: input patch resident in LDS, weights streamed per tap (last number: patch slices
     // per wave and step, 2 for wide images)
-    case 14: return launchPatch<T, TOut, 128, 256, 4, 2, 2, 1>(a, groups, st);
-    case 15: return launchPatch<T, TOut, 128, 256, 4, 2, 2, 2>(a, groups, st);
-    case 16: return launchPatch<T, TOut, 128, 128, 4, 2, 2, 1>(a, groups, st);
-    case 17: return launchPatch<T, TOut, 256, 128, 4, 2, 2, 1>(a, groups, st);
-    case 18: return launchPatch<T, TOut, 64, 256, 4, 1, 4, 1>(a, groups, st);
-    case 19: return launchPatch<T, TOut, 128, 128, 4, 2, 2, 2>(a, groups, st);
+    case 14: if constexpr (14 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 256, 4, 2, 2, 1>(a, groups, st); else break;
+    case 15: if constexpr (15 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 256, 4, 2, 2, 2>(a, groups, st); else break;
+    case 16: if constexpr (16 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 128, 4, 2, 2, 1>(a, groups, st); else break;
+    case 17: if constexpr (17 % kIgemmParts == PART) return launchPatch<T, TOut, 256, 128, 4, 2, 2, 1>(a, groups, st); else break;
+    case 18: if constexpr (18 % kIgemmParts == PART) return launchPatch<T, TOut, 64, 256, 4, 1, 4, 1>(a, groups, st); else break;
+    case 19: if constexpr (19 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 128, 4, 2, 2, 2>(a, groups, st); else break;
     // two LDS stages, 128-byte rows
-    case 20: return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 2>(a, groups, st);
-    case 21: return launchIgemm<T, TOut, 256, 128, 8, 2, 2, 2>(a, groups, st);
-    case 22: return launchIgemm<T, TOut, 128, 256, 8, 2, 2, 2>(a, groups, st);
-    case 23: return launchIgemm<T, TOut, 128, 64, 8, 2, 2, 2>(a, groups, st);
-    case 24: return launchIgemm<T, TOut, 64, 128, 8, 1, 4, 2>(a, groups, st);
+    case 20: if constexpr (20 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 2>(a, groups, st); else break;
+    case 21: if constexpr (21 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 8, 2, 2, 2>(a, groups, st); else break;
+    case 22: if constexpr (22 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 256, 8, 2, 2, 2>(a, groups, st); else break;
+    case 23: if constexpr (23 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 2, 2, 2>(a, groups, st); else break;
+    case 24: if constexpr (24 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 1, 4, 2>(a, groups, st); else break;
     // deeper prefetch
-    case 25: return launchIgemm<T, TOut, 128, 128, 4, 2, 2, 4>(a, groups, st);
-    case 26: return launchIgemm<T, TOut, 256, 128, 4, 2, 2, 6>(a, groups, st);
-    case 27: return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 4>(a, groups, st);
-    case 28: return launchIgemm<T, TOut, 128, 128, 4, 2, 2, 5>(a, groups, st);
+    case 25: if constexpr (25 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 4, 2, 2, 4>(a, groups, st); else break;
+    case 26: if constexpr (26 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 4, 2, 2, 6>(a, groups, st); else break;
+    case 27: if constexpr (27 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 4>(a, groups, st); else break;
+    case 28: if constexpr (28 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 4, 2, 2, 5>(a, groups, st); else break;
     // small tiles at high occupancy for bandwidth-bound short-K layers
-    case 29: return launchIgemm<T, TOut, 64, 128, 4, 1, 4, 2>(a, groups, st);
-    case 30: return launchIgemm<T, TOut, 64, 64, 4, 2, 2, 2>(a, groups, st);
-    case 31: return launchIgemm<T, TOut, 128, 64, 4, 2, 2, 2>(a, groups, st);
+    case 29: if constexpr (29 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 4, 1, 4, 2>(a, groups, st); else break;
+    case 30: if constexpr (30 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 4, 2, 2, 2>(a, groups, st); else break;
+    case 31: if constexpr (31 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 4, 2, 2, 2>(a, groups, st); else break;
     // eight wavefronts (512 threads, two per SIMD): a second wave per SIMD covers the first one's barrier and LDS waits where
     // the launch has at most one workgroup per CU; pixel tiles of 192 and 96 bring the tile count of the 76x76 and 38x38
     // layers at batch 8 just under the CU count (241 and 242 tiles instead of 361 and 182)
-    case 32: return launchIgemm<T, TOut, 256, 128, 8, 4, 2, 3>(a, groups, st);
-    case 33: return launchIgemm<T, TOut, 128, 128, 8, 2, 4, 4>(a, groups, st);
-    case 34: return launchIgemm<T, TOut, 256, 192, 8, 4, 2, 2>(a, groups, st);
-    case 35: return launchIgemm<T, TOut, 256, 192, 4, 4, 2, 4>(a, groups, st);
-    case 36: return launchIgemm<T, TOut, 256, 96, 8, 8, 1, 3>(a, groups, st);
+    case 32: if constexpr (32 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 8, 4, 2, 3>(a, groups, st); else break;
+    case 33: if constexpr (33 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 4, 4>(a, groups, st); else break;
+    case 34: if constexpr (34 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 192, 8, 4, 2, 2>(a, groups, st); else break;
+    case 35: if constexpr (35 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 192, 4, 4, 2, 4>(a, groups, st); else break;
+    case 36: if constexpr (36 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 96, 8, 8, 1, 3>(a, groups, st); else break;
     // twelve wavefronts (768 threads, three per SIMD) over 192-pixel tiles: 64 x 64 and 32 x 64 wave tiles
-    case 37: return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2>(a, groups, st);
-    case 38: return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 3>(a, groups, st);
+    case 37: if constexpr (37 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2>(a, groups, st); else break;
+    case 38: if constexpr (38 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 3>(a, groups, st); else break;
     // the LDS-patch kernel with eight wavefronts
-    case 39: return launchPatch<T, TOut, 128, 384, 4, 2, 4, 1>(a, groups, st);
-    case 40: return launchIgemm<T, TOut, 128, 128, 8, 2, 4, 3>(a, groups, st);
+    case 39: if constexpr (39 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 384, 4, 2, 4, 1>(a, groups, st); else break;
+    case 40: if constexpr (40 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 4, 3>(a, groups, st); else break;
     // 64 channels x 256 pixels with eight wavefronts side by side, for the first layers of the detectors (32 -> 64 channels)
-    case 41: return launchIgemm<T, TOut, 64, 256, 4, 1, 8, 3>(a, groups, st);
+    case 41: if constexpr (41 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 4, 1, 8, 3>(a, groups, st); else break;
     // 128 channels x 384 pixels with twelve wavefronts: one round of tiles for 128-filter layers over many pixels
-    case 42: return launchIgemm<T, TOut, 128, 384, 8, 2, 6, 2>(a, groups, st);
+    case 42: if constexpr (42 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 384, 8, 2, 6, 2>(a, groups, st); else break;
     // 3x3 stride-1 pad-1 only: input patch resident in LDS with 128-byte rows (last three numbers: wavefront grid rows x columns,
     // weight stages, patch slices per wavefront and tap step)
-    case 43: return launchPatch8<T, TOut, 128, 192, 4, 3, 3, 1>(a, groups, st);
-    case 44: return launchPatch8<T, TOut, 128, 192, 4, 2, 4, 1>(a, groups, st);
-    case 45: return launchPatch8<T, TOut, 128, 192, 2, 2, 4, 2>(a, groups, st);
-    case 46: return launchPatch8<T, TOut, 64, 384, 2, 6, 3, 1>(a, groups, st);
-    case 47: return launchPatch8<T, TOut, 64, 384, 2, 4, 4, 2>(a, groups, st);
-    case 48: return launchPatch8<T, TOut, 64, 256, 2, 4, 4, 1>(a, groups, st);
-    case 49: return launchPatch8<T, TOut, 128, 256, 4, 2, 3, 1>(a, groups, st);
-    case 50: return launchPatch8<T, TOut, 64, 192, 2, 2, 4, 2>(a, groups, st);
-    case 51: return launchPatch8<T, TOut, 128, 384, 2, 4, 3, 2>(a, groups, st);
+    case 43: if constexpr (43 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 4, 3, 3, 1>(a, groups, st); else break;
+    case 44: if constexpr (44 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 4, 2, 4, 1>(a, groups, st); else break;
+    case 45: if constexpr (45 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 2, 2, 4, 2>(a, groups, st); else break;
+    case 46: if constexpr (46 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 2, 6, 3, 1>(a, groups, st); else break;
+    case 47: if constexpr (47 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 2, 4, 4, 2>(a, groups, st); else break;
+    case 48: if constexpr (48 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 256, 2, 4, 4, 1>(a, groups, st); else break;
+    case 49: if constexpr (49 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 256, 4, 2, 3, 1>(a, groups, st); else break;
+    case 50: if constexpr (50 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 192, 2, 2, 4, 2>(a, groups, st); else break;
+    case 51: if constexpr (51 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 384, 2, 4, 3, 2>(a, groups, st); else break;
     // the same with the k-blocks of a tap step split between two groups of wavefronts over 64 x 64 wave tiles (the numbers are
     // the grid of wave tiles; twice as many wavefronts run)
-    case 52: return launchPatch8<T, TOut, 64, 384, 1, 6, 3, 1, 0, 2>(a, groups, st);
-    case 53: return launchPatch8<T, TOut, 128, 192, 2, 3, 3, 1, 0, 2>(a, groups, st);
-    case 54: return launchPatch8<T, TOut, 64, 256, 1, 4, 4, 1, 0, 2>(a, groups, st);
-    case 55: return launchPatch8<T, TOut, 128, 128, 2, 2, 4, 1, 0, 2>(a, groups, st);
-    case 56: return launchPatch8<T, TOut, 64, 384, 1, 6, 4, 1, 0, 2>(a, groups, st);
+    case 52: if constexpr (52 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 1, 6, 3, 1, 0, 2>(a, groups, st); else break;
+    case 53: if constexpr (53 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 2, 3, 3, 1, 0, 2>(a, groups, st); else break;
+    case 54: if constexpr (54 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 256, 1, 4, 4, 1, 0, 2>(a, groups, st); else break;
+    case 55: if constexpr (55 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 128, 2, 2, 4, 1, 0, 2>(a, groups, st); else break;
+    case 56: if constexpr (56 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 1, 6, 4, 1, 0, 2>(a, groups, st); else break;
     // the generic kernel with the same split (numbers: tile, 16-byte vectors of K per step, grid of 64 x 64 wave tiles, LDS stages)
-    case 57: return launchIgemm<T, TOut, 128, 192, 8, 2, 3, 3, 2>(a, groups, st);
-    case 58: return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 4, 2>(a, groups, st);
-    case 59: return launchIgemm<T, TOut, 64, 128, 8, 1, 2, 4, 2>(a, groups, st);
-    case 60: return launchIgemm<T, TOut, 128, 64, 8, 2, 1, 4, 2>(a, groups, st);
-    case 61: return launchIgemm<T, TOut, 64, 256, 8, 1, 4, 3, 2>(a, groups, st);
-    case 62: return launchIgemm<T, TOut, 64, 384, 8, 1, 6, 2, 2>(a, groups, st);
+    case 57: if constexpr (57 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 192, 8, 2, 3, 3, 2>(a, groups, st); else break;
+    case 58: if constexpr (58 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 4, 2>(a, groups, st); else break;
+    case 59: if constexpr (59 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 1, 2, 4, 2>(a, groups, st); else break;
+    case 60: if constexpr (60 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 2, 1, 4, 2>(a, groups, st); else break;
+    case 61: if constexpr (61 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 8, 1, 4, 3, 2>(a, groups, st); else break;
+    case 62: if constexpr (62 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 384, 8, 1, 6, 2, 2>(a, groups, st); else break;
     // the LDS-patch kernel over 256 channels x 192 pixels with twelve wavefronts: one round of tiles for the 76x76 128 -> 256 layers at batch 8
     // like tile 37, with a third fewer bytes delivered to LDS per tap step.  It fits the LDS with two weight stages only, the weight
     // tile of step it + 2 asked for behind the barrier of step it (see LATE in conv_patch8.hpp)
-    case 63: return launchPatch8<T, TOut, 256, 192, 4, 3, 2, 1>(a, groups, st);
+    case 63: if constexpr (63 % kIgemmParts == PART) return launchPatch8<T, TOut, 256, 192, 4, 3, 2, 1>(a, groups, st); else break;
+    // small images (one to a few pictures): 64 x 64 with 256-byte rows, half the barriers per K; 64 x 128 and 128 x 64 with eight wavefronts
+    // over 32 x 32 wave tiles, two per SIMD where the launch has at most one workgroup per CU
+    case 64: if constexpr (64 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 16, 2, 2, 3>(a, groups, st); else break;
+    case 65: if constexpr (65 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 2, 4, 4>(a, groups, st); else break;
+    case 66: if constexpr (66 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 4, 2, 4>(a, groups, st); else break;
     // tiles whose epilogue also computes the 1x1 convolution that follows (msnh_hip_conv2d_tail only; float16): the tile holds every
     // output channel of the first convolution (at most 256 / 128)
-    case 64:
-    case 65:
-        if constexpr (std::is_same<T, f16>::value && std::is_same<TOut, f16>::value)
-        {
-            if (tile == 64) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
-            return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
-        }
-        else
+    case 67:
+    case 68:
+        if constexpr (!(std::is_same<T, f16>::value && std::is_same<TOut, f16>::value))
         {
             setError("conv2d: this tile needs float16 tensors and a 1x1 convolution behind it (msnh_hip_conv2d_tail)");
             return 3;
         }
+        else if constexpr (67 % kIgemmParts == PART)
+        {
+            if (tile == 67) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
+            break;
+        }
+        else if constexpr (68 % kIgemmParts == PART)
+        {
+            if (tile == 68) return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
+            break;
+        }
+        else break;
     default: break;
     }
     setError("igemm: unknown tile %d", tile);
     return 2;
 }
 
+// (each picks its part: conv_igemm.hip)
 int igemmF16F16(IgemmArgs &a, int groups, int tile, hipStream_t st);
 int igemmF16F32(IgemmArgs &a, int groups, int tile, hipStream_t st);
 int igemmF32F32(IgemmArgs &a, int groups, int tile, hipStream_t st);

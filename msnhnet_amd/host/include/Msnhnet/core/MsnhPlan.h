@@ -180,6 +180,8 @@ private:
     void launch(PlanOp &op, msnh_stream_t s);
     void applyTails();                      // after the search: the 1x1 ops computed by their producer's launch become dead, the others alive
     DeviceBuffer _arena, _exportScratch, _convWorkspace;
+    DeviceBuffer _sliceWorkspace;           // MSNH_CONV_IGEMM_FUSEDK: zeroed when allocated, its counters are zero between launches
+    void reserveSliceWorkspace(size_t bytes, msnh_stream_t s);
     bool _tailWriteAll = false;             // runs that look at every tensor (calibration, float16 headroom): tailSkipY is ignored
 };
 }

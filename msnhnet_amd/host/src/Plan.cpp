@@ -996,8 +996,8 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
             const size_t bar = ok ? line.find(" | ") : std::string::npos;
             ok = ok && bar != std::string::npos && line.substr(0, bar) == tuneSignature(*this, ops[tunedOps[k]]);
             int algo = 0, tile = 0;
-            ok = ok && std::sscanf(line.c_str() + bar + 3, "%d %d", &algo, &tile) == 2 && tile >= 0 && tile <= nTiles &&
-                 (algo == MSNH_CONV_IGEMM || algo == MSNH_CONV_WINOGRAD || algo == MSNH_CONV_IGEMM_SPLITK || algo == MSNH_CONV_POINTWISE ||
+            ok = ok && std::sscanf(line.c_str() + bar + 3, "%d %d", &algo, &tile) == 2 && tile >= 0 && (tile <= nTiles || algo == MSNH_CONV_IGEMM_FUSEDK) &&
+                 (algo == MSNH_CONV_IGEMM || algo == MSNH_CONV_WINOGRAD || algo == MSNH_CONV_IGEMM_FUSEDK || algo == MSNH_CONV_POINTWISE ||
                   (algo == MSNH_CONV_IGEMM_TAIL && ops[tunedOps[k]].tail >= 0));
             if (ok) picks.emplace_back(algo, tile);
         }
@@ -1005,7 +1005,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         {
             // the library must still accept every recorded choice; otherwise the defaults come back and the search runs
             std::vector<std::pair<int, int>> before;
-            size_t need = 0;
+            size_t need = 0, needSliced = 0;
             for (size_t k = 0; k < tunedOps.size(); ++k)
             {
                 PlanOp &op = ops[tunedOps[k]];
@@ -1026,11 +1026,13 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
                 }
                 if (!msnh_hip_conv2d_tile_supported(&d, op.tile)) ok = false;
                 if (op.kind == PlanOp::CONV && op.wDev.bytes() != msnh_hip_conv2d_packed_weight_elems(&d, op.algo) * (d.dtype == MSNH_F16 ? 2u : 4u)) ok = false;
-                need = std::max(need, msnh_hip_conv2d_workspace_bytes(&d, op.algo));
+                size_t &most = op.algo == MSNH_CONV_IGEMM_FUSEDK ? needSliced : need;
+                most = std::max(most, msnh_hip_conv2d_workspace_bytes(&d, op.algo));
             }
             if (ok)
             {
                 if (need > _convWorkspace.bytes()) _convWorkspace.alloc(need);
+                reserveSliceWorkspace(needSliced, s);
                 applyTails();
                 return true;
             }
@@ -1095,9 +1097,11 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
             if (!(m.first == key)) continue;
             // same launch as one searched before: take its result, if the library accepts it for this op as well
             const int wasAlgo = op.algo, wasTile = op.tile;
-            op.algo = m.second / 1000; op.tile = m.second % 1000;
+            op.algo = m.second >> 16; op.tile = m.second & 0xffff;
             const msnh_conv_desc d = convDesc(*this, op);
-            if (msnh_hip_conv2d_tile_supported(&d, op.tile) && msnh_hip_conv2d_workspace_bytes(&d, op.algo) <= _convWorkspace.bytes()) found = true;
+            if (msnh_hip_conv2d_tile_supported(&d, op.tile) &&
+                msnh_hip_conv2d_workspace_bytes(&d, op.algo) <= (op.algo == MSNH_CONV_IGEMM_FUSEDK ? _sliceWorkspace : _convWorkspace).bytes())
+                found = true;
             else { op.algo = wasAlgo; op.tile = wasTile; }
             break;
         }
@@ -1132,19 +1136,27 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         };
         const int baseAlgo = op.algo;
         search(baseAlgo);
-        if (baseAlgo == MSNH_CONV_IGEMM)
+        // Layers whose output tiles do not fill the chip or fill it unevenly: the K loop cut into slices, summed inside the launch.  Tried on
+        // the tiles that came out best uncut and on the small ones, which win most of these layers; the library refuses what cannot help.
+        if (baseAlgo == MSNH_CONV_IGEMM && !op.up2)
         {
-            // layers with few output tiles: the K loop cut over several workgroups, if its workspace is modest
-            op.tile = 0;
-            op.algo = baseAlgo;
-            const msnh_conv_desc d = convDesc(*this, op);
-            const size_t need = msnh_hip_conv2d_workspace_bytes(&d, MSNH_CONV_IGEMM_SPLITK);
-            if (out.c % 4 == 0 && need <= (static_cast<size_t>(256) << 20))
-            {
-                MSNH_DEV(msnh_hip_stream_sync(s));
-                if (need > _convWorkspace.bytes()) _convWorkspace.alloc(need);
-                search(MSNH_CONV_IGEMM_SPLITK);
-            }
+            std::vector<int> tiles = {6, 12, 30, 64, 65, 66};
+            std::vector<Cand> plain = cands;
+            std::sort(plain.begin(), plain.end(), [](const Cand &x, const Cand &y) { return x.ms < y.ms; });
+            for (size_t i = 0; i < plain.size() && i < 6; ++i)
+                if (plain[i].tile > 0 && std::find(tiles.begin(), tiles.end(), plain[i].tile) == tiles.end()) tiles.push_back(plain[i].tile);
+            op.algo = MSNH_CONV_IGEMM_FUSEDK;
+            for (int tile : tiles)
+                for (int slices : {2, 3, 4, 5, 6, 8, 10, 12, 16})
+                {
+                    op.tile = tile + 256 * slices;
+                    const msnh_conv_desc probe = convDesc(*this, op);
+                    if (!msnh_hip_conv2d_tile_supported(&probe, op.tile)) continue;
+                    const size_t need = msnh_hip_conv2d_workspace_bytes(&probe, MSNH_CONV_IGEMM_FUSEDK);
+                    if (need == 0 || need > (static_cast<size_t>(64) << 20)) continue;
+                    reserveSliceWorkspace(need, s);
+                    cands.push_back({timeOne(MSNH_CONV_IGEMM_FUSEDK, tile + 256 * slices, 1, 3), MSNH_CONV_IGEMM_FUSEDK, tile + 256 * slices});
+                }
         }
         if (baseAlgo == MSNH_CONV_IGEMM && op.kind == PlanOp::CONV) search(MSNH_CONV_POINTWISE);      // (refused by the library unless the shape fits)
         int best = 0, bestAlgo = baseAlgo;
@@ -1161,7 +1173,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         }
         op.algo = bestAlgo;
         op.tile = best;
-        memo.emplace_back(key, bestAlgo * 1000 + best);
+        memo.emplace_back(key, (bestAlgo << 16) | best);
     }
     // Pairs marked by fuse (e): the two launches as chosen above, back to back, against one launch on every tile that carries a tail.
     {
@@ -1169,11 +1181,11 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         std::vector<PairKey> pairMemo;              // identical pairs share one comparison; tile 0 = two launches
         for (PlanOp &a : ops)
         {
-            if (a.dead || a.tail < 0 || a.kind != PlanOp::CONV || a.algo != MSNH_CONV_IGEMM) continue;
+            if (a.dead || a.tail < 0 || a.kind != PlanOp::CONV || (a.algo != MSNH_CONV_IGEMM && a.algo != MSNH_CONV_IGEMM_FUSEDK)) continue;
             PlanOp &b = ops[static_cast<size_t>(a.tail)];
-            if (b.dead || (b.algo != MSNH_CONV_IGEMM && b.algo != MSNH_CONV_POINTWISE)) continue;
+            if (b.dead || (b.algo != MSNH_CONV_IGEMM && b.algo != MSNH_CONV_IGEMM_FUSEDK && b.algo != MSNH_CONV_POINTWISE)) continue;
             const std::string ka = tuneSignature(*this, a), kb = tuneSignature(*this, b);
-            const int twoTile = a.tile;
+            const int twoAlgo = a.algo, twoTile = a.tile;
             bool found = false;
             for (const PairKey &m : pairMemo)
                 if (m.a == ka && m.b == kb)
@@ -1208,7 +1220,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
                 if (ms < bestMs || (forceTail && bestTile == 0)) { bestMs = ms; bestTile = tile; }
             }
             if (bestTile > 0) { a.algo = MSNH_CONV_IGEMM_TAIL; a.tile = bestTile; }
-            else { a.algo = MSNH_CONV_IGEMM; a.tile = twoTile; }
+            else { a.algo = twoAlgo; a.tile = twoTile; }
             pairMemo.push_back({ka, kb, bestTile});
         }
     }
@@ -1314,8 +1326,9 @@ void Plan::launch(PlanOp &op, msnh_stream_t s)
         const msnh_conv_desc d = convDesc(*this, op);
         if (op.wDev.bytes() != msnh_hip_conv2d_packed_weight_elems(&d, op.algo) * (d.dtype == MSNH_F16 ? 2u : 4u))
             MSNH_THROW("conv weights on the device are not packed for the algorithm of this launch (" + op.name + ")");
+        const DeviceBuffer &ws = op.algo == MSNH_CONV_IGEMM_FUSEDK ? _sliceWorkspace : _convWorkspace;
         MSNH_DEV(msnh_hip_conv2d(&d, ptr(op.in0), op.wDev.ptr(), op.scaleDev.as<float>(), op.shiftDev.as<float>(),
-                                 op.in1 >= 0 ? ptr(op.in1) : nullptr, ptr(op.out), _convWorkspace.ptr(), _convWorkspace.bytes(), s));
+                                 op.in1 >= 0 ? ptr(op.in1) : nullptr, ptr(op.out), ws.ptr(), ws.bytes(), s));
         break;
     }
     case PlanOp::AFFINE:
@@ -1381,11 +1394,11 @@ void Plan::launch(PlanOp &op, msnh_stream_t s)
                                             mulOf(op.in0) / mulOf(op.out), ptr(op.out), ld(op.out), s));
         break;
     case PlanOp::CONNECTED:
-        if (op.algo == MSNH_CONV_IGEMM || op.algo == MSNH_CONV_IGEMM_SPLITK)
+        if (op.algo == MSNH_CONV_IGEMM || op.algo == MSNH_CONV_IGEMM_FUSEDK)
         {
             const msnh_conv_desc d = convDesc(*this, op);
             MSNH_DEV(msnh_hip_conv2d(&d, ptr(op.in0), op.wDev.ptr(), nullptr, op.shiftDev.as<float>(), nullptr, ptr(op.out),
-                                     _convWorkspace.ptr(), _convWorkspace.bytes(), s));
+                                     _sliceWorkspace.ptr(), _sliceWorkspace.bytes(), s));
             break;
         }
         if (ld(op.in0) != in.c && in.n > 1 && in.h * in.w == 1) MSNH_THROW("connected input must be densely packed");
@@ -1466,6 +1479,14 @@ void Plan::run(size_t opBegin, size_t opEnd, msnh_stream_t s)
         if (!ops[i].dead) launch(ops[i], s);
 }
 
+void Plan::reserveSliceWorkspace(size_t bytes, msnh_stream_t s)
+{
+    if (bytes <= _sliceWorkspace.bytes()) return;
+    MSNH_DEV(msnh_hip_stream_sync(s));
+    _sliceWorkspace.alloc(bytes);
+    MSNH_DEV(msnh_hip_fill_zero(_sliceWorkspace.ptr(), static_cast<size_t>(64) << 10, s));
+}
+
 void Plan::clearCandidates(msnh_stream_t s)
 {
     const DeviceBuffer &cnt = yoloCandCnt[yoloSlot];
@@ -1492,7 +1513,7 @@ void Plan::exportTensor(int t, std::vector<float> &dst, msnh_stream_t s)
 std::string Plan::describe() const
 {
     static const char *kinds[] = {"conv", "affine", "add", "copy", "maxpool", "avgpool", "upsample", "connected", "input_cast", "yolo_decode", "pad", "slice", "bilinear", "softmax", "col2im"};
-    static const char *algos[] = {"auto", "direct", "igemm", "depthwise", "winograd", "stem", "igemm_splitk", "pointwise", "stem+down", "winograd_fused", "mbconv", "igemm+1x1"};
+    static const char *algos[] = {"auto", "direct", "igemm", "depthwise", "winograd", "stem", "igemm_splitk", "pointwise", "stem+down", "winograd_fused", "mbconv", "igemm+1x1", "igemm_fusedk"};
     std::ostringstream os;
     os << "plan: " << liveOps() << " launches, " << tensors.size() << " tensors, arena " << _arena.bytes() / (1024.0 * 1024.0) << " MiB, dtype "
        << (computeDtype == MSNH_F16 ? "f16" : "f32") << "\n";

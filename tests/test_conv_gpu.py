@@ -389,6 +389,59 @@ def test_conv_split_k(case, dtype):
     assert tried >= 3
 
 
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F16])
+@pytest.mark.parametrize("case", SPLITK_CASES)
+def test_conv_fused_k(case, dtype):
+    """K slices summed inside the launch: oracle result for tiles of every wavefront grid (with and without the k-block split) and slice
+    counts up to one or two steps per slice, bit-identical when the same workspace serves launch after launch, counters left zero"""
+    import ctypes
+    import torch
+    import gpuutil as gu
+    b, c, h, w, oc, k, stride, pad, groups = case
+    rng = np.random.default_rng(sum(case) + 1)
+    x, wt = _case(rng, b, c, h, w, oc, k, groups)
+    oh = (h + 2 * pad - k) // stride + 1
+    ow = (w + 2 * pad - k) // stride + 1
+    res = rng.standard_normal((b, oc, oh, ow), dtype=np.float32)
+    scale = rng.uniform(0.5, 1.5, oc).astype(np.float32)
+    shift = (rng.standard_normal(oc) * 0.1).astype(np.float32)
+    if dtype == abi.F16:
+        x, wt, res = gu.round_f16(x), gu.round_f16(wt), gu.round_f16(res)
+    ref = _ref(x, wt, stride, pad, 1, groups, scale, shift, "leaky", 0.1, res, "relu", 2.0, 0.5)
+    L = abi.lib()
+    algo = abi.ALGO["igemm_fusedk"]
+    d = abi.ConvDesc(dtype, dtype, b, h, w, c, c, oc, oh, ow, oc + 8, k, stride, pad, 1, groups, abi.ACT["leaky"], 0.1, 1, oc + 8, abi.ACT["relu"], 0.1, 2.0, 0.5, algo, 0)
+    packed = np.zeros(L.msnh_hip_conv2d_packed_weight_elems(ctypes.byref(d), algo), np.float32 if dtype == abi.F32 else np.float16)
+    wf = np.ascontiguousarray(wt, np.float32)
+    abi.check(L.msnh_hip_conv2d_pack_weights(ctypes.byref(d), algo, wf.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), packed.ctypes.data_as(ctypes.c_void_p)))
+    xd, wd, rd, sd, hd = gu.nhwc_dev(x, dtype), gu.dev(packed), gu.nhwc_dev(res, dtype, oc + 8), gu.dev(scale), gu.dev(shift)
+    assert L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), 12) == 0          # a tile without slices is not this algorithm
+    ws = torch.zeros(64 << 20, dtype=torch.uint8).cuda()
+    tried = 0
+    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66):
+        for slices in (2, 3, 7, 16):
+            d.tile = tile + 256 * slices
+            need = L.msnh_hip_conv2d_workspace_bytes(ctypes.byref(d), algo)
+            if not L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), d.tile):
+                assert need == 0
+                continue
+            if need > ws.numel():
+                continue
+            got = []
+            for rep in range(3):
+                y = torch.full((b, oh, ow, oc + 8), 3.0, dtype=gu.TORCH_DT[dtype]).cuda()
+                gu.sync()
+                abi.check(L.msnh_hip_conv2d(ctypes.byref(d), gu.ptr(xd), gu.ptr(wd), gu.ptr(sd), gu.ptr(hd), gu.ptr(rd), gu.ptr(y), gu.ptr(ws), need, None))
+                gu.sync()
+                assert (y[..., oc:] == 3.0).all()
+                got.append(gu.nchw_host(y, oc))
+            assert gu.rel_err(got[0], ref) <= TOL[dtype], (tile, slices, gu.rel_err(got[0], ref))
+            assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2]), (tile, slices)
+            assert not ws[:65536].any(), (tile, slices)
+            tried += 1
+    assert tried >= 3
+
+
 def test_conv_split_k_rejects():
     """Split-K needs its workspace, a K loop long enough to cut, and few enough output tiles to be worth cutting."""
     import ctypes
