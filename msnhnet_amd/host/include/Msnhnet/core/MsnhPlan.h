@@ -73,6 +73,9 @@ struct PlanOp
     int  tile = 0;                          // CONV/IGEMM: tile configuration chosen by Plan::tuneConvs (0 = library default)
     BaseLayer *src = nullptr;               // layer that owns the host weights of this op
     BaseLayer *src2 = nullptr;              // batch-norm layer folded into a CONV
+    int  src2Offset = 0;                    // ... whose first output channel is that channel of the layer (Plan::fuse a2)
+    int  focusAt[4] = {-1, -1, -1, -1};     // CONV over the network input in place of a focus opening (Plan::fuse g): channel of the concatenated slices at which
+                                            // the slice of rows r and columns c starts, at [2 r + c]; the layer's own filter is 3x3 over all of them
     int  chainHead = -1;                    // MAXPOOL: >= 0 = this pool's result is written by the launch of op chainHead (a chain of stride-1 pools in one launch)
     int  chainNext = -1;                    // MAXPOOL at the head or inside such a chain: the op whose pool follows
     int  stemOp = -1;                       // CONV 3x3 stride 2: the (dead) first-layer op computed in front of it by the same launch (Plan::fuse c)

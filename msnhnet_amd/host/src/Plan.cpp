@@ -159,6 +159,44 @@ void Plan::fuse()
         conv.out = aff.out;
         aff.dead = true;
     }
+    // (a2) CONVs (no activation) -> channel concatenation -> AFFINE that is its only reader (the batch norm behind the two halves of a
+    // cross-stage block): every convolution takes its channels of the affine into its epilogue, and the copies fill the affine's result.  The
+    // affine's pass over the tensor goes: eight launches of 4 to 10 us each in a YOLOv5s forward of three 544 x 544 images.
+    for (PlanOp &aff : ops)
+    {
+        if (aff.dead || aff.kind != PlanOp::AFFINE || tensors[static_cast<size_t>(aff.in0)].pinned || consumerCount(aff.in0) != 1) continue;
+        const int joined = aff.in0;
+        std::vector<PlanOp *> copies, convs;
+        int covered = 0;
+        bool ok = true;
+        for (PlanOp &op : ops)
+        {
+            if (op.dead || op.out != joined) continue;
+            ok = ok && op.kind == PlanOp::COPY && !tensors[static_cast<size_t>(op.in0)].pinned && consumerCount(op.in0) == 1;
+            const int p = ok ? producerOf(op.in0) : -1;
+            ok = ok && p >= 0 && ops[static_cast<size_t>(p)].kind == PlanOp::CONV && ops[static_cast<size_t>(p)].act == NONE &&
+                 ops[static_cast<size_t>(p)].src2 == nullptr && ops[static_cast<size_t>(p)].in1 < 0;
+            if (!ok) break;
+            copies.push_back(&op);
+            convs.push_back(&ops[static_cast<size_t>(p)]);
+            covered += tensors[static_cast<size_t>(op.in0)].c;
+        }
+        if (!ok || copies.empty() || covered != tensors[static_cast<size_t>(joined)].c ||
+            tensors[static_cast<size_t>(joined)].dtype != tensors[static_cast<size_t>(aff.out)].dtype)
+            continue;
+        for (size_t k = 0; k < copies.size(); ++k)
+        {
+            if (!aff.pureAct)
+            {
+                convs[k]->src2 = aff.src;
+                convs[k]->src2Offset = copies[k]->dstChanOffset;
+            }
+            convs[k]->act = aff.act;
+            convs[k]->actParam = aff.actParam;
+            copies[k]->out = aff.out;
+        }
+        aff.dead = true;
+    }
     // (b) CONV -> ADD(conv output, other) : the add and the block activation move into the conv epilogue.
     for (size_t i = 0; i < ops.size(); ++i)
     {
@@ -188,6 +226,56 @@ void Plan::fuse()
             break;
         }
     }
+    // (g) float16: network input -> four slices that take every second row and column -> concatenation of the four -> 3x3 convolution (the
+    // focus opening of YOLOv5): the rows 2y - 2 .. 2y + 3 of the input meet in one output row, so the convolution reads the input itself as
+    // a 7x7 convolution of stride 2 and padding 3 whose first filter row and column are zero -- the first-layer kernel takes that.  Ten
+    // launches and 140 us (three images of 544 x 544) become one.
+    if (computeDtype == MSNH_F16)
+        for (PlanOp &conv : ops)
+        {
+            if (conv.dead || conv.kind != PlanOp::CONV || conv.ksize != 3 || conv.stride != 1 || conv.pad != 1 || conv.dilation != 1 || conv.groups != 1 || conv.in1 >= 0) continue;
+            const PlanTensor &out = tensors[static_cast<size_t>(conv.out)];
+            const PlanTensor &joined = tensors[static_cast<size_t>(conv.in0)];
+            if (joined.pinned || consumerCount(conv.in0) != 1 || out.dtype != MSNH_F16 || out.layout != PlanTensor::NHWC) continue;
+            int at[4] = {-1, -1, -1, -1}, image = -1;
+            std::vector<PlanOp *> gone;
+            bool ok = true;
+            for (PlanOp &cp : ops)
+            {
+                if (cp.dead || cp.out != conv.in0) continue;
+                const int p = cp.kind == PlanOp::COPY ? producerOf(cp.in0) : -1;
+                ok = ok && p >= 0 && consumerCount(cp.in0) == 1 && !tensors[static_cast<size_t>(cp.in0)].pinned;
+                if (!ok) break;
+                PlanOp &sl = ops[static_cast<size_t>(p)];
+                ok = sl.kind == PlanOp::SLICE && (image < 0 || sl.in0 == image) && sl.slice[0] == 0 && sl.slice[1] == 1 && sl.slice[3] == 2 && sl.slice[5] == 2 &&
+                     sl.slice[2] < 2 && sl.slice[4] < 2;
+                if (!ok) break;
+                image = sl.in0;
+                at[sl.slice[2] * 2 + sl.slice[4]] = cp.dstChanOffset;
+                gone.push_back(&sl);
+                gone.push_back(&cp);
+            }
+            if (!ok || gone.size() != 8 || *std::min_element(at, at + 4) < 0) continue;
+            const int cast = producerOf(image);
+            const PlanTensor &img = tensors[static_cast<size_t>(image)];
+            if (cast < 0 || ops[static_cast<size_t>(cast)].kind != PlanOp::INPUT_CAST || img.pinned || img.h % 2 != 0 || img.w % 2 != 0 || consumerCount(image) != 4) continue;
+            msnh_conv_desc d;
+            std::memset(&d, 0, sizeof(d));
+            d.dtype = d.out_dtype = MSNH_F16;
+            d.batch = img.n; d.in_h = img.h; d.in_w = img.w; d.in_c = d.in_ld = img.c;
+            d.out_c = out.c; d.out_h = out.h; d.out_w = out.w; d.out_ld = (out.c + 7) / 8 * 8;
+            d.ksize = 7; d.stride = 2; d.pad = 3; d.dilation = 1; d.groups = 1;
+            // (packed filters beyond the scalar kernel's: the matrix-core first-layer kernel takes the shape; the scalar one would lose)
+            if (msnh_hip_conv2d_select_algo(&d) != MSNH_CONV_STEM ||
+                msnh_hip_conv2d_packed_weight_elems(&d, MSNH_CONV_STEM) <= static_cast<size_t>(49) * img.c * out.c * 2)
+                continue;
+            gone.push_back(&ops[static_cast<size_t>(cast)]);
+            for (PlanOp *op : gone) op->dead = true;
+            conv.in0 = ops[static_cast<size_t>(cast)].in0;
+            conv.ksize = 7; conv.stride = 2; conv.pad = 3;
+            std::copy(at, at + 4, conv.focusAt);
+            break;
+        }
     // (c) float16: first layer (3x3 stride 1, 32 filters, over the NCHW network input) -> 3x3 stride-2 convolution that is its only
     // consumer: one launch; the full-resolution 32-channel tensor between them stays on the chip (it keeps its place in the tensor
     // list: its calibrated scale is the scale of the values in LDS)
@@ -493,7 +581,8 @@ uint64_t Plan::structureHash() const
     for (const PlanOp &op : ops)
         os << static_cast<int>(op.kind) << ' ' << op.in0 << ' ' << op.in1 << ' ' << op.out << ' ' << (op.dead && op.tailOf < 0) << ' ' << op.layerIndex << ' ' << op.ksize << ' ' << op.stride << ' '
            << op.pad << ' ' << op.dilation << ' ' << op.groups << ' ' << static_cast<int>(op.act) << ' ' << static_cast<int>(op.act2) << ' ' << op.in1Sign << ' ' << (op.src2 != nullptr)
-           << ' ' << op.dstChanOffset << ' ' << op.stemOp << ' ' << op.chainHead << ' ' << op.mbExpand << ' ' << op.tail << ' ' << op.stemTail << ' ' << op.up2 << ';';
+           << ' ' << op.dstChanOffset << ' ' << op.stemOp << ' ' << op.chainHead << ' ' << op.mbExpand << ' ' << op.tail << ' ' << op.stemTail << ' ' << op.up2 << ' ' << op.src2Offset << ' ' << op.focusAt[0]
+           << ';';
     const std::string text = os.str();
     return PackFile::hash(text.data(), text.size());
 }
@@ -669,7 +758,9 @@ static void foldAffine(const PlanOp &o, int channels, float inMul, std::vector<f
         o.src2->foldedAffine(s2, h2);
         if (scale.empty()) scale.assign(static_cast<size_t>(channels), 1.f);
         if (shift.empty()) shift.assign(static_cast<size_t>(channels), 0.f);
-        for (size_t c = 0; c < static_cast<size_t>(channels); ++c) { scale[c] = s2[c] * scale[c]; shift[c] = s2[c] * shift[c] + h2[c]; }
+        const size_t from = static_cast<size_t>(o.src2Offset);
+        if (s2.size() < from + scale.size() || h2.size() < from + scale.size()) MSNH_THROW("batch-norm weights are not loaded (" + o.name + ")");
+        for (size_t c = 0; c < static_cast<size_t>(channels); ++c) { scale[c] = s2[from + c] * scale[c]; shift[c] = s2[from + c] * shift[c] + h2[from + c]; }
     }
     if (inMul != 1.f)
     {
@@ -702,20 +793,7 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             op.wDev.upload(p2.data(), p2.size() * 2);
             const auto affine = [&](const PlanOp &o, int channels, float inMul, DeviceBuffer &scaleDev, DeviceBuffer &shiftDev) {
                 std::vector<float> scale, shift;
-                o.src->foldedAffine(scale, shift);
-                if (o.src2)
-                {
-                    std::vector<float> s2, h2;
-                    o.src2->foldedAffine(s2, h2);
-                    if (scale.empty()) scale.assign(static_cast<size_t>(channels), 1.f);
-                    if (shift.empty()) shift.assign(static_cast<size_t>(channels), 0.f);
-                    for (size_t c = 0; c < static_cast<size_t>(channels); ++c) { scale[c] = s2[c] * scale[c]; shift[c] = s2[c] * shift[c] + h2[c]; }
-                }
-                if (inMul != 1.f)
-                {
-                    if (scale.empty()) scale.assign(static_cast<size_t>(channels), 1.f);
-                    for (float &v : scale) v *= inMul;
-                }
+                foldAffine(o, channels, inMul, scale, shift);
                 if (!scale.empty()) scaleDev.upload(scale.data(), scale.size() * sizeof(float));
                 if (!shift.empty()) shiftDev.upload(shift.data(), shift.size() * sizeof(float));
             };
@@ -788,9 +866,23 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             }
             d.algo = op.algo;
             workspace = std::max(workspace, msnh_hip_conv2d_workspace_bytes(&d, op.algo));
-            const std::vector<float> &w = op.src->kernelWeights();
-            const size_t expect = static_cast<size_t>(d.out_c) * (d.in_c / d.groups) * d.ksize * d.ksize;
-            if (w.size() != expect) MSNH_THROW("conv weights are not loaded (" + op.name + ")");
+            const std::vector<float> &w0 = op.src->kernelWeights();
+            const bool focus = op.focusAt[0] >= 0;
+            const size_t expect = static_cast<size_t>(d.out_c) * (focus ? 4 * d.in_c * 9 : (d.in_c / d.groups) * d.ksize * d.ksize);
+            if (w0.size() != expect) MSNH_THROW("conv weights are not loaded (" + op.name + ")");
+            std::vector<float> wide;
+            if (focus)
+            {
+                // filter row 1 + 2 fy + dy, column 1 + 2 fx + dx: tap (fy, fx) of the channels that the slice of rows dy and columns dx filled
+                wide.assign(static_cast<size_t>(d.out_c) * d.in_c * 49, 0.f);
+                for (int oc = 0; oc < d.out_c; ++oc)
+                    for (int ci = 0; ci < d.in_c; ++ci)
+                        for (int ky = 0; ky < 6; ++ky)
+                            for (int kx = 0; kx < 6; ++kx)
+                                wide[(static_cast<size_t>(oc) * d.in_c + ci) * 49 + (ky + 1) * 7 + kx + 1] =
+                                    w0[(static_cast<size_t>(oc) * 4 * d.in_c + op.focusAt[ky % 2 * 2 + kx % 2] + ci) * 9 + ky / 2 * 3 + kx / 2];
+            }
+            const std::vector<float> &w = focus ? wide : w0;
             const size_t elems = msnh_hip_conv2d_packed_weight_elems(&d, op.algo);
             const size_t el = d.dtype == MSNH_F16 ? 2 : 4;
             const unsigned char *kept = from ? from->blob(static_cast<uint32_t>(opIndex), static_cast<uint32_t>(op.algo), elems * el) : nullptr;
@@ -804,29 +896,10 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             }
 
             std::vector<float> scale, shift;
-            op.src->foldedAffine(scale, shift);
-            if (op.src2)
-            {
-                std::vector<float> s2, h2;
-                op.src2->foldedAffine(s2, h2);
-                if (scale.empty()) scale.assign(static_cast<size_t>(d.out_c), 1.f);
-                if (shift.empty()) shift.assign(static_cast<size_t>(d.out_c), 0.f);
-                for (int c = 0; c < d.out_c; ++c)
-                {
-                    const size_t i = static_cast<size_t>(c);
-                    scale[i] = s2[i] * scale[i];
-                    shift[i] = s2[i] * shift[i] + h2[i];
-                }
-            }
-            const float inMul = in.layout == PlanTensor::NCHW_INPUT ? 1.f : mulOf(op.in0);
-            if (inMul != 1.f)
-            {
-                if (scale.empty()) scale.assign(static_cast<size_t>(d.out_c), 1.f);
-                for (float &v : scale) v *= inMul;
-            }
+            foldAffine(op, d.out_c, in.layout == PlanTensor::NCHW_INPUT ? 1.f : mulOf(op.in0), scale, shift);
             if (!scale.empty()) op.scaleDev.upload(scale.data(), scale.size() * sizeof(float));
             if (!shift.empty()) op.shiftDev.upload(shift.data(), shift.size() * sizeof(float));
-            op.flops = 2.0 * d.batch * d.out_c * d.out_h * d.out_w * (d.in_c / d.groups) * d.ksize * d.ksize;
+            op.flops = 2.0 * d.batch * d.out_h * d.out_w * static_cast<double>(w0.size());
         }
         else if (op.kind == PlanOp::COL2IM)
         {

@@ -669,6 +669,27 @@ def test_conv_writes_the_upsampled_tensor(fp16):
         assert len(b) > 0 and abs(len(a) - len(b)) <= (max(2, len(b) // 100) if fp16 else 0)
 
 
+@pytest.mark.parametrize("size,batch,fp16", [(32, 1, True), (96, 3, True), (160, 2, True), (96, 2, False)])
+def test_focus_and_concatenated_norms_are_fused(size, batch, fp16):
+    """YOLOv5s: the focus opening (four slices, concatenation, 3x3 convolution) is one first-layer launch in float16, and the batch norms behind
+    the concatenated halves of the cross-stage blocks ride in their convolutions' epilogues (Plan::fuse g, a2).  The head logits against the
+    oracle's, image edges included (a head cell of a 32 x 32 image sees all four)."""
+    net, binp, g = nu.model("yolov5s", batch, size, seed=3)
+    x = zoo.seeded_input(batch, 3, size, size, seed=4)
+    ref, _ = _oracle_layers("yolov5s", size, binp, x)
+    m = netapi.Net(net, binp, fp16=fp16)
+    detail = m.plan_detail()
+    assert " affine" not in detail and ("conv[stem" in detail) == fp16, detail
+    assert not fp16 or not any(k in detail for k in (" slice", " input_cast")), detail
+    m.run_yolo(x)
+    yolo = [i for i in range(m.num_layers()) if m.layer_info(i)["type"] == "yolo"]
+    for h, i in enumerate(yolo):
+        got = m.yolo_head_logits(h).reshape(batch, -1)
+        for b in range(batch):
+            e = nu.rel_err(got[b], ref[b][i - 1])
+            assert e <= (2e-2 if fp16 else 1e-4), (h, b, e)
+
+
 def test_image_in_boxes_out():
     """8-bit images of different shapes -> device letterbox -> forward -> boxes in original-image pixels: equals the
     float path fed with the restatement's letterbox, followed by the restatement's rescale."""
