@@ -265,6 +265,14 @@ int msnh_hip_mbconv_pack(const msnh_mbconv_desc *d, const float *w_expand, const
  * with the output's geometry and pixel stride res_ld, or NULL; y: NHWC float16 with pixel stride out_ld. */
 int msnh_hip_mbconv(const msnh_mbconv_desc *d, const void *x, const void *packed, const float *scale3, const float *shift3, const void *residual,
                     void *y, msnh_stream_t s);
+/* The same with the widened channels of every output tile dealt to `slices` workgroups (for launches of few tiles); their partial results are
+ * summed in a fixed order inside the launch.  _slices: how many the library recommends for the descriptor (1: no workspace needed).
+ * workspace: _workspace_bytes() bytes, 16-byte aligned, the first 64 KiB zero before the first use; a launch leaves them zero.  One workspace
+ * serves launches that follow each other on one stream, MSNH_CONV_IGEMM_FUSEDK's included. */
+int msnh_hip_mbconv_slices(const msnh_mbconv_desc *d);
+size_t msnh_hip_mbconv_workspace_bytes(const msnh_mbconv_desc *d, int slices);
+int msnh_hip_mbconv_sliced(const msnh_mbconv_desc *d, const void *x, const void *packed, const float *scale3, const float *shift3, const void *residual,
+                           void *y, int slices, void *workspace, size_t workspace_bytes, msnh_stream_t s);
 
 /* ------------------------------------------------------------------------------------------------
  * Element-wise / bandwidth-bound layers (all NHWC, any ld).

@@ -269,14 +269,16 @@ template <int BM, int TM, int NW = 4> constexpr size_t igemmEpilogueLds() { retu
 constexpr size_t kFusedKHead = 64 * 1024;          // counters at the start of the workspace, zero between launches
 constexpr int kCpolAgent = 16;                     // sc1
 
+// (waves past nWaves hold nothing and only keep the barriers)
 template <int A, int B>
-__device__ __forceinline__ bool splitKCombine(const IgemmArgs &a, f32x16 (&acc)[A][B], int tileIdx, int nTiles, int wave, int nWaves, int lane, int *flag)
+__device__ __forceinline__ bool splitKCombine(float *ws, int slices, f32x16 (&acc)[A][B], int tileIdx, int nTiles, int wave, int nWaves, int lane, int *flag)
 {
     constexpr int V = A * B * 4;                   // 16-byte vectors per lane
     const size_t slot = static_cast<size_t>(nWaves) * V * 1024;
-    unsigned char *part = reinterpret_cast<unsigned char *>(a.ws) + kFusedKHead + static_cast<size_t>(tileIdx) * slot;
+    unsigned char *part = reinterpret_cast<unsigned char *>(ws) + kFusedKHead + static_cast<size_t>(tileIdx) * slot;
     const size_t step = static_cast<size_t>(nTiles) * slot;        // from a slice to the next one's partial sums of the same tile
     const int off = wave * V * 1024 + lane * 16;
+    if (wave < nWaves)
     {
         const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + blockIdx.y * step, static_cast<unsigned>(slot));
         staticFor<0, V>([&](auto vTag) {
@@ -291,25 +293,26 @@ __device__ __forceinline__ bool splitKCombine(const IgemmArgs &a, f32x16 (&acc)[
     __syncthreads();
     if (wave == 0 && lane == 0)
     {
-        int *count = reinterpret_cast<int *>(a.ws) + tileIdx;
+        int *count = reinterpret_cast<int *>(ws) + tileIdx;
         const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool last = before == a.splitK - 1;
+        const bool last = before == slices - 1;
         if (last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         *flag = last ? 1 : 0;
     }
     __syncthreads();
     if (*flag == 0) return false;
-    for (int s = 0; s < a.splitK; ++s)
-    {
-        const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + s * step, static_cast<unsigned>(slot));
-        staticFor<0, V>([&](auto vTag) {
-            constexpr int v = decltype(vTag)::value;
-            constexpr int ij = v / 4, q = v % 4;
-            const f32x4 d = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + v * 1024, 0, kCpolAgent));
+    if (wave < nWaves)
+        for (int s = 0; s < slices; ++s)
+        {
+            const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + s * step, static_cast<unsigned>(slot));
+            staticFor<0, V>([&](auto vTag) {
+                constexpr int v = decltype(vTag)::value;
+                constexpr int ij = v / 4, q = v % 4;
+                const f32x4 d = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + v * 1024, 0, kCpolAgent));
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[ij / B][ij % B][q * 4 + e] = s == 0 ? d[e] : acc[ij / B][ij % B][q * 4 + e] + d[e];
-        });
-    }
+                for (int e = 0; e < 4; ++e) acc[ij / B][ij % B][q * 4 + e] = s == 0 ? d[e] : acc[ij / B][ij % B][q * 4 + e] + d[e];
+            });
+        }
     return true;
 }
 
@@ -525,7 +528,7 @@ __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&a
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (a.fusedK > 1 && !splitKCombine(a, mine, tileIdx, nTiles, wave, nWaves, lane, reinterpret_cast<int *>(ss + 2 * BM))) return;
+    if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, mine, tileIdx, nTiles, wave, nWaves, lane, reinterpret_cast<int *>(ss + 2 * BM))) return;
     igemmEpilogue<T, TOut, BM, BN, 64, 32>(a, mine, smemRaw, chScale, chShift, m0, p0, wm, wn * 2 + kg, wave, lane, g, ss, stageOwn);
 }
 
@@ -1119,7 +1122,7 @@ void convIgemmKernel(IgemmArgs a)
         return;
     }
     if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles);
-    else if (a.fusedK > 1 && !splitKCombine(a, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + igemmEpilogueLds<BM, TM, NT / 64>()))) return;
+    else if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + igemmEpilogueLds<BM, TM, NT / 64>()))) return;
     else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g);
 }
 

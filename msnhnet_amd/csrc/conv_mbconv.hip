@@ -14,6 +14,9 @@
 // Everything a chunk needs beside the activations -- both 1x1 filters in matrix-core fragment order (rows permuted so that a lane's 16
 // accumulators are 16 consecutive channels), the depthwise taps, the two affines -- is one contiguous record of the packed weights,
 // copied into LDS by 16-byte-per-lane loads that deliver straight into LDS while the chunk before it is computed.
+//
+// One image of 14 x 14 pixels is four such workgroups on 256 CUs, each a serial chain of six or nine chunks.  There the chunks are dealt to
+// several workgroups per tile (grid y), whose partial projections are summed inside the launch (splitKCombine) before the epilogue.
 #include "conv_igemm.hpp"
 
 namespace msnh {
@@ -41,6 +44,8 @@ struct MbArgs
     int ks;                 // 16-wide K steps of the expand GEMM: ceil(in_c / 16)
     int mb;                 // 32-row blocks of the project GEMM: ceil(out_c / 32)
     int chunks;
+    int slices, perSlice;   // slices > 1: workgroups per tile, and chunks of each (the last may have fewer)
+    float *ws;
     unsigned chunkBytes;    // one chunk's record in the packed weights
     unsigned xBytes, blobBytes;
     int act1, act2, act3, act4, hasRes;
@@ -115,7 +120,9 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
             dmaLoad16(rb, static_cast<unsigned>(p) * 1024u + static_cast<unsigned>(lane) * 16u, static_cast<unsigned>(chunk) * a.chunkBytes,
                       ldsBase + dst + static_cast<unsigned>(p) * 1024u);
     };
-    issueBlob(0, bOff);
+    const int cBegin = static_cast<int>(blockIdx.y) * a.perSlice;
+    const int cEnd = min(a.chunks, cBegin + a.perSlice);
+    issueBlob(cBegin, bOff + static_cast<unsigned>(cBegin & 1) * a.chunkBytes);
 
     // ---- the input tile, zeros outside the image and past in_c: delivered straight into LDS, 1 KiB per wavefront and load; a pixel's row
     // is 2 ks + 1 slots of 16 bytes, the last one padding (an out-of-range offset delivers zeros) -------------------------------------
@@ -149,9 +156,9 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
         if (px < IP && gy >= 0 && gy < a.H && gx >= 0 && gx < a.W) inImage |= 1u << j;
     }
 
-    f32x16 accP;                                      // project: wavefront w owns block w / 2 of the output channels x column block w % 2
+    f32x16 accP[1][1];                                  // project: wavefront w owns block w / 2 of the output channels x column block w % 2
 #pragma unroll
-    for (int e = 0; e < 16; ++e) accP[e] = 0.f;
+    for (int e = 0; e < 16; ++e) accP[0][0][e] = 0.f;
 
     dmaWait<0>();
     __syncthreads();
@@ -208,15 +215,15 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
             *reinterpret_cast<f16x8 *>(ep + 16) = o1;
         }
     };
-    expandChunk(0);
-    for (int c = 0; c < a.chunks; ++c)
+    expandChunk(cBegin);
+    for (int c = cBegin; c < cEnd; ++c)
     {
         const unsigned cur = bOff + static_cast<unsigned>(c & 1) * a.chunkBytes;
         const unsigned char *rec = smem + cur;
         const float *aff = reinterpret_cast<const float *>(rec + mbAffOff(a.ks, a.mb));
         const int left = a.cexp - c * MB_CH;
         __syncthreads();
-        if (c + 1 < a.chunks) issueBlob(c + 1, bOff + static_cast<unsigned>((c + 1) & 1) * a.chunkBytes);
+        if (c + 1 < cEnd) issueBlob(c + 1, bOff + static_cast<unsigned>((c + 1) & 1) * a.chunkBytes);
 
         // ---- 2. depthwise (the threads share out the channel vectors that exist) ---------------------------------------------------------
         {
@@ -265,11 +272,13 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
             const unsigned char *bp = smem + yOff + (32 * j + n) * MB_ROW + h * 16;
 #pragma unroll
             for (int s = 0; s < MB_CH / 16; ++s)
-                mfmaBlock(*reinterpret_cast<const f16x8 *>(ap + s * 1024), *reinterpret_cast<const f16x8 *>(bp + s * 32), accP);
+                mfmaBlock(*reinterpret_cast<const f16x8 *>(ap + s * 1024), *reinterpret_cast<const f16x8 *>(bp + s * 32), accP[0][0]);
         }
-        if (c + 1 < a.chunks) expandChunk(c + 1);
+        if (c + 1 < cEnd) expandChunk(c + 1);
     }
 
+    // (the depthwise buffer's last readers are behind the barrier inside)
+    if (a.slices > 1 && !splitKCombine(a.ws, a.slices, accP, logical, a.total, wave, 2 * a.mb, lane, reinterpret_cast<int *>(smem + eOff))) return;
     // ---- epilogue: affine, activation, residual, second activation, scale; two 16-byte stores per lane ------------------------------
     if (wave < 2 * a.mb)
     {
@@ -291,8 +300,8 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                 {
-                    v[e]     = accP[8 * g + e] * s0[e] + h0[e];
-                    v[4 + e] = accP[8 * g + 4 + e] * s1[e] + h1[e];
+                    v[e]     = accP[0][0][8 * g + e] * s0[e] + h0[e];
+                    v[4 + e] = accP[0][0][8 * g + 4 + e] * s1[e] + h1[e];
                 }
                 activateArray<8>(v, a.act3, a.act3Param);
                 if (a.hasRes)
@@ -397,8 +406,36 @@ int msnh_hip_mbconv_pack(const msnh_mbconv_desc *d, const float *w_expand, const
     return 0;
 }
 
+int msnh_hip_mbconv_slices(const msnh_mbconv_desc *d)
+{
+    if (!msnh_hip_mbconv_supported(d)) return 0;
+    const long long tiles = static_cast<long long>((d->out_w + MB_TO - 1) / MB_TO) * ((d->out_h + MB_TO - 1) / MB_TO) * d->batch;
+    const int chunks = (d->exp_c + MB_CH - 1) / MB_CH;
+    // One workgroup per CU at most, and no more than six slices: past that the partial sums' way through memory costs what a shorter chain
+    // saves.  Two slices gain nothing over one (7.8 us either way for 24 -> 144 -> 24 channels at 56 x 56).  One image of 14 x 14,
+    // 96 -> 576 -> 96 channels: 18.9 us unsliced, 13.7 with two, 10.8 with three, 9.9 with five; eight images 19.1 and 10.7.
+    const int most = static_cast<int>(std::min<long long>(6, 256 / tiles));
+    if (most < 3 || chunks < 3) return 1;
+    const int per = (chunks + most - 1) / most;
+    const int slices = (chunks + per - 1) / per;
+    return slices < 3 ? 1 : slices;
+}
+
+size_t msnh_hip_mbconv_workspace_bytes(const msnh_mbconv_desc *d, int slices)
+{
+    if (!msnh_hip_mbconv_supported(d) || slices < 2) return 0;
+    const size_t tiles = static_cast<size_t>((d->out_w + MB_TO - 1) / MB_TO) * ((d->out_h + MB_TO - 1) / MB_TO) * d->batch;
+    return kFusedKHead + tiles * slices * 2 * ((d->out_c + 31) / 32) * 4096;
+}
+
 int msnh_hip_mbconv(const msnh_mbconv_desc *d, const void *x, const void *packed, const float *scale3, const float *shift3, const void *residual,
                     void *y, msnh_stream_t s)
+{
+    return msnh_hip_mbconv_sliced(d, x, packed, scale3, shift3, residual, y, 1, nullptr, 0, s);
+}
+
+int msnh_hip_mbconv_sliced(const msnh_mbconv_desc *d, const void *x, const void *packed, const float *scale3, const float *shift3, const void *residual,
+                           void *y, int slices, void *workspace, size_t workspace_bytes, msnh_stream_t s)
 {
     MSNH_REQUIRE(msnh_hip_mbconv_supported(d), "mbconv: block not supported (channels, stride or sizes)");
     MSNH_REQUIRE(x && packed && y && (!d->has_residual || residual), "mbconv: null pointer");
@@ -414,6 +451,12 @@ int msnh_hip_mbconv(const msnh_mbconv_desc *d, const void *x, const void *packed
     MSNH_REQUIRE(total < (1ll << 30), "mbconv: too many tiles");
     a.total = static_cast<int>(total);
     a.ks = (d->in_c + 15) / 16; a.mb = (d->out_c + 31) / 32; a.chunks = (d->exp_c + MB_CH - 1) / MB_CH;
+    MSNH_REQUIRE(slices >= 1 && slices <= a.chunks, "mbconv: %d slices of %d chunks", slices, a.chunks);
+    a.perSlice = (a.chunks + slices - 1) / slices;
+    a.slices = (a.chunks + a.perSlice - 1) / a.perSlice;          // none of them empty
+    a.ws = static_cast<float *>(workspace);
+    MSNH_REQUIRE(a.slices == 1 || (workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= msnh_hip_mbconv_workspace_bytes(d, a.slices) &&
+                                   total <= static_cast<long long>(kFusedKHead / 4)), "mbconv: sliced launch without its workspace");
     a.chunkBytes = mbChunkBytes(a.ks, a.mb);
     a.xBytes = static_cast<unsigned>((static_cast<unsigned long long>(d->batch) * d->in_h * d->in_w - 1) * d->in_ld * 2ull + d->in_c * 2ull);
     a.blobBytes = static_cast<unsigned>(static_cast<size_t>(a.chunks) * a.chunkBytes);
@@ -429,13 +472,13 @@ int msnh_hip_mbconv(const msnh_mbconv_desc *d, const void *x, const void *packed
     {
         static bool raised = false;
         if (!raised) { MSNH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mbconvKernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); raised = true; }
-        hipLaunchKernelGGL((mbconvKernel<1>), dim3(blocks), dim3(64 * MB_NW), lds, st, a);
+        hipLaunchKernelGGL((mbconvKernel<1>), dim3(blocks, static_cast<unsigned>(a.slices)), dim3(64 * MB_NW), lds, st, a);
     }
     else
     {
         static bool raised = false;
         if (!raised) { MSNH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mbconvKernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); raised = true; }
-        hipLaunchKernelGGL((mbconvKernel<2>), dim3(blocks), dim3(64 * MB_NW), lds, st, a);
+        hipLaunchKernelGGL((mbconvKernel<2>), dim3(blocks, static_cast<unsigned>(a.slices)), dim3(64 * MB_NW), lds, st, a);
     }
     MSNH_LAUNCH_CHECK();
     return 0;

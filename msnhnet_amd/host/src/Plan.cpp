@@ -773,7 +773,7 @@ static std::vector<uint16_t> toHalf(const std::vector<float> &v);
 
 void Plan::prepareWeights(PackFile *from, PackFile *to)
 {
-    size_t workspace = 0;
+    size_t workspace = 0, sliceWorkspace = 0;
     for (size_t opIndex = 0; opIndex < ops.size(); ++opIndex)
     {
         PlanOp &op = ops[opIndex];
@@ -838,6 +838,7 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             if (!s3.empty()) op.scaleDev.upload(s3.data(), s3.size() * sizeof(float));
             if (!h3.empty()) op.shiftDev.upload(h3.data(), h3.size() * sizeof(float));
             op.algo = MSNH_CONV_MBCONV;
+            sliceWorkspace = std::max(sliceWorkspace, msnh_hip_mbconv_workspace_bytes(&d, msnh_hip_mbconv_slices(&d)));
             const PlanTensor &wide = tensors[static_cast<size_t>(ex.out)];
             const PlanTensor &narrow = tensors[static_cast<size_t>(dw.out)];
             op.flops = 2.0 * d.batch * (static_cast<double>(wide.h) * wide.w * d.exp_c * d.in_c + static_cast<double>(narrow.h) * narrow.w * d.exp_c * 9 +
@@ -971,6 +972,7 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
         }
     }
     if (workspace > _convWorkspace.bytes()) _convWorkspace.alloc(workspace);
+    reserveSliceWorkspace(sliceWorkspace, nullptr);
 }
 
 // Tune cache, one line per tuned launch: what identifies the launch (shape, dtype, epilogue kind) and what the search chose for it.
@@ -1379,7 +1381,8 @@ void Plan::launch(PlanOp &op, msnh_stream_t s)
         {
             const msnh_mbconv_desc md = mbconvDesc(*this, op);
             if (op.wDev.bytes() != msnh_hip_mbconv_packed_bytes(&md)) MSNH_THROW("mbconv weights on the device do not fit this launch (" + op.name + ")");
-            MSNH_DEV(msnh_hip_mbconv(&md, ptr(op.in0), op.wDev.ptr(), op.scaleDev.as<float>(), op.shiftDev.as<float>(), op.in1 >= 0 ? ptr(op.in1) : nullptr, ptr(op.out), s));
+            MSNH_DEV(msnh_hip_mbconv_sliced(&md, ptr(op.in0), op.wDev.ptr(), op.scaleDev.as<float>(), op.shiftDev.as<float>(), op.in1 >= 0 ? ptr(op.in1) : nullptr, ptr(op.out),
+                                            msnh_hip_mbconv_slices(&md), _sliceWorkspace.ptr(), _sliceWorkspace.bytes(), s));
             break;
         }
         if (op.algo == MSNH_CONV_IGEMM_TAIL)
@@ -1558,6 +1561,7 @@ void Plan::reserveSliceWorkspace(size_t bytes, msnh_stream_t s)
     MSNH_DEV(msnh_hip_stream_sync(s));
     _sliceWorkspace.alloc(bytes);
     MSNH_DEV(msnh_hip_fill_zero(_sliceWorkspace.ptr(), static_cast<size_t>(64) << 10, s));
+    MSNH_DEV(msnh_hip_stream_sync(s));          // (the launches that use it may go to another stream)
 }
 
 void Plan::clearCandidates(msnh_stream_t s)

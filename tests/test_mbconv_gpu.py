@@ -132,3 +132,45 @@ def test_mbconv_activations_and_limits():
         assert L.msnh_hip_mbconv_supported(ctypes.byref(d)) == 0, change
         assert L.msnh_hip_mbconv_packed_bytes(ctypes.byref(d)) == 0
         assert L.msnh_hip_mbconv(ctypes.byref(d), None, None, None, None, None, None, None) != 0
+
+
+@pytest.mark.parametrize("case,slices", [((1, 96, 14, 14, 576, 96, 1, True), 9), ((2, 64, 14, 14, 384, 64, 1, True), 4), ((1, 24, 21, 28, 144, 32, 2, False), 3),
+                                         ((1, 8, 10, 13, 136, 8, 1, True), 2), ((3, 16, 7, 7, 64, 24, 1, False), 1)])
+def test_mbconv_sliced(case, slices):
+    """the widened channels dealt to several workgroups per tile: float32 sums in another order than the unsliced launch, so equal to it within
+    one rounding of the output; equal to itself bit for bit, whoever arrives last, with the workspace's counters left at zero"""
+    import torch
+    import gpuutil as gu
+    gu.init()
+    L = abi.lib()
+    b, cin, h, w, cexp, cout, stride, with_res = case
+    oh, ow = (h - 1) // stride + 1, (w - 1) // stride + 1
+    rng = np.random.default_rng(sum(case) + 3)
+    d = abi.MbconvDesc(b, h, w, cin, cin, cexp, stride, cout, oh, ow, cout, abi.ACT["relu6"], abi.ACT["relu6"], abi.ACT["none"], abi.ACT["none"],
+                       0.1, 0.1, 0.1, 0.1, 1 if with_res else 0, cout, 1.0, 1.0, 1.0, 1.0)
+    f = lambda *shape, k=1.0: np.ascontiguousarray(rng.standard_normal(shape) * k, np.float32)
+    we, wd, wp = f(cexp, cin, k=(2.0 / cin) ** 0.5), f(cexp, 9, k=0.4), f(cout, cexp, k=(1.0 / cexp) ** 0.5)
+    packed = np.zeros(L.msnh_hip_mbconv_packed_bytes(ctypes.byref(d)), np.uint8)
+    vp = lambda a: a.ctypes.data_as(ctypes.c_void_p)
+    abi.check(L.msnh_hip_mbconv_pack(ctypes.byref(d), vp(we), None, None, vp(wd), None, None, vp(wp), vp(packed)))
+    xd, rd = gu.nhwc_dev(f(b, cin, h, w), abi.F16, cin), gu.nhwc_dev(f(b, cout, oh, ow), abi.F16, cout)
+    pd, shift = torch.from_numpy(packed).cuda(), gu.dev(f(cout))
+    need = L.msnh_hip_mbconv_workspace_bytes(ctypes.byref(d), slices)
+    ws = torch.zeros(max(need, 16), dtype=torch.uint8).cuda()
+
+    def run(n, space):
+        y = torch.full((b, oh, ow, cout), 5.0, dtype=torch.float16).cuda()
+        abi.check(L.msnh_hip_mbconv_sliced(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), None, gu.ptr(shift), gu.ptr(rd) if with_res else None, gu.ptr(y), n,
+                                           gu.ptr(ws) if space else None, need if space else 0, None))
+        gu.sync()
+        return gu.nchw_host(y, cout)
+
+    print("mbconv sliced", case, slices, flush=True)
+    assert 1 <= L.msnh_hip_mbconv_slices(ctypes.byref(d)) <= (cexp + 63) // 64
+    whole, parts = run(1, False), run(slices, True)
+    assert gu.rel_err(parts, whole) <= 1e-3
+    assert all(np.array_equal(run(slices, True), parts) for _ in range(3))
+    assert not ws[:65536].any().item()
+    if slices > 1:
+        assert L.msnh_hip_mbconv_sliced(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), None, gu.ptr(shift), None, gu.ptr(xd), slices, gu.ptr(ws), need - 1, None) != 0
+    assert L.msnh_hip_mbconv_sliced(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), None, gu.ptr(shift), None, gu.ptr(xd), (cexp + 63) // 64 + 1, gu.ptr(ws), need, None) != 0
