@@ -93,6 +93,7 @@ int msnh_hip_host_free(void *hptr);
 int msnh_hip_memcpy_h2d(void *dst, const void *src, size_t bytes, msnh_stream_t s);
 int msnh_hip_memcpy_d2h(void *dst, const void *src, size_t bytes, msnh_stream_t s);
 int msnh_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, msnh_stream_t s);
+int msnh_hip_copy(void *dst, const void *src, size_t bytes, msnh_stream_t s);   /* by a kernel: device and pinned host memory, 16-byte aligned; safe under graph capture */
 int msnh_hip_fill_zero(void *dst, size_t bytes, msnh_stream_t s); /* a fill kernel, safe under graph capture */
 int msnh_hip_stream_create(msnh_stream_t *s);
 int msnh_hip_stream_destroy(msnh_stream_t s);

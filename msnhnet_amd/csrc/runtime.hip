@@ -22,6 +22,15 @@ hipStream_t resolveStream(msnh_stream_t s)
     return s ? static_cast<hipStream_t>(s) : g_defaultStream;
 }
 
+// Device <-> pinned host memory by the compute units: bound by the bus (3 MB in 57 us, 52 GB/s, as the copy engine), but without the engine's
+// start (10 us per transfer in front of a kernel that waits for it), so a transfer can be cut into pieces that follow each other.
+__global__ __launch_bounds__(256) void copyKernel(unsigned char *dst, const unsigned char *src, size_t bytes)
+{
+    const size_t vecs = bytes / 16, at = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x, stride = static_cast<size_t>(gridDim.x) * 256;
+    for (size_t i = at; i < vecs; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    if (at < bytes % 16) dst[vecs * 16 + at] = src[vecs * 16 + at];
+}
+
 __global__ void fillZeroKernel(uint32_t *dst, size_t words)
 {
     size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -125,6 +134,18 @@ int msnh_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, msnh_stream_t 
     if (bytes == 0) return 0;
     MSNH_REQUIRE(dst && src, "memcpy_d2d: NULL pointer");
     MSNH_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, resolveStream(s)));
+    return 0;
+}
+
+int msnh_hip_copy(void *dst, const void *src, size_t bytes, msnh_stream_t s)
+{
+    if (bytes == 0) return 0;
+    MSNH_REQUIRE(dst && src, "copy: NULL pointer");
+    MSNH_REQUIRE(reinterpret_cast<uintptr_t>(dst) % 16 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0, "copy: need 16-byte alignment");
+    const size_t blocks = (bytes + 4095) / 4096;
+    hipLaunchKernelGGL(copyKernel, dim3(static_cast<unsigned>(blocks < 256 ? blocks : 256)), dim3(256), 0, resolveStream(s), static_cast<unsigned char *>(dst),
+                       static_cast<const unsigned char *>(src), bytes);
+    MSNH_LAUNCH_CHECK();
     return 0;
 }
 

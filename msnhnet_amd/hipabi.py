@@ -51,7 +51,7 @@ _lib = None
 SYMBOLS = [
     "msnh_hip_last_error", "msnh_hip_init", "msnh_hip_device_count", "msnh_hip_device_name", "msnh_hip_malloc", "msnh_hip_free",
     "msnh_hip_host_alloc", "msnh_hip_host_free", "msnh_hip_memcpy_h2d", "msnh_hip_memcpy_d2h", "msnh_hip_memcpy_d2d",
-    "msnh_hip_fill_zero", "msnh_hip_stream_create", "msnh_hip_stream_destroy", "msnh_hip_stream_sync", "msnh_hip_event_create",
+    "msnh_hip_copy", "msnh_hip_fill_zero", "msnh_hip_stream_create", "msnh_hip_stream_destroy", "msnh_hip_stream_sync", "msnh_hip_event_create",
     "msnh_hip_event_destroy", "msnh_hip_event_record", "msnh_hip_stream_wait_event", "msnh_hip_event_sync", "msnh_hip_event_elapsed_ms", "msnh_hip_graph_begin",
     "msnh_hip_graph_end", "msnh_hip_graph_launch", "msnh_hip_graph_destroy", "msnh_hip_conv_stem_down_supported", "msnh_hip_conv_stem_down_packed_elems", "msnh_hip_conv_stem_down_pack", "msnh_hip_conv_stem_down", "msnh_hip_conv_stem_down_tail_supported", "msnh_hip_conv_stem_down_tail_packed_elems", "msnh_hip_conv_stem_down_tail_pack", "msnh_hip_conv_stem_down_tail", "msnh_hip_mbconv_supported", "msnh_hip_mbconv_packed_bytes", "msnh_hip_mbconv_pack", "msnh_hip_mbconv", "msnh_hip_mbconv_slices", "msnh_hip_mbconv_workspace_bytes", "msnh_hip_mbconv_sliced", "msnh_hip_conv2d_tile_count", "msnh_hip_conv2d_pack_layout_version", "msnh_hip_conv2d_tile_supported", "msnh_hip_conv2d_select_algo",
     "msnh_hip_conv2d_packed_weight_elems", "msnh_hip_conv2d_pack_weights", "msnh_hip_conv2d_workspace_bytes", "msnh_hip_conv2d",
@@ -88,6 +88,7 @@ def lib():
     L.msnh_hip_host_free.argtypes = [vp]
     for n in ("h2d", "d2h", "d2d"):
         getattr(L, "msnh_hip_memcpy_" + n).argtypes = [vp, vp, sz, vp]
+    L.msnh_hip_copy.argtypes = [vp, vp, sz, vp]
     L.msnh_hip_fill_zero.argtypes = [vp, sz, vp]
     L.msnh_hip_stream_create.argtypes = [ctypes.POINTER(vp)]
     L.msnh_hip_stream_destroy.argtypes = [vp]

@@ -143,8 +143,15 @@ private:
     bool   _planReady = false;
     std::vector<std::vector<float>> _layerOutputs;
     DeviceBuffer _inputDev, _imageDev;
-    PinnedBuffer _imagePinned;
+    PinnedBuffer _imagePinned;                 // 8-bit images on their way to _imageDev: [0, _imageUsed) of both belongs to uploads that may still run
+    size_t _imageUsed = 0;
+    long long _imageForward = 0;               // number of the forward enqueued behind the last of them
+    long long _enqueued = 0;                   // forwards enqueued so far
+    void imagesDone(long long forward);        // forward number `forward` is known to have finished
     PinnedBuffer _inputPinned, _outputPinned;
+    bool _outputReady = false;                 // _outputPinned receives the result of the last forward enqueued
+    size_t outputBytes() const;                // size of a classifier's result if the forward itself delivers it to _outputPinned, else 0
+    void upload(void *dst, void *stage, const void *src, size_t bytes);
     msnh_stream_t _stream = nullptr;
     // The captured forward.  Detectors have one per copy-back slot and per place of the NMS (inside the forward or behind it), captured
     // when first needed; [0][0] is the only one of a classifier.

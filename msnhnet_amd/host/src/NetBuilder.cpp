@@ -74,6 +74,7 @@ void NetBuilder::clearLayers()
     _layerOutputs.clear();
     _nextSlot = 0;
     _inFlight = 0;
+    _outputReady = false;
 }
 
 // ---- build -----------------------------------------------------------------------------------------------------------
@@ -460,6 +461,8 @@ void NetBuilder::finalizePlan()
     const float calMs = msSince(t0);
     t0 = Clock::now();
     plan->place();
+    _outputReady = false;
+    if (const size_t bytes = plan->tensors[static_cast<size_t>(plan->layerOut.back())].elems() * sizeof(float); bytes <= static_cast<size_t>(1) << 20) _outputPinned.reserve(bytes);
     setupYoloBuffers(*plan, _net->batch);
     plan->preferWinograd = winograd;
     plan->sparseYolo = !_saveLayerOutput;         // layer dumps read the whole decoded tensors
@@ -513,11 +516,29 @@ void NetBuilder::checkInput(size_t given) const
 std::vector<float> NetBuilder::runClassify(std::vector<float>) { MSNH_THROW("Gpu mode , can not run with cpu"); }
 std::vector<std::vector<YoloBox>> NetBuilder::runYolo(std::vector<float>) { MSNH_THROW("Gpu mode , can not run with cpu"); }
 
-// Host floats -> pinned staging buffer -> device, in pieces: the workers copy piece k + 1 into the staging buffer while the
-// DMA engine moves piece k (a batch of YOLOv3-608 is 35 MB: one thread's memcpy alone would take longer than the forward).
+// Host memory -> pinned staging buffer -> device, in pieces that a kernel moves while the next one is copied into the staging buffer: up to a
+// few MB the engine's start per transfer is what counts, not the bus (3 MB with the wait for it 129 -> 99 us, 4.4 MB 172 -> 138).
+void NetBuilder::upload(void *dst, void *stage, const void *src, size_t bytes)
+{
+    const size_t piece = static_cast<size_t>(512) << 10;
+    for (size_t off = 0; off < bytes; off += piece)
+    {
+        const size_t len = std::min(piece, bytes - off);
+        std::memcpy(static_cast<char *>(stage) + off, static_cast<const char *>(src) + off, len);
+        MSNH_DEV(msnh_hip_copy(static_cast<char *>(dst) + off, static_cast<char *>(stage) + off, len, _stream));
+    }
+}
+
+// A larger batch: the workers copy piece k + 1 into the staging buffer while the DMA engine moves piece k (a batch of YOLOv3-608 is 35 MB: one
+// thread's memcpy alone would take longer than the forward).
 void NetBuilder::uploadInput(const float *img, size_t count)
 {
     const size_t bytes = count * sizeof(float);
+    if (bytes <= static_cast<size_t>(8) << 20)
+    {
+        upload(_inputDev.ptr(), _inputPinned.ptr(), img, bytes);
+        return;
+    }
     const size_t piece = static_cast<size_t>(4) << 20, slice = static_cast<size_t>(512) << 10;
     const char *src = reinterpret_cast<const char *>(img);
     char *stage = static_cast<char *>(_inputPinned.ptr());
@@ -549,15 +570,28 @@ void NetBuilder::setInputImage(int index, const unsigned char *rgbHwc, int width
     if (index < 0 || index >= _net->batch) MSNH_THROW("image index outside the batch");
     if (preproc == MSNH_PRE_TRANSFORMED && (mean == nullptr || std == nullptr)) MSNH_THROW("mean or std can't be null");
     const size_t bytes = static_cast<size_t>(width) * height * 3;
-    // the pinned staging buffer is reused by the next call: wait for the previous upload before overwriting it
-    MSNH_DEV(msnh_hip_stream_sync(_stream));
-    _imagePinned.reserve(bytes);
-    if (_imageDev.bytes() < bytes) _imageDev.alloc(bytes);
-    std::memcpy(_imagePinned.ptr(), rgbHwc, bytes);
-    MSNH_DEV(msnh_hip_memcpy_h2d(_imageDev.ptr(), _imagePinned.ptr(), bytes, _stream));
+    // The images of a batch follow each other in the staging buffer; what earlier uploads still read is not overwritten before they are done.
+    const size_t space = (bytes + 15) / 16 * 16, most = static_cast<size_t>(64) << 20;
+    if (_imageUsed + space > _imagePinned.bytes())
+    {
+        if (_imageUsed > 0) MSNH_DEV(msnh_hip_stream_sync(_stream));
+        _imageUsed = 0;
+        const size_t want = std::max(space, std::min(most, space * static_cast<size_t>(_net->batch)));
+        _imagePinned.reserve(want);
+        if (_imageDev.bytes() < want) _imageDev.alloc(want);
+    }
+    const size_t at = _imageUsed;
+    _imageUsed += space;
+    _imageForward = _enqueued + 1;
+    upload(_imageDev.as<char>() + at, _imagePinned.as<char>() + at, rgbHwc, bytes);
     float *dst = _inputDev.as<float>() + static_cast<size_t>(index) * 3 * _net->height * _net->width;
-    MSNH_DEV(msnh_hip_image_u8_to_input(static_cast<const unsigned char *>(_imageDev.ptr()), width, height, _net->width, _net->height, preproc, mean, std,
+    MSNH_DEV(msnh_hip_image_u8_to_input(_imageDev.as<unsigned char>() + at, width, height, _net->width, _net->height, preproc, mean, std,
                                         shuffleRGB ? 1 : 0, dst, _stream));
+}
+
+void NetBuilder::imagesDone(long long forward)
+{
+    if (forward >= _imageForward) _imageUsed = 0;
 }
 
 static std::vector<float> yoloLayerDump(Plan &plan, const YoloLayer *yl, const PlanOp &op, int batch, msnh_stream_t s)
@@ -581,6 +615,7 @@ static std::vector<float> yoloLayerDump(Plan &plan, const YoloLayer *yl, const P
 void NetBuilder::runLayersEager()
 {
     Plan &plan = *_net->plan;
+    _outputReady = false;
     plan.yoloSlot = 0;
     plan.clearCandidates(_stream);
     _layerOutputs.assign(_net->layers.size(), std::vector<float>());
@@ -653,6 +688,8 @@ void NetBuilder::enqueueForward(const float *deviceInput)
         MSNH_DEV(msnh_hip_graph_end(_stream, &graph));
     }
     if (!eager) MSNH_DEV(msnh_hip_graph_launch(graph, _stream));
+    ++_enqueued;
+    _outputReady = outputBytes() > 0;
     if (yout)
     {
         _countsClear[slot] = inForward;
@@ -671,6 +708,17 @@ void NetBuilder::issueForward(YoloOutLayer *yout, bool inForward, msnh_stream_t 
     plan.runAll(s);
     if (yout) yout->enqueueGather(s);
     if (inForward) yout->enqueueImageNms(s, plan.yoloSlot);
+    if (const size_t bytes = outputBytes()) MSNH_DEV(msnh_hip_copy(_outputPinned.ptr(), plan.ptr(plan.layerOut.back()), bytes, s));
+}
+
+// A classifier's logits leave the device with the forward's last launch: a copy asked for behind it would wait for the copy engine's start.
+size_t NetBuilder::outputBytes() const
+{
+    const Plan &plan = *_net->plan;
+    if (_net->layers.back()->type() == LayerType::YOLO_OUT) return 0;
+    const PlanTensor &t = plan.tensors[static_cast<size_t>(plan.layerOut.back())];
+    const size_t bytes = t.elems() * sizeof(float);
+    return t.layout == PlanTensor::FLAT && t.dtype == MSNH_F32 && t.parent < 0 && bytes <= _outputPinned.bytes() ? bytes : 0;
 }
 
 void NetBuilder::dropGraphs()
@@ -687,7 +735,14 @@ std::vector<float> NetBuilder::fetchClassify()
 {
     Plan &plan = *_net->plan;
     std::vector<float> out;
-    plan.exportTensor(plan.layerOut.back(), out, _stream);
+    if (_outputReady)
+    {
+        MSNH_DEV(msnh_hip_stream_sync(_stream));
+        const float *r = _outputPinned.as<float>();
+        out.assign(r, r + outputBytes() / sizeof(float));
+    }
+    else plan.exportTensor(plan.layerOut.back(), out, _stream);
+    imagesDone(_enqueued);
     return out;
 }
 
@@ -706,6 +761,7 @@ const std::vector<std::vector<YoloBox>> &NetBuilder::fetchYoloResult()
     const int slot = (_nextSlot + 2 - _inFlight) & 1;          // oldest outstanding
     yout->finish(slot);
     --_inFlight;
+    imagesDone(_enqueued - _inFlight);
     return yout->finalOut;
 }
 
@@ -787,6 +843,7 @@ float NetBuilder::fp16Headroom(const std::vector<float> &img)
     checkInput(img.size());
     if (_inFlight > 0) MSNH_THROW("fetch the outstanding results first");
     uploadInput(img.data(), img.size());
+    _outputReady = false;
     return _net->plan->fp16Headroom(_stream);
 }
 
@@ -893,6 +950,7 @@ static double opBytes(const Plan &plan, const PlanOp &op)
 float NetBuilder::profileOps(int kind, int reps, int *launches, double *flops, double *bytes)
 {
     if (!_planReady) MSNH_THROW("weights are not loaded");
+    _outputReady = false;
     Plan &plan = *_net->plan;
     msnh_event_t e0 = nullptr, e1 = nullptr;
     MSNH_DEV(msnh_hip_event_create(&e0));
@@ -927,6 +985,7 @@ float NetBuilder::profileOps(int kind, int reps, int *launches, double *flops, d
 std::string NetBuilder::profileEachOp(int reps, std::vector<double> *values)
 {
     if (!_planReady) MSNH_THROW("weights are not loaded");
+    _outputReady = false;
     Plan &plan = *_net->plan;
     static const char *kinds[] = {"conv", "affine", "add", "copy", "maxpool", "avgpool", "upsample", "connected", "input_cast", "yolo_decode", "pad", "slice", "bilinear", "softmax", "col2im"};
     static const char *algos[] = {"auto", "direct", "igemm", "depthwise", "winograd", "stem", "igemm_splitk", "pointwise", "stem+down", "winograd_fused", "mbconv", "igemm+1x1", "igemm_fusedk"};

@@ -228,7 +228,14 @@ class Net:
             pass
 
     def build(self, path):
+        self._fixed = None
         _check(self.L.msnhnet_build(self.h, path.encode()))
+
+    def _result_shape(self):
+        """(batch, values per image of the last layer): asked once per built graph, not on each call"""
+        if getattr(self, "_fixed", None) is None:
+            self._fixed = (self.dims()[0], self.layer_info(self.num_layers() - 1)["outputNum"])
+        return self._fixed
 
     def load(self, path):
         _check(self.L.msnhnet_load(self.h, path.encode()))
@@ -314,25 +321,25 @@ class Net:
 
     def run_classify(self, img):
         x = np.ascontiguousarray(img, np.float32).ravel()
-        b = self.dims()[0]
-        last = self.layer_info(self.num_layers() - 1)
-        out = np.empty(b * last["outputNum"], np.float32)
+        b, per = self._result_shape()
+        out = np.empty(b * per, np.float32)
         n = ctypes.c_longlong()
         _check(self.L.msnhnet_run_classify_gpu(self.h, _fp(x), x.size, _fp(out), out.size, ctypes.byref(n)))
         return out[:n.value].reshape(b, -1)
 
     def _boxes(self, fn, *head):
-        b = self.dims()[0]
+        b = self._result_shape()[0]
         counts = (ctypes.c_int * b)()
         total = ctypes.c_longlong()
         if getattr(self, "_box_buf", None) is None:
             self._box_buf = np.zeros((max(int(self.L.msnhnet_yolo_max_boxes(self.h)), 1), 7), np.float32)
+            self._box_ptr = _fp(self._box_buf)
         boxes = self._box_buf
-        _check(fn(self.h, *head, counts, _fp(boxes), boxes.shape[0], ctypes.byref(total)))
+        _check(fn(self.h, *head, counts, self._box_ptr, boxes.shape[0], ctypes.byref(total)))
         out, at = [], 0
-        for i in range(b):
-            out.append(boxes[at:at + counts[i]].copy())
-            at += counts[i]
+        for n in counts:
+            out.append(boxes[at:at + n].copy())
+            at += n
         return out
 
     def run_yolo(self, img):
@@ -379,9 +386,8 @@ class Net:
         _check(self.L.msnhnet_sync(self.h))
 
     def fetch_classify(self):
-        b = self.dims()[0]
-        last = self.layer_info(self.num_layers() - 1)
-        out = np.empty(b * last["outputNum"], np.float32)
+        b, per = self._result_shape()
+        out = np.empty(b * per, np.float32)
         n = ctypes.c_longlong()
         _check(self.L.msnhnet_fetch_classify(self.h, _fp(out), out.size, ctypes.byref(n)))
         return out[:n.value].reshape(b, -1)

@@ -803,3 +803,21 @@ def test_timing_diagnostics_patch_kernel(tile):
     assert D.msnh_hip_diag_empty_launch(256, 256, None) == 0
     assert D.msnh_hip_diag_empty_launch(0, 256, None) != 0
     abi.check(L.msnh_hip_stream_sync(None))
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 4111, (1 << 20) + 16, (3 << 20) + 7])
+def test_copy_kernel(n):
+    """pinned -> device -> pinned by the copy kernel: every byte arrives, none beyond the end is touched"""
+    import torch
+    import gpuutil as gu
+    gu.init()
+    L = abi.lib()
+    src = torch.randint(0, 256, (n + 16,), dtype=torch.uint8).pin_memory()
+    mid = torch.full((n + 16,), 7, dtype=torch.uint8, device="cuda")
+    back = torch.full((n + 16,), 9, dtype=torch.uint8).pin_memory()
+    gu.sync()
+    abi.check(L.msnh_hip_copy(gu.ptr(mid), gu.ptr(src), n, None))
+    abi.check(L.msnh_hip_copy(gu.ptr(back), gu.ptr(mid), n, None))
+    gu.sync()
+    assert torch.equal(back[:n], src[:n]) and (back[n:] == 9).all() and (mid[n:] == 7).all().item()
+    assert L.msnh_hip_copy(ctypes.c_void_p(mid.data_ptr() + 4), gu.ptr(src), 4, None) != 0
