@@ -35,6 +35,10 @@ int    convDepthwise3x3(const msnh_conv_desc *d, const void *x, const void *w, c
 bool   stemMfmaOk(const msnh_conv_desc *d);
 size_t stemMfmaElems(const msnh_conv_desc *d);
 void   stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed);
+bool   stemMfmaF32Ok(const msnh_conv_desc *d);
+size_t stemMfmaF32Elems(const msnh_conv_desc *d);
+void   stemMfmaF32Pack(const msnh_conv_desc *d, const float *oihw, float *packed);
+int    convStemMfmaF32(const msnh_conv_desc *d, const float *x, const float *wA, const float *scale, const float *shift, float *y, hipStream_t st);
 int    convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, const float *scale, const float *shift, void *y, hipStream_t st);
 
 struct EpiArgs
@@ -333,9 +337,12 @@ static bool depthwiseOk(const msnh_conv_desc *d)
 
 static bool stemOk(const msnh_conv_desc *d)
 {
-    return d->in_c <= 4 && d->groups == 1 && d->dilation == 1 && d->out_c % 32 == 0 && d->out_ld % 4 == 0 &&
+    return d->in_c <= 4 && d->groups == 1 && d->dilation == 1 && (d->out_c % 32 == 0 || stemMfmaOk(d) || stemMfmaF32Ok(d)) && d->out_ld % 4 == 0 &&
            !d->has_residual && static_cast<size_t>(d->ksize) * d->ksize * d->in_c * 32 * 4 <= 60 * 1024;
 }
+
+// float32 values in front of the matrix-core kernel's
+static size_t stemScalarElems(const msnh_conv_desc *d) { return static_cast<size_t>(d->ksize) * d->ksize * d->in_c * d->out_c; }
 
 static bool winogradOk(const msnh_conv_desc *d)
 {
@@ -352,7 +359,7 @@ extern "C" {
 int msnh_hip_conv2d_tile_count(void) { return igemmTileCount(); }
 
 // Bumped whenever msnh_hip_conv2d_pack_weights changes what it writes for some (descriptor, algorithm).
-int msnh_hip_conv2d_pack_layout_version(void) { return 1; }
+int msnh_hip_conv2d_pack_layout_version(void) { return 2; }
 
 int msnh_hip_conv2d_tile_supported(const msnh_conv_desc *d, int tile)
 {
@@ -422,7 +429,7 @@ size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo)
     const size_t cinG = static_cast<size_t>(d->in_c / d->groups);
     if (algo == MSNH_CONV_WINOGRAD || algo == MSNH_CONV_WINOGRAD_FUSED) return static_cast<size_t>(16) * d->out_c * d->in_c;
     // float32 payload for the scalar kernel, followed (float16 plans) by the MFMA operand fragments
-    if (algo == MSNH_CONV_STEM) return kk * d->in_c * d->out_c * (d->dtype == MSNH_F16 ? 2 : 1) + (stemMfmaOk(d) ? stemMfmaElems(d) : 0);
+    if (algo == MSNH_CONV_STEM) return kk * d->in_c * d->out_c * (d->dtype == MSNH_F16 ? 2 : 1) + (stemMfmaOk(d) ? stemMfmaElems(d) : stemMfmaF32Ok(d) ? stemMfmaF32Elems(d) : 0);
     return static_cast<size_t>(d->out_c) * kk * cinG;
 }
 
@@ -462,6 +469,7 @@ int msnh_hip_conv2d_pack_weights(const msnh_conv_desc *d, int algo, const float 
                 for (int t = 0; t < kk; ++t)
                     o[(static_cast<size_t>(t) * d->in_c + ci) * d->out_c + oc] = oihw[(static_cast<size_t>(oc) * d->in_c + ci) * kk + t];
         if (stemMfmaOk(d)) stemMfmaPack(d, oihw, static_cast<_Float16 *>(packed) + static_cast<size_t>(kk) * d->in_c * d->out_c * 2);
+        if (stemMfmaF32Ok(d)) stemMfmaF32Pack(d, oihw, o + stemScalarElems(d));
         return 0;
     }
     case MSNH_CONV_WINOGRAD:
@@ -548,6 +556,8 @@ int msnh_hip_conv2d(const msnh_conv_desc *d, const void *x, const void *w, const
         if (stemMfmaOk(d))
             return convStemMfma(d, static_cast<const float *>(x), static_cast<const _Float16 *>(w) + static_cast<size_t>(d->ksize) * d->ksize * d->in_c * d->out_c * 2,
                                 scale, shift, y, st);
+        if (stemMfmaF32Ok(d))
+            return convStemMfmaF32(d, static_cast<const float *>(x), static_cast<const float *>(w) + stemScalarElems(d), scale, shift, static_cast<float *>(y), st);
         // a lane owns one pixel and OCT output channels: 32 when there are pixels enough to fill the chip, 8 for small images
         // (a single 224 x 224 image gives 98 workgroups at 32 channels per lane, 392 at 8)
 #define MSNH_STEM(TO, OCT)                                                                                              \

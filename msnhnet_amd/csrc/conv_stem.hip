@@ -58,8 +58,8 @@ __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
         reinterpret_cast<f16x8 *>(wl)[i] = reinterpret_cast<const f16x8 *>(a.wA)[i];
     for (int i = threadIdx.x; i < MBLK * 32; i += 256)
     {
-        ssl[i] = a.scale ? a.scale[i] : 1.f;
-        ssl[MBLK * 32 + i] = a.shift ? a.shift[i] : 0.f;
+        ssl[i] = a.scale && i < a.outC ? a.scale[i] : 1.f;
+        ssl[MBLK * 32 + i] = a.shift && i < a.outC ? a.shift[i] : 0.f;
     }
     __syncthreads();
 
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
                 acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wa1, b1, acc[mb], 0, 0, 0);
             }
         });
-        if (ox < a.OW)
+        if (ox < a.OW && (!hi || a.outC > 16))
         {
             f16 *yp = a.y + (static_cast<size_t>(row) * a.OW + ox) * a.outLd + (hi ? 16 : 0);
 #pragma unroll
@@ -214,7 +214,7 @@ struct StemRowsArgs
     const float *scale;
     const float *shift;
     f16         *y;
-    int B, H, W, OH, OW, outLd, stride, pad;
+    int B, H, W, OH, OW, outLd, outC, stride, pad;
     int groupsPerRow, nGroups;
     unsigned xBytes;
     int act;
@@ -233,8 +233,8 @@ __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
         reinterpret_cast<f16x8 *>(wl)[i] = reinterpret_cast<const f16x8 *>(a.wA)[i];
     for (int i = threadIdx.x; i < MBLK * 32; i += 256)
     {
-        ssl[i] = a.scale ? a.scale[i] : 1.f;
-        ssl[MBLK * 32 + i] = a.shift ? a.shift[i] : 0.f;
+        ssl[i] = a.scale && i < a.outC ? a.scale[i] : 1.f;
+        ssl[MBLK * 32 + i] = a.shift && i < a.outC ? a.shift[i] : 0.f;
     }
     __syncthreads();
 
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
                 acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wa, bf, acc[mb], 0, 0, 0);
             }
         });
-        if (ox < a.OW)
+        if (ox < a.OW && (!hi || a.outC > 16))
         {
             f16 *yp = a.y + (static_cast<size_t>(row) * a.OW + ox) * a.outLd + (hi ? 16 : 0);
 #pragma unroll
@@ -358,21 +358,221 @@ inline bool stemRowsOk(const msnh_conv_desc *d)
     return d->ksize == 7 && d->in_c == 3 && static_cast<long long>(d->batch) * 3 * d->in_h * d->in_w * 4 < 0x7fffffffLL;
 }
 
+// ---- float32 networks ---------------------------------------------------------------------------------------------------------------
+// 32x32x2 float32 MFMAs (a lane of the upper half holds the odd K index of a step), 64 clocks per step, block and SIMD: 7x7x3 -> 64 channels of one
+// 224 x 224 image are 1.5 us of matrix-core time.  K is laid out by image rows as above: a step multiplies tap e of two (channel, filter row) pairs, the
+// lower half of the wavefront holding the first pair's value and the upper half the second's, so a lane fetches the taps of its row with one or two
+// 16-byte loads.  (The scalar kernel before it: one LDS broadcast and one FMA per filter value, 22.5 us for that image; K in tap order with a
+// gather per value on the same MFMAs: 17.2; this one: 7.9, five images 54.8 -> 22.8.)  A small image is split over the channel blocks too (grid y), so that every SIMD has a wavefront.
+struct StemF32Args
+{
+    const float *x;
+    const float *wA;        // [mBlocks][ceil(steps / 4)][64 lanes][4]: four K steps per 16 bytes
+    const float *scale;
+    const float *shift;
+    float       *y;
+    int H, W, OH, OW, outLd, outC, stride, pad;
+    int groupsPerRow, nGroups;
+    int act;
+    float actParam, outMul;
+};
+
+constexpr int stemF32Steps(int ks, int cin) { return (cin * ks + 1) / 2 * ks; }
+
+template <int KS, int CIN, int MBLK>
+__global__ __launch_bounds__(256) void convStemMfmaF32Kernel(StemF32Args a)
+{
+    constexpr int ROWS = CIN * KS, CHUNKS = (ROWS + 1) / 2, QUADS = (stemF32Steps(KS, CIN) + 3) / 4;
+    constexpr int GC = 4;                                                          // chunks per group; 4 KS steps are whole quads
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    f32x4 *wl = reinterpret_cast<f32x4 *>(smem);                                  // [MBLK][QUADS][64]
+    float *ssl = reinterpret_cast<float *>(smem + MBLK * QUADS * 1024);            // [2][MBLK*32]
+    const int c0 = static_cast<int>(blockIdx.y) * MBLK * 32;
+    for (int i = threadIdx.x; i < MBLK * QUADS * 64; i += 256) wl[i] = reinterpret_cast<const f32x4 *>(a.wA)[static_cast<size_t>(blockIdx.y) * MBLK * QUADS * 64 + i];
+    for (int i = threadIdx.x; i < MBLK * 32; i += 256)
+    {
+        ssl[i] = a.scale && c0 + i < a.outC ? a.scale[c0 + i] : 1.f;
+        ssl[MBLK * 32 + i] = a.shift && c0 + i < a.outC ? a.shift[c0 + i] : 0.f;
+    }
+    __syncthreads();
+
+    const int lane = threadIdx.x & 63;
+    const int n = lane & 31;
+    const bool hi = lane >= 32;
+    const int nBlocks = static_cast<int>(gridDim.x);
+    const int perXcd = (nBlocks + 7) / 8;
+    const int logical = static_cast<int>(blockIdx.x % 8) * perXcd + static_cast<int>(blockIdx.x / 8);     // (see convStemMfmaKernel)
+    const int perBlock = (a.nGroups + nBlocks - 1) / nBlocks;
+    const int gBegin = logical < nBlocks ? logical * perBlock : a.nGroups;
+    const int gEnd = min(a.nGroups, gBegin + perBlock);
+    const int planes = CIN * a.H * a.W;
+    const bool lin = (a.act == MSNH_ACT_LEAKY || a.act == MSNH_ACT_RELU || a.act == MSNH_ACT_NONE);
+    const float slope = a.act == MSNH_ACT_LEAKY ? a.actParam : (a.act == MSNH_ACT_RELU ? 0.f : 1.f);
+
+    for (int g = gBegin + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)); g < gEnd; g += 4)
+    {
+        const int gx = g % a.groupsPerRow;
+        const int row = g / a.groupsPerRow;
+        const int oy = row % a.OH;
+        const int b = row / a.OH;
+        const int ox = gx * 32 + n;
+        const int iy0 = oy * a.stride - a.pad;
+        const int ix0 = ox * a.stride - a.pad;
+        const __amdgpu_buffer_rsrc_t rx = stemRsrc(a.x + static_cast<size_t>(b) * planes, static_cast<unsigned>(planes) * 4u);
+        const int base = iy0 * a.W + ix0;                          // element index of the window's corner in the image; may be negative
+        f32x16 acc[MBLK];
+#pragma unroll
+        for (int mb = 0; mb < MBLK; ++mb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
+        const int ixFirst = gx * 32 * a.stride - a.pad;
+        const int ixLast  = (gx * 32 + 31) * a.stride - a.pad;
+        const bool interior = iy0 >= 0 && iy0 + KS <= a.H && ixFirst >= 0 && ixLast + KS <= a.W && gx * 32 + 31 < a.OW;
+        // the rows' values are fetched a group of chunks ahead of the MFMAs that use them (all at once they would take the registers of a second wavefront)
+        float v[2][GC][KS];
+        const auto fetch = [&](auto gTag) {
+            constexpr int g0 = decltype(gTag)::value;
+            staticFor<g0 * GC, (g0 + 1) * GC < CHUNKS ? (g0 + 1) * GC : CHUNKS>([&](auto cTag) {
+                constexpr int c = decltype(cTag)::value;
+                constexpr int r0 = 2 * c, r1 = 2 * c + 1 < ROWS ? 2 * c + 1 : 2 * c;  // (a padding pair reads the last row again; its filter values are zero)
+                float (&t)[KS] = v[g0 % 2][c - g0 * GC];
+                const int off = base + (hi ? (r1 / KS * a.H + r1 % KS) * a.W : (r0 / KS * a.H + r0 % KS) * a.W);
+                const unsigned voff = static_cast<unsigned>(off) * 4u;                // a negative index wraps past the end of the buffer: zeros
+                const f32x4 lo4 = stemLoad16(rx, voff);
+                f32x4 hi4 = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (KS > 5) hi4 = stemLoad16(rx, voff + 16u);
+                else if constexpr (KS > 4) hi4[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, static_cast<int>(voff + 16u), 0, 0));
+#pragma unroll
+                for (int e = 0; e < KS; ++e) t[e] = e < 4 ? lo4[e & 3] : hi4[e & 3];
+                if (!interior)
+                {
+                    const bool rowOk = static_cast<unsigned>(iy0 + (hi ? r1 % KS : r0 % KS)) < static_cast<unsigned>(a.H);
+                    if (off < 0 && rowOk)
+                    {
+                        // the first image row of the first plane, left border: the 16-byte vectors would start in front of the tensor
+#pragma unroll
+                        for (int e = 0; e < KS; ++e)
+                            t[e] = off + e >= 0 ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (off + e) * 4, 0, 0)) : 0.f;
+                    }
+#pragma unroll
+                    for (int e = 0; e < KS; ++e) t[e] = (rowOk && static_cast<unsigned>(ix0 + e) < static_cast<unsigned>(a.W)) ? t[e] : 0.f;
+                }
+            });
+        };
+        fetch(std::integral_constant<int, 0>());
+        staticFor<0, (CHUNKS + GC - 1) / GC>([&](auto gTag) {
+            constexpr int g0 = decltype(gTag)::value;
+            if constexpr ((g0 + 1) * GC < CHUNKS) fetch(std::integral_constant<int, g0 + 1>());
+            __builtin_amdgcn_sched_barrier(0);
+            staticFor<g0 * GC * KS / 4, ((g0 + 1) * GC < CHUNKS ? (g0 + 1) * GC * KS / 4 : QUADS)>([&](auto qTag) {
+                constexpr int q = decltype(qTag)::value;
+#pragma unroll
+                for (int mb = 0; mb < MBLK; ++mb)
+                {
+                    const f32x4 w4 = wl[(mb * QUADS + q) * 64 + lane];
+                    staticFor<0, 4>([&](auto eTag) {
+                        constexpr int s = 4 * q + decltype(eTag)::value;
+                        if constexpr (s < CHUNKS * KS) acc[mb] = __builtin_amdgcn_mfma_f32_32x32x2f32(w4[s % 4], v[g0 % 2][s / KS - g0 * GC][s % KS], acc[mb], 0, 0, 0);
+                    });
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if (ox < a.OW && (!hi || a.outC > 16))
+        {
+            float *yp = a.y + (static_cast<size_t>(row) * a.OW + ox) * a.outLd + c0 + (hi ? 16 : 0);
+#pragma unroll
+            for (int mb = 0; mb < MBLK; ++mb)
+            {
+                const float *scp = ssl + mb * 32 + (hi ? 16 : 0);
+                const float *shp = scp + MBLK * 32;
+                float t[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) t[r] = acc[mb][r] * scp[r] + shp[r];
+                if (lin)
+                {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) t[r] = t[r] > 0.f ? t[r] : slope * t[r];
+                }
+                else activateArray<16>(t, a.act, a.actParam);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f32x4 *>(yp + mb * 32 + 4 * q) = f32x4{t[4 * q] * a.outMul, t[4 * q + 1] * a.outMul, t[4 * q + 2] * a.outMul, t[4 * q + 3] * a.outMul};
+            }
+        }
+    }
+}
+
+template <int KS, int CIN, int MBLK>
+int launchStemF32(const StemF32Args &a, unsigned blocks, hipStream_t st)
+{
+    const size_t smem = static_cast<size_t>(MBLK) * ((stemF32Steps(KS, CIN) + 3) / 4) * 1024 + 2 * MBLK * 32 * sizeof(float);
+    auto kern = convStemMfmaF32Kernel<KS, CIN, MBLK>;
+    if (smem > 48 * 1024)
+    {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
+        if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
+    }
+    hipLaunchKernelGGL(kern, dim3((blocks + 7) / 8 * 8, static_cast<unsigned>((a.outC + 31) / (32 * MBLK))), dim3(256), smem, st, a);
+    MSNH_LAUNCH_CHECK();
+    return 0;
+}
+
+// where K index k = tap * Cin + ci lies: offset inside one image's planes, and its filter row and column
+inline void stemTaps(const msnh_conv_desc *d, int *koff, int *kyx)
+{
+    const int K = d->ksize * d->ksize * d->in_c;
+    for (int k = 0; k < kStemMaxK; ++k)
+    {
+        const int tap = k / d->in_c, ci = k % d->in_c;
+        const int ky = tap / d->ksize, kx = tap % d->ksize;
+        koff[k] = k < K ? (ci * d->in_h + ky) * d->in_w + kx : 0;
+        kyx[k] = k < K ? ky << 8 | kx : 32767 << 8;
+    }
+}
+
+inline int stemMBlocks(const msnh_conv_desc *d) { return (d->out_c + 31) / 32; }
 inline int stemKBlocks(const msnh_conv_desc *d) { return (d->ksize * d->ksize * d->in_c + 31) / 32; }
 
 } // namespace
 
 bool stemMfmaOk(const msnh_conv_desc *d)
 {
-    const int mb = d->out_c / 32;
+    const int mb = d->out_c / 32;              // (16 channels: half a block, the other half of its rows zero)
     return d->dtype == MSNH_F16 && d->out_dtype == MSNH_F16 && (d->ksize == 3 || d->ksize == 5 || d->ksize == 7) && d->in_c >= 1 && d->in_c <= 4 &&
-           d->ksize * d->ksize * d->in_c <= kStemMaxK && d->groups == 1 && d->dilation == 1 && d->out_c % 32 == 0 && (mb == 1 || mb == 2 || mb == 4) &&
+           d->ksize * d->ksize * d->in_c <= kStemMaxK && d->groups == 1 && d->dilation == 1 && (d->out_c == 16 || (d->out_c % 32 == 0 && (mb == 1 || mb == 2 || mb == 4))) &&
            d->out_ld % 8 == 0 && !d->has_residual && d->in_h < 30000;
+}
+
+bool stemMfmaF32Ok(const msnh_conv_desc *d)
+{
+    return d->dtype == MSNH_F32 && d->out_dtype == MSNH_F32 && (d->ksize == 3 || d->ksize == 5 || d->ksize == 7) && d->in_c >= 1 && d->in_c <= 4 &&
+           d->ksize * d->ksize * d->in_c <= kStemMaxK && d->groups == 1 && d->dilation == 1 && (d->out_c == 16 || d->out_c % 32 == 0) && d->out_ld % 4 == 0 && !d->has_residual &&
+           d->in_h < 30000 && static_cast<long long>(d->in_c) * d->in_h * d->in_w * 4 < 0x7fffffffLL;
+}
+
+size_t stemMfmaF32Elems(const msnh_conv_desc *d) { return static_cast<size_t>(stemMBlocks(d)) * ((stemF32Steps(d->ksize, d->in_c) + 3) / 4) * 256; }
+
+// packed[mb][step / 4][lane][step % 4] = W[channel(mb, lane % 32)][ci][ky][kx], kx = step % ksize, (ci, ky) = pair 2 * (step / ksize) + lane / 32
+void stemMfmaF32Pack(const msnh_conv_desc *d, const float *oihw, float *packed)
+{
+    const int ks = d->ksize, steps = stemF32Steps(ks, d->in_c), quads = (steps + 3) / 4;
+    for (int mb = 0; mb < stemMBlocks(d); ++mb)
+        for (int s = 0; s < quads * 4; ++s)
+            for (int lane = 0; lane < 64; ++lane)
+            {
+                const int m = lane % 32;
+                const int oc = mb * 32 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
+                const int pair = 2 * (s / ks) + lane / 32;
+                const bool real = s < steps && pair < d->in_c * ks && oc < d->out_c;
+                packed[(static_cast<size_t>(mb * quads + s / 4) * 64 + lane) * 4 + s % 4] =
+                    real ? oihw[((static_cast<size_t>(oc) * d->in_c + pair / ks) * ks + pair % ks) * ks + s % ks] : 0.f;
+            }
 }
 
 size_t stemMfmaElems(const msnh_conv_desc *d)
 {
-    return static_cast<size_t>(d->out_c / 32) * (stemRowsOk(d) ? kRowChunks : stemKBlocks(d) * 2) * 64 * 8;
+    return static_cast<size_t>(stemMBlocks(d)) * (stemRowsOk(d) ? kRowChunks : stemKBlocks(d) * 2) * 64 * 8;
 }
 
 // packed[mb][kb16][lane][e] = W[channel(mb, lane % 32)][k = kb16*16 + 8*(lane/32) + e], k = tap*Cin + ci
@@ -382,7 +582,7 @@ void stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed)
     if (stemRowsOk(d))
     {
         // packed[mb][chunk][lane][e] = W[channel(mb, lane % 32)][ci][ky][kx = e], (ci, ky) = pair 2 * chunk + lane / 32
-        for (int mb = 0; mb < d->out_c / 32; ++mb)
+        for (int mb = 0; mb < stemMBlocks(d); ++mb)
             for (int c = 0; c < kRowChunks; ++c)
                 for (int lane = 0; lane < 64; ++lane)
                     for (int e = 0; e < 8; ++e)
@@ -391,12 +591,12 @@ void stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed)
                         const int oc = mb * 32 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
                         const int pair = 2 * c + lane / 32;
                         float v = 0.f;
-                        if (pair < 21 && e < 7) v = oihw[(static_cast<size_t>(oc) * 3 + pair / 7) * 49 + (pair % 7) * 7 + e];
+                        if (pair < 21 && e < 7 && oc < d->out_c) v = oihw[(static_cast<size_t>(oc) * 3 + pair / 7) * 49 + (pair % 7) * 7 + e];
                         packed[((static_cast<size_t>(mb) * kRowChunks + c) * 64 + lane) * 8 + e] = static_cast<_Float16>(v);
                     }
         return;
     }
-    for (int mb = 0; mb < d->out_c / 32; ++mb)
+    for (int mb = 0; mb < stemMBlocks(d); ++mb)
         for (int kb = 0; kb < KB2; ++kb)
             for (int lane = 0; lane < 64; ++lane)
                 for (int e = 0; e < 8; ++e)
@@ -405,7 +605,7 @@ void stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed)
                     const int oc = mb * 32 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
                     const int k = kb * 16 + 8 * (lane / 32) + e;
                     float v = 0.f;
-                    if (k < K)
+                    if (k < K && oc < d->out_c)
                     {
                         const int tap = k / cin, ci = k % cin;
                         v = oihw[(static_cast<size_t>(oc) * cin + ci) * kk + tap];
@@ -428,7 +628,7 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
         MSNH_REQUIRE(groups < (1LL << 31), "conv2d: stem tensor too large");
         r.nGroups = static_cast<int>(groups);
         r.xBytes = static_cast<unsigned>(static_cast<long long>(d->batch) * 3 * d->in_h * d->in_w * 4);
-        r.act = d->act; r.actParam = d->act_param; r.outMul = d->out_mul;
+        r.outC = d->out_c; r.act = d->act; r.actParam = d->act_param; r.outMul = d->out_mul;
         for (int p = 0; p < 2 * kRowChunks; ++p)
         {
             r.rowOff[p] = p < 21 ? ((p / 7) * d->in_h + p % 7) * d->in_w : 0;
@@ -436,7 +636,7 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
         }
         const long long want = (groups + 3) / 4;
         const unsigned blocks = static_cast<unsigned>(want < 256 * 4 ? (want < 1 ? 1 : want) : 256 * 4);     // (2..8 workgroups per CU measure alike)
-        switch (d->out_c / 32)
+        switch (stemMBlocks(d))
         {
         case 1: return launchStemRows<1>(r, blocks, st);
         case 2: return launchStemRows<2>(r, blocks, st);
@@ -452,21 +652,10 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
     MSNH_REQUIRE(groups < (1LL << 31) && static_cast<long long>(d->in_c) * d->in_h * d->in_w < (1LL << 31), "conv2d: stem tensor too large");
     a.nGroups = static_cast<int>(groups);
     a.act = d->act; a.actParam = d->act_param; a.outMul = d->out_mul;
-    const int K = d->ksize * d->ksize * d->in_c;
-    for (int k = 0; k < kStemMaxK; ++k)
-    {
-        if (k < K)
-        {
-            const int tap = k / d->in_c, ci = k % d->in_c;
-            const int ky = tap / d->ksize, kx = tap % d->ksize;
-            a.koff[k] = (ci * d->in_h + ky) * d->in_w + kx;
-            a.kyx[k] = ky << 8 | kx;
-        }
-        else { a.koff[k] = 0; a.kyx[k] = 32767 << 8; }
-    }
+    stemTaps(d, a.koff, a.kyx);
     // several wavefronts per SIMD hide the gather latency; every wavefront walks the pixel groups with a grid stride
     const long long want = (groups + 3) / 4;
-    const int kb = stemKBlocks(d), mb = d->out_c / 32;
+    const int kb = stemKBlocks(d), mb = stemMBlocks(d);
     const long long cap = 256 * (kb <= 2 ? 8 : 4);             // measured: short K wants more wavefronts in flight
     const unsigned blocks = static_cast<unsigned>(want < cap ? (want < 1 ? 1 : want) : cap);
 #define MSNH_STEM(KBV, MBV) if (kb == KBV && mb == MBV) return launchStem<KBV, MBV>(a, blocks, st)
@@ -475,6 +664,32 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
     MSNH_STEM(3, 1); MSNH_STEM(3, 2); MSNH_STEM(3, 4);
     MSNH_STEM(4, 1); MSNH_STEM(4, 2); MSNH_STEM(4, 4);
     MSNH_STEM(5, 1); MSNH_STEM(5, 2); MSNH_STEM(5, 4);
+#undef MSNH_STEM
+    setError("conv2d: stem shape not instantiated");
+    return 2;
+}
+
+int convStemMfmaF32(const msnh_conv_desc *d, const float *x, const float *wA, const float *scale, const float *shift, float *y, hipStream_t st)
+{
+    MSNH_REQUIRE(stemMfmaF32Ok(d), "conv2d: shape not supported by the matrix-core stem kernel");
+    MSNH_REQUIRE(reinterpret_cast<uintptr_t>(y) % 16 == 0 && reinterpret_cast<uintptr_t>(wA) % 16 == 0, "conv2d: stem needs 16-byte aligned output and weights");
+    StemF32Args a;
+    a.x = x; a.wA = wA; a.scale = scale; a.shift = shift; a.y = y;
+    a.H = d->in_h; a.W = d->in_w; a.OH = d->out_h; a.OW = d->out_w; a.outLd = d->out_ld; a.outC = d->out_c;
+    a.stride = d->stride; a.pad = d->pad;
+    a.groupsPerRow = (d->out_w + 31) / 32;
+    const long long groups = static_cast<long long>(d->batch) * d->out_h * a.groupsPerRow;
+    MSNH_REQUIRE(groups < (1LL << 31), "conv2d: stem tensor too large");
+    a.nGroups = static_cast<int>(groups);
+    a.act = d->act; a.actParam = d->act_param; a.outMul = d->out_mul;
+    const long long want = (groups + 3) / 4;
+    const unsigned blocks = static_cast<unsigned>(want < 256 * 4 ? (want < 1 ? 1 : want) : 256 * 4);
+    // two channel blocks per wavefront share a gather where that still leaves two wavefronts per SIMD
+    const int ks = d->ksize, cin = d->in_c, mb = d->out_c % 64 == 0 && groups * (d->out_c / 64) >= 2048 ? 2 : 1;
+#define MSNH_STEM(KSV, CV) if (ks == KSV && cin == CV) return mb == 2 ? launchStemF32<KSV, CV, 2>(a, blocks, st) : launchStemF32<KSV, CV, 1>(a, blocks, st)
+    MSNH_STEM(3, 1); MSNH_STEM(3, 2); MSNH_STEM(3, 3); MSNH_STEM(3, 4);
+    MSNH_STEM(5, 1); MSNH_STEM(5, 2); MSNH_STEM(5, 3); MSNH_STEM(5, 4);
+    MSNH_STEM(7, 1); MSNH_STEM(7, 2); MSNH_STEM(7, 3);
 #undef MSNH_STEM
     setError("conv2d: stem shape not instantiated");
     return 2;

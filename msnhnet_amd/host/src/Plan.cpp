@@ -226,56 +226,55 @@ void Plan::fuse()
             break;
         }
     }
-    // (g) float16: network input -> four slices that take every second row and column -> concatenation of the four -> 3x3 convolution (the
+    // (g) network input -> four slices that take every second row and column -> concatenation of the four -> 3x3 convolution (the
     // focus opening of YOLOv5): the rows 2y - 2 .. 2y + 3 of the input meet in one output row, so the convolution reads the input itself as
     // a 7x7 convolution of stride 2 and padding 3 whose first filter row and column are zero -- the first-layer kernel takes that.  Ten
-    // launches and 140 us (three images of 544 x 544) become one.
-    if (computeDtype == MSNH_F16)
-        for (PlanOp &conv : ops)
+    // launches and 140 us (float16, three images of 544 x 544) become one of 17 us.
+    for (PlanOp &conv : ops)
+    {
+        if (conv.dead || conv.kind != PlanOp::CONV || conv.ksize != 3 || conv.stride != 1 || conv.pad != 1 || conv.dilation != 1 || conv.groups != 1 || conv.in1 >= 0) continue;
+        const PlanTensor &out = tensors[static_cast<size_t>(conv.out)];
+        const PlanTensor &joined = tensors[static_cast<size_t>(conv.in0)];
+        if (joined.pinned || consumerCount(conv.in0) != 1 || out.dtype != computeDtype || out.layout != PlanTensor::NHWC) continue;
+        int at[4] = {-1, -1, -1, -1}, image = -1;
+        std::vector<PlanOp *> gone;
+        bool ok = true;
+        for (PlanOp &cp : ops)
         {
-            if (conv.dead || conv.kind != PlanOp::CONV || conv.ksize != 3 || conv.stride != 1 || conv.pad != 1 || conv.dilation != 1 || conv.groups != 1 || conv.in1 >= 0) continue;
-            const PlanTensor &out = tensors[static_cast<size_t>(conv.out)];
-            const PlanTensor &joined = tensors[static_cast<size_t>(conv.in0)];
-            if (joined.pinned || consumerCount(conv.in0) != 1 || out.dtype != MSNH_F16 || out.layout != PlanTensor::NHWC) continue;
-            int at[4] = {-1, -1, -1, -1}, image = -1;
-            std::vector<PlanOp *> gone;
-            bool ok = true;
-            for (PlanOp &cp : ops)
-            {
-                if (cp.dead || cp.out != conv.in0) continue;
-                const int p = cp.kind == PlanOp::COPY ? producerOf(cp.in0) : -1;
-                ok = ok && p >= 0 && consumerCount(cp.in0) == 1 && !tensors[static_cast<size_t>(cp.in0)].pinned;
-                if (!ok) break;
-                PlanOp &sl = ops[static_cast<size_t>(p)];
-                ok = sl.kind == PlanOp::SLICE && (image < 0 || sl.in0 == image) && sl.slice[0] == 0 && sl.slice[1] == 1 && sl.slice[3] == 2 && sl.slice[5] == 2 &&
-                     sl.slice[2] < 2 && sl.slice[4] < 2;
-                if (!ok) break;
-                image = sl.in0;
-                at[sl.slice[2] * 2 + sl.slice[4]] = cp.dstChanOffset;
-                gone.push_back(&sl);
-                gone.push_back(&cp);
-            }
-            if (!ok || gone.size() != 8 || *std::min_element(at, at + 4) < 0) continue;
-            const int cast = producerOf(image);
-            const PlanTensor &img = tensors[static_cast<size_t>(image)];
-            if (cast < 0 || ops[static_cast<size_t>(cast)].kind != PlanOp::INPUT_CAST || img.pinned || img.h % 2 != 0 || img.w % 2 != 0 || consumerCount(image) != 4) continue;
-            msnh_conv_desc d;
-            std::memset(&d, 0, sizeof(d));
-            d.dtype = d.out_dtype = MSNH_F16;
-            d.batch = img.n; d.in_h = img.h; d.in_w = img.w; d.in_c = d.in_ld = img.c;
-            d.out_c = out.c; d.out_h = out.h; d.out_w = out.w; d.out_ld = (out.c + 7) / 8 * 8;
-            d.ksize = 7; d.stride = 2; d.pad = 3; d.dilation = 1; d.groups = 1;
-            // (packed filters beyond the scalar kernel's: the matrix-core first-layer kernel takes the shape; the scalar one would lose)
-            if (msnh_hip_conv2d_select_algo(&d) != MSNH_CONV_STEM ||
-                msnh_hip_conv2d_packed_weight_elems(&d, MSNH_CONV_STEM) <= static_cast<size_t>(49) * img.c * out.c * 2)
-                continue;
-            gone.push_back(&ops[static_cast<size_t>(cast)]);
-            for (PlanOp *op : gone) op->dead = true;
-            conv.in0 = ops[static_cast<size_t>(cast)].in0;
-            conv.ksize = 7; conv.stride = 2; conv.pad = 3;
-            std::copy(at, at + 4, conv.focusAt);
-            break;
+            if (cp.dead || cp.out != conv.in0) continue;
+            const int p = cp.kind == PlanOp::COPY ? producerOf(cp.in0) : -1;
+            ok = ok && p >= 0 && consumerCount(cp.in0) == 1 && !tensors[static_cast<size_t>(cp.in0)].pinned;
+            if (!ok) break;
+            PlanOp &sl = ops[static_cast<size_t>(p)];
+            ok = sl.kind == PlanOp::SLICE && (image < 0 || sl.in0 == image) && sl.slice[0] == 0 && sl.slice[1] == 1 && sl.slice[3] == 2 && sl.slice[5] == 2 &&
+                 sl.slice[2] < 2 && sl.slice[4] < 2;
+            if (!ok) break;
+            image = sl.in0;
+            at[sl.slice[2] * 2 + sl.slice[4]] = cp.dstChanOffset;
+            gone.push_back(&sl);
+            gone.push_back(&cp);
         }
+        if (!ok || gone.size() != 8 || *std::min_element(at, at + 4) < 0) continue;
+        const int cast = producerOf(image);
+        const PlanTensor &img = tensors[static_cast<size_t>(image)];
+        if (cast < 0 || ops[static_cast<size_t>(cast)].kind != PlanOp::INPUT_CAST || img.pinned || img.h % 2 != 0 || img.w % 2 != 0 || consumerCount(image) != 4) continue;
+        msnh_conv_desc d;
+        std::memset(&d, 0, sizeof(d));
+        d.dtype = d.out_dtype = computeDtype;
+        d.batch = img.n; d.in_h = img.h; d.in_w = img.w; d.in_c = d.in_ld = img.c;
+        d.out_c = out.c; d.out_h = out.h; d.out_w = out.w; d.out_ld = (out.c + 7) / 8 * 8;
+        d.ksize = 7; d.stride = 2; d.pad = 3; d.dilation = 1; d.groups = 1;
+        // (packed filters beyond the scalar kernel's: the matrix-core first-layer kernel takes the shape; the scalar one would lose)
+        if (msnh_hip_conv2d_select_algo(&d) != MSNH_CONV_STEM ||
+            msnh_hip_conv2d_packed_weight_elems(&d, MSNH_CONV_STEM) <= static_cast<size_t>(49) * img.c * out.c * (computeDtype == MSNH_F16 ? 2 : 1))
+            continue;
+        gone.push_back(&ops[static_cast<size_t>(cast)]);
+        for (PlanOp *op : gone) op->dead = true;
+        conv.in0 = ops[static_cast<size_t>(cast)].in0;
+        conv.ksize = 7; conv.stride = 2; conv.pad = 3;
+        std::copy(at, at + 4, conv.focusAt);
+        break;
+    }
     // (c) float16: first layer (3x3 stride 1, 32 filters, over the NCHW network input) -> 3x3 stride-2 convolution that is its only
     // consumer: one launch; the full-resolution 32-channel tensor between them stays on the chip (it keeps its place in the tensor
     // list: its calibrated scale is the scale of the values in LDS)

@@ -283,6 +283,25 @@ def test_conv_stem(h, w, oc, k, stride, pad, out_dtype):
     assert gu.rel_err(y, ref) <= (1e-5 if out_dtype == abi.F32 else 1e-3)
 
 
+@pytest.mark.parametrize("dtype,b,c,h,w,oc,k,stride,pad", [(abi.F16, 2, 3, 33, 31, 16, 3, 1, 1), (abi.F16, 1, 3, 21, 70, 16, 7, 2, 3), (abi.F16, 1, 1, 9, 40, 16, 5, 1, 2),
+                                                          (abi.F32, 1, 1, 9, 40, 32, 3, 1, 1), (abi.F32, 2, 3, 33, 31, 16, 3, 1, 1), (abi.F32, 2, 2, 17, 33, 96, 5, 2, 2), (abi.F32, 1, 4, 40, 64, 32, 3, 1, 0),
+                                                          (abi.F32, 9, 3, 96, 96, 128, 7, 1, 3)])
+def test_conv_stem_channel_counts(dtype, b, c, h, w, oc, k, stride, pad):
+    """half a block of filters (float16), 1 to 4 input channels, one and two blocks per wavefront and blocks that the grid deals out (float32)"""
+    import gpuutil as gu
+    rng = np.random.default_rng(oc + k + c)
+    x, wt = _case(rng, b, c, h, w, oc, k)
+    if dtype == abi.F16:
+        x, wt = gu.round_f16(x), gu.round_f16(wt)
+    scale = rng.uniform(0.5, 1.5, oc).astype(np.float32)
+    shift = (rng.standard_normal(oc) * 0.1).astype(np.float32)
+    print("stem", dtype, b, c, h, w, oc, k, flush=True)
+    y, used = gu.conv2d(x, wt, dtype=dtype, stride=stride, pad=pad, scale=scale, shift=shift, act="mish", out_mul=0.5, out_ld=oc + 8)
+    assert used == "stem"
+    ref = _ref(x, wt, stride, pad, 1, 1, scale, shift, "mish", 0.1, None, "none", 1.0, 0.5)
+    assert gu.rel_err(y, ref) <= (1e-5 if dtype == abi.F32 else 1e-3)
+
+
 @pytest.mark.parametrize("b,c,h,w,oc", [(2, 16, 12, 10, 24), (1, 32, 19, 19, 64), (3, 8, 7, 9, 8), (1, 64, 38, 38, 128)])
 @pytest.mark.parametrize("with_res", [False, True])
 def test_conv_winograd(b, c, h, w, oc, with_res):
