@@ -459,15 +459,17 @@ size_t msnh_hip_yolo_nms_static_max_bytes(void);
 int msnh_hip_yolo_nms_static(int batch, int classes, const float *rows, int cand_cap, const int *cand_cnt, float nms_thresh, float *kept,
                              int kept_cap, int *kept_cnt, msnh_stream_t s);
 
-/* The NMS of every image whose candidates are at most msnh_hip_yolo_nms_images_cap() = 1024 in one launch (a workgroup per image), results in
+/* The NMS of every image whose candidates are at most msnh_hip_yolo_nms_images_cap() = 1024, in two launches, results in
  * output order: what msnh_hip_yolo_nms followed by the reference's ordering of its records gives (src/layers/MsnhYoloOutLayer.cpp:175-194
  * and :381-461).  rows / cand_cap / cand_cnt as for msnh_hip_yolo_nms; cand_cnt is set to zero again.  out_rows: [batch][1024][8] float32,
  * the kept rows of image b from out_rows + b * 8192 on; out_hdr: int32 [batch][4] = { candidates found, rows kept, flag, 0 }, flag != 0:
  * more than 1024 candidates (1) or a NaN score (2), no rows were written and the caller runs the procedure itself.  Both are 16-byte
- * aligned memory that the device can write, device memory or pinned host memory. */
+ * aligned memory that the device can write, device memory or pinned host memory.  workspace: _workspace_bytes() bytes, 16-byte aligned, zero before
+ * its first use; calls that share one follow each other on one stream. */
 int msnh_hip_yolo_nms_images_cap(void);
+size_t msnh_hip_yolo_nms_images_workspace_bytes(int batch);
 int msnh_hip_yolo_nms_images(int batch, const float *rows, int cand_cap, int *cand_cnt, float nms_thresh, float *out_rows, int *out_hdr,
-                             msnh_stream_t s);
+                             void *workspace, size_t workspace_bytes, msnh_stream_t s);
 
 /* Matrix-core ceiling probe (measurement only, no counterpart in the reference): every SIMD runs `iters` rounds of four independent
  * 32x32x16 float16 MFMAs per wavefront with waves_per_simd (1..8) wavefronts resident, no memory traffic.  Reports the rate

@@ -2,6 +2,7 @@
 // the objectness threshold.  The NHWC head tensor already stores the (5+classes) values of one anchor of
 // one pixel contiguously, so both the read and the write of a wavefront are contiguous runs.
 #include "common.hpp"
+#include <algorithm>
 #include <mutex>
 
 namespace msnh {
@@ -923,36 +924,19 @@ __global__ __launch_bounds__(256) void yoloNmsScanKernel(const unsigned long lon
 // What a detector's real scenes give: tens to some hundreds of candidates per image.  The launches above serve them badly -- a workgroup
 // per (class, image) of which all but a few are empty, one barrier per kept box (169 kept boxes of one class: 171 us), three further
 // launches from 257 members up (722 members: 105 us in all), records in no order behind a counter that has to be cleared first and
-// copied back.  Here the workgroup holds one candidate per lane:
-//   1. bitonic sort by (class, objectness, score, cell): partners less than a wavefront apart exchange registers, the others go through LDS;
-//   2. for every pair of 64-member chunks with a class in common, a word per member of the later one: which members of the earlier one would
-//      erase it (one wavefront per pair of chunks, lane = victim);
-//   3. the first wavefront walks the chunks: a member is out if one of its words meets a kept member of an earlier chunk, the rest of the
+// copied back.  Here an image takes two launches, whose pair-wise work is spread over many CUs:
+//   1. yoloNmsRankKernel: a member's place in the order (class, objectness, score, cell) is the number of members above it; 64 members per
+//      workgroup, the others dealt to its wavefronts; corners, class and key go to the member's place in the workspace;
+//   2. yoloNmsImageKernel, a wavefront per pair of 64-member chunks with a class in common: a word per member of the later chunk, which members
+//      of the earlier one would erase it.  The workgroup of an image that finishes last goes on alone:
+//   3. its first wavefront walks the chunks: a member is out if one of its words meets a kept member of an earlier chunk, the rest of the
 //      chunk is resolved by fixed-point iteration on its own words (bit masks only, no barrier);
 //   4. the classes ordered by their best (score, cell), rows written where the reference's output has them -- straight into the caller's
 //      pinned memory when it passes such -- and the image's candidate counter reset for the next forward.
-// Bound by the instruction issue of the one CU in steps 1 and 2; 27 us for 338 candidates of one class and 64 us for 722, launch included,
-// where the launches above took 181 and 114 (trace) plus four copies and two stream hand-overs.
+// One workgroup for all of it, with a bitonic sort for step 1, was bound by the instruction issue of its CU: 64 us for 722 candidates of one
+// class and 27 us for 338; the two launches take 30 and 22 us (14 for a single candidate, the timing events included).
 constexpr int NMS_IMG = 1024;
 constexpr int NMS_IMG_LDS = (NMS_IMG / 64) * (NMS_IMG / 64 + 1) / 2 * 64 * 8;      // one word per member and chunk at or before its own
-
-// The value of lane ^ J, without LDS: quad permutes, mirrors of half rows (lane ^ 7) and rows (lane ^ 15), row and half-wave swaps.
-template <int J>
-__device__ __forceinline__ unsigned xorLane(unsigned v)
-{
-    const int x = static_cast<int>(v);
-    if (J == 1) return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);
-    if (J == 2) return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);
-    if (J == 4) return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, x, 0x1B, 0xf, 0xf, false), 0x141, 0xf, 0xf, false);
-    if (J == 8) return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, false), 0x140, 0xf, 0xf, false);
-    if (J == 16)
-    {
-        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-        return (threadIdx.x & 16) ? r[0] : r[1];
-    }
-    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return (threadIdx.x & 32) ? r[0] : r[1];
-}
 
 // iouAbove(kept, victim) for the lanes with `mine`, without a branch unless some lane's quotient stands next to the threshold.
 __device__ __forceinline__ bool iouAboveFlat(const float4 &k, float karea, const float4 &j, float jarea, float thr, bool mine)
@@ -975,133 +959,118 @@ __device__ __forceinline__ bool iouAboveFlat(const float4 &k, float karea, const
     return hit;
 }
 
-struct NmsKey
+// An image's part of the workspace.
+struct NmsImageWs
 {
-    unsigned long long hi, lo;
-    unsigned ix;
+    unsigned arrived, bad;                                         // zero between calls
+    unsigned pad[14];
+    float4 corner[NMS_IMG];                                        // members in order
+    unsigned long long lo[NMS_IMG];                                // score, cell
+    int cls[NMS_IMG];
+    unsigned row[NMS_IMG];
+    unsigned long long erasedBy[NMS_IMG_LDS / 8];                  // [c (c + 1) / 2 + rc][64], rc <= c
 };
 
-__device__ __forceinline__ void nmsSortStep(NmsKey &e, const NmsKey &o, int j, int k2)
+struct __attribute__((aligned(16))) NmsKey
 {
-    const bool less = e.hi < o.hi || (e.hi == o.hi && (e.lo < o.lo || (e.lo == o.lo && e.ix > o.ix)));
-    const bool wantMax = ((threadIdx.x & j) == 0) == ((threadIdx.x & k2) == 0);
-    if (less == wantMax) e = o;
-}
+    unsigned long long hi, lo;
+};
 
-template <int J>
-__device__ __forceinline__ void nmsSortLanes(NmsKey &e, int k2)
+__global__ __launch_bounds__(NMS_IMG) void yoloNmsRankKernel(const float *__restrict__ rows, int candCap, const int *__restrict__ candCnt, NmsImageWs *__restrict__ ws)
 {
-    NmsKey o;
-    o.hi = (static_cast<unsigned long long>(xorLane<J>(static_cast<unsigned>(e.hi >> 32))) << 32) | xorLane<J>(static_cast<unsigned>(e.hi));
-    o.lo = (static_cast<unsigned long long>(xorLane<J>(static_cast<unsigned>(e.lo >> 32))) << 32) | xorLane<J>(static_cast<unsigned>(e.lo));
-    o.ix = xorLane<J>(e.ix);
-    nmsSortStep(e, o, J, k2);
+#pragma clang fp contract(off)
+    __shared__ NmsKey key[NMS_IMG];
+    __shared__ int above[64];
+    const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int found = candCnt[b];
+    const int n = found < candCap ? found : candCap;
+    const int i0 = static_cast<int>(blockIdx.x) * 64;
+    if (n > NMS_IMG || i0 >= n) return;
+    const float *r = rows + static_cast<size_t>(b) * candCap * 8;
+    if (tid < n)
+    {
+        const float4 q = *reinterpret_cast<const float4 *>(r + static_cast<size_t>(tid) * 8 + 4);    // objectness, class score, class, cell
+        const float score = q.x * q.y;
+        if (!(score == score) || !(q.x == q.x)) ws[b].bad = 1u;
+        // (class numbers are not negative)
+        key[tid].hi = (static_cast<unsigned long long>(~static_cast<unsigned>(static_cast<int>(q.z))) << 32) | orderedBits(q.x);
+        key[tid].lo = (static_cast<unsigned long long>(orderedBits(score)) << 32) | ~static_cast<unsigned>(q.w);
+    }
+    if (tid < 64) above[tid] = 0;
+    __syncthreads();
+    const int i = i0 + lane;
+    const NmsKey mine = key[i < n ? i : n - 1];
+    // this wavefront's share of the others: [j0, j1)
+    const int per = (n + NMS_IMG / 64 - 1) / (NMS_IMG / 64), j0 = wave * per, j1 = j0 + per < n ? j0 + per : n;
+    int count = 0;
+#pragma unroll 4
+    for (int j = j0; j < j1; ++j)
+    {
+        const NmsKey o = key[j];
+        const bool higher = o.hi > mine.hi || (o.hi == mine.hi && (o.lo > mine.lo || (o.lo == mine.lo && j < i)));
+        count += higher ? 1 : 0;
+    }
+    atomicAdd(&above[lane], count);
+    __syncthreads();
+    if (tid < 64 && i < n)
+    {
+        const int at = above[tid];
+        const float4 q = *reinterpret_cast<const float4 *>(r + static_cast<size_t>(i) * 8);
+        ws[b].corner[at] = make_float4(q.x - q.z / 2.f, q.y - q.w / 2.f, q.x + q.z / 2.f, q.y + q.w / 2.f);
+        ws[b].lo[at] = mine.lo;
+        ws[b].cls[at] = static_cast<int>(~static_cast<unsigned>(mine.hi >> 32));
+        ws[b].row[at] = static_cast<unsigned>(i);
+    }
 }
 
 __global__ __launch_bounds__(NMS_IMG) void yoloNmsImageKernel(const float *__restrict__ rows, int candCap, int *__restrict__ candCnt, float thr,
-                                                              float *__restrict__ outRows, int *__restrict__ outHdr)
+                                                              NmsImageWs *__restrict__ ws, float *__restrict__ outRows, int *__restrict__ outHdr)
 {
 #pragma clang fp contract(off)
     constexpr int NW = NMS_IMG / 64;
-    __shared__ unsigned long long hiS[NMS_IMG], loS[NMS_IMG];      // sort exchange; afterwards hiS: the best key of a class segment
-    __shared__ unsigned ixS[NMS_IMG];                              // row of a sorted member
-    __shared__ float4 corner[NMS_IMG];                             // sorted members
+    __shared__ unsigned long long segTop[NMS_IMG];                 // the best key of a class segment
+    __shared__ float4 corner[NMS_IMG];
     __shared__ float area[NMS_IMG];
-    __shared__ int seg[NMS_IMG];                                   // class segment of a sorted member
+    __shared__ int seg[NMS_IMG];                                   // class of a member; later its class segment
     __shared__ int segStart[NMS_IMG + 1], segOut[NMS_IMG];         // first kept member of a segment; where its rows go
     __shared__ unsigned short keptPos[NMS_IMG];
-    __shared__ int heads[NW], nKept, bad;
-    extern __shared__ __attribute__((aligned(16))) unsigned long long erasedBy[];      // [c (c + 1) / 2 + rc][64], rc <= c
-    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ int heads[NW], nKept, last;
+    extern __shared__ __attribute__((aligned(16))) unsigned long long erasedBy[];      // the image's words, in its last workgroup
+    const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int found = candCnt[b];
     const int n = found < candCap ? found : candCap;
     const float *r = rows + static_cast<size_t>(b) * candCap * 8;
     int *hdr = outHdr + b * 4;
+    NmsImageWs &w = ws[b];
     if (n == 0 || n > NMS_IMG)
     {
+        // (a workgroup that arrives after the counter's reset reads zero candidates and leaves here)
         __syncthreads();                                           // every lane has read the counter
-        if (tid == 0)
+        if (tid == 0 && blockIdx.x == 0)
         {
             *reinterpret_cast<int4 *>(hdr) = make_int4(found, 0, n > NMS_IMG ? 1 : 0, 0);
             candCnt[b] = 0;
         }
         return;
     }
-    if (tid == 0) bad = 0;
-    __syncthreads();
-    NmsKey e = {0ull, 0ull, static_cast<unsigned>(tid)};           // below every real key (class numbers are not negative)
+    const int W = (n + 63) / 64, items = W * (W + 1) / 2;
+    const int item = static_cast<int>(blockIdx.x) * NW + wave;
+    if (static_cast<int>(blockIdx.x) * NW >= items) return;
+    int cls = 0;
     if (tid < n)
     {
-        const float4 q = *reinterpret_cast<const float4 *>(r + static_cast<size_t>(tid) * 8 + 4);    // objectness, class score, class, cell
-        const float score = q.x * q.y;
-        if (!(score == score) || !(q.x == q.x)) bad = 1;
-        e.hi = (static_cast<unsigned long long>(~static_cast<unsigned>(static_cast<int>(q.z))) << 32) | orderedBits(q.x);
-        e.lo = (static_cast<unsigned long long>(orderedBits(score)) << 32) | ~static_cast<unsigned>(q.w);
-    }
-    int S = 64;
-    while (S < n) S <<= 1;
-    for (int k2 = 2; k2 <= S; k2 <<= 1)
-    {
-        for (int j = k2 >> 1; j >= 64; j >>= 1)
-        {
-            __syncthreads();
-            if (tid < S) { hiS[tid] = e.hi; loS[tid] = e.lo; ixS[tid] = e.ix; }
-            __syncthreads();
-            if (tid < S) nmsSortStep(e, {hiS[tid ^ j], loS[tid ^ j], ixS[tid ^ j]}, j, k2);
-        }
-        if (tid >= S) continue;
-        if (k2 > 32) nmsSortLanes<32>(e, k2);
-        if (k2 > 16) nmsSortLanes<16>(e, k2);
-        if (k2 > 8) nmsSortLanes<8>(e, k2);
-        if (k2 > 4) nmsSortLanes<4>(e, k2);
-        if (k2 > 2) nmsSortLanes<2>(e, k2);
-        nmsSortLanes<1>(e, k2);
-    }
-    const unsigned long long hi = e.hi, lo = e.lo;
-    const int ix = static_cast<int>(e.ix);
-    __syncthreads();
-    if (bad)
-    {
-        if (tid == 0)
-        {
-            *reinterpret_cast<int4 *>(hdr) = make_int4(found, 0, 2, 0);
-            candCnt[b] = 0;
-        }
-        return;
-    }
-    hiS[tid] = hi;
-    ixS[tid] = ix;
-    if (tid < n)
-    {
-        const float4 q = *reinterpret_cast<const float4 *>(r + static_cast<size_t>(ix) * 8);
-        const float ax1 = q.x - q.z / 2.f, ax2 = q.x + q.z / 2.f, ay1 = q.y - q.w / 2.f, ay2 = q.y + q.w / 2.f;
-        corner[tid] = make_float4(ax1, ay1, ax2, ay2);
-        area[tid] = (ax2 - ax1 + 1) * (ay2 - ay1 + 1);
+        const float4 k = w.corner[tid];
+        corner[tid] = k;
+        area[tid] = (k.z - k.x + 1) * (k.w - k.y + 1);
+        cls = w.cls[tid];
+        seg[tid] = cls;
     }
     __syncthreads();
-    const bool head = tid < n && (tid == 0 || (hiS[tid - 1] >> 32) != (hi >> 32));
-    const unsigned long long headMask = __ballot(head);
-    if (lane == 0) heads[wave] = __popcll(headMask);
-    __syncthreads();
-    int before = 0, nSeg = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-    {
-        before += w < wave ? heads[w] : 0;
-        nSeg += heads[w];
-    }
-    const int mySeg = before + __popcll(headMask & ((2ull << lane) - 1ull)) - 1;       // (2 << 63 wraps to 0: every lane up to 63)
-    seg[tid] = mySeg;
-    unsigned long long *segTop = hiS;
-    segTop[tid] = 0ull;                                            // (the neighbour's key was read before the last barrier)
-    __syncthreads();
-    if (tid < n) atomicMax(&segTop[mySeg], lo);
-    const int W = (n + 63) / 64;
     // Boxes more than a unit apart in x or y have no intersection (inter = 0, never above a threshold >= 0): most pairs, decided for the
     // whole wavefront by four comparisons.  The margin of 2 instead of the "+ 1" of the extents keeps the skip on the safe side of any
     // rounding; a comparison with a NaN corner is false, which does not skip.
     const bool skipOk = thr >= 0.f;
-    for (int item = __builtin_amdgcn_readfirstlane(wave); item < W * (W + 1) / 2; item += NW)
+    if (item < items)
     {
         int c = 0;
         while ((c + 1) * (c + 2) / 2 <= item) ++c;
@@ -1109,7 +1078,7 @@ __global__ __launch_bounds__(NMS_IMG) void yoloNmsImageKernel(const float *__res
         const int j = c * 64 + lane, jSafe = j < n ? j : n - 1;
         const int i0 = rc * 64, iEnd = n - i0 < 64 ? n - i0 : 64;
         unsigned long long word = 0ull;
-        if (seg[i0 + iEnd - 1] >= seg[c * 64])                     // (segments ascend: else no class in common)
+        if (seg[i0 + iEnd - 1] >= seg[c * 64])                     // (classes ascend: else none in common)
         {
             const float4 jc = corner[jSafe];
             const float ja = area[jSafe];
@@ -1145,8 +1114,51 @@ __global__ __launch_bounds__(NMS_IMG) void yoloNmsImageKernel(const float *__res
                 todo &= todo - 1ull;
             }
         }
-        erasedBy[item * 64 + lane] = word;
+        __hip_atomic_store(&w.erasedBy[item * 64 + lane], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    // the last workgroup of the image goes on (the words are stored past the L2, which other XCDs do not share, and complete before a workgroup
+    // counts itself in)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0)
+    {
+        const unsigned groups = static_cast<unsigned>((items + NW - 1) / NW);
+        last = __hip_atomic_fetch_add(&w.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1 ? 1 : 0;
+    }
+    __syncthreads();
+    if (!last) return;
+    const unsigned bad = w.bad;
+    __syncthreads();
+    if (tid == 0)
+    {
+        __hip_atomic_store(&w.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        w.bad = 0u;
+    }
+    if (bad)
+    {
+        if (tid == 0)
+        {
+            *reinterpret_cast<int4 *>(hdr) = make_int4(found, 0, 2, 0);
+            candCnt[b] = 0;
+        }
+        return;
+    }
+    for (int k = tid; k < items * 64; k += NMS_IMG) erasedBy[k] = __hip_atomic_load(&w.erasedBy[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool head = tid < n && (tid == 0 || seg[tid - 1] != cls);
+    const unsigned long long headMask = __ballot(head);
+    if (lane == 0) heads[wave] = __popcll(headMask);
+    segTop[tid] = 0ull;
+    __syncthreads();
+    int before = 0, nSeg = 0;
+#pragma unroll
+    for (int v = 0; v < NW; ++v)
+    {
+        before += v < wave ? heads[v] : 0;
+        nSeg += heads[v];
+    }
+    const int mySeg = before + __popcll(headMask & ((2ull << lane) - 1ull)) - 1;       // (2 << 63 wraps to 0: every lane up to 63)
+    seg[tid] = mySeg;
+    if (tid < n) atomicMax(&segTop[mySeg], w.lo[tid]);
     __syncthreads();
     if (wave == 0)
     {
@@ -1198,7 +1210,7 @@ __global__ __launch_bounds__(NMS_IMG) void yoloNmsImageKernel(const float *__res
     if (tid < picks)
     {
         const int at = keptPos[tid], s = seg[at];
-        const float4 *q = reinterpret_cast<const float4 *>(r + static_cast<size_t>(ixS[at]) * 8);
+        const float4 *q = reinterpret_cast<const float4 *>(r + static_cast<size_t>(w.row[at]) * 8);
         float4 *o = reinterpret_cast<float4 *>(outRows + (static_cast<size_t>(b) * NMS_IMG + segOut[s] + tid - segStart[s]) * 8);
         o[0] = q[0];
         o[1] = q[1];
@@ -1562,11 +1574,15 @@ extern "C" int msnh_hip_yolo_nms(int batch, int classes, const float *rows, int 
 
 extern "C" int msnh_hip_yolo_nms_images_cap(void) { return NMS_IMG; }
 
+extern "C" size_t msnh_hip_yolo_nms_images_workspace_bytes(int batch) { return batch > 0 ? static_cast<size_t>(batch) * sizeof(NmsImageWs) : 0; }
+
 extern "C" int msnh_hip_yolo_nms_images(int batch, const float *rows, int cand_cap, int *cand_cnt, float nms_thresh, float *out_rows, int *out_hdr,
-                                        msnh_stream_t s)
+                                        void *workspace, size_t workspace_bytes, msnh_stream_t s)
 {
     MSNH_REQUIRE(batch > 0 && batch <= 65535 && cand_cap > 0 && cand_cap <= (1 << 24), "yolo_nms_images: bad geometry");
-    MSNH_REQUIRE(rows && cand_cnt && out_rows && out_hdr, "yolo_nms_images: NULL pointer");
+    MSNH_REQUIRE(rows && cand_cnt && out_rows && out_hdr && workspace, "yolo_nms_images: NULL pointer");
+    MSNH_REQUIRE(workspace_bytes >= msnh_hip_yolo_nms_images_workspace_bytes(batch) && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+                 "yolo_nms_images: workspace too small (msnh_hip_yolo_nms_images_workspace_bytes) or not 16-byte aligned");
     MSNH_REQUIRE(reinterpret_cast<uintptr_t>(rows) % 16 == 0 && reinterpret_cast<uintptr_t>(out_rows) % 16 == 0 && reinterpret_cast<uintptr_t>(out_hdr) % 16 == 0,
                  "yolo_nms_images: rows, out_rows and out_hdr must be 16-byte aligned");
     int dev = -1;
@@ -1575,7 +1591,12 @@ extern "C" int msnh_hip_yolo_nms_images(int batch, const float *rows, int cand_c
         std::lock_guard<std::mutex> lock(g_nmsMutex);
         MSNH_REQUIRE(ensureNmsAttributes(g_nms[dev]), "%s", g_nms[dev].error);
     }
-    hipLaunchKernelGGL(yoloNmsImageKernel, dim3(batch), dim3(NMS_IMG), NMS_IMG_LDS, resolveStream(s), rows, cand_cap, cand_cnt, nms_thresh, out_rows, out_hdr);
+    const unsigned most = static_cast<unsigned>(std::min(NMS_IMG, cand_cap)), chunks = (most + 63) / 64;
+    NmsImageWs *ws = static_cast<NmsImageWs *>(workspace);
+    hipLaunchKernelGGL(yoloNmsRankKernel, dim3(chunks, batch), dim3(NMS_IMG), 0, resolveStream(s), rows, cand_cap, cand_cnt, ws);
+    MSNH_LAUNCH_CHECK();
+    hipLaunchKernelGGL(yoloNmsImageKernel, dim3((chunks * (chunks + 1) / 2 + NMS_IMG / 64 - 1) / (NMS_IMG / 64), batch), dim3(NMS_IMG), NMS_IMG_LDS, resolveStream(s), rows, cand_cap,
+                       cand_cnt, nms_thresh, ws, out_rows, out_hdr);
     MSNH_LAUNCH_CHECK();
     return 0;
 }

@@ -138,6 +138,7 @@ public:
     // candidate counts and rows, one set per copy-back slot: a forward writes the set of its own slot, so what an earlier forward left
     // for the host or the NMS is read in place while the next one runs
     DeviceBuffer yoloCandCnt[2], yoloRows[2];
+    DeviceBuffer yoloNmsWs;                 // msnh_hip_yolo_nms_images: zeroed when allocated
     int yoloSlot = 0;                       // the set that the launches issued now write
     int   *candCnt() const { return yoloCandCnt[yoloSlot].as<int>(); }
     float *candRows() const { return yoloRows[yoloSlot].as<float>(); }

@@ -370,8 +370,8 @@ public:
     // placement with the shorter time between results stays.
     static int deviceNms;
     static const int kDeviceNmsFew = 2048;
-    // Up to kImageNms candidates per image (msnh_hip_yolo_nms_images_cap) the NMS is the last launch of the forward itself: one workgroup
-    // per image takes about as long as the copies and stream hand-overs that a stream of its own would need.
+    // Up to kImageNms candidates per image (msnh_hip_yolo_nms_images_cap) the NMS is the last two launches of the forward itself, which
+    // take less time than the copies and stream hand-overs that a stream of its own would need.
     static const int kImageNms = 1024;
     static const int kDeviceNmsCandidates = 6144;
     static const int kTrialBatches = 16;

@@ -1433,7 +1433,8 @@ void YoloOutLayer::enqueueImageNms(msnh_stream_t s, int slot)
 {
     Plan &pl = *plan;
     Slot &sl = _slots[slot & 1];
-    MSNH_DEV(msnh_hip_yolo_nms_images(_batch, pl.candRows(), pl.yoloCells, pl.candCnt(), _nmsThresh, sl.imageRows.as<float>(), sl.imageHdr.as<int>(), s));
+    MSNH_DEV(msnh_hip_yolo_nms_images(_batch, pl.candRows(), pl.yoloCells, pl.candCnt(), _nmsThresh, sl.imageRows.as<float>(), sl.imageHdr.as<int>(),
+                                      pl.yoloNmsWs.ptr(), pl.yoloNmsWs.bytes(), s));
 }
 
 // Everything a slot needs, at its full size, before the slot is first used.  An allocation or a free of device or pinned memory

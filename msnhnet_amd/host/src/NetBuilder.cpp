@@ -388,6 +388,9 @@ static void setupYoloBuffers(Plan &plan, int batch)
         plan.yoloCandCnt[k].alloc(sizeof(int) * static_cast<size_t>(std::max(batch, 64)));
         plan.yoloRows[k].alloc(sizeof(float) * 8 * cells * static_cast<size_t>(batch));
     }
+    plan.yoloNmsWs.alloc(msnh_hip_yolo_nms_images_workspace_bytes(batch));
+    MSNH_DEV(msnh_hip_fill_zero(plan.yoloNmsWs.ptr(), plan.yoloNmsWs.bytes(), nullptr));
+    MSNH_DEV(msnh_hip_stream_sync(nullptr));
     plan.findYoloHeads();
 }
 

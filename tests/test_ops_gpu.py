@@ -626,7 +626,7 @@ def test_yolo_nms():
 
 @pytest.mark.parametrize("classes,spread", [(1, 120.0), (3, 300.0), (90, 60.0), (1, 1e4)])
 def test_yolo_nms_images(classes, spread):
-    """one-launch NMS per image against the host procedure, rows bit for bit and in output order: candidate counts around the chunk and
+    """two-launch NMS per image against the host procedure, rows bit for bit and in output order: candidate counts around the chunk and
     sort sizes, ties in both sort keys, infinite boxes; 1025 candidates and a NaN score are flagged; the counters come back zero"""
     import gpuutil as gu
     from msnhnet_amd import netapi
@@ -646,9 +646,14 @@ def test_yolo_nms_images(classes, spread):
     rd, cd = gu.dev(rows), gu.dev(np.array(counts, np.int32))
     out = torch.full((len(counts), abi.lib().msnh_hip_yolo_nms_images_cap(), 8), -7.0).cuda()
     hdr = torch.full((len(counts), 4), -7, dtype=torch.int32).cuda()
+    ws = torch.zeros(abi.lib().msnh_hip_yolo_nms_images_workspace_bytes(len(counts)), dtype=torch.uint8).cuda()
     gu.sync()
-    abi.check(abi.lib().msnh_hip_yolo_nms_images(len(counts), gu.ptr(rd), cap, gu.ptr(cd), 0.45, gu.ptr(out), gu.ptr(hdr), None))
-    gu.sync()
+    for again in range(2):                  # (the second call finds the workspace as the first left it)
+        out.fill_(-7.0)
+        cd.copy_(torch.tensor(counts, dtype=torch.int32))
+        gu.sync()
+        abi.check(abi.lib().msnh_hip_yolo_nms_images(len(counts), gu.ptr(rd), cap, gu.ptr(cd), 0.45, gu.ptr(out), gu.ptr(hdr), gu.ptr(ws), ws.numel(), None))
+        gu.sync()
     assert not cd.cpu().numpy().any()
     for b, (n, h) in enumerate(zip(counts, hdr.cpu().numpy())):
         assert h[0] == n and h[2] == (1 if n > 1024 else 2 if b == 14 else 0), (b, h)
