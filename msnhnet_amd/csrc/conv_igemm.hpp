@@ -532,6 +532,44 @@ __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&a
     igemmEpilogue<T, TOut, BM, BN, 64, 32>(a, mine, smemRaw, chScale, chShift, m0, p0, wm, wn * 2 + kg, wave, lane, g, ss, stageOwn);
 }
 
+// Epilogue of the kernels whose four wavefronts multiplied different k-blocks of the one wave tile: wavefront 0 adds what the others park in LDS
+// and finishes alone (the tile is small: 1024 or 2048 results).
+template <int BM, int BN> constexpr size_t igemmGatherLds() { return (static_cast<size_t>(3) * BM * BN + 2 * BM) * sizeof(float); }       // (fusedK: a flag behind it)
+
+template <typename T, typename TOut, int BM, int BN>
+__device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (&acc)[BM / 32][BN / 32], unsigned char *smemRaw, float chScale, float chShift,
+                                                    int m0, int p0, int wave, int lane, int g, int tileIdx, int nTiles)
+{
+    constexpr int MB = BM / 32, NB = BN / 32;
+    float *xch = reinterpret_cast<float *>(smemRaw);
+    float *ss  = xch + 3 * BM * BN;
+    const int tid = wave * 64 + lane;
+    if (tid < BM) { ss[tid] = chScale; ss[BM + tid] = chShift; }
+    if (wave > 0)
+        staticFor<0, MB * NB>([&](auto ijTag) {
+            constexpr int ij = decltype(ijTag)::value;
+            float *put = xch + (wave - 1) * BM * BN + ij * 1024 + lane;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) put[r * 64] = acc[ij / NB][ij % NB][r];
+        });
+    __syncthreads();
+    if (wave == 0)
+        for (int k = 0; k < 3; ++k)
+            staticFor<0, MB * NB>([&](auto ijTag) {
+                constexpr int ij = decltype(ijTag)::value;
+                const float *get = xch + k * BM * BN + ij * 1024 + lane;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[ij / NB][ij % NB][r] += get[r * 64];
+            });
+    if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, 1, lane, reinterpret_cast<int *>(ss + 2 * BM))) return;
+    if (wave > 0) return;
+    // (the parked sums are in registers before the staging writes reach their region: one wavefront's LDS accesses are served in order)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    igemmEpilogue<T, TOut, BM, BN, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, 0, 0, 0, lane, g, ss, xch);
+}
+
 // Register budget: two workgroups per CU (one wave of each per SIMD) so that one workgroup's barrier and epilogue
 // are covered by the other's MFMAs; smaller tiles, which serve the short-K bandwidth-bound layers, get three to six.
 constexpr int igemmWavesPerSimd(int bm, int bn, int kv = 8, int ns = 3, int nw = 4)
@@ -834,11 +872,12 @@ __device__ __forceinline__ void igemmTailEpilogue(const IgemmArgs &a, f32x16 (&a
 
 // KG = 2: two groups of wavefronts share the WM x WN grid of (then 64 x 64) wave tiles and split the k-blocks of every tile step
 // between them, which takes a third off the LDS fragment reads per MFMA against 32 x 64 wave tiles of the same workgroup tile.
+// KG = 4: the four wavefronts multiply one k-block each of every step for the workgroup's only wave tile.
 // TAIL = 1: the epilogue also computes the 1x1 convolution that reads this one's result (igemmTailEpilogue); float16 only.
 template <typename T, typename TOut, int BM, int BN, int KV, int WM, int WN, int NS, int KG = 1, int TAIL = 0>
 __global__ __launch_bounds__(64 * WM * WN * KG)
-__attribute__((amdgpu_waves_per_eu(KG == 2 ? (WM * WN * KG) / 4 : igemmWavesPerSimd(BM, BN, KV, NS, WM * WN),
-                                   KG == 2 ? (WM * WN * KG == 4 ? 3 : (WM * WN * KG) / 4) : igemmWavesPerSimd(BM, BN, KV, NS, WM * WN))))
+__attribute__((amdgpu_waves_per_eu(KG == 4 ? 1 : KG == 2 ? (WM * WN * KG) / 4 : igemmWavesPerSimd(BM, BN, KV, NS, WM * WN),
+                                   KG == 4 ? 4 : KG == 2 ? (WM * WN * KG == 4 ? 3 : (WM * WN * KG) / 4) : igemmWavesPerSimd(BM, BN, KV, NS, WM * WN))))
 void convIgemmKernel(IgemmArgs a)
 {
     typedef typename Frag<T>::V V;
@@ -863,7 +902,7 @@ void convIgemmKernel(IgemmArgs a)
     constexpr int A_BYTES = BML * ROWB;
     constexpr unsigned STAGE = (BML + BNL) * ROWB; // one LDS stage: A rows, then B rows
     static_assert(TM % 32 == 0 && TN % 32 == 0 && (NT == 256 || NT == 512 || NT == 768) && S % 2 == 0, "wave grid");
-    static_assert(KG == 1 || (KG == 2 && TM == 64 && TN == 64), "the K-split variant works on 64 x 64 wave tiles");
+    static_assert(KG == 1 || (KG == 2 && TM == 64 && TN == 64) || (KG == 4 && NWT == 1), "the K-split variants work on 64 x 64 wave tiles or on one wave tile");
     static_assert(NS >= 2 && NS <= 8, "LDS stages");
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smemRaw[];
@@ -1117,11 +1156,13 @@ void convIgemmKernel(IgemmArgs a)
         e.y = a.ws + static_cast<size_t>(blockIdx.y) * a.P * a.wsLd;
         e.outLd = a.wsLd;
         e.vecOk = (a.wsLd % 8 == 0) && (a.coutG % 8 == 0 || gridDim.z == 1);
-        if constexpr (KG == 2) igemmEpilogueSwap<T, float, BM, BN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64);
+        if constexpr (KG == 4) igemmEpilogueGather<T, float, BM, BN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wave, lane, g, 0, 0);
+        else if constexpr (KG == 2) igemmEpilogueSwap<T, float, BM, BN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64);
         else igemmEpilogue<T, float, BM, BN, TM, TN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wm, wn, wave, lane, g);
         return;
     }
-    if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles);
+    if constexpr (KG == 4) igemmEpilogueGather<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wave, lane, g, tileIdx, nTiles);
+    else if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles);
     else if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + igemmEpilogueLds<BM, TM, NT / 64>()))) return;
     else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g);
 }
@@ -1182,6 +1223,13 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         setError("conv2d: the implicit GEMM needs at most 64 filter taps and tensors below 2 GiB");
         return 3;
     }
+    // Below 1024 products per result a float16 tile has at most eight k-steps, so parking and adding the three partial tiles costs what the smaller tile
+    // saves (level with 64 x 64), and float16 results keep one summation order over all tiles there.  float32 steps take half the channels: no line.
+    if (KG == 4 && sizeof(T) == 2 && a.taps * a.cinG < 1024)
+    {
+        setError("conv2d: this tile needs float32 tensors or a float16 convolution of at least 1024 products per result");
+        return 3;
+    }
     constexpr int RPP = 64 * WM * WN * KG / KV;
     const size_t smemLoop = static_cast<size_t>(NS) * ((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16;
     size_t smemEpi = 0;
@@ -1190,7 +1238,7 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         constexpr unsigned STAGE = static_cast<unsigned>(((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16);
         smemEpi = TailLds<BM, BN, STAGE>::bytes();
     }
-    else smemEpi = std::max(igemmEpilogueLds<BM, BM / WM, WM * WN * KG>(), KG == 2 ? igemmSwapLds<WM * WN * KG, BM>() : size_t(0));
+    else smemEpi = std::max(igemmEpilogueLds<BM, BM / WM, WM * WN * KG>(), KG == 4 ? igemmGatherLds<BM, BN>() : KG == 2 ? igemmSwapLds<WM * WN * KG, BM>() : size_t(0));
     if (a.fusedK > 1) smemEpi += 16;                  // the flag of splitKCombine
     const size_t smem = smemLoop > smemEpi ? smemLoop : smemEpi;
     a.mTiles = (a.coutG + BM - 1) / BM;
@@ -1257,8 +1305,8 @@ namespace msnh {
 // Tile configurations (BM x BN output tile, KV 16-byte vectors of K per step, WM x WN wavefront grid).
 // Index 0 is "choose for me"; the others can be forced through msnh_conv_desc::tile, which is how the host
 // library's per-layer search picks the fastest one at load time.
-constexpr int kIgemmTiles = 68;
-constexpr int kIgemmTailTileFirst = 67;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
+constexpr int kIgemmTiles = 71;
+constexpr int kIgemmTailTileFirst = 70;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
 
 // One translation unit instantiates every third configuration of one type pair (tile % kIgemmParts == PART), so that they compile in parallel.
 constexpr int kIgemmParts = 3;
@@ -1356,23 +1404,29 @@ int igemmDispatch(IgemmArgs &a, int groups, int tile, hipStream_t st)
     case 64: if constexpr (64 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 16, 2, 2, 3>(a, groups, st); else break;
     case 65: if constexpr (65 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 2, 4, 4>(a, groups, st); else break;
     case 66: if constexpr (66 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 4, 2, 4>(a, groups, st); else break;
+    // 32 x 32 and 32 x 64 with the k-blocks of a step dealt to the four wavefronts: a 32 x 32 tile is a quarter of the work of 64 x 64 for its CU,
+    // so the layers of one small picture fill the chip with a third of the slices -- and of the partial sums -- that 64 x 64 needs, or with none.
+    // float32, one 224 x 224 picture: 3x3 64 -> 64 at 56 x 56 10.5 -> 8.7 us, 256 -> 256 at 14 x 14 14.7 -> 10.9, 512 -> 512 at 7 x 7 17.3 -> 12.6
+    case 67: if constexpr (67 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 32, 16, 1, 1, 3, 4>(a, groups, st); else break;
+    case 68: if constexpr (68 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 32, 16, 1, 1, 2, 4>(a, groups, st); else break;
+    case 69: if constexpr (69 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 64, 16, 1, 1, 2, 4>(a, groups, st); else break;
     // tiles whose epilogue also computes the 1x1 convolution that follows (msnh_hip_conv2d_tail only; float16): the tile holds every
     // output channel of the first convolution (at most 256 / 128)
-    case 67:
-    case 68:
+    case 70:
+    case 71:
         if constexpr (!(std::is_same<T, f16>::value && std::is_same<TOut, f16>::value))
         {
             setError("conv2d: this tile needs float16 tensors and a 1x1 convolution behind it (msnh_hip_conv2d_tail)");
             return 3;
         }
-        else if constexpr (67 % kIgemmParts == PART)
+        else if constexpr (70 % kIgemmParts == PART)
         {
-            if (tile == 67) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
+            if (tile == 70) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
             break;
         }
-        else if constexpr (68 % kIgemmParts == PART)
+        else if constexpr (71 % kIgemmParts == PART)
         {
-            if (tile == 68) return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
+            if (tile == 71) return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
             break;
         }
         else break;

@@ -1214,7 +1214,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         // the tiles that came out best uncut and on the small ones, which win most of these layers; the library refuses what cannot help.
         if (baseAlgo == MSNH_CONV_IGEMM && !op.up2)
         {
-            std::vector<int> tiles = {6, 12, 30, 64, 65, 66};
+            std::vector<int> tiles = {6, 12, 64, 66, 67, 68};
             std::vector<Cand> plain = cands;
             std::sort(plain.begin(), plain.end(), [](const Cand &x, const Cand &y) { return x.ms < y.ms; });
             for (size_t i = 0; i < plain.size() && i < 6; ++i)

@@ -437,7 +437,7 @@ def test_conv_fused_k(case, dtype):
     assert L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), 12) == 0          # a tile without slices is not this algorithm
     ws = torch.zeros(64 << 20, dtype=torch.uint8).cuda()
     tried = 0
-    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66):
+    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66, 67, 68, 69):
         for slices in (2, 3, 7, 16):
             d.tile = tile + 256 * slices
             need = L.msnh_hip_conv2d_workspace_bytes(ctypes.byref(d), algo)
