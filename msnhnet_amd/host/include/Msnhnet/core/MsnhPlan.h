@@ -140,6 +140,9 @@ public:
     DeviceBuffer yoloCandCnt[2], yoloRows[2];
     DeviceBuffer yoloNmsWs;                 // msnh_hip_yolo_nms_images: zeroed when allocated
     int yoloSlot = 0;                       // the set that the launches issued now write
+    // The set's counts are zero on the device (a forward that suppresses its own candidates leaves them so).  Every launch that appends candidates drops
+    // the flag, whoever issues it: launch() sees them all but a replayed graph's, whose caller drops it.
+    bool countsClear[2] = {false, false};
     int   *candCnt() const { return yoloCandCnt[yoloSlot].as<int>(); }
     float *candRows() const { return yoloRows[yoloSlot].as<float>(); }
     void clearCandidates(msnh_stream_t s);  // the counts of the current set to zero: the start of every forward

@@ -156,7 +156,6 @@ private:
     // The captured forward.  Detectors have one per copy-back slot and per place of the NMS (inside the forward or behind it), captured
     // when first needed; [0][0] is the only one of a classifier.
     msnh_graph_t  _graphs[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
-    bool _countsClear[2] = {false, false};     // the slot's candidate counts are zero on the device (the NMS inside a forward leaves them so)
     void dropGraphs();
     void issueForward(YoloOutLayer *yout, bool inForward, msnh_stream_t s);
     int _nextSlot = 0, _inFlight = 0;          // copy-back slots of the detection post-processing

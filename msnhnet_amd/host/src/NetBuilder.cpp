@@ -672,7 +672,8 @@ void NetBuilder::enqueueForward(const float *deviceInput)
     const int slot = yout ? _nextSlot : 0;
     const bool inForward = yout && yout->nmsInForward();
     plan.yoloSlot = slot;
-    if (inForward && !_countsClear[slot]) plan.clearCandidates(_stream);
+    if (inForward && !plan.countsClear[slot]) plan.clearCandidates(_stream);
+    plan.countsClear[slot] = false;             // (a replayed graph appends as well; until the forward that leaves zero behind is on its way)
     static const bool eager = std::getenv("MSNH_EAGER") != nullptr;
     msnh_graph_t &graph = _graphs[slot][inForward ? 1 : 0];
     if (eager) issueForward(yout, inForward, _stream);
@@ -695,7 +696,7 @@ void NetBuilder::enqueueForward(const float *deviceInput)
     _outputReady = outputBytes() > 0;
     if (yout)
     {
-        _countsClear[slot] = inForward;
+        plan.countsClear[slot] = inForward;
         // results leave the device right behind the forward, so the next forward can start while the host sorts
         yout->enqueueCopyBack(_stream, slot, inForward);
         _nextSlot ^= 1;
@@ -729,7 +730,6 @@ void NetBuilder::dropGraphs()
     for (auto &perSlot : _graphs)
         for (msnh_graph_t &g : perSlot)
             if (g) { msnh_hip_graph_destroy(g); g = nullptr; }
-    _countsClear[0] = _countsClear[1] = false;
 }
 
 void NetBuilder::sync() { MSNH_DEV(msnh_hip_stream_sync(_stream)); }

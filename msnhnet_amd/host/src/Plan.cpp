@@ -1489,6 +1489,7 @@ void Plan::launch(PlanOp &op, msnh_stream_t s)
         const int per = 5 + op.classes;
         float *decoded = yoloDecoded.as<float>() + static_cast<size_t>(op.cellBase) * per;
         const bool cand = op.confThresh < 1.5f;
+        if (cand) countsClear[yoloSlot] = false;
         if (sparseYolo && cand && !yoloHeadOps.empty())
         {
             // all heads in one launch, issued where the last of them stands in the plan (nothing between the heads reads their lists)
