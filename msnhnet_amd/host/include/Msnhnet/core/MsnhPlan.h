@@ -136,13 +136,26 @@ public:
     int  yoloClasses = 0;
     DeviceBuffer yoloDecoded, yoloCandIdx;
     // candidate counts and rows, one set per copy-back slot: a forward writes the set of its own slot, so what an earlier forward left
-    // for the host or the NMS is read in place while the next one runs
-    DeviceBuffer yoloCandCnt[2], yoloRows[2];
+    // for the host or the NMS is read in place while the next one runs.  The third set belongs to launches outside the forwards (SideRun).
+    DeviceBuffer yoloCandCnt[3], yoloRows[3];
     DeviceBuffer yoloNmsWs;                 // msnh_hip_yolo_nms_images: zeroed when allocated
     int yoloSlot = 0;                       // the set that the launches issued now write
     // The set's counts are zero on the device (a forward that suppresses its own candidates leaves them so).  Every launch that appends candidates drops
     // the flag, whoever issues it: launch() sees them all but a replayed graph's, whose caller drops it.
-    bool countsClear[2] = {false, false};
+    bool countsClear[3] = {false, false, false};
+    // Runs of single launches outside the forwards (the profiles, the headroom check): while one of these lives the heads append to a set of their own,
+    // empty at its start, so that neither the counts a forward starts from nor the rows of a result that nobody has fetched yet change.
+    class SideRun
+    {
+    public:
+        SideRun(Plan &plan, msnh_stream_t s);
+        ~SideRun() { _plan.yoloSlot = _slot; }
+        SideRun(const SideRun &) = delete;
+        SideRun &operator=(const SideRun &) = delete;
+    private:
+        Plan &_plan;
+        int _slot;
+    };
     int   *candCnt() const { return yoloCandCnt[yoloSlot].as<int>(); }
     float *candRows() const { return yoloRows[yoloSlot].as<float>(); }
     void clearCandidates(msnh_stream_t s);  // the counts of the current set to zero: the start of every forward

@@ -344,6 +344,7 @@ public:
     void enqueueImageNms(msnh_stream_t s, int slot);       // device: NMS of every image, kept boxes straight into the slot's pinned memory
     void enqueueCopyBack(msnh_stream_t s, int slot, bool inForward);   // device -> pinned host, asynchronous (inForward: enqueueImageNms has done it)
     void finish(int slot);                                 // host: wait, sort, NMS -> finalOut
+    bool outstanding(int slot) const { return _slots[slot & 1].pending; }   // enqueueCopyBack without a finish()
 
     static std::vector<YoloBox> nms(const std::vector<YoloBox> &bboxes, const float &nmsThresh, const bool &useSoftNms, const float &sigma = 0.3f);
     // hard NMS with the same result as nms(), restructured for speed (see the definition)

@@ -618,6 +618,8 @@ static std::vector<float> yoloLayerDump(Plan &plan, const YoloLayer *yl, const P
 void NetBuilder::runLayersEager()
 {
     Plan &plan = *_net->plan;
+    // (the layers run into the first slot: not while a result in it is on its way)
+    if (_net->layers.back()->type() == LayerType::YOLO_OUT && static_cast<YoloOutLayer *>(_net->layers.back())->outstanding(0)) MSNH_THROW("fetch the outstanding results first");
     _outputReady = false;
     plan.yoloSlot = 0;
     plan.clearCandidates(_stream);
@@ -955,6 +957,7 @@ float NetBuilder::profileOps(int kind, int reps, int *launches, double *flops, d
     if (!_planReady) MSNH_THROW("weights are not loaded");
     _outputReady = false;
     Plan &plan = *_net->plan;
+    Plan::SideRun side(plan, _stream);
     msnh_event_t e0 = nullptr, e1 = nullptr;
     MSNH_DEV(msnh_hip_event_create(&e0));
     MSNH_DEV(msnh_hip_event_create(&e1));
@@ -990,6 +993,7 @@ std::string NetBuilder::profileEachOp(int reps, std::vector<double> *values)
     if (!_planReady) MSNH_THROW("weights are not loaded");
     _outputReady = false;
     Plan &plan = *_net->plan;
+    Plan::SideRun side(plan, _stream);
     static const char *kinds[] = {"conv", "affine", "add", "copy", "maxpool", "avgpool", "upsample", "connected", "input_cast", "yolo_decode", "pad", "slice", "bilinear", "softmax", "col2im"};
     static const char *algos[] = {"auto", "direct", "igemm", "depthwise", "winograd", "stem", "igemm_splitk", "pointwise", "stem+down", "winograd_fused", "mbconv", "igemm+1x1", "igemm_fusedk"};
     msnh_event_t e0 = nullptr, e1 = nullptr;

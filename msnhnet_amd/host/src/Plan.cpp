@@ -545,7 +545,7 @@ float Plan::fp16Headroom(msnh_stream_t s)
     struct WriteAll { bool &f; explicit WriteAll(bool &x) : f(x) { f = true; } ~WriteAll() { f = false; } } writeAll(_tailWriteAll);
     DeviceBuffer res(sizeof(float) * 2);
     MSNH_DEV(msnh_hip_fill_zero(res.ptr(), sizeof(float) * 2, s));
-    clearCandidates(s);
+    SideRun side(*this, s);
     for (PlanOp &op : ops)
     {
         if (op.dead) continue;
@@ -1568,6 +1568,14 @@ void Plan::clearCandidates(msnh_stream_t s)
 {
     const DeviceBuffer &cnt = yoloCandCnt[yoloSlot];
     if (cnt.ptr()) MSNH_DEV(msnh_hip_fill_zero(cnt.ptr(), cnt.bytes(), s));
+}
+
+Plan::SideRun::SideRun(Plan &plan, msnh_stream_t s) : _plan(plan), _slot(plan.yoloSlot)
+{
+    for (DeviceBuffer *set : {plan.yoloCandCnt, plan.yoloRows})
+        if (set[0].ptr() && !set[2].ptr()) set[2].alloc(set[0].bytes());
+    plan.yoloSlot = 2;
+    plan.clearCandidates(s);
 }
 
 void Plan::exportTensor(int t, std::vector<float> &dst, msnh_stream_t s)
