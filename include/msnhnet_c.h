@@ -193,8 +193,8 @@ long long msnhnet_time_detail(msnhnet_t net, char *dst, long long cap);       /*
  * its own stream, arena and graph (one packed copy of the weights serves all), driven by its own host thread with `depth` batches in flight (detectors 1 or
  * 2, classifiers 1); the device runs the forwards of different instances side by side, which fills the gaps between the launches
  * of one forward.  The switches of msnhnet_set_* apply as for msnhnet_create + build + load.
- *   msnhnet_group_prime  : one forward of the device-resident float32 NCHW batch on every instance, on the calling thread
- *                          (fills each instance's input buffer, captures its graph); call once before submitting.
+ *   msnhnet_group_prime  : one forward (a detector: two, one per copy-back slot) of the device-resident float32 NCHW batch on every
+ *                          instance, on the calling thread (fills each instance's input buffer); call once before submitting.
  *   msnhnet_group_submit : hands the next batch to the next instance; device_input as for msnhnet_enqueue (NULL = run on what
  *                          the instance's input buffer holds), valid until the batch's result has been fetched.
  *   msnhnet_group_flush  : every instance fetches what it still holds in flight now (it otherwise keeps depth - 1 results back

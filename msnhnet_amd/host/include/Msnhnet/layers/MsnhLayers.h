@@ -340,6 +340,7 @@ public:
     // The stages of forwardGPU, separately, so that a caller can overlap the host stage of one batch with
     // the device work of the next (two copy-back slots):
     bool nmsInForward();                                   // the next forward ends with the NMS itself (enqueueImageNms)
+    bool canSuppressInForward();                           // ... some forward may (and the buffers for it are there afterwards)
     void enqueueGather(msnh_stream_t s);                   // device: compact the candidate rows
     void enqueueImageNms(msnh_stream_t s, int slot);       // device: NMS of every image, kept boxes straight into the slot's pinned memory
     void enqueueCopyBack(msnh_stream_t s, int slot, bool inForward);   // device -> pinned host, asynchronous (inForward: enqueueImageNms has done it)

@@ -62,6 +62,9 @@ public:
     // Detection networks may have two forwards in flight (enqueue, enqueue, fetch, enqueue, fetch, ...): the
     // host-side sort / NMS of one batch then overlaps the device work of the next.
     void enqueueForward(const float *deviceInput);
+    // Records the launches of the forwards that enqueueForward replays (a load ends with it; not needed before a forward, which records what is missing).
+    void recordForwards();
+    bool recordAtLoad = true;                 // false: whoever loads the network changes it afterwards and calls recordForwards() then (NetGroup)
     void sync();
     std::vector<float> fetchClassify();
     std::vector<std::vector<YoloBox>> fetchYolo();
@@ -127,7 +130,7 @@ private:
     std::string _weightsPath;               // set while loadWeightsFromMsnhBin runs: where the tune cache goes
     uint64_t _graphTextHash = 0, _weightsHash = 0;
     float _readMs = 0.f;
-    std::string _loadDetail;
+    std::string _loadDetail, _packState;
     std::unique_ptr<Plan> lowerNetwork(int dtype);
     void uploadInput(const float *img, size_t count);
     void runLayersEager();
@@ -153,10 +156,14 @@ private:
     size_t outputBytes() const;                // size of a classifier's result if the forward itself delivers it to _outputPinned, else 0
     void upload(void *dst, void *stage, const void *src, size_t bytes);
     msnh_stream_t _stream = nullptr;
-    // The captured forward.  Detectors have one per copy-back slot and per place of the NMS (inside the forward or behind it), captured
-    // when first needed; [0][0] is the only one of a classifier.
+    // The recorded forward.  Detectors have one per copy-back slot and per place of the NMS (behind the forward or inside it), recorded at load
+    // and, when the settings have changed since, when first needed; [0][0] is the only one of a classifier.
     msnh_graph_t  _graphs[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};
+    int   _recorded = 0;                       // forwards recorded since the network was loaded
+    float _recordMs = 0.f;
     void dropGraphs();
+    void settleKeepDecoded(YoloOutLayer *yout);
+    void recordForward(YoloOutLayer *yout, int slot, bool inForward);
     void issueForward(YoloOutLayer *yout, bool inForward, msnh_stream_t s);
     int _nextSlot = 0, _inFlight = 0;          // copy-back slots of the detection post-processing
 };

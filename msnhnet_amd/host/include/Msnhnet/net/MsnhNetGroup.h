@@ -34,8 +34,9 @@ public:
     bool isDetector() const { return _detect; }
     NetBuilder &instance(int i) { return *_lanes.at(static_cast<size_t>(i))->net; }
 
-    // One forward of the float32 NCHW batch at deviceInput on every instance, one after the other on the calling thread: every
-    // instance's input buffer then holds that batch (submit(nullptr) runs on it), its graph is captured and its buffers exist.
+    // One forward (a detector: two, one per copy-back slot) of the float32 NCHW batch at deviceInput on every instance, one after the other on the calling
+    // thread: every instance's input buffer then holds that batch (submit(nullptr) runs on it) and its buffers exist.  (Its forwards were recorded when the
+    // group was made.)
     void prime(const float *deviceInput);
     // Hands the next batch to the next instance.  deviceInput: device pointer to the batch (copied into the instance's input buffer on
     // its stream; must stay valid until the result has been fetched) or nullptr to run on what that buffer holds.

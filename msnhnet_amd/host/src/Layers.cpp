@@ -1420,10 +1420,12 @@ void YoloOutLayer::enqueueGather(msnh_stream_t s)
                                   pl.yoloCandIdx.as<int>(), pl.yoloCells, pl.candCnt(), pl.candRows(), s));
 }
 
-bool YoloOutLayer::nmsInForward()
+bool YoloOutLayer::nmsInForward() { return _lastMaxCandidates <= kImageNms && canSuppressInForward(); }
+
+bool YoloOutLayer::canSuppressInForward()
 {
     if (plan == nullptr) MSNH_THROW("YoloOut: layer is not part of a planned network");
-    if (deviceNms == 0 || _useSoftNms || keepClassScores || !plan->sparseYolo || _lastMaxCandidates > kImageNms) return false;
+    if (deviceNms == 0 || _useSoftNms || keepClassScores || !plan->sparseYolo) return false;
     prepareSlot(_slots[0], true);           // (not inside the capture of the forward: allocations)
     prepareSlot(_slots[1], true);
     return true;

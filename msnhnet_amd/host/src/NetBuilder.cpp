@@ -404,6 +404,7 @@ void NetBuilder::finalizePlan()
     _inputPinned.reserve(inBytes);
     _netState->gpuInput = _inputDev.as<float>();
     dropGraphs();
+    _recorded = 0;
     _nextSlot = 0;
     _inFlight = 0;
 
@@ -486,8 +487,9 @@ void NetBuilder::finalizePlan()
     {
         std::ostringstream os;
         os << "load: read+hash " << _readMs << " ms, lower " << lowerMs << " ms, pack file open " << openMs << " ms, calibrate " << calMs << " ms, place+pack+upload "
-           << packMs << " ms, tune " << tuneMs << " ms; pack file " << packState;
+           << packMs << " ms, tune " << tuneMs << " ms";
         _loadDetail = os.str();
+        _packState = packState;
     }
 
     // hand every layer its slice of the op list
@@ -504,6 +506,12 @@ void NetBuilder::finalizePlan()
     }
     _net->plan = std::move(plan);
     _planReady = true;
+    if (recordAtLoad)
+    {
+        t0 = Clock::now();
+        recordForwards();
+        _recordMs = msSince(t0);
+    }
 }
 
 // ---- run -------------------------------------------------------------------------------------------------------------
@@ -657,6 +665,54 @@ void NetBuilder::runLayersEager()
     msnh_hip_event_destroy(e1);
 }
 
+static bool eagerForwards()
+{
+    static const bool eager = std::getenv("MSNH_EAGER") != nullptr;
+    return eager;
+}
+
+// The full decoded rows are only written for YoloBox::classesVal; the recorded launches carry the choice.
+void NetBuilder::settleKeepDecoded(YoloOutLayer *yout)
+{
+    Plan &plan = *_net->plan;
+    if (!yout || !plan.sparseYolo || plan.yoloKeepDecoded == YoloOutLayer::keepClassScores) return;
+    plan.yoloKeepDecoded = YoloOutLayer::keepClassScores;
+    dropGraphs();
+}
+
+// Records one whole forward; enqueueForward replays it with a single launch.
+void NetBuilder::recordForward(YoloOutLayer *yout, int slot, bool inForward)
+{
+    _net->plan->yoloSlot = slot;
+    MSNH_DEV(msnh_hip_graph_begin(_stream));
+    try { issueForward(yout, inForward, _stream); }
+    catch (...)
+    {
+        msnh_graph_t junk = nullptr;
+        msnh_hip_graph_end(_stream, &junk);
+        if (junk) msnh_hip_graph_destroy(junk);
+        throw;
+    }
+    MSNH_DEV(msnh_hip_graph_end(_stream, &_graphs[slot][inForward ? 1 : 0]));
+    ++_recorded;
+}
+
+// All the forwards that this network replays under the present settings, so that none of them is recorded in the middle of serving (a scene that crosses
+// the line between the two places of the suppression would be the first to need its form; 0.3 to 0.7 ms for the 76 launches of YOLOv3).  A forward that cannot
+// be recorded is left to the call that needs it, which reports why.
+void NetBuilder::recordForwards()
+try
+{
+    if (!_planReady || eagerForwards() || _saveLayerOutput) return;
+    YoloOutLayer *yout = _net->layers.back()->type() == LayerType::YOLO_OUT ? static_cast<YoloOutLayer *>(_net->layers.back()) : nullptr;
+    settleKeepDecoded(yout);
+    const bool both = yout && yout->canSuppressInForward();
+    for (int slot = 0; slot < (yout ? 2 : 1); ++slot)
+        for (int form = 0; form < (both ? 2 : 1); ++form)
+            if (_graphs[slot][form] == nullptr) recordForward(yout, slot, form != 0);
+}
+catch (const std::exception &) {}
+
 void NetBuilder::enqueueForward(const float *deviceInput)
 {
     if (!_planReady) MSNH_THROW("weights are not loaded");
@@ -665,35 +721,18 @@ void NetBuilder::enqueueForward(const float *deviceInput)
     if (yout && _inFlight >= 2) MSNH_THROW("two forwards are already in flight: fetch a result first");
     if (deviceInput != nullptr && deviceInput != _inputDev.as<float>())
         MSNH_DEV(msnh_hip_memcpy_d2d(_inputDev.ptr(), deviceInput, sizeof(float) * static_cast<size_t>(_net->inputNum), _stream));
-    if (yout && plan.sparseYolo && plan.yoloKeepDecoded != YoloOutLayer::keepClassScores)
-    {
-        // the full decoded rows are only written for YoloBox::classesVal; the recorded launches carry the choice
-        plan.yoloKeepDecoded = YoloOutLayer::keepClassScores;
-        dropGraphs();
-    }
+    settleKeepDecoded(yout);
     const int slot = yout ? _nextSlot : 0;
     const bool inForward = yout && yout->nmsInForward();
     plan.yoloSlot = slot;
     if (inForward && !plan.countsClear[slot]) plan.clearCandidates(_stream);
     plan.countsClear[slot] = false;             // (a replayed graph appends as well; until the forward that leaves zero behind is on its way)
-    static const bool eager = std::getenv("MSNH_EAGER") != nullptr;
-    msnh_graph_t &graph = _graphs[slot][inForward ? 1 : 0];
-    if (eager) issueForward(yout, inForward, _stream);
-    else if (graph == nullptr)
+    if (eagerForwards()) issueForward(yout, inForward, _stream);
+    else
     {
-        // Record the whole forward once; later calls replay it with a single launch.
-        MSNH_DEV(msnh_hip_graph_begin(_stream));
-        try { issueForward(yout, inForward, _stream); }
-        catch (...)
-        {
-            msnh_graph_t junk = nullptr;
-            msnh_hip_graph_end(_stream, &junk);
-            if (junk) msnh_hip_graph_destroy(junk);
-            throw;
-        }
-        MSNH_DEV(msnh_hip_graph_end(_stream, &graph));
+        if (_graphs[slot][inForward ? 1 : 0] == nullptr) recordForward(yout, slot, inForward);
+        MSNH_DEV(msnh_hip_graph_launch(_graphs[slot][inForward ? 1 : 0], _stream));
     }
-    if (!eager) MSNH_DEV(msnh_hip_graph_launch(graph, _stream));
     ++_enqueued;
     _outputReady = outputBytes() > 0;
     if (yout)
@@ -1042,7 +1081,10 @@ std::string NetBuilder::profileEachOp(int reps, std::vector<double> *values)
     return os.str();
 }
 
-std::string NetBuilder::getLoadDetail() const { return _loadDetail; }
+std::string NetBuilder::getLoadDetail() const
+{
+    return _loadDetail.empty() ? _loadDetail : _loadDetail + ", record " + std::to_string(_recordMs) + " ms; " + std::to_string(_recorded) + " forwards recorded; pack file " + _packState;
+}
 std::string NetBuilder::getPlanDetail() const { return _net->plan ? _net->plan->describe() : std::string(); }
 double NetBuilder::getConvFlops() const { return _net->plan ? _net->plan->totalConvFlops() : 0.0; }
 }

@@ -12,6 +12,7 @@ NetGroup::NetGroup(const std::string &msnhnetPath, const std::string &msnhbinPat
     {
         std::unique_ptr<Lane> lane(new Lane());
         lane->net.reset(new NetBuilder());
+        lane->net->recordAtLoad = false;                    // (the packed weights move below)
         lane->net->buildNetFromMsnhNet(msnhnetPath);
         lane->net->loadWeightsFromMsnhBin(msnhbinPath);
         if (instances > 1)
@@ -45,6 +46,7 @@ NetGroup::NetGroup(const std::string &msnhnetPath, const std::string &msnhbinPat
             }
         }
     }
+    for (std::unique_ptr<Lane> &lane : _lanes) lane->net->recordForwards();
     Network *n = _lanes[0]->net->getNet();
     _detect = !n->layers.empty() && n->layers.back()->type() == LayerType::YOLO_OUT;
     _depth = _detect ? std::max(1, std::min(depth, 2)) : 1;
@@ -140,12 +142,14 @@ void NetGroup::drive(Lane &lane)
 void NetGroup::prime(const float *deviceInput)
 {
     if (outstanding() != 0) MSNH_THROW("NetGroup: fetch the outstanding results before prime()");
+    // (a detector's instance alternates between two copy-back slots: one forward in each)
     for (std::unique_ptr<Lane> &lane : _lanes)
-    {
-        lane->net->enqueueForward(deviceInput);
-        if (_detect) lane->net->fetchYolo();
-        else lane->net->fetchClassify();
-    }
+        for (int k = 0; k < (_detect ? 2 : 1); ++k)
+        {
+            lane->net->enqueueForward(deviceInput);
+            if (_detect) lane->net->fetchYolo();
+            else lane->net->fetchClassify();
+        }
 }
 
 void NetGroup::submit(const float *deviceInput)

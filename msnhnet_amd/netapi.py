@@ -456,7 +456,7 @@ class NetGroup:
     device then runs the forwards of different instances side by side: the launch gaps, prologues and write bursts of one
     forward's kernels are filled by another's, which a single stream cannot do.  Results come back in submission order.
 
-    prime(ptr) runs the device-resident float32 NCHW batch at `ptr` once on every instance (call it before the first submit).
+    prime(ptr) runs the device-resident float32 NCHW batch at `ptr` on every instance, once per copy-back slot (call it before the first submit).
     submit(ptr) hands the next batch to the next instance: a device pointer (copied into the instance's input buffer on its
     stream; keep it valid until the result is fetched) or None to run on what that buffer holds.  flush() makes the instances
     deliver what they still hold in flight now (a fetch of a held-back result asks for it by itself).  fetch() returns the oldest outstanding result (boxes per image for a detector,

@@ -1,6 +1,9 @@
 """Detectors across forwards: where the candidates of a result are suppressed -- inside the forward, behind it on the device, on the host --
 and what runs between two forwards must not show in the boxes.  Every result is compared with the one a network gives that has run nothing
 else (the same kernels: a load takes the tile choices of an earlier load of the same plan), bit for bit."""
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -13,6 +16,43 @@ pytestmark = pytest.mark.gpu
 
 def same(got, want):
     return len(got) == len(want) and all(np.array_equal(a, b, equal_nan=True) for a, b in zip(got, want))
+
+
+GRID, CLASSES, LOGIT = 32, 3, 20.0          # a scene network's head: GRID x GRID cells, three anchors; pixel value v stands for the logit LOGIT * (v - 0.5)
+
+
+def scene_net(batch, tag=""):
+    """a detector whose only convolution (8 x 8, stride 8) hands the pixels on as logits: value m of anchor a in a cell is pixel m of the first
+    row of the cell's patch in channel a -- any scene can be painted"""
+    per = 5 + CLASSES
+    g = zoo.GraphWriter(batch, 3, 8 * GRID, 8 * GRID)
+    g.conv(3 * per, k=8, stride=8, bn=0, act="none")
+    g.yolo([14, 17, 22, 31, 40, 26], class_num=CLASSES)
+    g.yoloout([1], conf=0.5, nms=0.45)
+    w = np.zeros((3 * per, 3, 8, 8), np.float32)
+    for a in range(3):
+        for m in range(per):
+            w[a * per + m, a, 0, m] = LOGIT
+    path = os.path.join(nu.workdir(), f"scenes_b{batch}{tag}")
+    with open(path + ".msnhnet", "w") as f:
+        f.write(g.text())
+    np.concatenate([w.ravel(), np.full(3 * per, -LOGIT / 2, np.float32)]).tofile(path + ".msnhbin")
+    return path + ".msnhnet", path + ".msnhbin"
+
+
+def scene(counts, seed):
+    """a batch with counts[b] candidates in image b, of all classes, many of them overlapping"""
+    per, cells = 5 + CLASSES, 3 * GRID * GRID
+    rng = np.random.default_rng(seed)
+    x = np.zeros((len(counts), 3, GRID, 8, GRID, 8), np.float32)
+    for b, n in enumerate(counts):
+        t = rng.uniform(-2.0, 2.0, (cells, per))
+        t[:, 4] = -6.0
+        t[rng.permutation(cells)[:n], 4] = rng.uniform(0.5, 6.0, n)
+        t[:, 2:4] *= 0.5
+        v = (t / LOGIT + 0.5).reshape(3, GRID, GRID, per)
+        x[b, :, :, 0, :, :per] = v
+    return x.reshape(len(counts), 3, 8 * GRID, 8 * GRID)
 
 
 BETWEEN = {
@@ -84,3 +124,46 @@ def test_layer_dumps_wait_for_outstanding_results():
         m.run_yolo(xs[1])
     assert same(m.fetch_yolo(), want[0])
     assert same(m.run_yolo(xs[1]), want[1])
+
+
+def recorded(m):
+    return int(re.search(r"(\d+) forwards recorded", m.load_detail()).group(1))
+
+
+def test_forwards_are_recorded_before_they_are_needed():
+    """a load records every forward that its network replays (a detector: two copy-back slots, the suppression inside and behind), so that neither
+    the first batches nor the first crowded scene wait for it; a group's instances the same, over the weights they share"""
+    net, binp = scene_net(2)
+    quiet, crowded = scene((300, 900), 1), scene((1500, 2500), 2)
+    m = netapi.Net(net, binp)
+    assert recorded(m) == 4
+    for x in (quiet, quiet, crowded, crowded, crowded, quiet, quiet, quiet):
+        assert all(len(b) > 0 for b in m.run_yolo(x))
+    assert recorded(m) == 4
+    xd = [torch.from_numpy(x).cuda() for x in (quiet, crowded, quiet)]
+    torch.cuda.synchronize()
+    want = [m.run_yolo(x) for x in (quiet, crowded, quiet)]
+    grp = netapi.NetGroup(net, binp, instances=2, depth=2)
+    try:
+        assert [recorded(n) for n in grp.nets] == [4, 4]
+        grp.prime(xd[0].data_ptr())
+        for i in (0, 1, 2, 1, 1, 1, 0, 0, 0, 2, 1):
+            grp.submit(xd[i].data_ptr())
+            assert same(grp.fetch(), want[i])
+        assert [recorded(n) for n in grp.nets] == [4, 4]
+    finally:
+        grp.close()
+    netapi.set_device_nms(0)
+    try:
+        m = netapi.Net(net, binp)
+        assert recorded(m) == 2
+        m.run_yolo(quiet)
+    finally:
+        netapi.set_device_nms(1)
+    assert same(m.run_yolo(quiet), want[0]) and same(m.run_yolo(quiet), want[0])      # (a form that the settings did not allow before: recorded now)
+    assert recorded(m) == 4
+    assert recorded(netapi.Net(*nu.model("resnet18", 1, 224, seed=3)[:2])) == 1
+    small = netapi.Net(*nu.model("resnet18", 1, 64, seed=3)[:2])                       # (its 7 x 7 pool does not fit a 2 x 2 tensor: loads, does not run)
+    assert recorded(small) == 0
+    with pytest.raises(netapi.MsnhnetError, match="window larger"):
+        small.run_classify(zoo.seeded_input(1, 3, 64, 64, 1))
