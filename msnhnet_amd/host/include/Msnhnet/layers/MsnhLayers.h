@@ -372,9 +372,10 @@ public:
     // placement with the shorter time between results stays.
     static int deviceNms;
     static const int kDeviceNmsFew = 2048;
-    // Up to kImageNms candidates per image (msnh_hip_yolo_nms_images_cap) the NMS is the last two launches of the forward itself, which
-    // take less time than the copies and stream hand-overs that a stream of its own would need.
+    // Up to kImageNms candidates per image (msnh_hip_yolo_nms_images_cap: one thread of a workgroup per candidate) the NMS is the last two launches of the
+    // forward itself, which take less time than the copies and stream hand-overs that a stream of its own would need; notePlace() says when.
     static const int kImageNms = 1024;
+    static const int kQuietResults = 8, kQuietResultsMost = 256;          // notePlace
     static const int kDeviceNmsCandidates = 6144;
     static const int kTrialBatches = 16;
 
@@ -425,8 +426,13 @@ private:
     bool _haveLastFinish = false, _lastFinishHost = false;
     void noteResult(const Slot &sl, bool pipelined);
     void prepareSlot(Slot &sl, bool deviceNmsBuffers);
-    void finishImages(const Slot &sl, const DeviceBuffer &devRows);
-    std::vector<YoloBox> hostNmsOfImage(const DeviceBuffer &devRows, int image, int candidates);
+    bool _inside = true;                   // the next forward suppresses its own candidates (if the settings allow it)
+    int _quietNeeded = kQuietResults, _quietSeen = 0, _insideRun = 0;
+    void notePlace(bool inForward);
+    void finishImages(Slot &sl, const DeviceBuffer &devRows);
+    void fetchRows(Slot &sl, const DeviceBuffer &devRows, const std::vector<int> &images, const std::vector<int> &counts, size_t from);
+    void suppressOnHost(const std::vector<int> &images, const std::vector<int> &counts, const float *rows, const float *decoded, double *candidatesDone = nullptr,
+                        double *suppressionDone = nullptr);
     Slot _slots[2];
 };
 }

@@ -3,6 +3,7 @@
 // MsnhLayers.h); none of its compute code exists here -- the arithmetic lives in the device kernels.
 #include "Msnhnet/layers/MsnhLayers.h"
 #include <algorithm>
+#include <numeric>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1420,7 +1421,7 @@ void YoloOutLayer::enqueueGather(msnh_stream_t s)
                                   pl.yoloCandIdx.as<int>(), pl.yoloCells, pl.candCnt(), pl.candRows(), s));
 }
 
-bool YoloOutLayer::nmsInForward() { return _lastMaxCandidates <= kImageNms && canSuppressInForward(); }
+bool YoloOutLayer::nmsInForward() { return _inside && canSuppressInForward(); }
 
 bool YoloOutLayer::canSuppressInForward()
 {
@@ -1618,31 +1619,95 @@ void YoloOutLayer::noteResult(const Slot &sl, bool pipelined)
     _lastFinishHost = !sl.onDevice;
 }
 
-// An image whose candidates the device did not suppress itself: its rows are still in the slot's set on the device.
-std::vector<YoloBox> YoloOutLayer::hostNmsOfImage(const DeviceBuffer &devRows, int image, int candidates)
+// Candidates, suppression and output of the given images of a batch on the host.  Three flat parallel phases: candidates per image; NMS per
+// (image, class) -- the classes of an image are independent, and a batch has far fewer images than the host has cores; concatenation per image.
+void YoloOutLayer::suppressOnHost(const std::vector<int> &images, const std::vector<int> &counts, const float *rows, const float *decoded, double *candidatesDone, double *suppressionDone)
 {
-    std::vector<float> rows(static_cast<size_t>(candidates) * 8);
-    if (_fetchStream == nullptr) MSNH_DEV(msnh_hip_stream_create(&_fetchStream));
-    MSNH_DEV(msnh_hip_memcpy_d2h(rows.data(), devRows.as<float>() + static_cast<size_t>(image) * static_cast<size_t>(plan->yoloCells) * 8, rows.size() * sizeof(float), _fetchStream));
-    MSNH_DEV(msnh_hip_stream_sync(_fetchStream));
-    return nmsSorted(boxesFromRows(rows.data(), candidates, nullptr), _nmsThresh);
+    const size_t cells = static_cast<size_t>(plan->yoloCells);
+    const int n = static_cast<int>(images.size());
+    std::vector<std::vector<YoloBox>> cand(images.size());
+    std::vector<std::vector<std::vector<int>>> groups(images.size());
+    TaskPool &pool = TaskPool::instance();
+    const auto start = TimeUtil::startRecord();
+    pool.parallelFor(n, [&](int i) {
+        const size_t b = static_cast<size_t>(images[static_cast<size_t>(i)]);
+        cand[static_cast<size_t>(i)] = boxesFromRows(rows + b * cells * 8, counts[b], decoded ? decoded + b * cells * static_cast<size_t>(_channel) : nullptr);
+        if (_useSoftNms) finalOut[b] = nms(cand[static_cast<size_t>(i)], _nmsThresh, true);
+        else groups[static_cast<size_t>(i)] = groupByClass(cand[static_cast<size_t>(i)]);
+    });
+    if (candidatesDone) *candidatesDone = *suppressionDone = TimeUtil::getElapsedTime(start);
+    if (_useSoftNms) return;
+    std::vector<std::pair<int, int>> tasks;
+    for (int i = 0; i < n; ++i)
+        for (size_t g = 0; g < groups[static_cast<size_t>(i)].size(); ++g) tasks.emplace_back(i, static_cast<int>(g));
+    // largest classes first, one task at a time: a crowded class costs as much as all the small ones together
+    std::stable_sort(tasks.begin(), tasks.end(), [&groups](const std::pair<int, int> &x, const std::pair<int, int> &y) {
+        return groups[static_cast<size_t>(x.first)][static_cast<size_t>(x.second)].size() > groups[static_cast<size_t>(y.first)][static_cast<size_t>(y.second)].size();
+    });
+    pool.parallelFor(static_cast<int>(tasks.size()), [&](int t) {
+        const size_t i = static_cast<size_t>(tasks[static_cast<size_t>(t)].first);
+        nmsClass(cand[i], groups[i][static_cast<size_t>(tasks[static_cast<size_t>(t)].second)], _nmsThresh);
+    });
+    if (suppressionDone) *suppressionDone = TimeUtil::getElapsedTime(start);
+    pool.parallelFor(n, [&](int i) {
+        std::vector<YoloBox> &out = finalOut[static_cast<size_t>(images[static_cast<size_t>(i)])];
+        for (const std::vector<int> &m : groups[static_cast<size_t>(i)])
+            for (int j : m) out.push_back(cand[static_cast<size_t>(i)][static_cast<size_t>(j)]);
+    });
+}
+
+// Whether the next forwards suppress their own candidates.  Eight images of a 3072-cell head: up to kImageNms candidates per image (950) a batch takes 185 us
+// with the suppression inside and 395 behind the forward (with two in flight 123 and 228); an image above the line inside costs the host's suppression,
+// 730 us against 470 for 1500 candidates and 1250 against 635 for 2900.  So one crowded result sends the next ones behind, and they come back after
+// _quietNeeded quiet results in a row: at least kQuietResults, whose gain pays for the crossing, and twice as many whenever the stay inside was shorter than
+// the wait for it -- scenes that keep crossing the line settle behind the forward and cost there what they cost before there was an inside.
+void YoloOutLayer::notePlace(bool inForward)
+{
+    const bool crowded = _lastMaxCandidates > kImageNms;
+    if (inForward && crowded && _inside)
+    {
+        _quietNeeded = _insideRun < _quietNeeded ? std::min(2 * _quietNeeded, kQuietResultsMost) : kQuietResults;
+        _inside = false;
+    }
+    _insideRun = _inside && !crowded ? _insideRun + 1 : 0;
+    _quietSeen = crowded ? 0 : _quietSeen + 1;
+    if (!_inside && _quietSeen >= _quietNeeded) _inside = true;
+}
+
+// Brings the rows [from, counts[b]) of images that have that many to the slot's place for them (the slot's set on the device is intact until its next forward).
+void YoloOutLayer::fetchRows(Slot &sl, const DeviceBuffer &devRows, const std::vector<int> &images, const std::vector<int> &counts, size_t from)
+{
+    bool any = false;
+    for (int b : images)
+    {
+        const size_t n = static_cast<size_t>(counts[static_cast<size_t>(b)]);
+        if (n <= from) continue;
+        // (its own stream: the copy stream may already hold the next forward's work)
+        if (_fetchStream == nullptr) MSNH_DEV(msnh_hip_stream_create(&_fetchStream));
+        const size_t off = (static_cast<size_t>(b) * static_cast<size_t>(plan->yoloCells) + from) * 8;
+        MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.as<float>() + off, devRows.as<float>() + off, sizeof(float) * 8 * (n - from), _fetchStream));
+        any = true;
+    }
+    if (any) MSNH_DEV(msnh_hip_stream_sync(_fetchStream));
 }
 
 // Results of enqueueImageNms: the rows are the kept boxes in output order.
-void YoloOutLayer::finishImages(const Slot &sl, const DeviceBuffer &devRows)
+void YoloOutLayer::finishImages(Slot &sl, const DeviceBuffer &devRows)
 {
     const int *hdr = sl.imageHdr.as<int>();
     batchHasBox.assign(static_cast<size_t>(_batch), false);
     finalOut.resize(static_cast<size_t>(_batch));
     _lastMaxCandidates = 0;
-    _lastKept = 0;
+    std::vector<int> left, counts(static_cast<size_t>(_batch));        // images that the kernel left to the host: more candidates than it takes, or NaN scores
     for (int b = 0; b < _batch; ++b, hdr += 4)
     {
         const int candidates = std::min(hdr[0], plan->yoloCells);
         _lastMaxCandidates = std::max(_lastMaxCandidates, candidates);
         batchHasBox[static_cast<size_t>(b)] = candidates > 0;
+        counts[static_cast<size_t>(b)] = candidates;
         std::vector<YoloBox> &out = finalOut[static_cast<size_t>(b)];
-        if (hdr[2] != 0) out = hostNmsOfImage(devRows, b, candidates);        // more candidates than the kernel takes, or NaN scores
+        out.clear();
+        if (hdr[2] != 0) left.push_back(b);
         else
         {
             out.assign(static_cast<size_t>(hdr[1]), YoloBox());
@@ -1656,8 +1721,12 @@ void YoloOutLayer::finishImages(const Slot &sl, const DeviceBuffer &devRows)
                 r += 8;
             }
         }
-        _lastKept += out.size();
     }
+    fetchRows(sl, devRows, left, counts, 0);
+    if (!left.empty()) suppressOnHost(left, counts, sl.rows.as<float>(), nullptr);
+    _lastKept = 0;
+    for (const std::vector<YoloBox> &out : finalOut) _lastKept += out.size();
+    notePlace(true);
 }
 
 void YoloOutLayer::finish(int slot)
@@ -1679,10 +1748,11 @@ void YoloOutLayer::finish(int slot)
         return;
     }
     const int cells = plan->yoloCells;
-    const int per = _channel;
     const int *cnt = sl.cnt.as<int>();
-    _lastMaxCandidates = 0;
-    for (int b = 0; b < _batch; ++b) _lastMaxCandidates = std::max(_lastMaxCandidates, std::min(cnt[b], cells));
+    std::vector<int> counts(static_cast<size_t>(_batch));
+    for (int b = 0; b < _batch; ++b) counts[static_cast<size_t>(b)] = std::min(cnt[b], cells);
+    _lastMaxCandidates = *std::max_element(counts.begin(), counts.end());
+    notePlace(false);
     if (sl.onDevice)
     {
         const int *keptCnt = sl.keptCnt.as<int>();
@@ -1711,67 +1781,25 @@ void YoloOutLayer::finish(int slot)
         TaskPool::instance().parallelFor(_batch, [&](int b) {
             if (keptCnt[1 + b] == 0) finalOut[static_cast<size_t>(b)] = boxesFromKept(perImage[static_cast<size_t>(b)]);
         });
+        std::vector<int> left;                     // images that the device left to the host: a class with very many candidates, or NaN scores
         for (int b = 0; b < _batch; ++b)
         {
             batchHasBox[static_cast<size_t>(b)] = cnt[b] > 0;
-            // the device left this image to the host (a class with very many candidates, or NaN scores)
-            if (keptCnt[1 + b] != 0) finalOut[static_cast<size_t>(b)] = hostNmsOfImage(devRows, b, std::min(cnt[b], cells));
+            if (keptCnt[1 + b] != 0) left.push_back(b);
         }
+        fetchRows(sl, devRows, left, counts, 0);   // (over the records above, which are boxes by now)
+        if (!left.empty()) suppressOnHost(left, counts, sl.rows.as<float>(), nullptr);
         if (std::getenv("MSNH_DEBUG_TIMING")) std::fprintf(stderr, "yoloout finish (device NMS, %zu boxes): wait %.3f ms, host %.3f ms\n", total, dbgWait, TimeUtil::getElapsedTime(dbg0) - dbgWait);
         return;
     }
-    {
-        // rows beyond the prefix that was copied ahead of time (the slot's set on the device is still intact)
-        bool more = false;
-        for (int b = 0; b < _batch; ++b)
-        {
-            const size_t n = static_cast<size_t>(std::min(cnt[b], cells));
-            if (n <= sl.rowsCopied) continue;
-            if (_fetchStream == nullptr) MSNH_DEV(msnh_hip_stream_create(&_fetchStream));
-            const size_t off = (static_cast<size_t>(b) * static_cast<size_t>(cells) + sl.rowsCopied) * 8;
-            MSNH_DEV(msnh_hip_memcpy_d2h(sl.rows.as<float>() + off, devRows.as<float>() + off, sizeof(float) * 8 * (n - sl.rowsCopied), _fetchStream));
-            more = true;
-        }
-        if (more) MSNH_DEV(msnh_hip_stream_sync(_fetchStream));
-    }
-    const float *decodedHost = keepClassScores ? sl.decoded.as<float>() : nullptr;
+    std::vector<int> all(static_cast<size_t>(_batch));
+    std::iota(all.begin(), all.end(), 0);
+    fetchRows(sl, devRows, all, counts, sl.rowsCopied);        // what is beyond the prefix that was copied ahead of time
     batchHasBox.assign(static_cast<size_t>(_batch), false);
     finalOut.assign(static_cast<size_t>(_batch), std::vector<YoloBox>());
-    // three flat parallel phases: candidates per image; NMS per (image, class) -- the classes of an image are
-    // independent, and a batch has far fewer images than the host has cores; concatenation per image
-    std::vector<std::vector<YoloBox>> cand(static_cast<size_t>(_batch));
-    std::vector<std::vector<std::vector<int>>> groups(static_cast<size_t>(_batch));
-    TaskPool &pool = TaskPool::instance();
-    pool.parallelFor(_batch, [&](int b) {
-        const int n = std::min(cnt[b], cells);
-        const float *dec = decodedHost ? decodedHost + static_cast<size_t>(b) * cells * per : nullptr;
-        cand[static_cast<size_t>(b)] = boxesFromRows(sl.rows.as<float>() + static_cast<size_t>(b) * cells * 8, n, dec);
-        if (_useSoftNms) finalOut[static_cast<size_t>(b)] = nms(cand[static_cast<size_t>(b)], _nmsThresh, true);
-        else groups[static_cast<size_t>(b)] = groupByClass(cand[static_cast<size_t>(b)]);
-    });
-    const double dbgA = TimeUtil::getElapsedTime(dbg0);
-    double dbgB = dbgA;
-    if (!_useSoftNms)
-    {
-        std::vector<std::pair<int, int>> tasks;
-        for (int b = 0; b < _batch; ++b)
-            for (size_t g = 0; g < groups[static_cast<size_t>(b)].size(); ++g) tasks.emplace_back(b, static_cast<int>(g));
-        // largest classes first, one task at a time: a crowded class costs as much as all the small ones together
-        std::stable_sort(tasks.begin(), tasks.end(), [&groups](const std::pair<int, int> &x, const std::pair<int, int> &y) {
-            return groups[static_cast<size_t>(x.first)][static_cast<size_t>(x.second)].size() > groups[static_cast<size_t>(y.first)][static_cast<size_t>(y.second)].size();
-        });
-        const int nTasks = static_cast<int>(tasks.size());
-        pool.parallelFor(nTasks, [&](int t) {
-            const size_t b = static_cast<size_t>(tasks[static_cast<size_t>(t)].first);
-            nmsClass(cand[b], groups[b][static_cast<size_t>(tasks[static_cast<size_t>(t)].second)], _nmsThresh);
-        });
-        dbgB = TimeUtil::getElapsedTime(dbg0);
-        pool.parallelFor(_batch, [&](int b) {
-            std::vector<YoloBox> &out = finalOut[static_cast<size_t>(b)];
-            for (const std::vector<int> &m : groups[static_cast<size_t>(b)])
-                for (int j : m) out.push_back(cand[static_cast<size_t>(b)][static_cast<size_t>(j)]);
-        });
-    }
+    double dbgA = 0.0, dbgB = 0.0;
+    const double dbgRows = TimeUtil::getElapsedTime(dbg0);
+    suppressOnHost(all, counts, sl.rows.as<float>(), keepClassScores ? sl.decoded.as<float>() : nullptr, &dbgA, &dbgB);
     for (int b = 0; b < _batch; ++b) batchHasBox[static_cast<size_t>(b)] = cnt[b] > 0;
     {
         // did the device make the host wait?  If it has not for eight batches in a row, the host stage may be what bounds the
@@ -1786,7 +1814,7 @@ void YoloOutLayer::finish(int slot)
     }
     if (std::getenv("MSNH_DEBUG_TIMING"))
         std::fprintf(stderr, "yoloout finish: wait %.3f ms, host %.3f ms (candidates %.3f, suppression %.3f, output %.3f)\n", dbgWait,
-                     TimeUtil::getElapsedTime(dbg0) - dbgWait, dbgA - dbgWait, dbgB - dbgA, TimeUtil::getElapsedTime(dbg0) - dbgB);
+                     TimeUtil::getElapsedTime(dbg0) - dbgWait, dbgRows + dbgA - dbgWait, dbgB - dbgA, TimeUtil::getElapsedTime(dbg0) - dbgRows - dbgB);
 }
 
 std::vector<float> YoloOutLayer::lastCandidateRows(int image) const

@@ -167,3 +167,43 @@ def test_forwards_are_recorded_before_they_are_needed():
     assert recorded(small) == 0
     with pytest.raises(netapi.MsnhnetError, match="window larger"):
         small.run_classify(zoo.seeded_input(1, 3, 64, 64, 1))
+
+
+QUIET, CROWDED = [(0, 700, 1024), (1024, 3, 900), (500, 0, 1)], [(1025, 20, 3000), (1100, 1500, 2048), (10, 3072, 1024), (2049, 1024, 1025)]
+
+
+@pytest.mark.parametrize("depth", [1, 2])
+@pytest.mark.parametrize("own_stream", [True, False])
+def test_scenes_that_cross_the_line_both_ways(depth, own_stream):
+    """candidate counts on both sides of 1024 in one batch and from batch to batch, long enough for the suppression to go inside, behind and inside
+    again several times: the boxes are the host's, wherever they were suppressed"""
+    net, binp = scene_net(3)
+    counts = QUIET + CROWDED
+    xs = [scene(c, 10 + i) for i, c in enumerate(counts)]
+    netapi.set_device_nms(0)
+    try:
+        host = netapi.Net(net, binp)
+        want = [host.run_yolo(x) for x in xs]
+        for i, c in enumerate(counts):
+            host.run_yolo(xs[i])
+            assert [len(host.yolo_candidates(b)) for b in range(3)] == list(c)
+    finally:
+        netapi.set_device_nms(1)
+    assert all(len(np.unique(b[:, 6])) == CLASSES for b in want[3][2:])
+    xd = [torch.from_numpy(x).cuda() for x in xs]
+    torch.cuda.synchronize()
+    m = netapi.Net(net, binp)
+    m.set_copy_on_forward_stream(not own_stream)
+    rng = np.random.default_rng(7)
+    order = [0, 1, 3, 0, 4, 2, 5, 6, 6]
+    for rounds in range(3):
+        order += list(rng.integers(0, 3, 12)) + [3 + rounds, 6, 3, 1, 4]           # a quiet stretch, then back and forth
+    order += list(rng.integers(0, len(xs), 40)) + [0] * 70 + [5, 0, 0]
+    print("crossing", depth, own_stream, flush=True)
+    sent = 0
+    for k, i in enumerate(order):
+        while sent < len(order) and sent < k + depth:
+            m.enqueue(xd[order[sent]].data_ptr())
+            sent += 1
+        assert same(m.fetch_yolo(), want[i]), (k, i)
+    assert recorded(m) == 4
