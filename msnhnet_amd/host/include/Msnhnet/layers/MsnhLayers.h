@@ -375,7 +375,7 @@ public:
     // Up to kImageNms candidates per image (msnh_hip_yolo_nms_images_cap: one thread of a workgroup per candidate) the NMS is the last two launches of the
     // forward itself, which take less time than the copies and stream hand-overs that a stream of its own would need; notePlace() says when.
     static const int kImageNms = 1024;
-    static const int kQuietResults = 8, kQuietResultsMost = 256;          // notePlace
+    static constexpr int kQuietResults = 8, kQuietResultsMost = 256;          // notePlace
     static const int kDeviceNmsCandidates = 6144;
     static const int kTrialBatches = 16;
 
