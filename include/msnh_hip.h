@@ -55,7 +55,7 @@ enum msnh_conv_algo
     MSNH_CONV_IGEMM     = 2,   /* implicit GEMM on MFMA, LDS-staged tiles; needs (in_c/groups) % 8 == 0 (f16) or % 4 (f32) */
     MSNH_CONV_DEPTHWISE = 3,   /* groups == in_c == out_c, bandwidth-bound direct kernel */
     MSNH_CONV_WINOGRAD  = 4,   /* F(2x2,3x3): ksize 3, stride 1, dilation 1, groups 1 */
-    MSNH_CONV_STEM      = 5,   /* in_c <= 4 first layer: reads NCHW float32 input directly (cast fused) */
+    MSNH_CONV_STEM      = 5,   /* in_c <= 4 first layer: reads NCHW float32 input directly (cast fused); msnh_hip_conv2d_stem_supported */
     MSNH_CONV_POINTWISE = 7,   /* 1x1 stride 1, float16, in_c and out_c <= 128 and multiples of 8: weights resident in LDS, pixels
                                   straight from memory into MFMA fragments, no tiles (tile must be 0).  IGEMM weight packing.
                                   Never chosen by AUTO. */
@@ -167,8 +167,11 @@ int msnh_hip_conv2d_pack_layout_version(void);
 /* 1 if IGEMM tile configuration `tile` can run this shape (some configurations are specialised, e.g. for 3x3
  * stride-1 layers whose input patch fits in LDS), else 0.  Pure host function. */
 int msnh_hip_conv2d_tile_supported(const msnh_conv_desc *d, int tile);
-/* Which algorithm MSNH_CONV_AUTO resolves to for this shape (never AUTO).  Pure host function. */
+/* Which algorithm MSNH_CONV_AUTO resolves to for this shape (never AUTO).  STEM, whose input is NCHW float32, only where out_c is a
+ * multiple of 32; the other filter counts that STEM takes are given to it by asking for MSNH_CONV_STEM.  Pure host function. */
 int msnh_hip_conv2d_select_algo(const msnh_conv_desc *d);
+/* 1 if MSNH_CONV_STEM can run this shape (d->algo is not looked at): out_c a multiple of 32, or 16 filters of size 3, 5 or 7.  Pure host function. */
+int msnh_hip_conv2d_stem_supported(const msnh_conv_desc *d);
 /* Number of elements (of d->dtype) of the packed weight buffer for `algo`.  Pure host function. */
 size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo);
 /* Host-side weight packing from the `.msnhbin` order w[out_c][in_c/groups][k][k] float32

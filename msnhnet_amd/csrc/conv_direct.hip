@@ -341,6 +341,10 @@ static bool stemOk(const msnh_conv_desc *d)
            !d->has_residual && static_cast<size_t>(d->ksize) * d->ksize * d->in_c * 32 * 4 <= 60 * 1024;
 }
 
+// What AUTO takes it for: an AUTO caller prepares the input for what it knows AUTO to be (STEM reads NCHW float32, DIRECT the descriptor's NHWC), so the set
+// stays what it was when STEM learned more filter counts.
+static bool stemAuto(const msnh_conv_desc *d) { return d->out_c % 32 == 0 && stemOk(d); }
+
 // float32 values in front of the matrix-core kernel's
 static size_t stemScalarElems(const msnh_conv_desc *d) { return static_cast<size_t>(d->ksize) * d->ksize * d->in_c * d->out_c; }
 
@@ -416,11 +420,13 @@ int msnh_hip_conv2d_select_algo(const msnh_conv_desc *d)
     if (!d) return MSNH_CONV_DIRECT;
     if (d->algo != MSNH_CONV_AUTO) return d->algo;
     if (d->out_upsample == 2) return MSNH_CONV_IGEMM;
-    if (stemOk(d)) return MSNH_CONV_STEM;
+    if (stemAuto(d)) return MSNH_CONV_STEM;
     if (depthwiseOk(d)) return MSNH_CONV_DEPTHWISE;
     if (igemmOk(d)) return MSNH_CONV_IGEMM;
     return MSNH_CONV_DIRECT;
 }
+
+int msnh_hip_conv2d_stem_supported(const msnh_conv_desc *d) { return d && !validate(d) && stemOk(d) ? 1 : 0; }
 
 size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo)
 {

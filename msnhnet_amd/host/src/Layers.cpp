@@ -229,7 +229,7 @@ int ConvolutionalLayer::lower(Plan &plan, int in, int layerIndex)
         d.out_c = _outChannel; d.out_h = _outHeight; d.out_w = _outWidth; d.out_ld = (_outChannel + 7) / 8 * 8;
         d.ksize = _kSizeX; d.stride = _strideX; d.pad = _paddingX; d.dilation = _dilationX; d.groups = _groups;
         d.act = NONE; d.act2 = NONE; d.res_ld = d.out_c; d.res_mul = 1.f; d.out_mul = 1.f; d.algo = MSNH_CONV_AUTO;
-        if (msnh_hip_conv2d_select_algo(&d) != MSNH_CONV_STEM)
+        if (!msnh_hip_conv2d_stem_supported(&d))
         {
             const int cast = plan.addTensor(_batch, _height, _width, _channel, dtype, "input_nhwc");
             plan.addOp(PlanOp::INPUT_CAST, in, -1, cast, layerIndex, "input_cast");

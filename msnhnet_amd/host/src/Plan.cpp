@@ -265,7 +265,7 @@ void Plan::fuse()
         d.out_c = out.c; d.out_h = out.h; d.out_w = out.w; d.out_ld = (out.c + 7) / 8 * 8;
         d.ksize = 7; d.stride = 2; d.pad = 3; d.dilation = 1; d.groups = 1;
         // (packed filters beyond the scalar kernel's: the matrix-core first-layer kernel takes the shape; the scalar one would lose)
-        if (msnh_hip_conv2d_select_algo(&d) != MSNH_CONV_STEM ||
+        if (!msnh_hip_conv2d_stem_supported(&d) ||
             msnh_hip_conv2d_packed_weight_elems(&d, MSNH_CONV_STEM) <= static_cast<size_t>(49) * img.c * out.c * (computeDtype == MSNH_F16 ? 2 : 1))
             continue;
         gone.push_back(&ops[static_cast<size_t>(cast)]);

@@ -129,6 +129,8 @@ def conv2d(x, w_oihw, *, dtype, out_dtype=None, stride=1, pad=0, dil=1, groups=1
     d = abi.ConvDesc(dtype, out_dtype, b, h, wd, c, in_ld or c, oc, oh, ow, out_ld or oc, k, stride, pad, dil, groups,
                      abi.ACT[act], act_param, 1 if residual is not None else 0, res_ld or oc, abi.ACT[act2], act2_param,
                      res_mul, out_mul, abi.ALGO[algo], tile, 2 if upsample == 2 else 0, xcd_blocks)
+    if algo == "auto" and L.msnh_hip_conv2d_stem_supported(ctypes.byref(d)):
+        d.algo = abi.ALGO["stem"]                  # (asked for where it applies, as the plans do)
     resolved = L.msnh_hip_conv2d_select_algo(ctypes.byref(d))
     n = L.msnh_hip_conv2d_packed_weight_elems(ctypes.byref(d), resolved)
     host_dt = np.float32 if (dtype == abi.F32 or resolved == abi.ALGO["stem"]) else np.float16
