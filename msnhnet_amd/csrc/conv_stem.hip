@@ -27,6 +27,8 @@ template <int I, int N, typename F> __device__ __forceinline__ void staticFor(F 
     }
 }
 
+typedef unsigned stemU32x4 __attribute__((ext_vector_type(4)));
+
 constexpr int kStemMaxK = 160;          // 7x7x3 = 147 padded to five 32-wide K blocks
 
 struct StemArgs
@@ -47,10 +49,26 @@ struct StemArgs
     int kyx[kStemMaxK];     // ky << 8 | kx; K padding: ky = 32767 (never inside the image)
 };
 
-// KB: 32-wide K blocks; MBLK: 32-channel output blocks
-template <int KB, int MBLK>
+// operand B of 16 K indices (8 per half of the wavefront) with everything from the K-th on set to zero
+template <int K> __device__ __forceinline__ f16x8 stemKeepTaps(f16x8 b, bool hi)
+{
+    stemU32x4 v = __builtin_bit_cast(stemU32x4, b);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+    {
+        const unsigned lo = (2 * j < K ? 0xffffu : 0u) | (2 * j + 1 < K ? 0xffff0000u : 0u), up = (2 * j + 8 < K ? 0xffffu : 0u) | (2 * j + 9 < K ? 0xffff0000u : 0u);
+        if (lo != ~0u || up != ~0u) v[j] &= hi ? up : lo;
+    }
+    return __builtin_bit_cast(f16x8, v);
+}
+
+// TAPS: ksize^2 * Cin, in KB 32-wide K blocks; MBLK: 32-channel output blocks.  What fills the last block up has zero weights, but zero times an
+// infinite pixel is not zero: its operand is blanked too, by masks that the number of taps makes constants (a mask per dword that holds padding; as
+// kernel arguments they cost 3 us of 4 for MobileNetV2's first layer, one image, computed in the kernel 3 % of 28 at batch 64).
+template <int TAPS, int MBLK>
 __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
 {
+    constexpr int KB = (TAPS + 31) / 32;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     f16 *wl = reinterpret_cast<f16 *>(smem);                                  // [MBLK][KB*2][64][8]
     float *ssl = reinterpret_cast<float *>(smem + MBLK * KB * 2 * 1024);       // [2][MBLK*32]
@@ -109,9 +127,9 @@ __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
                 {
-                    // lanes 0-31 hold K index kLo, lanes 32-63 kLo + 8; K padding has offset 0 and a zero weight
+                    // lanes 0-31 hold K index kLo, lanes 32-63 kLo + 8; K padding has offset 0, its value is blanked below
                     const int kLo = kb * 32 + (i / 8) * 16 + (i % 8);
-                    v[i] = xb[hi ? a.koff[kLo + 8] : a.koff[kLo]];
+                    v[i] = kLo >= TAPS ? 0.f : xb[hi ? a.koff[kLo + 8] : a.koff[kLo]];
                 }
             }
             else
@@ -129,6 +147,11 @@ __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
             f16x8 b0, b1;
 #pragma unroll
             for (int e = 0; e < 8; ++e) { b0[e] = static_cast<f16>(v[e]); b1[e] = static_cast<f16>(v[8 + e]); }
+            if constexpr (kb == KB - 1)
+            {
+                b0 = stemKeepTaps<TAPS - kb * 32>(b0, hi);
+                b1 = stemKeepTaps<TAPS - kb * 32 - 16>(b1, hi);
+            }
 #pragma unroll
             for (int mb = 0; mb < MBLK; ++mb)
             {
@@ -169,11 +192,12 @@ __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
     }
 }
 
-template <int KB, int MBLK>
+template <int TAPS, int MBLK>
 int launchStem(const StemArgs &a, unsigned blocks, hipStream_t st)
 {
+    constexpr int KB = (TAPS + 31) / 32;
     const size_t smem = static_cast<size_t>(MBLK) * KB * 2 * 1024 + 2 * MBLK * 32 * sizeof(float);
-    auto kern = convStemMfmaKernel<KB, MBLK>;
+    auto kern = convStemMfmaKernel<TAPS, MBLK>;
     if (smem > 48 * 1024)
     {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
@@ -191,7 +215,8 @@ int launchStem(const StemArgs &a, unsigned blocks, hipStream_t st)
 // its half of a 16-wide K chunk with two 16-byte loads and converts it in place.  11 chunks (K = 176 with zero weights in
 // the padding) instead of 10, but a fifth of the instructions.  Loads go through a buffer resource: a vector that starts
 // left of the image or ends past the tensor reads zeros or a neighbouring row, and whatever lies outside the image is
-// blanked before the conversion (only in groups that touch the border), the eighth value always.
+// blanked before the conversion (only in groups that touch the border), what is no tap -- the eighth value, the 22nd pair -- always: its
+// weights are zero, but zero times an infinite pixel is not.
 // 16-byte load through a buffer resource: the hardware checks the byte offset against the resource size and returns zeros
 // beyond it (an index that went negative wraps to an offset past the end)
 typedef int stemI32x4 __attribute__((ext_vector_type(4)));
@@ -277,7 +302,8 @@ __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
         staticFor<0, kRowChunks>([&](auto cTag) {
             constexpr int c = decltype(cTag)::value;
             const int off = base + (hi ? a.rowOff[2 * c + 1] : a.rowOff[2 * c]);
-            const unsigned voff = static_cast<unsigned>(off) * 4u;  // a negative index wraps past the end of the buffer: zeros
+            // a negative index wraps past the end of the buffer: zeros; so does the padding pair's
+            const unsigned voff = 2 * c + 1 >= 21 && hi ? 0x80000000u : static_cast<unsigned>(off) * 4u;
             f32x4 lo4 = stemLoad16(rx, voff);
             f32x4 hi4 = stemLoad16(rx, voff + 16u);
             float v[8] = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], 0.f};
@@ -434,10 +460,13 @@ __global__ __launch_bounds__(256) void convStemMfmaF32Kernel(StemF32Args a)
             constexpr int g0 = decltype(gTag)::value;
             staticFor<g0 * GC, (g0 + 1) * GC < CHUNKS ? (g0 + 1) * GC : CHUNKS>([&](auto cTag) {
                 constexpr int c = decltype(cTag)::value;
-                constexpr int r0 = 2 * c, r1 = 2 * c + 1 < ROWS ? 2 * c + 1 : 2 * c;  // (a padding pair reads the last row again; its filter values are zero)
+                constexpr int r0 = 2 * c, r1 = 2 * c + 1 < ROWS ? 2 * c + 1 : 2 * c;
                 float (&t)[KS] = v[g0 % 2][c - g0 * GC];
                 const int off = base + (hi ? (r1 / KS * a.H + r1 % KS) * a.W : (r0 / KS * a.H + r0 % KS) * a.W);
-                const unsigned voff = static_cast<unsigned>(off) * 4u;                // a negative index wraps past the end of the buffer: zeros
+                // a negative index wraps past the end of the buffer: zeros; so does the padding pair's (zero filter values alone would not do: zero times
+                // an infinite pixel is not zero)
+                const bool padded = 2 * c + 1 >= ROWS && hi;
+                const unsigned voff = padded ? 0x80000000u : static_cast<unsigned>(off) * 4u;
                 const f32x4 lo4 = stemLoad16(rx, voff);
                 f32x4 hi4 = {0.f, 0.f, 0.f, 0.f};
                 if constexpr (KS > 5) hi4 = stemLoad16(rx, voff + 16u);
@@ -446,7 +475,7 @@ __global__ __launch_bounds__(256) void convStemMfmaF32Kernel(StemF32Args a)
                 for (int e = 0; e < KS; ++e) t[e] = e < 4 ? lo4[e & 3] : hi4[e & 3];
                 if (!interior)
                 {
-                    const bool rowOk = static_cast<unsigned>(iy0 + (hi ? r1 % KS : r0 % KS)) < static_cast<unsigned>(a.H);
+                    const bool rowOk = !padded && static_cast<unsigned>(iy0 + (hi ? r1 % KS : r0 % KS)) < static_cast<unsigned>(a.H);
                     if (off < 0 && rowOk)
                     {
                         // the first image row of the first plane, left border: the 16-byte vectors would start in front of the tensor
@@ -655,15 +684,13 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
     stemTaps(d, a.koff, a.kyx);
     // several wavefronts per SIMD hide the gather latency; every wavefront walks the pixel groups with a grid stride
     const long long want = (groups + 3) / 4;
-    const int kb = stemKBlocks(d), mb = stemMBlocks(d);
-    const long long cap = 256 * (kb <= 2 ? 8 : 4);             // measured: short K wants more wavefronts in flight
+    const int taps = d->ksize * d->ksize * d->in_c, mb = stemMBlocks(d);
+    const long long cap = 256 * (taps <= 64 ? 8 : 4);             // measured: short K wants more wavefronts in flight
     const unsigned blocks = static_cast<unsigned>(want < cap ? (want < 1 ? 1 : want) : cap);
-#define MSNH_STEM(KBV, MBV) if (kb == KBV && mb == MBV) return launchStem<KBV, MBV>(a, blocks, st)
-    MSNH_STEM(1, 1); MSNH_STEM(1, 2); MSNH_STEM(1, 4);
-    MSNH_STEM(2, 1); MSNH_STEM(2, 2); MSNH_STEM(2, 4);
-    MSNH_STEM(3, 1); MSNH_STEM(3, 2); MSNH_STEM(3, 4);
-    MSNH_STEM(4, 1); MSNH_STEM(4, 2); MSNH_STEM(4, 4);
-    MSNH_STEM(5, 1); MSNH_STEM(5, 2); MSNH_STEM(5, 4);
+#define MSNH_STEM(T) if (taps == T) return mb <= 1 ? launchStem<T, 1>(a, blocks, st) : mb == 2 ? launchStem<T, 2>(a, blocks, st) : launchStem<T, 4>(a, blocks, st)
+    MSNH_STEM(9); MSNH_STEM(18); MSNH_STEM(27); MSNH_STEM(36);                  // 3x3 over 1 to 4 channels
+    MSNH_STEM(25); MSNH_STEM(50); MSNH_STEM(75); MSNH_STEM(100);                // 5x5
+    MSNH_STEM(49); MSNH_STEM(98); MSNH_STEM(147);                               // 7x7 (over 3 channels a tensor too large for the row-ordered kernel)
 #undef MSNH_STEM
     setError("conv2d: stem shape not instantiated");
     return 2;
