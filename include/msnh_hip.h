@@ -74,6 +74,10 @@ enum msnh_conv_algo
                                   epilogue.  desc.tile = tile configuration + 256 * slices, both given (2..32 slices).  The workspace's
                                   first 64 KiB must be zero before the first launch that uses it; every launch leaves them zero.
                                   Same weight packing as IGEMM.  Never chosen by AUTO. */
+    MSNH_CONV_STEM_FOCUS = 13, /* the focus opening of YOLOv5 -- four slices of every second row and column, concatenated, under a 3x3 convolution -- as the
+                                  6x6 stride-2 pad-2 convolution over the image that it is (in_c <= 3, float16 or float32 throughout, out_c as for STEM on
+                                  the matrix cores: 16, or a multiple of 32 and in float16 one of 32, 64, 128).  Input NCHW float32 like STEM; weights
+                                  packed for it.  Never chosen by AUTO. */
     MSNH_CONV_MBCONV = 10      /* not an algorithm of msnh_hip_conv2d: the label of a launch of msnh_hip_mbconv (1x1 expand, 3x3 depthwise
                                   and 1x1 project convolution of an inverted-residual block as one) */
 };
@@ -170,7 +174,8 @@ int msnh_hip_conv2d_tile_supported(const msnh_conv_desc *d, int tile);
 /* Which algorithm MSNH_CONV_AUTO resolves to for this shape (never AUTO).  STEM, whose input is NCHW float32, only where out_c is a
  * multiple of 32; the other filter counts that STEM takes are given to it by asking for MSNH_CONV_STEM.  Pure host function. */
 int msnh_hip_conv2d_select_algo(const msnh_conv_desc *d);
-/* 1 if MSNH_CONV_STEM can run this shape (d->algo is not looked at): out_c a multiple of 32, or 16 filters of size 3, 5 or 7.  Pure host function. */
+/* 1 if MSNH_CONV_STEM can run this shape: out_c a multiple of 32, or 16 filters of size 3, 5 or 7.  With d->algo MSNH_CONV_STEM_FOCUS the same for
+ * that (other values of d->algo are not looked at).  Pure host function. */
 int msnh_hip_conv2d_stem_supported(const msnh_conv_desc *d);
 /* Number of elements (of d->dtype) of the packed weight buffer for `algo`.  Pure host function. */
 size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo);
@@ -179,12 +184,13 @@ size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo);
  *   DIRECT / IGEMM : [out_c][k*k][in_c/groups], tap-major, channel fastest
  *   DEPTHWISE      : [k*k][channels]
  *   WINOGRAD       : [16][out_c][in_c]  = G g G^T per (oc,ic), G of F(2x2,3x3)
- *   STEM           : [k*k*in_c][out_c] float32 regardless of dtype
+ *   STEM           : [k*k*in_c][out_c] float32 regardless of dtype, then the operands of the matrix-core kernel where it takes the shape
+ *   STEM_FOCUS     : the operands of the matrix-core kernel
  * `packed` is host memory of msnh_hip_conv2d_packed_weight_elems() elements; upload it afterwards. */
 int msnh_hip_conv2d_pack_weights(const msnh_conv_desc *d, int algo, const float *oihw, void *packed);
 /* Scratch bytes `workspace` must provide for `algo` (0 for all but WINOGRAD, IGEMM_SPLITK and IGEMM_FUSEDK). */
 size_t msnh_hip_conv2d_workspace_bytes(const msnh_conv_desc *d, int algo);
-/* x: NHWC d->dtype (STEM: NCHW float32); w: packed for the resolved algo; scale/shift: float32[out_c] or NULL;
+/* x: NHWC d->dtype (STEM, STEM_FOCUS: NCHW float32); w: packed for the resolved algo; scale/shift: float32[out_c] or NULL;
  * residual: NHWC d->dtype with pixel stride res_ld, or NULL; y: NHWC d->out_dtype with pixel stride out_ld. */
 int msnh_hip_conv2d(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                     const void *residual, void *y, void *workspace, size_t workspace_bytes, msnh_stream_t s);

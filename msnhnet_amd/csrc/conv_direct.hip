@@ -36,6 +36,7 @@ bool   stemMfmaOk(const msnh_conv_desc *d);
 size_t stemMfmaElems(const msnh_conv_desc *d);
 void   stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed);
 bool   stemMfmaF32Ok(const msnh_conv_desc *d);
+bool   stemFocusOk(const msnh_conv_desc *d);
 size_t stemMfmaF32Elems(const msnh_conv_desc *d);
 void   stemMfmaF32Pack(const msnh_conv_desc *d, const float *oihw, float *packed);
 int    convStemMfmaF32(const msnh_conv_desc *d, const float *x, const float *wA, const float *scale, const float *shift, float *y, hipStream_t st);
@@ -426,7 +427,10 @@ int msnh_hip_conv2d_select_algo(const msnh_conv_desc *d)
     return MSNH_CONV_DIRECT;
 }
 
-int msnh_hip_conv2d_stem_supported(const msnh_conv_desc *d) { return d && !validate(d) && stemOk(d) ? 1 : 0; }
+int msnh_hip_conv2d_stem_supported(const msnh_conv_desc *d)
+{
+    return d && !validate(d) && (d->algo == MSNH_CONV_STEM_FOCUS ? stemFocusOk(d) : stemOk(d)) ? 1 : 0;
+}
 
 size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo)
 {
@@ -436,6 +440,7 @@ size_t msnh_hip_conv2d_packed_weight_elems(const msnh_conv_desc *d, int algo)
     if (algo == MSNH_CONV_WINOGRAD || algo == MSNH_CONV_WINOGRAD_FUSED) return static_cast<size_t>(16) * d->out_c * d->in_c;
     // float32 payload for the scalar kernel, followed (float16 plans) by the MFMA operand fragments
     if (algo == MSNH_CONV_STEM) return kk * d->in_c * d->out_c * (d->dtype == MSNH_F16 ? 2 : 1) + (stemMfmaOk(d) ? stemMfmaElems(d) : stemMfmaF32Ok(d) ? stemMfmaF32Elems(d) : 0);
+    if (algo == MSNH_CONV_STEM_FOCUS) return !stemFocusOk(d) ? 0 : d->dtype == MSNH_F16 ? stemMfmaElems(d) : stemMfmaF32Elems(d);
     return static_cast<size_t>(d->out_c) * kk * cinG;
 }
 
@@ -478,6 +483,11 @@ int msnh_hip_conv2d_pack_weights(const msnh_conv_desc *d, int algo, const float 
         if (stemMfmaF32Ok(d)) stemMfmaF32Pack(d, oihw, o + stemScalarElems(d));
         return 0;
     }
+    case MSNH_CONV_STEM_FOCUS:
+        MSNH_REQUIRE(stemFocusOk(d), "pack_weights: shape not supported by the stem kernel");
+        if (d->dtype == MSNH_F16) stemMfmaPack(d, oihw, static_cast<_Float16 *>(packed));
+        else stemMfmaF32Pack(d, oihw, static_cast<float *>(packed));
+        return 0;
     case MSNH_CONV_WINOGRAD:
     case MSNH_CONV_WINOGRAD_FUSED:
         MSNH_REQUIRE(winogradOk(d), "pack_weights: shape not supported by the Winograd kernel");
@@ -510,7 +520,7 @@ int msnh_hip_conv2d(const msnh_conv_desc *d, const void *x, const void *w, const
     e.actParam = d->act_param; e.act2Param = d->act2_param; e.resMul = d->res_mul; e.outMul = d->out_mul;
     const int cinG = d->in_c / d->groups, coutG = d->out_c / d->groups;
     const long long P = static_cast<long long>(d->batch) * d->out_h * d->out_w;
-    if (algo != MSNH_CONV_STEM) MSNH_REQUIRE(d->in_ld >= d->in_c, "conv2d: in_ld < in_c");
+    if (algo != MSNH_CONV_STEM && algo != MSNH_CONV_STEM_FOCUS) MSNH_REQUIRE(d->in_ld >= d->in_c, "conv2d: in_ld < in_c");
 
     switch (algo)
     {
@@ -580,6 +590,10 @@ int msnh_hip_conv2d(const msnh_conv_desc *d, const void *x, const void *w, const
         MSNH_LAUNCH_CHECK();
         return 0;
     }
+    case MSNH_CONV_STEM_FOCUS:
+        MSNH_REQUIRE(stemFocusOk(d), "conv2d: shape not supported by the stem kernel");
+        return d->dtype == MSNH_F16 ? convStemMfma(d, static_cast<const float *>(x), static_cast<const _Float16 *>(w), scale, shift, y, st)
+                                    : convStemMfmaF32(d, static_cast<const float *>(x), static_cast<const float *>(w), scale, shift, static_cast<float *>(y), st);
     case MSNH_CONV_DIRECT:
     {
         const int Kdir = d->ksize * d->ksize * cinG;

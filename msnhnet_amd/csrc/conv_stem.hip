@@ -1,5 +1,5 @@
-// First-layer convolution on the matrix cores: 3x3 / 5x5 / 7x7 filter over <= 4 input channels (7x7 over 3 channels has a
-// kernel of its own further down), read straight from
+// First-layer convolution on the matrix cores: 3x3 / 5x5 / 7x7 filter over <= 4 input channels, and the 6x6 stride-2 filter of the focus opening
+// (7x7 and 6x6 over 3 channels have a kernel of their own further down), read straight from
 // the NCHW float32 network input (layout conversion and cast to float16 fused), NHWC float16 out.
 //
 // GEMM view: all output channels (32, 64 or 128) x 32 consecutive output pixels of one row per wavefront,
@@ -208,15 +208,15 @@ int launchStem(const StemArgs &a, unsigned blocks, hipStream_t st)
     return 0;
 }
 
-// ---- 7x7 filters over 3 channels (the ResNet stems): K ordered by image rows ------------------------------------------------
+// ---- 7x7 and 6x6 filters over 3 channels (the ResNet stems, the focus opening): K ordered by image rows ----------------------
 // The gather kernel above issues one 4-byte load, one conversion and one select per K index and lane: 147 of each for a
-// 7x7x3 filter, and the vector ALU, not memory, sets its time.  Here K is laid out as 21 (channel, filter row) pairs of
+// 7x7x3 filter, and the vector ALU, not memory, sets its time.  Here K is laid out as 21 (6x6: 18) (channel, filter row) pairs of
 // 8 values each (7 taps + one zero): the 7 taps of a pair are 7 consecutive floats of one image row, so a lane fetches
-// its half of a 16-wide K chunk with two 16-byte loads and converts it in place.  11 chunks (K = 176 with zero weights in
-// the padding) instead of 10, but a fifth of the instructions.  Loads go through a buffer resource: a vector that starts
+// its half of a 16-wide K chunk with two 16-byte loads and converts it in place.  11 chunks (K = 176; 6x6: 9, K = 144) instead
+// of 10, but a fifth of the instructions.  Loads go through a buffer resource: a vector that starts
 // left of the image or ends past the tensor reads zeros or a neighbouring row, and whatever lies outside the image is
-// blanked before the conversion (only in groups that touch the border), what is no tap -- the eighth value, the 22nd pair -- always: its
-// weights are zero, but zero times an infinite pixel is not.
+// blanked before the conversion (only in groups that touch the border), what is no tap -- the values behind the filter row, the 22nd pair of
+// a 7x7 filter -- always: its weights are zero, but zero times an infinite pixel is not.
 // 16-byte load through a buffer resource: the hardware checks the byte offset against the resource size and returns zeros
 // beyond it (an index that went negative wraps to an offset past the end)
 typedef int stemI32x4 __attribute__((ext_vector_type(4)));
@@ -230,12 +230,13 @@ __device__ __forceinline__ f32x4 stemLoad16(__amdgpu_buffer_rsrc_t r, unsigned v
     return __builtin_bit_cast(f32x4, v);
 }
 
-constexpr int kRowChunks = 11;          // ceil(3 * 7 / 2) chunks of two (channel, filter row) pairs
+constexpr int stemRowChunks(int ks) { return (3 * ks + 1) / 2; }       // chunks of two (channel, filter row) pairs
+constexpr int kRowChunksMost = stemRowChunks(7);
 
 struct StemRowsArgs
 {
     const float *x;
-    const f16   *wA;        // [mBlocks][kRowChunks][64 lanes][8]
+    const f16   *wA;        // [mBlocks][stemRowChunks(KS)][64 lanes][8]
     const float *scale;
     const float *shift;
     f16         *y;
@@ -244,13 +245,14 @@ struct StemRowsArgs
     unsigned xBytes;
     int act;
     float actParam, outMul;
-    int rowOff[2 * kRowChunks];     // (ci * H + ky) * W of pair r; padding pair: 0
-    int rowKy[2 * kRowChunks];      // ky of pair r; padding pair: 32767 (never inside the image)
+    int rowOff[2 * kRowChunksMost]; // (ci * H + ky) * W of pair r; padding pair: 0
+    int rowKy[2 * kRowChunksMost];  // ky of pair r; padding pair: 32767 (never inside the image)
 };
 
-template <int MBLK>
+template <int KS, int MBLK>
 __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
 {
+    constexpr int kRowChunks = stemRowChunks(KS);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     f16 *wl = reinterpret_cast<f16 *>(smem);                                        // [MBLK][kRowChunks][64][8]
     float *ssl = reinterpret_cast<float *>(smem + MBLK * kRowChunks * 1024);         // [2][MBLK*32]
@@ -298,15 +300,15 @@ __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
         // wave-uniform: every tap of every pixel of the group lies inside the image (no blanking then)
         const int ixFirst = gx * 32 * a.stride - a.pad;
         const int ixLast  = (gx * 32 + 31) * a.stride - a.pad;
-        const bool interior = iy0 >= 0 && iy0 + 7 <= a.H && ixFirst >= 0 && ixLast + 7 <= a.W && gx * 32 + 31 < a.OW;
+        const bool interior = iy0 >= 0 && iy0 + KS <= a.H && ixFirst >= 0 && ixLast + KS <= a.W && gx * 32 + 31 < a.OW;
         staticFor<0, kRowChunks>([&](auto cTag) {
             constexpr int c = decltype(cTag)::value;
             const int off = base + (hi ? a.rowOff[2 * c + 1] : a.rowOff[2 * c]);
             // a negative index wraps past the end of the buffer: zeros; so does the padding pair's
-            const unsigned voff = 2 * c + 1 >= 21 && hi ? 0x80000000u : static_cast<unsigned>(off) * 4u;
+            const unsigned voff = 2 * c + 1 >= 3 * KS && hi ? 0x80000000u : static_cast<unsigned>(off) * 4u;
             f32x4 lo4 = stemLoad16(rx, voff);
             f32x4 hi4 = stemLoad16(rx, voff + 16u);
-            float v[8] = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], 0.f};
+            float v[8] = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], KS > 6 ? hi4[2] : 0.f, 0.f};
             if (!interior)
             {
                 const int ky = hi ? a.rowKy[2 * c + 1] : a.rowKy[2 * c];
@@ -316,11 +318,11 @@ __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
                     // the first image row of the first plane, left border: the 16-byte vectors would start in front of the
                     // tensor (and their offsets wrap), so the taps that exist are fetched one by one
 #pragma unroll
-                    for (int e = 0; e < 7; ++e)
+                    for (int e = 0; e < KS; ++e)
                         v[e] = off + e >= 0 ? __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, (off + e) * 4, 0, 0)) : 0.f;
                 }
 #pragma unroll
-                for (int e = 0; e < 7; ++e) v[e] = (rowOk && static_cast<unsigned>(ix0 + e) < static_cast<unsigned>(a.W)) ? v[e] : 0.f;
+                for (int e = 0; e < KS; ++e) v[e] = (rowOk && static_cast<unsigned>(ix0 + e) < static_cast<unsigned>(a.W)) ? v[e] : 0.f;
             }
             f16x8 bf;
 #pragma unroll
@@ -363,11 +365,11 @@ __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
     }
 }
 
-template <int MBLK>
+template <int KS, int MBLK>
 int launchStemRows(const StemRowsArgs &a, unsigned blocks, hipStream_t st)
 {
-    const size_t smem = static_cast<size_t>(MBLK) * kRowChunks * 1024 + 2 * MBLK * 32 * sizeof(float);
-    auto kern = convStemRowsKernel<MBLK>;
+    const size_t smem = static_cast<size_t>(MBLK) * stemRowChunks(KS) * 1024 + 2 * MBLK * 32 * sizeof(float);
+    auto kern = convStemRowsKernel<KS, MBLK>;
     if (smem > 48 * 1024)
     {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
@@ -378,10 +380,10 @@ int launchStemRows(const StemRowsArgs &a, unsigned blocks, hipStream_t st)
     return 0;
 }
 
-// the row-ordered kernel takes 7x7 filters over 3 channels whose whole input is addressable with 32-bit byte offsets
+// the row-ordered kernel takes 7x7 and 6x6 filters over 3 channels whose whole input is addressable with 32-bit byte offsets
 inline bool stemRowsOk(const msnh_conv_desc *d)
 {
-    return d->ksize == 7 && d->in_c == 3 && static_cast<long long>(d->batch) * 3 * d->in_h * d->in_w * 4 < 0x7fffffffLL;
+    return (d->ksize == 7 || d->ksize == 6) && d->in_c == 3 && static_cast<long long>(d->batch) * 3 * d->in_h * d->in_w * 4 < 0x7fffffffLL;
 }
 
 // ---- float32 networks ---------------------------------------------------------------------------------------------------------------
@@ -565,19 +567,28 @@ inline int stemKBlocks(const msnh_conv_desc *d) { return (d->ksize * d->ksize * 
 
 } // namespace
 
-bool stemMfmaOk(const msnh_conv_desc *d)
+static bool stemMfmaShape(const msnh_conv_desc *d)
 {
     const int mb = d->out_c / 32;              // (16 channels: half a block, the other half of its rows zero)
-    return d->dtype == MSNH_F16 && d->out_dtype == MSNH_F16 && (d->ksize == 3 || d->ksize == 5 || d->ksize == 7) && d->in_c >= 1 && d->in_c <= 4 &&
+    return d->dtype == MSNH_F16 && d->out_dtype == MSNH_F16 && d->in_c >= 1 && d->in_c <= 4 &&
            d->ksize * d->ksize * d->in_c <= kStemMaxK && d->groups == 1 && d->dilation == 1 && (d->out_c == 16 || (d->out_c % 32 == 0 && (mb == 1 || mb == 2 || mb == 4))) &&
            d->out_ld % 8 == 0 && !d->has_residual && d->in_h < 30000;
 }
 
-bool stemMfmaF32Ok(const msnh_conv_desc *d)
+static bool stemMfmaF32Shape(const msnh_conv_desc *d)
 {
-    return d->dtype == MSNH_F32 && d->out_dtype == MSNH_F32 && (d->ksize == 3 || d->ksize == 5 || d->ksize == 7) && d->in_c >= 1 && d->in_c <= 4 &&
+    return d->dtype == MSNH_F32 && d->out_dtype == MSNH_F32 && d->in_c >= 1 && d->in_c <= 4 &&
            d->ksize * d->ksize * d->in_c <= kStemMaxK && d->groups == 1 && d->dilation == 1 && (d->out_c == 16 || d->out_c % 32 == 0) && d->out_ld % 4 == 0 && !d->has_residual &&
            d->in_h < 30000 && static_cast<long long>(d->in_c) * d->in_h * d->in_w * 4 < 0x7fffffffLL;
+}
+
+static bool stemSize(const msnh_conv_desc *d) { return d->ksize == 3 || d->ksize == 5 || d->ksize == 7; }
+
+bool stemMfmaOk(const msnh_conv_desc *d) { return stemSize(d) && stemMfmaShape(d); }
+bool stemMfmaF32Ok(const msnh_conv_desc *d) { return stemSize(d) && stemMfmaF32Shape(d); }
+bool stemFocusOk(const msnh_conv_desc *d)
+{
+    return d->ksize == 6 && d->stride == 2 && d->pad == 2 && d->in_c <= 3 && (stemMfmaShape(d) || stemMfmaF32Shape(d));
 }
 
 size_t stemMfmaF32Elems(const msnh_conv_desc *d) { return static_cast<size_t>(stemMBlocks(d)) * ((stemF32Steps(d->ksize, d->in_c) + 3) / 4) * 256; }
@@ -601,7 +612,7 @@ void stemMfmaF32Pack(const msnh_conv_desc *d, const float *oihw, float *packed)
 
 size_t stemMfmaElems(const msnh_conv_desc *d)
 {
-    return static_cast<size_t>(stemMBlocks(d)) * (stemRowsOk(d) ? kRowChunks : stemKBlocks(d) * 2) * 64 * 8;
+    return static_cast<size_t>(stemMBlocks(d)) * (stemRowsOk(d) ? stemRowChunks(d->ksize) : stemKBlocks(d) * 2) * 64 * 8;
 }
 
 // packed[mb][kb16][lane][e] = W[channel(mb, lane % 32)][k = kb16*16 + 8*(lane/32) + e], k = tap*Cin + ci
@@ -611,8 +622,9 @@ void stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed)
     if (stemRowsOk(d))
     {
         // packed[mb][chunk][lane][e] = W[channel(mb, lane % 32)][ci][ky][kx = e], (ci, ky) = pair 2 * chunk + lane / 32
+        const int ks = d->ksize, chunks = stemRowChunks(ks);
         for (int mb = 0; mb < stemMBlocks(d); ++mb)
-            for (int c = 0; c < kRowChunks; ++c)
+            for (int c = 0; c < chunks; ++c)
                 for (int lane = 0; lane < 64; ++lane)
                     for (int e = 0; e < 8; ++e)
                     {
@@ -620,8 +632,8 @@ void stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed)
                         const int oc = mb * 32 + 16 * ((m >> 2) & 1) + 4 * (m >> 3) + (m & 3);
                         const int pair = 2 * c + lane / 32;
                         float v = 0.f;
-                        if (pair < 21 && e < 7 && oc < d->out_c) v = oihw[(static_cast<size_t>(oc) * 3 + pair / 7) * 49 + (pair % 7) * 7 + e];
-                        packed[((static_cast<size_t>(mb) * kRowChunks + c) * 64 + lane) * 8 + e] = static_cast<_Float16>(v);
+                        if (pair < 3 * ks && e < ks && oc < d->out_c) v = oihw[((static_cast<size_t>(oc) * 3 + pair / ks) * ks + pair % ks) * ks + e];
+                        packed[((static_cast<size_t>(mb) * chunks + c) * 64 + lane) * 8 + e] = static_cast<_Float16>(v);
                     }
         return;
     }
@@ -645,7 +657,7 @@ void stemMfmaPack(const msnh_conv_desc *d, const float *oihw, _Float16 *packed)
 
 int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, const float *scale, const float *shift, void *y, hipStream_t st)
 {
-    MSNH_REQUIRE(stemMfmaOk(d), "conv2d: shape not supported by the matrix-core stem kernel");
+    MSNH_REQUIRE(stemMfmaOk(d) || (stemFocusOk(d) && d->dtype == MSNH_F16), "conv2d: shape not supported by the matrix-core stem kernel");
     MSNH_REQUIRE(reinterpret_cast<uintptr_t>(y) % 16 == 0 && reinterpret_cast<uintptr_t>(wA) % 16 == 0, "conv2d: stem needs 16-byte aligned output and weights");
     if (stemRowsOk(d))
     {
@@ -658,18 +670,19 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
         r.nGroups = static_cast<int>(groups);
         r.xBytes = static_cast<unsigned>(static_cast<long long>(d->batch) * 3 * d->in_h * d->in_w * 4);
         r.outC = d->out_c; r.act = d->act; r.actParam = d->act_param; r.outMul = d->out_mul;
-        for (int p = 0; p < 2 * kRowChunks; ++p)
+        const int ks = d->ksize;
+        for (int p = 0; p < 2 * kRowChunksMost; ++p)
         {
-            r.rowOff[p] = p < 21 ? ((p / 7) * d->in_h + p % 7) * d->in_w : 0;
-            r.rowKy[p] = p < 21 ? p % 7 : 32767;
+            r.rowOff[p] = p < 3 * ks ? ((p / ks) * d->in_h + p % ks) * d->in_w : 0;
+            r.rowKy[p] = p < 3 * ks ? p % ks : 32767;
         }
         const long long want = (groups + 3) / 4;
         const unsigned blocks = static_cast<unsigned>(want < 256 * 4 ? (want < 1 ? 1 : want) : 256 * 4);     // (2..8 workgroups per CU measure alike)
         switch (stemMBlocks(d))
         {
-        case 1: return launchStemRows<1>(r, blocks, st);
-        case 2: return launchStemRows<2>(r, blocks, st);
-        default: return launchStemRows<4>(r, blocks, st);
+        case 1: return ks == 6 ? launchStemRows<6, 1>(r, blocks, st) : launchStemRows<7, 1>(r, blocks, st);
+        case 2: return ks == 6 ? launchStemRows<6, 2>(r, blocks, st) : launchStemRows<7, 2>(r, blocks, st);
+        default: return ks == 6 ? launchStemRows<6, 4>(r, blocks, st) : launchStemRows<7, 4>(r, blocks, st);
         }
     }
     StemArgs a;
@@ -690,6 +703,7 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
 #define MSNH_STEM(T) if (taps == T) return mb <= 1 ? launchStem<T, 1>(a, blocks, st) : mb == 2 ? launchStem<T, 2>(a, blocks, st) : launchStem<T, 4>(a, blocks, st)
     MSNH_STEM(9); MSNH_STEM(18); MSNH_STEM(27); MSNH_STEM(36);                  // 3x3 over 1 to 4 channels
     MSNH_STEM(25); MSNH_STEM(50); MSNH_STEM(75); MSNH_STEM(100);                // 5x5
+    MSNH_STEM(72); MSNH_STEM(108);                                              // 6x6 (over one channel: 36, above; over 3 a tensor too large for the row-ordered kernel)
     MSNH_STEM(49); MSNH_STEM(98); MSNH_STEM(147);                               // 7x7 (over 3 channels a tensor too large for the row-ordered kernel)
 #undef MSNH_STEM
     setError("conv2d: stem shape not instantiated");
@@ -698,7 +712,7 @@ int convStemMfma(const msnh_conv_desc *d, const float *x, const _Float16 *wA, co
 
 int convStemMfmaF32(const msnh_conv_desc *d, const float *x, const float *wA, const float *scale, const float *shift, float *y, hipStream_t st)
 {
-    MSNH_REQUIRE(stemMfmaF32Ok(d), "conv2d: shape not supported by the matrix-core stem kernel");
+    MSNH_REQUIRE(stemMfmaF32Ok(d) || (stemFocusOk(d) && d->dtype == MSNH_F32), "conv2d: shape not supported by the matrix-core stem kernel");
     MSNH_REQUIRE(reinterpret_cast<uintptr_t>(y) % 16 == 0 && reinterpret_cast<uintptr_t>(wA) % 16 == 0, "conv2d: stem needs 16-byte aligned output and weights");
     StemF32Args a;
     a.x = x; a.wA = wA; a.scale = scale; a.shift = shift; a.y = y;
@@ -716,6 +730,7 @@ int convStemMfmaF32(const msnh_conv_desc *d, const float *x, const float *wA, co
 #define MSNH_STEM(KSV, CV) if (ks == KSV && cin == CV) return mb == 2 ? launchStemF32<KSV, CV, 2>(a, blocks, st) : launchStemF32<KSV, CV, 1>(a, blocks, st)
     MSNH_STEM(3, 1); MSNH_STEM(3, 2); MSNH_STEM(3, 3); MSNH_STEM(3, 4);
     MSNH_STEM(5, 1); MSNH_STEM(5, 2); MSNH_STEM(5, 3); MSNH_STEM(5, 4);
+    MSNH_STEM(6, 1); MSNH_STEM(6, 2); MSNH_STEM(6, 3);
     MSNH_STEM(7, 1); MSNH_STEM(7, 2); MSNH_STEM(7, 3);
 #undef MSNH_STEM
     setError("conv2d: stem shape not instantiated");

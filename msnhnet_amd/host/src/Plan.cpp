@@ -228,8 +228,8 @@ void Plan::fuse()
     }
     // (g) network input -> four slices that take every second row and column -> concatenation of the four -> 3x3 convolution (the
     // focus opening of YOLOv5): the rows 2y - 2 .. 2y + 3 of the input meet in one output row, so the convolution reads the input itself as
-    // a 7x7 convolution of stride 2 and padding 3 whose first filter row and column are zero -- the first-layer kernel takes that.  Ten
-    // launches and 140 us (float16, three images of 544 x 544) become one of 17 us.
+    // a 6x6 convolution of stride 2 and padding 2 on the first-layer kernels (MSNH_CONV_STEM_FOCUS).  Ten launches and 140 us (float16, three
+    // images of 544 x 544) become one of 14 us.
     for (PlanOp &conv : ops)
     {
         if (conv.dead || conv.kind != PlanOp::CONV || conv.ksize != 3 || conv.stride != 1 || conv.pad != 1 || conv.dilation != 1 || conv.groups != 1 || conv.in1 >= 0) continue;
@@ -263,15 +263,13 @@ void Plan::fuse()
         d.dtype = d.out_dtype = computeDtype;
         d.batch = img.n; d.in_h = img.h; d.in_w = img.w; d.in_c = d.in_ld = img.c;
         d.out_c = out.c; d.out_h = out.h; d.out_w = out.w; d.out_ld = (out.c + 7) / 8 * 8;
-        d.ksize = 7; d.stride = 2; d.pad = 3; d.dilation = 1; d.groups = 1;
-        // (packed filters beyond the scalar kernel's: the matrix-core first-layer kernel takes the shape; the scalar one would lose)
-        if (!msnh_hip_conv2d_stem_supported(&d) ||
-            msnh_hip_conv2d_packed_weight_elems(&d, MSNH_CONV_STEM) <= static_cast<size_t>(49) * img.c * out.c * (computeDtype == MSNH_F16 ? 2 : 1))
-            continue;
+        d.ksize = 6; d.stride = 2; d.pad = 2; d.dilation = 1; d.groups = 1;
+        d.algo = MSNH_CONV_STEM_FOCUS;
+        if (!msnh_hip_conv2d_stem_supported(&d)) continue;
         gone.push_back(&ops[static_cast<size_t>(cast)]);
         for (PlanOp *op : gone) op->dead = true;
         conv.in0 = ops[static_cast<size_t>(cast)].in0;
-        conv.ksize = 7; conv.stride = 2; conv.pad = 3;
+        conv.ksize = 6; conv.stride = 2; conv.pad = 2;
         std::copy(at, at + 4, conv.focusAt);
         break;
     }
@@ -848,7 +846,7 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
         {
             const PlanTensor &in = tensors[static_cast<size_t>(op.in0)];
             msnh_conv_desc d = convDesc(*this, op);
-            if (in.layout == PlanTensor::NCHW_INPUT) d.algo = MSNH_CONV_STEM;
+            if (in.layout == PlanTensor::NCHW_INPUT) d.algo = op.focusAt[0] >= 0 ? MSNH_CONV_STEM_FOCUS : MSNH_CONV_STEM;
             op.algo = msnh_hip_conv2d_select_algo(&d);
             if (op.algo == MSNH_CONV_STEM && in.layout != PlanTensor::NCHW_INPUT)
             {
@@ -873,13 +871,13 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             std::vector<float> wide;
             if (focus)
             {
-                // filter row 1 + 2 fy + dy, column 1 + 2 fx + dx: tap (fy, fx) of the channels that the slice of rows dy and columns dx filled
-                wide.assign(static_cast<size_t>(d.out_c) * d.in_c * 49, 0.f);
+                // filter row 2 fy + dy, column 2 fx + dx: tap (fy, fx) of the channels that the slice of rows dy and columns dx filled
+                wide.resize(static_cast<size_t>(d.out_c) * d.in_c * 36);
                 for (int oc = 0; oc < d.out_c; ++oc)
                     for (int ci = 0; ci < d.in_c; ++ci)
                         for (int ky = 0; ky < 6; ++ky)
                             for (int kx = 0; kx < 6; ++kx)
-                                wide[(static_cast<size_t>(oc) * d.in_c + ci) * 49 + (ky + 1) * 7 + kx + 1] =
+                                wide[(static_cast<size_t>(oc) * d.in_c + ci) * 36 + ky * 6 + kx] =
                                     w0[(static_cast<size_t>(oc) * 4 * d.in_c + op.focusAt[ky % 2 * 2 + kx % 2] + ci) * 9 + ky / 2 * 3 + kx / 2];
             }
             const std::vector<float> &w = focus ? wide : w0;
@@ -1598,7 +1596,7 @@ void Plan::exportTensor(int t, std::vector<float> &dst, msnh_stream_t s)
 std::string Plan::describe() const
 {
     static const char *kinds[] = {"conv", "affine", "add", "copy", "maxpool", "avgpool", "upsample", "connected", "input_cast", "yolo_decode", "pad", "slice", "bilinear", "softmax", "col2im"};
-    static const char *algos[] = {"auto", "direct", "igemm", "depthwise", "winograd", "stem", "igemm_splitk", "pointwise", "stem+down", "winograd_fused", "mbconv", "igemm+1x1", "igemm_fusedk"};
+    static const char *algos[] = {"auto", "direct", "igemm", "depthwise", "winograd", "stem", "igemm_splitk", "pointwise", "stem+down", "winograd_fused", "mbconv", "igemm+1x1", "igemm_fusedk", "stem_focus"};
     std::ostringstream os;
     os << "plan: " << liveOps() << " launches, " << tensors.size() << " tensors, arena " << _arena.bytes() / (1024.0 * 1024.0) << " MiB, dtype "
        << (computeDtype == MSNH_F16 ? "f16" : "f32") << "\n";

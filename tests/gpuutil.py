@@ -133,6 +133,7 @@ def conv2d(x, w_oihw, *, dtype, out_dtype=None, stride=1, pad=0, dil=1, groups=1
         d.algo = abi.ALGO["stem"]                  # (asked for where it applies, as the plans do)
     resolved = L.msnh_hip_conv2d_select_algo(ctypes.byref(d))
     n = L.msnh_hip_conv2d_packed_weight_elems(ctypes.byref(d), resolved)
+    first_layer = resolved in (abi.ALGO["stem"], abi.ALGO["stem_focus"])            # (NCHW float32 input)
     host_dt = np.float32 if (dtype == abi.F32 or resolved == abi.ALGO["stem"]) else np.float16
     if resolved == abi.ALGO["stem"] and dtype == abi.F16:
         n //= 2
@@ -141,7 +142,7 @@ def conv2d(x, w_oihw, *, dtype, out_dtype=None, stride=1, pad=0, dil=1, groups=1
     abi.check(L.msnh_hip_conv2d_pack_weights(ctypes.byref(d), resolved, wf.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),
                                              packed.ctypes.data_as(ctypes.c_void_p)))
     wdev = dev(packed)
-    if resolved == abi.ALGO["stem"]:
+    if first_layer:
         xdev = dev(np.ascontiguousarray(x, np.float32))
     else:
         xdev = nhwc_dev(x, dtype, in_ld)

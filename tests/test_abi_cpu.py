@@ -8,11 +8,11 @@ from msnhnet_amd import hipabi as abi
 
 
 def _first_layer(dtype, in_c, out_c, k, **kw):
-    f = dict(batch=2, h=40, w=36, stride=1, groups=1, dil=1, out_ld=(out_c + 7) // 8 * 8, residual=0, out_dtype=dtype)
+    f = dict(batch=2, h=40, w=36, stride=1, pad=0, groups=1, dil=1, out_ld=(out_c + 7) // 8 * 8, residual=0, out_dtype=dtype)
     f.update(kw)
     ext = f["dil"] * (k - 1) + 1
-    oh, ow = (f["h"] - ext) // f["stride"] + 1, (f["w"] - ext) // f["stride"] + 1
-    return abi.ConvDesc(dtype, f["out_dtype"], f["batch"], f["h"], f["w"], in_c, in_c, out_c, oh, ow, f["out_ld"], k, f["stride"], 0, f["dil"], f["groups"], abi.ACT["none"], 0.1,
+    oh, ow = (f["h"] + 2 * f["pad"] - ext) // f["stride"] + 1, (f["w"] + 2 * f["pad"] - ext) // f["stride"] + 1
+    return abi.ConvDesc(dtype, f["out_dtype"], f["batch"], f["h"], f["w"], in_c, in_c, out_c, oh, ow, f["out_ld"], k, f["stride"], f["pad"], f["dil"], f["groups"], abi.ACT["none"], 0.1,
                         f["residual"], out_c, abi.ACT["none"], 0.1, 1.0, 1.0, abi.ALGO["auto"], 0, 0, 0)
 
 
@@ -38,3 +38,18 @@ def test_stem_refuses_what_it_cannot_run():
               _first_layer(abi.F16, 3, 16, 3, out_ld=18), _first_layer(abi.F16, 3, 16, 9)):
         assert ok(d) == 0
     assert L.msnh_hip_conv2d_stem_supported(None) == 0
+
+
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F16])
+def test_focus_opening_is_asked_for(dtype):
+    L = abi.lib()
+    for in_c, out_c in itertools.product((1, 2, 3, 4), (8, 16, 32, 48, 64, 96, 128)):
+        d = _first_layer(dtype, in_c, out_c, 6, stride=2, pad=2)
+        auto = L.msnh_hip_conv2d_select_algo(ctypes.byref(d))
+        assert auto != abi.ALGO["stem_focus"] and (auto == abi.ALGO["stem"]) == (out_c % 32 == 0)
+        d.algo = abi.ALGO["stem_focus"]
+        takes = in_c <= 3 and (out_c in (16, 32, 64, 128) or (out_c == 96 and dtype == abi.F32))
+        assert L.msnh_hip_conv2d_stem_supported(ctypes.byref(d)) == takes, (in_c, out_c)
+        assert (L.msnh_hip_conv2d_packed_weight_elems(ctypes.byref(d), d.algo) > 0) == takes
+        d.ksize, d.pad = 5, 2
+        assert L.msnh_hip_conv2d_stem_supported(ctypes.byref(d)) == 0

@@ -55,3 +55,32 @@ def _check(dtype, c, h, w, oc, k, stride, pad, algo="stem"):
                                                    (2, 20, 72, 16, 5, 1, 2), (3, 30, 150, 64, 7, 2, 3), (3, 30, 150, 16, 7, 2, 3), (3, 22, 70, 128, 7, 1, 3), (1, 22, 70, 16, 7, 2, 3)])
 def test_pixels_that_are_not_finite(dtype, c, h, w, oc, k, stride, pad):
     _check(dtype, c, h, w, oc, k, stride, pad)
+
+
+@pytest.mark.parametrize("dtype", [abi.F16, abi.F32])
+@pytest.mark.parametrize("c,h,w,oc", [(3, 32, 32, 32), (3, 30, 146, 32), (3, 26, 72, 16), (3, 64, 128, 64), (3, 12, 66, 128), (2, 20, 70, 32), (1, 22, 68, 16), (3, 2, 2, 32)])
+def test_focus_opening(dtype, c, h, w, oc):
+    """the 6x6 stride-2 filter: against slices, concatenation and a 3x3 convolution in float64, and the pixels that are not finite"""
+    import gpuutil as gu
+    rng = np.random.default_rng(oc + c + h)
+    w3 = (rng.standard_normal((oc, 4 * c, 3, 3)) / np.sqrt(36 * c)).astype(np.float32)
+    x = rng.uniform(-1.0, 1.0, (2, c, h, w)).astype(np.float32)
+    if dtype == abi.F16:
+        x, w3 = gu.round_f16(x), gu.round_f16(w3)
+    at = {(0, 0): 0, (1, 0): c, (0, 1): 2 * c, (1, 1): 3 * c}                     # row and column parity -> channel of the concatenation (YOLOv5's order)
+    joined = np.zeros((2, 4 * c, h // 2 + 2, w // 2 + 2))
+    w6 = np.zeros((oc, c, 6, 6), np.float32)
+    for (dy, dx), ch in at.items():
+        joined[:, ch:ch + c, 1:-1, 1:-1] = x[:, :, dy::2, dx::2]
+        w6[:, :, dy::2, dx::2] = w3[:, ch:ch + c]
+    ref = np.zeros((2, oc, h // 2, w // 2))
+    for ky in range(3):
+        for kx in range(3):
+            ref += np.einsum("oc,bchw->bohw", w3[:, :, ky, kx].astype(np.float64), joined[:, :, ky:ky + h // 2, kx:kx + w // 2])
+    print("focus", dtype, c, h, w, oc, flush=True)
+    got, used = gu.conv2d(x, w6, dtype=dtype, stride=2, pad=2, algo="stem_focus", out_ld=oc + 8)
+    assert used == "stem_focus" and got.shape == ref.shape
+    # float32: 36 c products summed in another order; float16: the result rounded to 11 bits
+    assert gu.rel_err(got, ref) <= (2e-6 if dtype == abi.F32 else 1e-3)
+    if h > 8:
+        _check(dtype, c, h, w, oc, 6, 2, 2, "stem_focus")
