@@ -78,7 +78,8 @@ def cpu_baseline(arch, size, tmp, seed, budget_s=30.0):
 # HBM bytes per launch (fetch + write) of the dominant kernels, measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this
 # script and kept in profiles/hbm_traffic.json, one entry per (workload, dtype, batch) with the hash of the plan it was measured
 # on (launch kinds, algorithms and shapes; not the tile choices, which the per-layer search may settle differently from run to
-# run).  A plan that hashes differently -- a kernel or a fusion changed since -- reports null instead of a stale figure.
+# run, but the K slices of a launch, which parks and re-reads that many partial results).  A plan that hashes differently -- a kernel or
+# a fusion changed since -- reports null instead of a stale figure.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 HBM_PEAK = 8000.0           # GB/s
 
@@ -87,8 +88,10 @@ def plan_hash(plan_text):
     """hash of a plan description without its tile numbers and arena size"""
     import hashlib
     import re
-    # (which of the GEMM-type kernels and which tile runs a layer is the per-layer search's choice and may differ between two runs)
-    lines = [re.sub(r"\[(igemm_fusedk|igemm_splitk|igemm|pointwise)", "[gemm", re.sub(r" t\d+", "", l)) for l in plan_text.splitlines()[1:]]
+    # (which of the GEMM-type kernels and which tile runs a layer is the per-layer search's choice and may differ between two runs; a sliced launch, whose
+    # number is tile + 256 * slices, moves other bytes than the layer's operands and result)
+    sliced = lambda m: f"[gemm in {int(m.group(1)) >> 8} slices"
+    lines = [re.sub(r"\[(igemm|pointwise)\b", "[gemm", re.sub(r" t\d+", "", re.sub(r"\[igemm_fusedk t(\d+)", sliced, l))) for l in plan_text.splitlines()[1:]]
     return hashlib.sha256("\n".join(lines).encode()).hexdigest()[:16]
 
 

@@ -16,6 +16,17 @@ def test_bench_refuses_more_than_one_gpu():
     assert "one GPU" in r.stdout
 
 
+def test_plan_hash_tells_sliced_launches_apart():
+    """measured traffic is shown for plans that move the same bytes: tile choices do not count, the K slices of a launch do"""
+    sys.path.insert(0, ROOT)
+    import bench
+    line = "  L4 conv[{} k3 s1 g1 +res] 32x14x14x256 -> 14x14x256 f16 e0"
+    h = {a: bench.plan_hash("plan: 1 launches, arena 3 MiB\n" + line.format(a)) for a in ("igemm t37", "igemm t6", "igemm", "pointwise", "igemm_fusedk t774", "igemm_fusedk t780", "igemm_fusedk t518", "igemm+1x1 t70")}
+    assert h["igemm t37"] == h["igemm t6"] == h["igemm"] == h["pointwise"]
+    assert h["igemm_fusedk t774"] == h["igemm_fusedk t780"]              # three slices each
+    assert len({h["igemm"], h["igemm_fusedk t774"], h["igemm_fusedk t518"], h["igemm+1x1 t70"]}) == 4
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("workload,instances", [("resnet18", 1), ("yolov3_tiny", 2)])
 def test_bench_prints_one_json_line_with_the_contract_keys(workload, instances):
