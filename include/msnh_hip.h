@@ -166,6 +166,9 @@ typedef struct msnh_conv_desc
  * speed per shape.  The host library times them per layer at load (the reference asks cuDNN for the fastest
  * algorithm the same way, src/layers/MsnhConvolutionalLayer.cpp:150-194). */
 int msnh_hip_conv2d_tile_count(void);
+/* The configurations on which slices of the K loop (IGEMM_FUSEDK) are worth timing whatever they do unsliced: writes up to cap of their numbers,
+ * returns how many there are.  Pure host function. */
+int msnh_hip_conv2d_sliced_tiles(int *tiles, int cap);
 /* Version of the layouts msnh_hip_conv2d_pack_weights writes: packed weights kept on disk are valid for the version they were made under. */
 int msnh_hip_conv2d_pack_layout_version(void);
 /* 1 if IGEMM tile configuration `tile` can run this shape (some configurations are specialised, e.g. for 3x3

@@ -16,6 +16,7 @@ int convIgemmTail(const msnh_conv_desc *d, const msnh_conv_tail_desc *tail, cons
 int igemmTailTileFirst();
 int convIgemmWs(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                 const void *residual, void *y, hipStream_t st, bool dryRun, void *splitWs, size_t splitWsBytes);
+int igemmSlicedTiles(int *tiles, int cap);
 size_t igemmSplitKWorkspaceBytes(const msnh_conv_desc *d);
 size_t igemmFusedKWorkspaceBytes(const msnh_conv_desc *d);
 bool pointwiseOk(const msnh_conv_desc *d);
@@ -362,6 +363,8 @@ using namespace msnh;
 extern "C" {
 
 int msnh_hip_conv2d_tile_count(void) { return igemmTileCount(); }
+
+int msnh_hip_conv2d_sliced_tiles(int *tiles, int cap) { return igemmSlicedTiles(tiles, tiles ? cap : 0); }
 
 // Bumped whenever msnh_hip_conv2d_pack_weights changes what it writes for some (descriptor, algorithm).
 int msnh_hip_conv2d_pack_layout_version(void) { return 2; }

@@ -46,6 +46,13 @@ int igemmHeuristicTile(const msnh_conv_desc *d)
 int igemmTileCount() { return kIgemmTiles; }
 int igemmTailTileFirst() { return kIgemmTailTileFirst; }
 
+int igemmSlicedTiles(int *tiles, int cap)
+{
+    const int n = static_cast<int>(sizeof(kIgemmSlicedTiles) / sizeof(kIgemmSlicedTiles[0]));
+    for (int i = 0; i < n && i < cap; ++i) tiles[i] = kIgemmSlicedTiles[i];
+    return n;
+}
+
 size_t igemmSplitKWorkspaceBytes(const msnh_conv_desc *d)
 {
     return static_cast<size_t>(kSplitKMax) * d->batch * d->out_h * d->out_w * d->out_c * sizeof(float);

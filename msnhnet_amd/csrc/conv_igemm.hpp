@@ -1308,130 +1308,133 @@ namespace msnh {
 constexpr int kIgemmTiles = 71;
 constexpr int kIgemmTailTileFirst = 70;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
 
+// The configurations on which a sliced launch (MSNH_CONV_IGEMM_FUSEDK) is worth timing whatever they do unsliced: 32 x 32 to 128 x 64, which give a layer of
+// few output tiles the most workgroups before it is cut.  (Larger ones are tried where they are among a layer's fastest unsliced.)  Over the layers of 16
+// networks at batch 1 to 32 in both types the search took 67 83 times, 68 20, 12 19, 65 16, 6 twice, 64 and 66 once; 30 (64 x 64 with two stages of
+// 64-byte rows) and 69 (32 x 64) never, and timing them costs a load 1 to 3 %.
+constexpr int kIgemmSlicedTiles[] = {6, 12, 64, 65, 66, 67, 68};
+
 // One translation unit instantiates every third configuration of one type pair (tile % kIgemmParts == PART), so that they compile in parallel.
 constexpr int kIgemmParts = 3;
 
 template <typename T, typename TOut, int PART>
 int igemmDispatch(IgemmArgs &a, int groups, int tile, hipStream_t st)
 {
+// (a configuration's number stands once: the case and the part that instantiates it follow from it)
+#define MSNH_TILE(N, LAUNCH, ...) case N: if constexpr ((N) % kIgemmParts == PART) return LAUNCH<T, TOut, __VA_ARGS__>(a, groups, st); else break;
+#define MSNH_TILE_TAIL(N, LAUNCH, ...)                                                                                                        \
+    case N:                                                                                                                                   \
+        if constexpr (!(std::is_same<T, f16>::value && std::is_same<TOut, f16>::value))                                                       \
+        {                                                                                                                                     \
+            setError("conv2d: this tile needs float16 tensors and a 1x1 convolution behind it (msnh_hip_conv2d_tail)");                        \
+            return 3;                                                                                                                         \
+        }                                                                                                                                     \
+        else if constexpr ((N) % kIgemmParts == PART) return LAUNCH<T, TOut, __VA_ARGS__>(a, groups, st);                                      \
+        else break;
     switch (tile)
     {
-    case 1:  if constexpr (1 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2>(a, groups, st); else break;
-    case 2:  if constexpr (2 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 4, 2, 2>(a, groups, st); else break;
-    case 3:  if constexpr (3 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 8, 1, 4>(a, groups, st); else break;
-    case 4:  if constexpr (4 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 4, 1, 4>(a, groups, st); else break;
-    case 5:  if constexpr (5 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 256, 8, 1, 4>(a, groups, st); else break;
-    case 6:  if constexpr (6 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 4, 2, 2>(a, groups, st); else break;
-    case 7:  if constexpr (7 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 4, 2, 2>(a, groups, st); else break;
-    case 8:  if constexpr (8 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 2, 2>(a, groups, st); else break;
-    case 9:  if constexpr (9 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 4, 2, 2>(a, groups, st); else break;
-    case 10: if constexpr (10 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 1, 4>(a, groups, st); else break;
-    case 11: if constexpr (11 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 4, 1, 4>(a, groups, st); else break;
-    case 12: if constexpr (12 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 8, 2, 2>(a, groups, st); else break;
-    case 13: if constexpr (13 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 256, 4, 2, 2>(a, groups, st); else break;
+    MSNH_TILE(1, launchIgemm, 128, 128, 8, 2, 2)
+    MSNH_TILE(2, launchIgemm, 128, 128, 4, 2, 2)
+    MSNH_TILE(3, launchIgemm, 64, 256, 8, 1, 4)
+    MSNH_TILE(4, launchIgemm, 64, 256, 4, 1, 4)
+    MSNH_TILE(5, launchIgemm, 32, 256, 8, 1, 4)
+    MSNH_TILE(6, launchIgemm, 64, 64, 4, 2, 2)
+    MSNH_TILE(7, launchIgemm, 256, 128, 4, 2, 2)
+    MSNH_TILE(8, launchIgemm, 128, 64, 8, 2, 2)
+    MSNH_TILE(9, launchIgemm, 128, 64, 4, 2, 2)
+    MSNH_TILE(10, launchIgemm, 64, 128, 8, 1, 4)
+    MSNH_TILE(11, launchIgemm, 64, 128, 4, 1, 4)
+    MSNH_TILE(12, launchIgemm, 64, 64, 8, 2, 2)
+    MSNH_TILE(13, launchIgemm, 128, 256, 4, 2, 2)
     // 3x3 stride-1 pad-1 only: input patch resident in LDS, weights streamed per tap (last number: patch slices
     // per wave and step, 2 for wide images)
-    case 14: if constexpr (14 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 256, 4, 2, 2, 1>(a, groups, st); else break;
-    case 15: if constexpr (15 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 256, 4, 2, 2, 2>(a, groups, st); else break;
-    case 16: if constexpr (16 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 128, 4, 2, 2, 1>(a, groups, st); else break;
-    case 17: if constexpr (17 % kIgemmParts == PART) return launchPatch<T, TOut, 256, 128, 4, 2, 2, 1>(a, groups, st); else break;
-    case 18: if constexpr (18 % kIgemmParts == PART) return launchPatch<T, TOut, 64, 256, 4, 1, 4, 1>(a, groups, st); else break;
-    case 19: if constexpr (19 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 128, 4, 2, 2, 2>(a, groups, st); else break;
+    MSNH_TILE(14, launchPatch, 128, 256, 4, 2, 2, 1)
+    MSNH_TILE(15, launchPatch, 128, 256, 4, 2, 2, 2)
+    MSNH_TILE(16, launchPatch, 128, 128, 4, 2, 2, 1)
+    MSNH_TILE(17, launchPatch, 256, 128, 4, 2, 2, 1)
+    MSNH_TILE(18, launchPatch, 64, 256, 4, 1, 4, 1)
+    MSNH_TILE(19, launchPatch, 128, 128, 4, 2, 2, 2)
     // two LDS stages, 128-byte rows
-    case 20: if constexpr (20 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 2>(a, groups, st); else break;
-    case 21: if constexpr (21 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 8, 2, 2, 2>(a, groups, st); else break;
-    case 22: if constexpr (22 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 256, 8, 2, 2, 2>(a, groups, st); else break;
-    case 23: if constexpr (23 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 2, 2, 2>(a, groups, st); else break;
-    case 24: if constexpr (24 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 1, 4, 2>(a, groups, st); else break;
+    MSNH_TILE(20, launchIgemm, 128, 128, 8, 2, 2, 2)
+    MSNH_TILE(21, launchIgemm, 256, 128, 8, 2, 2, 2)
+    MSNH_TILE(22, launchIgemm, 128, 256, 8, 2, 2, 2)
+    MSNH_TILE(23, launchIgemm, 128, 64, 8, 2, 2, 2)
+    MSNH_TILE(24, launchIgemm, 64, 128, 8, 1, 4, 2)
     // deeper prefetch
-    case 25: if constexpr (25 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 4, 2, 2, 4>(a, groups, st); else break;
-    case 26: if constexpr (26 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 4, 2, 2, 6>(a, groups, st); else break;
-    case 27: if constexpr (27 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 4>(a, groups, st); else break;
-    case 28: if constexpr (28 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 4, 2, 2, 5>(a, groups, st); else break;
+    MSNH_TILE(25, launchIgemm, 128, 128, 4, 2, 2, 4)
+    MSNH_TILE(26, launchIgemm, 256, 128, 4, 2, 2, 6)
+    MSNH_TILE(27, launchIgemm, 128, 128, 8, 2, 2, 4)
+    MSNH_TILE(28, launchIgemm, 128, 128, 4, 2, 2, 5)
     // small tiles at high occupancy for bandwidth-bound short-K layers
-    case 29: if constexpr (29 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 4, 1, 4, 2>(a, groups, st); else break;
-    case 30: if constexpr (30 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 4, 2, 2, 2>(a, groups, st); else break;
-    case 31: if constexpr (31 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 4, 2, 2, 2>(a, groups, st); else break;
+    MSNH_TILE(29, launchIgemm, 64, 128, 4, 1, 4, 2)
+    MSNH_TILE(30, launchIgemm, 64, 64, 4, 2, 2, 2)
+    MSNH_TILE(31, launchIgemm, 128, 64, 4, 2, 2, 2)
     // eight wavefronts (512 threads, two per SIMD): a second wave per SIMD covers the first one's barrier and LDS waits where
     // the launch has at most one workgroup per CU; pixel tiles of 192 and 96 bring the tile count of the 76x76 and 38x38
     // layers at batch 8 just under the CU count (241 and 242 tiles instead of 361 and 182)
-    case 32: if constexpr (32 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 128, 8, 4, 2, 3>(a, groups, st); else break;
-    case 33: if constexpr (33 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 4, 4>(a, groups, st); else break;
-    case 34: if constexpr (34 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 192, 8, 4, 2, 2>(a, groups, st); else break;
-    case 35: if constexpr (35 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 192, 4, 4, 2, 4>(a, groups, st); else break;
-    case 36: if constexpr (36 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 96, 8, 8, 1, 3>(a, groups, st); else break;
+    MSNH_TILE(32, launchIgemm, 256, 128, 8, 4, 2, 3)
+    MSNH_TILE(33, launchIgemm, 128, 128, 8, 2, 4, 4)
+    MSNH_TILE(34, launchIgemm, 256, 192, 8, 4, 2, 2)
+    MSNH_TILE(35, launchIgemm, 256, 192, 4, 4, 2, 4)
+    MSNH_TILE(36, launchIgemm, 256, 96, 8, 8, 1, 3)
     // twelve wavefronts (768 threads, three per SIMD) over 192-pixel tiles: 64 x 64 and 32 x 64 wave tiles
-    case 37: if constexpr (37 % kIgemmParts == PART) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2>(a, groups, st); else break;
-    case 38: if constexpr (38 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 3>(a, groups, st); else break;
+    MSNH_TILE(37, launchIgemm, 256, 192, 8, 4, 3, 2)
+    MSNH_TILE(38, launchIgemm, 128, 192, 8, 4, 3, 3)
     // the LDS-patch kernel with eight wavefronts
-    case 39: if constexpr (39 % kIgemmParts == PART) return launchPatch<T, TOut, 128, 384, 4, 2, 4, 1>(a, groups, st); else break;
-    case 40: if constexpr (40 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 4, 3>(a, groups, st); else break;
+    MSNH_TILE(39, launchPatch, 128, 384, 4, 2, 4, 1)
+    MSNH_TILE(40, launchIgemm, 128, 128, 8, 2, 4, 3)
     // 64 channels x 256 pixels with eight wavefronts side by side, for the first layers of the detectors (32 -> 64 channels)
-    case 41: if constexpr (41 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 4, 1, 8, 3>(a, groups, st); else break;
+    MSNH_TILE(41, launchIgemm, 64, 256, 4, 1, 8, 3)
     // 128 channels x 384 pixels with twelve wavefronts: one round of tiles for 128-filter layers over many pixels
-    case 42: if constexpr (42 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 384, 8, 2, 6, 2>(a, groups, st); else break;
+    MSNH_TILE(42, launchIgemm, 128, 384, 8, 2, 6, 2)
     // 3x3 stride-1 pad-1 only: input patch resident in LDS with 128-byte rows (last three numbers: wavefront grid rows x columns,
     // weight stages, patch slices per wavefront and tap step)
-    case 43: if constexpr (43 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 4, 3, 3, 1>(a, groups, st); else break;
-    case 44: if constexpr (44 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 4, 2, 4, 1>(a, groups, st); else break;
-    case 45: if constexpr (45 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 2, 2, 4, 2>(a, groups, st); else break;
-    case 46: if constexpr (46 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 2, 6, 3, 1>(a, groups, st); else break;
-    case 47: if constexpr (47 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 2, 4, 4, 2>(a, groups, st); else break;
-    case 48: if constexpr (48 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 256, 2, 4, 4, 1>(a, groups, st); else break;
-    case 49: if constexpr (49 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 256, 4, 2, 3, 1>(a, groups, st); else break;
-    case 50: if constexpr (50 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 192, 2, 2, 4, 2>(a, groups, st); else break;
-    case 51: if constexpr (51 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 384, 2, 4, 3, 2>(a, groups, st); else break;
+    MSNH_TILE(43, launchPatch8, 128, 192, 4, 3, 3, 1)
+    MSNH_TILE(44, launchPatch8, 128, 192, 4, 2, 4, 1)
+    MSNH_TILE(45, launchPatch8, 128, 192, 2, 2, 4, 2)
+    MSNH_TILE(46, launchPatch8, 64, 384, 2, 6, 3, 1)
+    MSNH_TILE(47, launchPatch8, 64, 384, 2, 4, 4, 2)
+    MSNH_TILE(48, launchPatch8, 64, 256, 2, 4, 4, 1)
+    MSNH_TILE(49, launchPatch8, 128, 256, 4, 2, 3, 1)
+    MSNH_TILE(50, launchPatch8, 64, 192, 2, 2, 4, 2)
+    MSNH_TILE(51, launchPatch8, 128, 384, 2, 4, 3, 2)
     // the same with the k-blocks of a tap step split between two groups of wavefronts over 64 x 64 wave tiles (the numbers are
     // the grid of wave tiles; twice as many wavefronts run)
-    case 52: if constexpr (52 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 1, 6, 3, 1, 0, 2>(a, groups, st); else break;
-    case 53: if constexpr (53 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 192, 2, 3, 3, 1, 0, 2>(a, groups, st); else break;
-    case 54: if constexpr (54 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 256, 1, 4, 4, 1, 0, 2>(a, groups, st); else break;
-    case 55: if constexpr (55 % kIgemmParts == PART) return launchPatch8<T, TOut, 128, 128, 2, 2, 4, 1, 0, 2>(a, groups, st); else break;
-    case 56: if constexpr (56 % kIgemmParts == PART) return launchPatch8<T, TOut, 64, 384, 1, 6, 4, 1, 0, 2>(a, groups, st); else break;
+    MSNH_TILE(52, launchPatch8, 64, 384, 1, 6, 3, 1, 0, 2)
+    MSNH_TILE(53, launchPatch8, 128, 192, 2, 3, 3, 1, 0, 2)
+    MSNH_TILE(54, launchPatch8, 64, 256, 1, 4, 4, 1, 0, 2)
+    MSNH_TILE(55, launchPatch8, 128, 128, 2, 2, 4, 1, 0, 2)
+    MSNH_TILE(56, launchPatch8, 64, 384, 1, 6, 4, 1, 0, 2)
     // the generic kernel with the same split (numbers: tile, 16-byte vectors of K per step, grid of 64 x 64 wave tiles, LDS stages)
-    case 57: if constexpr (57 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 192, 8, 2, 3, 3, 2>(a, groups, st); else break;
-    case 58: if constexpr (58 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 128, 8, 2, 2, 4, 2>(a, groups, st); else break;
-    case 59: if constexpr (59 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 1, 2, 4, 2>(a, groups, st); else break;
-    case 60: if constexpr (60 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 2, 1, 4, 2>(a, groups, st); else break;
-    case 61: if constexpr (61 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 256, 8, 1, 4, 3, 2>(a, groups, st); else break;
-    case 62: if constexpr (62 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 384, 8, 1, 6, 2, 2>(a, groups, st); else break;
+    MSNH_TILE(57, launchIgemm, 128, 192, 8, 2, 3, 3, 2)
+    MSNH_TILE(58, launchIgemm, 128, 128, 8, 2, 2, 4, 2)
+    MSNH_TILE(59, launchIgemm, 64, 128, 8, 1, 2, 4, 2)
+    MSNH_TILE(60, launchIgemm, 128, 64, 8, 2, 1, 4, 2)
+    MSNH_TILE(61, launchIgemm, 64, 256, 8, 1, 4, 3, 2)
+    MSNH_TILE(62, launchIgemm, 64, 384, 8, 1, 6, 2, 2)
     // the LDS-patch kernel over 256 channels x 192 pixels with twelve wavefronts: one round of tiles for the 76x76 128 -> 256 layers at batch 8
     // like tile 37, with a third fewer bytes delivered to LDS per tap step.  It fits the LDS with two weight stages only, the weight
     // tile of step it + 2 asked for behind the barrier of step it (see LATE in conv_patch8.hpp)
-    case 63: if constexpr (63 % kIgemmParts == PART) return launchPatch8<T, TOut, 256, 192, 4, 3, 2, 1>(a, groups, st); else break;
+    MSNH_TILE(63, launchPatch8, 256, 192, 4, 3, 2, 1)
     // small images (one to a few pictures): 64 x 64 with 256-byte rows, half the barriers per K; 64 x 128 and 128 x 64 with eight wavefronts
     // over 32 x 32 wave tiles, two per SIMD where the launch has at most one workgroup per CU
-    case 64: if constexpr (64 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 64, 16, 2, 2, 3>(a, groups, st); else break;
-    case 65: if constexpr (65 % kIgemmParts == PART) return launchIgemm<T, TOut, 64, 128, 8, 2, 4, 4>(a, groups, st); else break;
-    case 66: if constexpr (66 % kIgemmParts == PART) return launchIgemm<T, TOut, 128, 64, 8, 4, 2, 4>(a, groups, st); else break;
+    MSNH_TILE(64, launchIgemm, 64, 64, 16, 2, 2, 3)
+    MSNH_TILE(65, launchIgemm, 64, 128, 8, 2, 4, 4)
+    MSNH_TILE(66, launchIgemm, 128, 64, 8, 4, 2, 4)
     // 32 x 32 and 32 x 64 with the k-blocks of a step dealt to the four wavefronts: a 32 x 32 tile is a quarter of the work of 64 x 64 for its CU,
     // so the layers of one small picture fill the chip with a third of the slices -- and of the partial sums -- that 64 x 64 needs, or with none.
     // float32, one 224 x 224 picture: 3x3 64 -> 64 at 56 x 56 10.5 -> 8.7 us, 256 -> 256 at 14 x 14 14.7 -> 10.9, 512 -> 512 at 7 x 7 17.3 -> 12.6
-    case 67: if constexpr (67 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 32, 16, 1, 1, 3, 4>(a, groups, st); else break;
-    case 68: if constexpr (68 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 32, 16, 1, 1, 2, 4>(a, groups, st); else break;
-    case 69: if constexpr (69 % kIgemmParts == PART) return launchIgemm<T, TOut, 32, 64, 16, 1, 1, 2, 4>(a, groups, st); else break;
+    MSNH_TILE(67, launchIgemm, 32, 32, 16, 1, 1, 3, 4)
+    MSNH_TILE(68, launchIgemm, 32, 32, 16, 1, 1, 2, 4)
+    MSNH_TILE(69, launchIgemm, 32, 64, 16, 1, 1, 2, 4)
     // tiles whose epilogue also computes the 1x1 convolution that follows (msnh_hip_conv2d_tail only; float16): the tile holds every
     // output channel of the first convolution (at most 256 / 128)
-    case 70:
-    case 71:
-        if constexpr (!(std::is_same<T, f16>::value && std::is_same<TOut, f16>::value))
-        {
-            setError("conv2d: this tile needs float16 tensors and a 1x1 convolution behind it (msnh_hip_conv2d_tail)");
-            return 3;
-        }
-        else if constexpr (70 % kIgemmParts == PART)
-        {
-            if (tile == 70) return launchIgemm<T, TOut, 256, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
-            break;
-        }
-        else if constexpr (71 % kIgemmParts == PART)
-        {
-            if (tile == 71) return launchIgemm<T, TOut, 128, 192, 8, 4, 3, 2, 1, 1>(a, groups, st);
-            break;
-        }
-        else break;
+    MSNH_TILE_TAIL(70, launchIgemm, 256, 192, 8, 4, 3, 2, 1, 1)
+    MSNH_TILE_TAIL(71, launchIgemm, 128, 192, 8, 4, 3, 2, 1, 1)
     default: break;
     }
+#undef MSNH_TILE
+#undef MSNH_TILE_TAIL
     setError("igemm: unknown tile %d", tile);
     return 2;
 }

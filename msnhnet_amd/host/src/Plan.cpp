@@ -1209,10 +1209,12 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         const int baseAlgo = op.algo;
         search(baseAlgo);
         // Layers whose output tiles do not fill the chip or fill it unevenly: the K loop cut into slices, summed inside the launch.  Tried on
-        // the tiles that came out best uncut and on the small ones, which win most of these layers; the library refuses what cannot help.
+        // the tiles that came out best uncut and on the small ones that the library names, which win most of these layers; it refuses what cannot
+        // help, and slices under the upsampling epilogue altogether.
         if (baseAlgo == MSNH_CONV_IGEMM && !op.up2)
         {
-            std::vector<int> tiles = {6, 12, 64, 66, 67, 68};
+            std::vector<int> tiles(static_cast<size_t>(msnh_hip_conv2d_sliced_tiles(nullptr, 0)));
+            msnh_hip_conv2d_sliced_tiles(tiles.data(), static_cast<int>(tiles.size()));
             std::vector<Cand> plain = cands;
             std::sort(plain.begin(), plain.end(), [](const Cand &x, const Cand &y) { return x.ms < y.ms; });
             for (size_t i = 0; i < plain.size() && i < 6; ++i)

@@ -53,3 +53,22 @@ def test_focus_opening_is_asked_for(dtype):
         assert (L.msnh_hip_conv2d_packed_weight_elems(ctypes.byref(d), d.algo) > 0) == takes
         d.ksize, d.pad = 5, 2
         assert L.msnh_hip_conv2d_stem_supported(ctypes.byref(d)) == 0
+
+
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F16])
+def test_tiles_to_slice_take_slices(dtype):
+    """the configurations that the library names for sliced launches exist and take slices of a small, deep layer in both types; the upsampling epilogue
+    goes with unsliced launches only"""
+    L = abi.lib()
+    n = L.msnh_hip_conv2d_sliced_tiles(None, 0)
+    tiles = (ctypes.c_int * (n + 1))(*([-7] * (n + 1)))
+    assert L.msnh_hip_conv2d_sliced_tiles(tiles, n) == n and tiles[n] == -7
+    one = (ctypes.c_int * 2)(-7, -7)
+    assert L.msnh_hip_conv2d_sliced_tiles(one, 1) == n and (one[0], one[1]) == (tiles[0], -7)
+    assert len(set(tiles[:n])) == n and all(1 <= t <= L.msnh_hip_conv2d_tile_count() for t in tiles[:n])
+    for t in tiles[:n]:
+        d = abi.ConvDesc(dtype, dtype, 1, 13, 13, 512, 512, 256, 13, 13, 256, 3, 1, 1, 1, 1, abi.ACT["leaky"], 0.1, 0, 256, abi.ACT["none"], 0.1, 1.0, 1.0, abi.ALGO["igemm_fusedk"], t + 256 * 4, 0, 0)
+        assert L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), d.tile) == 1, t
+        assert L.msnh_hip_conv2d_workspace_bytes(ctypes.byref(d), d.algo) > 65536
+        d.out_upsample = 2
+        assert L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), d.tile) == 0
