@@ -1167,7 +1167,7 @@ void convIgemmKernel(IgemmArgs a)
     else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g);
 }
 
-// Split-K reduction: sums the K slices in slice order (so the result does not depend on timing) and applies the
+// MSNH_CONV_IGEMM_SPLITK (callers of the C interface; the plans use the sum inside the launch).  Split-K reduction: sums the K slices in slice order (so the result does not depend on timing) and applies the
 // convolution's epilogue.  One thread per (pixel, 4 channels).
 template <typename T, typename TOut>
 __global__ __launch_bounds__(256) void splitKReduceKernel(IgemmArgs a, int outC, long long total)
