@@ -28,7 +28,7 @@ def _reference(x, we, wd, wp, s1, h1, s2, h2, s3, h3, stride, acts, mul1, mul2, 
     return (np.float32(out_mul) * y).astype(np.float32)
 
 
-def run_mbconv(x, we, wd, wp, s1, h1, s2, h2, s3, h3, stride, acts, mul1, mul2, out_mul, res, res_mul, in_ld=None, out_ld=None, res_ld=None):
+def run_mbconv(x, we, wd, wp, s1, h1, s2, h2, s3, h3, stride, acts, mul1, mul2, out_mul, res, res_mul, in_ld=None, out_ld=None, res_ld=None, slices=1):
     import torch
     import gpuutil as gu
     gu.init()
@@ -50,7 +50,13 @@ def run_mbconv(x, we, wd, wp, s1, h1, s2, h2, s3, h3, stride, acts, mul1, mul2, 
     s3d, h3d = gu.dev(s3), gu.dev(h3)
     rd = gu.nhwc_dev(res, abi.F16, res_ld) if res is not None else None
     yd = torch.full((b, oh, ow, out_ld), 5.0, dtype=torch.float16).cuda()
-    abi.check(L.msnh_hip_mbconv(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), gu.ptr(s3d), gu.ptr(h3d), gu.ptr(rd), gu.ptr(yd), None))
+    if slices == 1:
+        abi.check(L.msnh_hip_mbconv(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), gu.ptr(s3d), gu.ptr(h3d), gu.ptr(rd), gu.ptr(yd), None))
+    else:
+        need = L.msnh_hip_mbconv_workspace_bytes(ctypes.byref(d), slices)
+        ws = torch.zeros(need, dtype=torch.uint8).cuda()
+        gu.sync()
+        abi.check(L.msnh_hip_mbconv_sliced(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), gu.ptr(s3d), gu.ptr(h3d), gu.ptr(rd), gu.ptr(yd), slices, gu.ptr(ws), need, None))
     gu.sync()
     if out_ld > cout:
         assert (yd[..., cout:] == 5.0).all().item(), "wrote past out_c"
@@ -73,8 +79,8 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES)
-def test_mbconv_block(case):
+def _block(case, slices=1):
+    """one block through the launch and through the three oracle layers"""
     import gpuutil as gu
     b, cin, h, w, cexp, cout, stride, with_res = case
     rng = np.random.default_rng(sum(case) + 11)
@@ -91,14 +97,29 @@ def test_mbconv_block(case):
     oh, ow = (h - 1) // stride + 1, (w - 1) // stride + 1
     res = gu.round_f16(rng.standard_normal((b, cout, oh, ow), dtype=np.float32)) if with_res else None
     acts = ("relu6", "relu6", "none", "none")
-    print("mbconv", case, flush=True)
+    print("mbconv", case, slices, flush=True)
     args = (x, we, wd, wp, s1, h1, s2, h2, s3, h3, stride, acts, mul1, mul2, out_mul, res, res_mul)
-    y = run_mbconv(*args, in_ld=cin + 8, out_ld=cout + 8, res_ld=cout + 16)
+    lds = dict(in_ld=cin + 8, out_ld=cout + 8, res_ld=cout + 16, slices=slices)
+    y = run_mbconv(*args, **lds)
     ref = _reference(*args)
     e = gu.rel_err(y, ref)
     print("error", e, flush=True)
     assert e <= 1e-3
-    assert np.array_equal(y, run_mbconv(*args, in_ld=cin + 8, out_ld=cout + 8, res_ld=cout + 16))
+    assert np.array_equal(y, run_mbconv(*args, **lds))
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_mbconv_block(case):
+    _block(case)
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("slices", [2, 3, 9])
+def test_mbconv_sliced_block(case, slices):
+    """the same with the widened channels dealt to several workgroups: as many as there are 64-channel chunks at most"""
+    slices = min(slices, (case[4] + 63) // 64)
+    if slices > 1:
+        _block(case, slices)
 
 
 def test_mbconv_activations_and_limits():
