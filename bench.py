@@ -348,8 +348,8 @@ def main():
                          "reference's own calling convention, a host float image per call (runYoloGPU / runClassifyGPU), PCIe "
                          "inclusive.  host_u8: 8-bit host images, letterboxed on the device, PCIe inclusive.")
     ap.add_argument("--nms", default="auto", choices=["host", "auto", "device"],
-                    help="detection workloads: sort + NMS on the host, on the device, or (library default) on the device while the "
-                         "previous result had at most 2048 candidates per image -- the seeded weights give 11k, so auto means host here")
+                    help="detection workloads: sort + NMS on the host, on the device, or (library default) by the results so far: inside the "
+                         "forward up to 1024 candidates per image, on the device up to 2048 -- the seeded weights give 4.5k, so auto means host here")
     ap.add_argument("--instances", type=int, default=3,
                     help="network instances on the GPU, each with its own stream and arena, fed round-robin by one host thread each "
                          "(netapi.NetGroup; device-resident input only).  The device runs their forwards side by side, which fills the launch gaps, "

@@ -86,8 +86,9 @@ int msnhnet_create(msnhnet_t *net);                       /* NetBuilder() */
 int msnhnet_destroy(msnhnet_t net);
 int msnhnet_set_use_fp16(int on);                         /* NetBuilder::setUseFp16, process-wide, before build */
 int msnhnet_set_device_nms(int mode);                     /* hard NMS: 0 = candidates copied back, sort + NMS on the host; 2 = on the device, only kept boxes cross
-                                                              PCIe; 1 (default) = chosen per batch from the previous result: on the device up to 2048 candidates per
-                                                              image, and up to 6144 unless forwards are pipelined and the host keeps up with them */
+                                                              PCIe; 1 (default) = chosen per batch from the results so far: inside the forward up to 1024 candidates per
+                                                              image, on the device up to 2048, and up to 6144 unless forwards are pipelined and the host keeps up
+                                                              with them */
 int msnhnet_set_tune_cache(int on);                       /* keep the per-layer tile search result in "<weights>.f16.tune" / ".f32.tune" next to the
                                                               .msnhbin file and reuse it on the next load (same graph, same device); off by default */
 int msnhnet_set_weight_cache(int on);                     /* keep the packed device-side kernels and the float16 calibration in "<weights>.f16.pack" /

@@ -365,7 +365,7 @@ public:
     bool lastOnDevice = false;             // where the NMS of the result fetched last ran
     bool copyOnForwardStream = false;      // copy-back (and device NMS) on the forward's stream instead of a stream of their own (NetGroup)
     // hard NMS on the device (only the kept boxes are copied back): 0 = never (sort + NMS on the host), 2 = always,
-    // 1 (default) = chosen per batch from the previous result: up to kDeviceNmsFew candidates per image on the device; up to
+    // 1 (default) = chosen per batch from the results so far: inside the forward (kImageNms); else up to kDeviceNmsFew candidates per image on the device; up to
     // kDeviceNmsCandidates (the largest class the device kernels take) on the device as well, except while forwards are pipelined and
     // the host stage keeps up with them -- the host then does it for free beside the next forward; more than that on the host.
     // "Keeps up" is measured: when the host stage stops waiting for the device, kTrialBatches batches run on the device and the

@@ -31,7 +31,8 @@ public:
     // keep the per-layer tile / algorithm choices next to the weights file ("<path>.msnhbin.tune"): the next load of the same
     // graph on the same device skips the search.  Off by default (the library then writes no files).
     // hard NMS of detection networks: 0 = candidates are copied back and sorted / suppressed on the host, 2 = on the device (only
-    // kept boxes are copied back), 1 (default) = on the device while the previous result had at most 2048 candidates per image
+    // kept boxes are copied back), 1 (default) = by the results so far: inside the forward up to 1024 candidates per image, on the device
+    // up to 2048 (YoloOutLayer::deviceNms)
     static void setDeviceNms(const int &mode);
     static void setTuneCache(const bool &on);
     static bool tuneCache;
