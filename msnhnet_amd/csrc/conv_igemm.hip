@@ -58,6 +58,52 @@ size_t igemmSplitKWorkspaceBytes(const msnh_conv_desc *d)
     return static_cast<size_t>(kSplitKMax) * d->batch * d->out_h * d->out_w * d->out_c * sizeof(float);
 }
 
+// MSNH_CONV_IGEMM_SPLITK (callers of the C interface; the plans use the sum inside the launch): the kernel with float32 results writes the raw partial sums
+// of its slices, slicePitch apart, and a second launch sums them in slice order (so the result does not depend on timing) and applies the
+// convolution's epilogue.  One thread per (pixel, 4 channels).
+template <typename T, typename TOut>
+__global__ __launch_bounds__(256) void splitKReduceKernel(IgemmArgs a, int outC, long long total)
+{
+    const long long idx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= total) return;
+    const int cq = outC / 4;
+    const int c = static_cast<int>(idx % cq) * 4;
+    const long long p = idx / cq;
+    const float *w = a.ws + static_cast<size_t>(p) * a.wsLd + c;
+    f32x4 acc = *reinterpret_cast<const f32x4 *>(w);
+    for (int s = 1; s < a.splitK; ++s) acc += *reinterpret_cast<const f32x4 *>(w + static_cast<size_t>(s) * a.P * a.wsLd);
+    const T *res = static_cast<const T *>(a.res);
+    TOut *y = static_cast<TOut *>(a.y);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        const float sc = a.scale ? a.scale[c + k] : 1.f;
+        const float sh = a.shift ? a.shift[c + k] : 0.f;
+        float v = activate(acc[k] * sc + sh, a.act, a.actParam);
+        if (a.hasRes) v = activate(v + a.resMul * toF(res[static_cast<size_t>(p) * a.resLd + c + k]), a.act2, a.act2Param);
+        y[static_cast<size_t>(p) * a.outLd + c + k] = fromF<TOut>(a.outMul * v);
+    }
+}
+
+static int convIgemmSplitK(IgemmArgs &a, const msnh_conv_desc *d, int tile, hipStream_t st)
+{
+    IgemmArgs e = a;
+    e.scale = e.shift = nullptr;
+    e.act = MSNH_ACT_NONE; e.hasRes = 0; e.res = nullptr; e.outMul = 1.f;
+    e.y = a.ws;
+    e.outLd = a.wsLd;
+    e.slicePitch = static_cast<size_t>(a.P) * a.wsLd;
+    e.vecOk = (a.wsLd % 8 == 0) && (a.coutG % 8 == 0 || d->groups == 1);
+    const int rc = d->dtype != MSNH_F16 ? igemmF32F32(e, d->groups, tile, st) : igemmF16F32(e, d->groups, tile, st);
+    if (rc != 0 || a.dryRun) return rc;
+    a.splitK = e.splitK;
+    const long long total = static_cast<long long>(a.P) * (d->out_c / 4);
+    const auto kern = d->dtype != MSNH_F16 ? splitKReduceKernel<float, float> : (d->out_dtype == MSNH_F16 ? splitKReduceKernel<f16, f16> : splitKReduceKernel<f16, float>);
+    hipLaunchKernelGGL(kern, dim3(gridFor(total, 256)), dim3(256), 0, st, a, d->out_c, total);
+    MSNH_LAUNCH_CHECK();
+    return 0;
+}
+
 // tail != nullptr: the launch also computes the 1x1 convolution described there (msnh_hip_conv2d_tail); d->tile then names one of the
 // tiles that carry a tail, 0 the first of them that takes the shape.
 static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
@@ -100,7 +146,7 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
     a.vecOk = (d->out_ld % 8 == 0) && ((d->out_c / d->groups) % 8 == 0 || d->groups == 1) &&
               (reinterpret_cast<uintptr_t>(y) % (8 * outEl) == 0) &&
               (!a.hasRes || (d->res_ld % 8 == 0 && reinterpret_cast<uintptr_t>(residual) % 16 == 0));
-    a.splitMax = 0; a.splitK = 1; a.fusedK = 0; a.wsNeed = a.wsBytes = 0; a.ws = nullptr; a.wsLd = d->out_c;
+    a.splitMax = 0; a.splitK = 1; a.fusedK = 0; a.wsNeed = a.wsBytes = 0; a.ws = nullptr; a.wsLd = d->out_c; a.slicePitch = 0;
     if (a.up2) MSNH_REQUIRE(d->algo != MSNH_CONV_IGEMM_SPLITK && !tail, "conv2d: the upsampling epilogue goes with the plain implicit GEMM");
     if (d->algo == MSNH_CONV_IGEMM_SPLITK)
     {
@@ -134,6 +180,7 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
     }
     if (tile <= 0 || tile > kIgemmTiles) tile = igemmHeuristicTile(d);
     MSNH_REQUIRE(d->dtype == MSNH_F16 || d->out_dtype == MSNH_F32, "igemm: float32 input needs float32 output");
+    if (a.splitMax > 1) return convIgemmSplitK(a, d, tile, st);
     const int rc = d->dtype != MSNH_F16 ? igemmF32F32(a, d->groups, tile, st)
                                         : (d->out_dtype == MSNH_F16 ? igemmF16F16(a, d->groups, tile, st) : igemmF16F32(a, d->groups, tile, st));
     if (wsNeed) *wsNeed = a.wsNeed;

@@ -47,6 +47,7 @@ struct IgemmArgs
     int fusedK;             // > 1: that many slices, summed inside the launch (splitKCombine)
     size_t wsNeed, wsBytes; // fusedK: workspace this launch needs / has
     float *ws;              // split-K: float32 partial sums [slice][pixel][out_c]
+    size_t slicePitch;      // elements of y between the results of two slices (split-K's partial sums; 0 otherwise)
     int wsLd;               // = out_c of the whole convolution
     int buffersOk;          // both extents fit a buffer resource
     int act, act2, hasRes, vecOk;
@@ -164,6 +165,10 @@ template <typename V> __device__ __forceinline__ V bufferLoad16(__amdgpu_buffer_
 // 3. every lane then owns 8 consecutive channels of a pixel: 16-byte residual loads and output stores through
 //    range-checked buffer resources (pixels past the end of the tensor are dropped by the hardware), the lanes of
 //    a pixel covering a contiguous run of channels.
+// Registers bound it: a 64 x 64 wave tile holds 64 accumulators of the 168 its three wavefronts per SIMD leave, and what does not fit goes through scratch
+// memory with a wait behind every residual load.  So there is one instance of it per kernel, a transcendental activation meets 16 values at a time, and the
+// rare paths are rolled loops.  (Raw partial sums as a second instance, 32 values per activation and the rare paths unrolled: 128 x 128 tile 27.8k instead
+// of 5.9k instructions and 218 instead of 0 values in scratch; yolov4 f16 b16 4396 -> 4204 us, yolov3 f16 b8 2076 -> 2011, resnet50 f16 b32 926 -> 897.)
 template <typename T> struct Raw8;               // 8 consecutive elements as loaded / stored
 template <> struct Raw8<f16>
 {
@@ -346,7 +351,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
     const bool full = a.vecOk && (mv + 7 < a.coutG);
     const unsigned ch = static_cast<unsigned>(chBase + mv);
     const int npix = min(a.P - p0, BN);
-    TOut    *yBlock = static_cast<TOut *>(a.y) + static_cast<size_t>(p0) * a.outLd;
+    TOut    *yBlock = static_cast<TOut *>(a.y) + blockIdx.y * a.slicePitch + static_cast<size_t>(p0) * a.outLd;
     const T *rBlock = static_cast<const T *>(a.res) + static_cast<size_t>(p0) * a.resLd;
     const __amdgpu_buffer_rsrc_t ry = a.up2 ? makeRsrc(a.y, a.yBytes) : makeRsrc(yBlock, static_cast<unsigned>(npix) * a.outLd * sizeof(TOut));
     const __amdgpu_buffer_rsrc_t rr = makeRsrc(a.hasRes ? rBlock : nullptr, a.hasRes ? static_cast<unsigned>(npix) * a.resLd * sizeof(T) : 0u);
@@ -358,7 +363,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
         constexpr int j = decltype(jTag)::value;
         const int pixBase = wn * TN + j * 32;         // first pixel of this column block inside the tile
         Raw8<T> resRaw[PASSES];
-        if (a.hasRes)
+        if (a.hasRes && lin2)
         {
 #pragma unroll
             for (int t = 0; t < PASSES; ++t)
@@ -367,45 +372,30 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
                 resRaw[t] = bufferLoad8<T>(rr, full ? (pl * a.resLd + ch) * static_cast<unsigned>(sizeof(T)) : kOobOffset);
             }
         }
-        auto stageBlock = [&](auto slopeTag) {
-            constexpr bool SL = decltype(slopeTag)::value;
-            if constexpr (SL)
-            {
-                staticFor<0, MB * 4>([&](auto iqTag) {
-                        constexpr int i = decltype(iqTag)::value / 4;
-                        constexpr int q = decltype(iqTag)::value % 4;
-                        const int ml = i * 32 + q * 8 + (lane >> 5) * 4;       // channel inside the wave tile
-                        const f32x4 sc = *reinterpret_cast<const f32x4 *>(ss + wm * TM + ml);
-                        const f32x4 sh = *reinterpret_cast<const f32x4 *>(ss + BM + wm * TM + ml);
-                        f32x4 v;
+        // (a 32 x 32 block at a time: with the transcendental activations over all blocks of the column at once the choice of the activation
+        // holds a wave tile's worth of values in registers that the tile has not got)
+        staticFor<0, MB>([&](auto iTag) {
+            constexpr int i = decltype(iTag)::value;
+            float v[16];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = activateSel<true>(acc[i][j][q * 4 + e] * sc[e] + sh[e], slope1, a.act, a.actParam);
-                        *reinterpret_cast<f32x4 *>(stage + (lane & 31) * LDE + ml) = v;
-                });
-            }
-            else
+            for (int q = 0; q < 4; ++q)
             {
-                // transcendental activations: affine on every accumulator first, then ONE choice of the activation for all of them
-                float t[MB * 16];
-                staticFor<0, MB * 4>([&](auto iqTag) {
-                        constexpr int iq = decltype(iqTag)::value;
-                        constexpr int i = iq / 4, q = iq % 4;
-                        const int ml = i * 32 + q * 8 + (lane >> 5) * 4;
-                        const f32x4 sc = *reinterpret_cast<const f32x4 *>(ss + wm * TM + ml);
-                        const f32x4 sh = *reinterpret_cast<const f32x4 *>(ss + BM + wm * TM + ml);
+                const int ml = i * 32 + q * 8 + (lane >> 5) * 4;       // channel inside the wave tile
+                const f32x4 sc = *reinterpret_cast<const f32x4 *>(ss + wm * TM + ml);
+                const f32x4 sh = *reinterpret_cast<const f32x4 *>(ss + BM + wm * TM + ml);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) t[iq * 4 + e] = acc[i][j][q * 4 + e] * sc[e] + sh[e];
-                });
-                activateArray<MB * 16>(t, a.act, a.actParam);
-                staticFor<0, MB * 4>([&](auto iqTag) {
-                        constexpr int iq = decltype(iqTag)::value;
-                        constexpr int i = iq / 4, q = iq % 4;
-                        const int ml = i * 32 + q * 8 + (lane >> 5) * 4;
-                        *reinterpret_cast<f32x4 *>(stage + (lane & 31) * LDE + ml) = f32x4{t[iq * 4], t[iq * 4 + 1], t[iq * 4 + 2], t[iq * 4 + 3]};
-                });
+                for (int e = 0; e < 4; ++e) v[q * 4 + e] = acc[i][j][q * 4 + e] * sc[e] + sh[e];
             }
-        };
-        if (lin1) stageBlock(std::true_type()); else stageBlock(std::false_type());
+            if (lin1)
+            {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) v[e] = activateSel<true>(v[e], slope1, a.act, a.actParam);
+            }
+            else activateArray<16>(v, a.act, a.actParam);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<f32x4 *>(stage + (lane & 31) * LDE + i * 32 + q * 8 + (lane >> 5) * 4) = f32x4{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
+        });
         // the staging area belongs to this wavefront alone, and the LDS serves a wavefront's accesses in the order it issued them: the
         // reads below see the writes above without a workgroup barrier (a barrier here kept the twelve wavefronts of a tile in step
         // through their stores)
@@ -413,73 +403,77 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
-        auto storeBlock = [&](auto slopeTag) {
-            constexpr bool SL = decltype(slopeTag)::value;
+        const auto readStaged = [&](int row, float (&v)[8]) {
+            const f32x4 lo = *reinterpret_cast<const f32x4 *>(stage + row * LDE + vcol);
+            const f32x4 hi = *reinterpret_cast<const f32x4 *>(stage + row * LDE + vcol + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+        };
+        const bool resLin = !a.hasRes || lin2;
+        if (full && resLin)
+        {
 #pragma unroll
             for (int t = 0; t < PASSES; ++t)
             {
                 const int row = t * RPI + lane / VPR;
                 const unsigned pl = pixBase + row;
                 float v[8];
-                const f32x4 lo = *reinterpret_cast<const f32x4 *>(stage + row * LDE + vcol);
-                const f32x4 hi = *reinterpret_cast<const f32x4 *>(stage + row * LDE + vcol + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
-                if (full)
+                readStaged(row, v);
+                if (a.hasRes)
                 {
-                    if (a.hasRes)
-                    {
-                        float r[8];
-                        resRaw[t].toFloat(r);
-                        if constexpr (SL)
-                        {
+                    float r[8];
+                    resRaw[t].toFloat(r);
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) v[e] = activateSel<true>(v[e] + a.resMul * r[e], slope2, a.act2, a.act2Param);
-                        }
-                        else
-                        {
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) v[e] += a.resMul * r[e];
-                            activateArray<8>(v, a.act2, a.act2Param);
-                        }
-                    }
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] *= a.outMul;
-                    Raw8<TOut> o;
-                    o.fromFloat(v);
-                    if (a.up2)
-                    {
-                        // pixel (image, row, column) -> the 2 x 2 pixels (2 row + dy, 2 column + dx) of the upsampled tensor
-                        const unsigned p = static_cast<unsigned>(p0) + pl;
-                        const unsigned t1 = fastDiv(p, a.byOW), bImg = fastDiv(t1, a.byOH);
-                        const unsigned ox = p - t1 * a.OW, oy = t1 - bImg * a.OH;
-                        const unsigned q = ((bImg * 2u * a.OH + 2u * oy) * 2u * a.OW + 2u * ox) * a.outLd + ch;
-                        const unsigned rowStep = 2u * a.OW * a.outLd;
-                        const unsigned es = static_cast<unsigned>(sizeof(TOut));
-                        const bool in = static_cast<int>(pl) < npix;
-                        bufferStore8<TOut>(o, ry, in ? q * es : kOobOffset);
-                        bufferStore8<TOut>(o, ry, in ? (q + a.outLd) * es : kOobOffset);
-                        bufferStore8<TOut>(o, ry, in ? (q + rowStep) * es : kOobOffset);
-                        bufferStore8<TOut>(o, ry, in ? (q + rowStep + a.outLd) * es : kOobOffset);
-                    }
-                    else bufferStore8<TOut>(o, ry, (pl * a.outLd + ch) * static_cast<unsigned>(sizeof(TOut)));
+                    for (int e = 0; e < 8; ++e) v[e] = activateSel<true>(v[e] + a.resMul * r[e], slope2, a.act2, a.act2Param);
                 }
-                else if (chOk && static_cast<int>(pl) < npix)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] *= a.outMul;
+                Raw8<TOut> o;
+                o.fromFloat(v);
+                if (a.up2)
                 {
-                    const T *rp = rBlock + static_cast<size_t>(pl) * a.resLd + ch;
-                    TOut *yp = yBlock + static_cast<size_t>(pl) * a.outLd + ch;
+                    // pixel (image, row, column) -> the 2 x 2 pixels (2 row + dy, 2 column + dx) of the upsampled tensor
+                    const unsigned p = static_cast<unsigned>(p0) + pl;
+                    const unsigned t1 = fastDiv(p, a.byOW), bImg = fastDiv(t1, a.byOH);
+                    const unsigned ox = p - t1 * a.OW, oy = t1 - bImg * a.OH;
+                    const unsigned q = ((bImg * 2u * a.OH + 2u * oy) * 2u * a.OW + 2u * ox) * a.outLd + ch;
+                    const unsigned rowStep = 2u * a.OW * a.outLd;
+                    const unsigned es = static_cast<unsigned>(sizeof(TOut));
+                    const bool in = static_cast<int>(pl) < npix;
+                    bufferStore8<TOut>(o, ry, in ? q * es : kOobOffset);
+                    bufferStore8<TOut>(o, ry, in ? (q + a.outLd) * es : kOobOffset);
+                    bufferStore8<TOut>(o, ry, in ? (q + rowStep) * es : kOobOffset);
+                    bufferStore8<TOut>(o, ry, in ? (q + rowStep + a.outLd) * es : kOobOffset);
+                }
+                else bufferStore8<TOut>(o, ry, (pl * a.outLd + ch) * static_cast<unsigned>(sizeof(TOut)));
+            }
+        }
+        else if (chOk)
+        {
+            // channels cut off inside a vector, unaligned rows, transcendental activations behind a residual: a pass at a time, the residual read where it
+            // is added (unrolled with the loads ahead, this is most of the kernel's instructions and the registers they need)
+#pragma unroll 1
+            for (int t = 0; t < PASSES; ++t)
+            {
+                const int row = t * RPI + lane / VPR;
+                const int pl = pixBase + row;
+                if (pl >= npix) continue;
+                float v[8];
+                readStaged(row, v);
+                const T *rp = rBlock + static_cast<size_t>(pl) * a.resLd + ch;
+                TOut *yp = yBlock + static_cast<size_t>(pl) * a.outLd + ch;
+                if (a.hasRes)
+                {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
-                        if (mv + e < a.coutG)
-                        {
-                            float o = v[e];
-                            if (a.hasRes) o = activateSel<SL>(o + a.resMul * toF(rp[e]), slope2, a.act2, a.act2Param);
-                            yp[e] = fromF<TOut>(a.outMul * o);
-                        }
+                        if (mv + e < a.coutG) v[e] += a.resMul * toF(rp[e]);
+                    activateArray<8>(v, a.act2, a.act2Param);
                 }
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (mv + e < a.coutG) yp[e] = fromF<TOut>(a.outMul * v[e]);
             }
-        };
-        if (lin2) storeBlock(std::true_type()); else storeBlock(std::false_type());
+        }
         if (j + 1 < NB)
         {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1148,49 +1142,10 @@ void convIgemmKernel(IgemmArgs a)
     }
     const int nTilesP = (a.P + BN - 1) / BN;
     const int nTiles = a.mTiles * nTilesP * static_cast<int>(gridDim.z), tileIdx = (g * nTilesP + pTile) * a.mTiles + mTile;
-    if (a.splitK > 1 && a.fusedK <= 1)
-    {
-        // raw float32 partial sums of this K slice; affine, activation and residual follow in the reduction pass
-        IgemmArgs e = a;
-        e.act = MSNH_ACT_NONE; e.hasRes = 0; e.outMul = 1.f;
-        e.y = a.ws + static_cast<size_t>(blockIdx.y) * a.P * a.wsLd;
-        e.outLd = a.wsLd;
-        e.vecOk = (a.wsLd % 8 == 0) && (a.coutG % 8 == 0 || gridDim.z == 1);
-        if constexpr (KG == 4) igemmEpilogueGather<T, float, BM, BN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wave, lane, g, 0, 0);
-        else if constexpr (KG == 2) igemmEpilogueSwap<T, float, BM, BN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64);
-        else igemmEpilogue<T, float, BM, BN, TM, TN>(e, acc, smemRaw, 1.f, 0.f, m0, p0, wm, wn, wave, lane, g);
-        return;
-    }
     if constexpr (KG == 4) igemmEpilogueGather<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wave, lane, g, tileIdx, nTiles);
     else if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles);
     else if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + igemmEpilogueLds<BM, TM, NT / 64>()))) return;
     else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g);
-}
-
-// MSNH_CONV_IGEMM_SPLITK (callers of the C interface; the plans use the sum inside the launch).  Split-K reduction: sums the K slices in slice order (so the result does not depend on timing) and applies the
-// convolution's epilogue.  One thread per (pixel, 4 channels).
-template <typename T, typename TOut>
-__global__ __launch_bounds__(256) void splitKReduceKernel(IgemmArgs a, int outC, long long total)
-{
-    const long long idx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int cq = outC / 4;
-    const int c = static_cast<int>(idx % cq) * 4;
-    const long long p = idx / cq;
-    const float *w = a.ws + static_cast<size_t>(p) * a.wsLd + c;
-    f32x4 acc = *reinterpret_cast<const f32x4 *>(w);
-    for (int s = 1; s < a.splitK; ++s) acc += *reinterpret_cast<const f32x4 *>(w + static_cast<size_t>(s) * a.P * a.wsLd);
-    const T *res = static_cast<const T *>(a.res);
-    TOut *y = static_cast<TOut *>(a.y);
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-    {
-        const float sc = a.scale ? a.scale[c + k] : 1.f;
-        const float sh = a.shift ? a.shift[c + k] : 0.f;
-        float v = activate(acc[k] * sc + sh, a.act, a.actParam);
-        if (a.hasRes) v = activate(v + a.resMul * toF(res[static_cast<size_t>(p) * a.resLd + c + k]), a.act2, a.act2Param);
-        y[static_cast<size_t>(p) * a.outLd + c + k] = fromF<TOut>(a.outMul * v);
-    }
 }
 
 constexpr int kSplitKMax = 8;
@@ -1285,13 +1240,6 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
     }
     hipLaunchKernelGGL(kern, grid, dim3(64 * WM * WN * KG), smem, st, a);
     MSNH_LAUNCH_CHECK();
-    if (a.splitK > 1 && a.fusedK <= 1)
-    {
-        const int outC = a.coutG * groups;
-        const long long total = static_cast<long long>(a.P) * (outC / 4);
-        hipLaunchKernelGGL((splitKReduceKernel<T, TOut>), dim3(gridFor(total, 256)), dim3(256), 0, st, a, outC, total);
-        MSNH_LAUNCH_CHECK();
-    }
     return 0;
 }
 

@@ -358,6 +358,36 @@ def test_conv_winograd_fused(b, c, h, w, oc, with_res):
     assert np.array_equal(y, y2)
 
 
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F16])
+@pytest.mark.parametrize("act,act2", [("mish", "none"), ("swish", "mish"), ("leaky", "swish"), ("relu6", "relu"), ("logistic", None)])
+@pytest.mark.parametrize("oc,pad_ld", [(200, 0), (93, 3)])
+def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
+    """The epilogue's paths on tiles of every wavefront grid: transcendental activations in front of and behind the residual, channel vectors cut off by
+    out_c, rows that are no multiple of eight channels, a last pixel tile of 13 x 11 pixels."""
+    import gpuutil as gu
+    b, c, h, w = 3, 72, 13, 11
+    rng = np.random.default_rng(oc + len(act))
+    x, wt = _case(rng, b, c, h, w, oc, 3)
+    res = rng.standard_normal((b, oc, h, w), dtype=np.float32) if act2 else None
+    scale = rng.uniform(0.5, 1.5, oc).astype(np.float32)
+    shift = (rng.standard_normal(oc) * 0.1).astype(np.float32)
+    if dtype == abi.F16:
+        x, wt = gu.round_f16(x), gu.round_f16(wt)
+        res = gu.round_f16(res) if act2 else None
+    ref = _ref(x, wt, 1, 1, 1, 1, scale, shift, act, 0.1, res, act2 or "none", 0.5, 2.0)
+    ran = 0
+    for tile in (1, 5, 6, 9, 13, 14, 31, 32, 36, 37, 38, 46, 52, 55, 58, 61, 64, 66, 67, 69):
+        try:
+            y, used = gu.conv2d(x, wt, dtype=dtype, stride=1, pad=1, scale=scale, shift=shift, act=act, residual=res, act2=act2 or "none", res_mul=0.5, out_mul=2.0,
+                                algo="igemm", tile=tile, out_ld=oc + pad_ld, res_ld=oc + pad_ld)
+        except abi.HipError as e:
+            assert "this tile" in str(e)
+            continue
+        ran += 1
+        assert gu.rel_err(y, ref) <= TOL[dtype], (tile, gu.rel_err(y, ref))
+    assert ran >= 15
+
+
 SPLITK_CASES = [
     # b, c, h, w, oc, k, stride, pad, groups
     (1, 512, 7, 7, 512, 3, 1, 1, 1),
