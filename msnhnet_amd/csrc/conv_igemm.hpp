@@ -139,6 +139,39 @@ __device__ __forceinline__ void mfmaBlock(const f32x4 &a, const f32x4 &b, f32x16
     c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[3], b[3], c, 0, 0, 0);
 }
 
+// float32 products on the bfloat16 matrix cores.  A float32 value is the sum of three bfloat16 values (8 + 8 + 8 significant bits, each the rounded
+// remainder of the one before), and of the nine products of two such sums the six largest carry all but 2^-26 of the product:
+//     a b  ~  ah bh + (ah bm + am bh) + (am bm + ah bl + al bh)
+// Six 32x32x16 bfloat16 MFMAs take 192 cycles for 16 k where the eight 32x32x2 float32 MFMAs take 512.  The five small products go into an
+// accumulator of their own: added to the large one they would be rounded at its magnitude five times per 16 k, apart from it they are not, and the
+// large one is rounded once per 16 k instead of eight times.  Against 64-bit sums, normal and rectified operands, K = 576 / 4608: 1.3e-7 / 4.2e-7 of
+// the results' rms, where the float32 MFMAs give 4.4e-7 / 1.2e-6 (one accumulator for all six: 3.7e-7 / 1.1e-6).
+// bfloat16 has float32's exponents, so nothing overflows that did not before, apart from values within a half of 2^-8 of the largest float32; an infinity
+// times a piece that is zero is NaN, however, where the float32 product is an infinity.  Every result that such an operand reaches is not finite
+// either way, so a workgroup that finds a result that is not finite multiplies its tile again with the float32 MFMAs.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// 8 values in 44 vector instructions: a conversion rounds two values, a shift and a mask widen them again.
+__device__ __forceinline__ void splitF32(const f32x4 &a, const f32x4 &b, bf16x8 &hi, bf16x8 &mid, bf16x8 &lo)
+{
+    u32x4 h, m, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+    {
+        const float v0 = e < 2 ? a[2 * e] : b[2 * e - 4], v1 = e < 2 ? a[2 * e + 1] : b[2 * e - 3];
+        h[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
+        const float r0 = v0 - __builtin_bit_cast(float, h[e] << 16), r1 = v1 - __builtin_bit_cast(float, h[e] & 0xffff0000u);
+        m[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
+        const float s0 = r0 - __builtin_bit_cast(float, m[e] << 16), s1 = r1 - __builtin_bit_cast(float, m[e] & 0xffff0000u);
+        l[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{s0, s1}, bf16x2));
+    }
+    hi = __builtin_bit_cast(bf16x8, h);
+    mid = __builtin_bit_cast(bf16x8, m);
+    lo = __builtin_bit_cast(bf16x8, l);
+}
+
 // 16-byte load through a buffer resource: the address is base + voffset + soffset with a hardware range check of
 // voffset against the resource size, so a lane whose row, tap or channel falls outside the tensor simply carries an
 // out-of-range voffset and reads zeros -- no branches, no 64-bit address arithmetic in the loop.
@@ -257,6 +290,27 @@ template <int I, int N, typename F> __device__ __forceinline__ void staticFor(F 
         f(std::integral_constant<int, I>());
         staticFor<I + 1, N>(f);
     }
+}
+
+template <int MB, int NB> __device__ __forceinline__ void clearBlocks(f32x16 (&c)[MB][NB])
+{
+    staticFor<0, MB * NB>([&](auto ijTag) {
+        constexpr int i = decltype(ijTag)::value / NB, j = decltype(ijTag)::value % NB;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) c[i][j][r] = 0.f;
+    });
+}
+
+// One 16-k block of the split product, products outermost so that an accumulator's MFMAs do not follow each other.  (Pieces: 0 high, 1 middle, 2 low.)
+template <int MB, int NB>
+__device__ __forceinline__ void mfmaSplit(const bf16x8 (&a)[3][MB], const bf16x8 (&b)[3][NB], f32x16 (&acc)[MB][NB], f32x16 (&low)[MB][NB])
+{
+    staticFor<0, 6 * MB * NB>([&](auto tTag) __attribute__((always_inline)) {
+        constexpr int t = decltype(tTag)::value / (MB * NB), i = decltype(tTag)::value / NB % MB, j = decltype(tTag)::value % NB;
+        constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+        if constexpr (t < 5) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[t]][i], b[pb[t]][j], low[i][j], 0, 0, 0);
+        else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[t]][i], b[pb[t]][j], acc[i][j], 0, 0, 0);
+    });
 }
 
 template <int BM, int TM, int NW = 4> constexpr size_t igemmEpilogueLds() { return (2 * BM + NW * 32 * (TM + 4)) * sizeof(float); }
@@ -505,17 +559,21 @@ __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&a
     auto swap = [&](auto gTag) {
         constexpr int q = decltype(gTag)::value;
         float *put = xch + (wt * 2 + q) * kSwapRegion + lane;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
+        staticFor<0, 2>([&](auto iTag) {
+            constexpr int i = decltype(iTag)::value;
 #pragma unroll
             for (int r = 0; r < 16; ++r) put[(i * 16 + r) * 64] = acc[i][1 - q][r];
+        });
         __syncthreads();
         stageOwn = xch + (wt * 2 + (1 - q)) * kSwapRegion;
         const float *get = stageOwn + lane;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
+        staticFor<0, 2>([&](auto iTag) {
+            constexpr int i = decltype(iTag)::value;
 #pragma unroll
             for (int r = 0; r < 16; ++r) mine[i][0][r] = acc[i][q][r] + get[(i * 16 + r) * 64];
+        });
+        // (differs between the groups, or their code is merged over a pointer to the accumulators, which then live in memory)
+        asm volatile("; k-group %0" ::"n"(q));
     };
     if (kg == 0) swap(std::integral_constant<int, 0>()); else swap(std::integral_constant<int, 1>());
     // (the partner's sums are in registers before the staging writes below reach the same region: one wavefront's LDS accesses are served in order)
@@ -576,6 +634,36 @@ constexpr int igemmWavesPerSimd(int bm, int bn, int kv = 8, int ns = 3, int nw =
     // live on memory bandwidth)
     if (ns == 2 && kv == 4 && bm * bn <= 64 * 128) return bm * bn > 64 * 64 ? 6 : 8;
     return bm * bn > 128 * 128 ? 2 : (bm * bn > 64 * 128 ? 3 : (bm * bn > 64 * 64 ? 4 : 6));
+}
+
+// float32 tiles whose wavefronts have the registers for the split product (splitF32): per 32 x 32 block two accumulators, per block row and column the
+// three pieces and the values they come from.  The others multiply with the float32 MFMAs, and so do those with one block per wavefront: there the split
+// of two operands (88 vector instructions) costs what the matrix cores save, 3x3 64 -> 64 at 56 x 56 8.66 -> 9.21 us, 256 -> 256 at 14 x 14 11.2 -> 11.9.
+// The others, start -> now: 3x3 256 -> 512 at 38 x 38 eight images 214 -> 172 us, one image 38.2 -> 32.2; 128 -> 256 at 76 x 76 eight images 223 -> 173;
+// 1x1 512 -> 256 at 38 x 38 eight images 32.3 -> 28.0.  What binds then is the bfloat16 rate under load: 159 x 6 = 954 TFLOP/s where a large matrix product gets 1120.
+constexpr int igemmSplitRegs(int mb, int nb) { return 32 * mb * nb + 20 * (mb + nb) + 40; }
+constexpr bool igemmSplits(int bm, int bn, int wm, int wn, int kg)
+{
+    const int mb = bm / wm / 32, nb = bn / wn / 32;
+    return mb * nb >= 2 && mb * nb <= 4 && igemmSplitRegs(mb, nb) <= 512 / ((wm * wn * kg + 3) / 4);
+}
+
+template <typename T> constexpr int igemmWavesMin(int bm, int bn, int kv, int wm, int wn, int ns, int kg)
+{
+    const int nw = wm * wn * kg;
+    if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg)) return (nw + 3) / 4;
+    return kg == 4 ? 1 : kg == 2 ? nw / 4 : igemmWavesPerSimd(bm, bn, kv, ns, nw);
+}
+
+template <typename T> constexpr int igemmWavesMax(int bm, int bn, int kv, int wm, int wn, int ns, int kg)
+{
+    const int nw = wm * wn * kg;
+    if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg))
+    {
+        const int fit = 512 / igemmSplitRegs(bm / wm / 32, bn / wn / 32);
+        return fit > nw / 4 ? fit : nw / 4;
+    }
+    return kg == 4 ? 4 : kg == 2 ? (nw == 4 ? 3 : nw / 4) : igemmWavesPerSimd(bm, bn, kv, ns, nw);
 }
 
 // 16-byte-per-lane load from a buffer resource straight into LDS: the 64 lanes of the wave fill 1 KiB starting at
@@ -870,8 +958,7 @@ __device__ __forceinline__ void igemmTailEpilogue(const IgemmArgs &a, f32x16 (&a
 // TAIL = 1: the epilogue also computes the 1x1 convolution that reads this one's result (igemmTailEpilogue); float16 only.
 template <typename T, typename TOut, int BM, int BN, int KV, int WM, int WN, int NS, int KG = 1, int TAIL = 0>
 __global__ __launch_bounds__(64 * WM * WN * KG)
-__attribute__((amdgpu_waves_per_eu(KG == 4 ? 1 : KG == 2 ? (WM * WN * KG) / 4 : igemmWavesPerSimd(BM, BN, KV, NS, WM * WN),
-                                   KG == 4 ? 4 : KG == 2 ? (WM * WN * KG == 4 ? 3 : (WM * WN * KG) / 4) : igemmWavesPerSimd(BM, BN, KV, NS, WM * WN))))
+__attribute__((amdgpu_waves_per_eu(igemmWavesMin<T>(BM, BN, KV, WM, WN, NS, KG), igemmWavesMax<T>(BM, BN, KV, WM, WN, NS, KG))))
 void convIgemmKernel(IgemmArgs a)
 {
     typedef typename Frag<T>::V V;
@@ -1044,12 +1131,7 @@ void convIgemmKernel(IgemmArgs a)
     };
 
     f32x16 acc[MB][NB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    clearBlocks(acc);
 
     // NS >= 3 LDS stages rotate: while tile step `it` is multiplied out of stage `cur`, steps it+1 .. it+NS-2 are
     // already (being) delivered into the following stages and the loads of step it+NS-1 go into the stage before
@@ -1073,66 +1155,150 @@ void convIgemmKernel(IgemmArgs a)
     constexpr int INFLIGHT = NS >= 3 ? (NS - 3) * NL + NPRE : 0;   // loads younger than step it+1's at the barrier
 
     const bool tailPrefetch = TAIL != 0 && a.hasRes && nLocal >= 2;
-    tapNext = tapFirst;
-    chunkNext = chunkFirst - 1;                               // advance() steps onto the first tile step
-    setTap(tapNext);
-    staticFor<0, AHEAD>([&](auto stTag) {
-        constexpr int st = decltype(stTag)::value;
-        advance(nLocal <= st);
-        staticFor<st == 0 ? AROWS : 0, NL>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, st * STAGE); });     // (step 0: the filters are on their way)
-    });
-    dmaWait<(AHEAD - 1) * NL>();                 // step 0 has landed
-    __syncthreads();
-    readFrags(0, std::integral_constant<int, 0>());
+    // The loads of the first AHEAD tile steps; skip: of the first one's, how many are on their way already.
+    auto fillStages = [&](auto skip) {
+        tapNext = tapFirst;
+        chunkNext = chunkFirst - 1;                           // advance() steps onto the first tile step
+        setTap(tapNext);
+        staticFor<0, AHEAD>([&](auto stTag) {
+            constexpr int st = decltype(stTag)::value;
+            advance(nLocal <= st);
+            staticFor<st == 0 ? decltype(skip)::value : 0, NL>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, st * STAGE); });
+        });
+        dmaWait<(AHEAD - 1) * NL>();             // step 0 has landed
+        __syncthreads();
+    };
 
-    // cur: stage of step it; nxt: of step it+1; nn: where the loads issued during step it go
-    unsigned cur = 0, nxt = STAGE, nn = NS >= 3 ? (NS - 1) * STAGE : 0;
-    for (int it = 0; it < nLocal; ++it)
-    {
-        advance(it + AHEAD >= nLocal);          // sANext / sBNext / cutNext now describe step it + AHEAD
-        readFrags(cur, std::integral_constant<int, 1>());
-        __builtin_amdgcn_sched_barrier(0);
-        staticFor<0, TOT>([&](auto gTag) {
-            constexpr int gi = decltype(gTag)::value;
-            constexpr int ks = gi / PER;
-            if constexpr (gi % PER == 0 && ks >= 1)
-            {
-                if constexpr (ks < S - 1)
-                    readFrags(cur, std::integral_constant<int, ks + 1>());
-                else
+    auto multiply = [&]() {
+        readFrags(0, std::integral_constant<int, 0>());
+
+        // cur: stage of step it; nxt: of step it+1; nn: where the loads issued during step it go
+        unsigned cur = 0, nxt = STAGE, nn = NS >= 3 ? (NS - 1) * STAGE : 0;
+        for (int it = 0; it < nLocal; ++it)
+        {
+            advance(it + AHEAD >= nLocal);          // sANext / sBNext / cutNext now describe step it + AHEAD
+            readFrags(cur, std::integral_constant<int, 1>());
+            __builtin_amdgcn_sched_barrier(0);
+            staticFor<0, TOT>([&](auto gTag) {
+                constexpr int gi = decltype(gTag)::value;
+                constexpr int ks = gi / PER;
+                if constexpr (gi % PER == 0 && ks >= 1)
                 {
-                    dmaWait<INFLIGHT>();         // all of step it+1 has landed; younger loads may be in flight
-                    __syncthreads();
-                    if constexpr (TAIL != 0)
+                    if constexpr (ks < S - 1)
+                        readFrags(cur, std::integral_constant<int, ks + 1>());
+                    else
                     {
-                        // the residual tile of the epilogue: the rows that lie behind the loop's stages right away, the others into the
-                        // stage of this step -- free from here on -- in the last step but one
-                        if (tailPrefetch && it == 0) tailIssueResidual<BM, BN, STAGE, NT / 64>(a, p0, ldsBase, wave, lane, true, 0u);
-                        if (tailPrefetch && it == nLocal - 2 && TailLds<BM, BN, STAGE>::LOWROWS > 0)
-                            tailIssueResidual<BM, BN, STAGE, NT / 64>(a, p0, ldsBase, wave, lane, false, TailLds<BM, BN, STAGE>::lowOff(nLocal & 1));
+                        dmaWait<INFLIGHT>();         // all of step it+1 has landed; younger loads may be in flight
+                        __syncthreads();
+                        if constexpr (TAIL != 0)
+                        {
+                            // the residual tile of the epilogue: the rows that lie behind the loop's stages right away, the others into the
+                            // stage of this step -- free from here on -- in the last step but one
+                            if (tailPrefetch && it == 0) tailIssueResidual<BM, BN, STAGE, NT / 64>(a, p0, ldsBase, wave, lane, true, 0u);
+                            if (tailPrefetch && it == nLocal - 2 && TailLds<BM, BN, STAGE>::LOWROWS > 0)
+                                tailIssueResidual<BM, BN, STAGE, NT / 64>(a, p0, ldsBase, wave, lane, false, TailLds<BM, BN, STAGE>::lowOff(nLocal & 1));
+                        }
+                        readFrags(nxt, std::integral_constant<int, 0>());
                     }
-                    readFrags(nxt, std::integral_constant<int, 0>());
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                mfmaBlock(fa[ks % 2][(gi % PER) / NB], fb[ks % 2][(gi % PER) % NB], acc[(gi % PER) / NB][(gi % PER) % NB]);
+                if constexpr (gi >= LBASE)
+                {
+                    // loads l with LBASE + l * LSPAN / NL == gi
+                    constexpr int first = ((gi - LBASE) * NL + LSPAN - 1) / LSPAN;
+                    constexpr int last  = ((gi - LBASE + 1) * NL + LSPAN - 1) / LSPAN;
+                    // (TAIL: the stages that steps past the end of K would zero receive residual rows instead)
+                    if (!(TAIL != 0 && pastEndNext))
+                        staticFor<first, last>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, nn); });
                 }
                 __builtin_amdgcn_sched_barrier(0);
-            }
-            mfmaBlock(fa[ks % 2][(gi % PER) / NB], fb[ks % 2][(gi % PER) % NB], acc[(gi % PER) / NB][(gi % PER) % NB]);
-            if constexpr (gi >= LBASE)
+            });
+            nn = NS >= 3 ? cur : nxt;
+            cur = nxt;
+            nxt = nxt + STAGE == NS * STAGE ? 0u : nxt + STAGE;
+        }
+    };
+
+    // The same over 16 k a time as split products (float32): the values of a pair of k-blocks are split as soon as they are in registers, and the next pair
+    // is read while the six products are multiplied.  The barrier sits behind the split of the step's last pair: its stage is free from there on.
+    [[maybe_unused]] auto multiplySplit = [&]() {
+        constexpr int S2     = S / 2;            // pairs of k-blocks per tile step and wavefront
+        constexpr int NPRE2  = NS >= 3 ? (S2 - 1) * NL / S2 : 0;              // loads of a step in front of its barrier
+        constexpr int INFL2  = NS >= 3 ? (NS - 3) * NL + NPRE2 : 0;
+        f32x16 low[MB][NB];
+        clearBlocks(low);
+        unsigned cur = 0, nxt = STAGE, nn = NS >= 3 ? (NS - 1) * STAGE : 0;
+        readFrags(0, std::integral_constant<int, 0>());
+        readFrags(0, std::integral_constant<int, 1>());
+        for (int it = 0; it < nLocal; ++it)
+        {
+            advance(it + AHEAD >= nLocal);
+            staticFor<0, S2>([&](auto pTag) {
+                constexpr int p = decltype(pTag)::value;
+                bf16x8 sa[3][MB], sb[3][NB];
+                if constexpr (std::is_same<T, float>::value)
+                {
+#pragma unroll
+                    for (int i = 0; i < MB; ++i) splitF32(fa[0][i], fa[1][i], sa[0][i], sa[1][i], sa[2][i]);
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) splitF32(fb[0][j], fb[1][j], sb[0][j], sb[1][j], sb[2][j]);
+                }
+                if constexpr (p < S2 - 1)
+                {
+                    readFrags(cur, std::integral_constant<int, 2 * p + 2>());
+                    readFrags(cur, std::integral_constant<int, 2 * p + 3>());
+                }
+                else
+                {
+                    dmaWait<INFL2>();
+                    __syncthreads();
+                    readFrags(nxt, std::integral_constant<int, 0>());
+                    readFrags(nxt, std::integral_constant<int, 1>());
+                }
+                // pair p of S2 takes loads [p NL / S2, (p + 1) NL / S2); two stages: all of them follow the barrier
+                constexpr int first = NS >= 3 ? p * NL / S2 : (p == S2 - 1 ? 0 : NL);
+                constexpr int last  = NS >= 3 ? (p + 1) * NL / S2 : NL;
+                staticFor<first, last>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, nn); });
+                mfmaSplit<MB, NB>(sa, sb, acc, low);
+            });
+            nn = NS >= 3 ? cur : nxt;
+            cur = nxt;
+            nxt = nxt + STAGE == NS * STAGE ? 0u : nxt + STAGE;
+        }
+        float probe = 0.f;                       // NaN from the first result that is not finite
+        staticFor<0, MB * NB>([&](auto ijTag) {
+            constexpr int i = decltype(ijTag)::value / NB, j = decltype(ijTag)::value % NB;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
             {
-                // loads l with LBASE + l * LSPAN / NL == gi
-                constexpr int first = ((gi - LBASE) * NL + LSPAN - 1) / LSPAN;
-                constexpr int last  = ((gi - LBASE + 1) * NL + LSPAN - 1) / LSPAN;
-                // (TAIL: the stages that steps past the end of K would zero receive residual rows instead)
-                if (!(TAIL != 0 && pastEndNext))
-                    staticFor<first, last>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, nn); });
+                acc[i][j][r] += low[i][j][r];
+                probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
             }
-            __builtin_amdgcn_sched_barrier(0);
         });
-        nn = NS >= 3 ? cur : nxt;
-        cur = nxt;
-        nxt = nxt + STAGE == NS * STAGE ? 0u : nxt + STAGE;
+        return probe != 0.f;
+    };
+
+    fillStages(std::integral_constant<int, AROWS>());         // (step 0: the filters are on their way)
+    if constexpr (std::is_same<T, float>::value && igemmSplits(BM, BN, WM, WN, KG))
+    {
+        const bool odd = multiplySplit();
+        dmaWait<0>();
+        if (__syncthreads_or(odd))
+        {
+            clearBlocks(acc);
+            fillStages(std::integral_constant<int, 0>());
+            multiply();
+            dmaWait<0>();
+            __syncthreads();
+        }
     }
-    dmaWait<0>();
-    __syncthreads();
+    else
+    {
+        multiply();
+        dmaWait<0>();
+        __syncthreads();
+    }
 
     if constexpr (TAIL != 0)
     {

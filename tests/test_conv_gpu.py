@@ -388,6 +388,46 @@ def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
     assert ran >= 15
 
 
+@pytest.mark.parametrize("tile", [1, 5, 9, 23, 32, 36, 38, 41, 58, 61, 69])
+@pytest.mark.parametrize("c,oc,k", [(256, 96, 3), (40, 72, 1), (64, 130, 3)])
+def test_conv_f32_split_products(c, oc, k, tile):
+    """float32 tiles that multiply bfloat16 pieces: their error against 64-bit sums is that of one float32 rounding per 16 products.  With partial sums that grow
+    like a random walk, n = K / 16 roundings of relative size 2^-24 / sqrt(3) leave 2^-24 / sqrt(3) * sqrt(n / 2) of the results' rms; 1.5 times that, and 2^-24
+    for the affine and the pieces left out."""
+    import torch
+    import gpuutil as gu
+    rng = np.random.default_rng(c + oc + tile)
+    x, wt = _case(rng, 2, c, 19, 17, oc, k)
+    y, _ = gu.conv2d(x, wt, dtype=abi.F32, stride=1, pad=k // 2, algo="igemm", tile=tile)
+    ref = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), padding=k // 2).numpy()
+    err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    assert err <= 2.0 ** -24 * (1.5 * np.sqrt(c * k * k / 16 / 6) + 1), err
+
+
+@pytest.mark.parametrize("tile", [2, 5, 23, 36, 38, 58, 61, 69])
+@pytest.mark.parametrize("slices", [0, 2])
+def test_conv_f32_split_products_not_finite(slices, tile):
+    """Infinities, NaN and the largest values, against filters with zero pieces: the same classes of results as float32 products give"""
+    import gpuutil as gu
+    rng = np.random.default_rng(tile)
+    x, wt = _case(rng, 1, 64, 12, 11, 72, 3)
+    wt[:, :8] = 0.5                                     # exact in bfloat16: middle and low piece are zero
+    for v, (ch, r, col) in zip((np.inf, -np.inf, np.nan, 3.4e38, np.inf), ((3, 2, 2), (5, 6, 9), (40, 10, 5), (7, 0, 0), (60, 11, 10))):
+        x[0, ch, r, col] = v
+    wt[9, 33, 1, 1] = np.inf
+    kw = dict(dtype=abi.F32, stride=1, pad=1)
+    L = abi.lib()
+    ref = _ref(x, wt, 1, 1, 1, 1, None, None, "none", 0.1, None, "none", 1.0, 1.0)
+    if slices:
+        d = abi.ConvDesc(abi.F32, abi.F32, 1, 12, 11, 64, 64, 72, 12, 11, 72, 3, 1, 1, 1, 1, 0, 0.1, 0, 72, 0, 0.1, 1.0, 1.0, abi.ALGO["igemm_splitk"], tile)
+        if not L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), tile):
+            pytest.skip("the tile takes no slices of this shape")
+        y, _ = gu.conv2d(x, wt, algo="igemm_splitk", tile=tile, **kw)
+    else:
+        y, _ = gu.conv2d(x, wt, algo="igemm", tile=tile, **kw)
+    assert gu.rel_err(y, ref) <= TOL[abi.F32]
+
+
 SPLITK_CASES = [
     # b, c, h, w, oc, k, stride, pad, groups
     (1, 512, 7, 7, 512, 3, 1, 1, 1),
