@@ -127,6 +127,10 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
     a.yBytes = a.up2 ? static_cast<unsigned>(static_cast<unsigned long long>(d->batch) * d->out_h * d->out_w * 4ull * d->out_ld * dtypeSize(d->out_dtype)) : 0u;
     a.byOW = makeFastDiv(static_cast<unsigned>(d->out_w));
     a.byOH = makeFastDiv(static_cast<unsigned>(d->out_h));
+    a.byKsize = makeFastDiv(static_cast<unsigned>(d->ksize));
+    a.tapRows = 0;
+    if (a.taps <= 64) for (int q = 0; q < d->ksize; ++q) a.tapRows |= 1ull << (q * d->ksize);      // (more taps are refused)
+    a.pointwise = d->ksize == 1 && d->stride == 1 && d->pad == 0 ? 1 : 0;
     a.patchOk = (d->ksize == 3 && d->stride == 1 && d->pad == 1 && d->dilation == 1 && d->groups == 1 && d->out_h == d->in_h && d->out_w == d->in_w) ? 1 : 0;
     a.patchRows = 0; a.mTiles = 0; a.cChunks = 0; a.nIter = 0;
     a.dryRun = dryRun ? 1 : 0;

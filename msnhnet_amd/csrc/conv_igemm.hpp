@@ -55,6 +55,12 @@ struct IgemmArgs
     FastDiv byOW, byOH;     // pixel index -> (image, row, column) without hardware-less integer division
     int xcdGm;              // > 1: the XCDs form an xcdGm x (8 / xcdGm) grid over (channel tiles, pixel tiles), see igemmTileOf
     int xcdMPer, xcdPPer;   // channel tiles / pixel tiles per XCD in that arrangement
+    int nTilesP, tiles;     // pixel tiles; channel tiles x pixel tiles
+    int tilesPerXcd, xcdGmLog2;
+    FastDiv byMTiles, byXcdMPer;
+    FastDiv bySplitK, byChunks, byKsize;
+    unsigned long long tapRows;   // bit ki * ksize for every filter row ki
+    int pointwise;          // 1x1, no padding, stride 1: the input pixel is the output pixel
     int up2;                // every result pixel goes to the 2 x 2 pixels of y it maps to under nearest-neighbour upsampling (y: [batch][2 OH][2 OW])
     unsigned yBytes;        // up2: extent of y in bytes
     // tail (tiles with TAIL = 1 only): a 1x1 stride-1 convolution z = zMul * act3(scale2 * (W2 . y) + shift2) of this convolution's
@@ -74,35 +80,46 @@ struct IgemmArgs
 // tile and XCD -- and every XCD fetches every filter.  Where the filters outweigh the input (512 -> 1024 channels over
 // 19 x 19 pixels: 9.4 MB against 3 MB) the host asks for an xcdGm x (8 / xcdGm) arrangement instead: an XCD owns a block of
 // channel tiles and a block of pixel tiles and fetches only that share of the filters and that share of the input.
-__device__ __forceinline__ bool igemmTileOf(const IgemmArgs &a, int nTilesP, int &mTile, int &pTile)
+__device__ __forceinline__ bool igemmTileOf(const IgemmArgs &a, int &mTile, int &pTile)
 {
-    const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
+    const unsigned xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
     if (a.xcdGm <= 1)
     {
-        const int total   = a.mTiles * nTilesP;
-        const int perXcd  = (total + 7) / 8;
-        const int logical = xcd * perXcd + idx;
-        mTile = logical % a.mTiles;
-        pTile = logical / a.mTiles;
-        return logical < total;                       // padding ids of the last round
+        const unsigned logical = xcd * a.tilesPerXcd + idx;
+        pTile = static_cast<int>(fastDiv(logical, a.byMTiles));
+        mTile = static_cast<int>(logical) - pTile * a.mTiles;
+        return static_cast<int>(logical) < a.tiles;   // padding ids of the last round
     }
-    const int lp = idx / a.xcdMPer;
-    mTile = (xcd % a.xcdGm) * a.xcdMPer + (idx - lp * a.xcdMPer);
-    pTile = (xcd / a.xcdGm) * a.xcdPPer + lp;
-    return lp < a.xcdPPer && mTile < a.mTiles && pTile < nTilesP;
+    const int lp = static_cast<int>(fastDiv(idx, a.byXcdMPer));
+    mTile = static_cast<int>(xcd & (a.xcdGm - 1)) * a.xcdMPer + (static_cast<int>(idx) - lp * a.xcdMPer);
+    pTile = static_cast<int>(xcd >> a.xcdGmLog2) * a.xcdPPer + lp;
+    return lp < a.xcdPPer && mTile < a.mTiles && pTile < a.nTilesP;
+}
+
+// One word of every 64-byte line of the arguments, so that all lines are in the scalar cache after one trip to memory.  The compiler loads a field where
+// it is used, and the cache is cold at the start of a launch: the chain tile -> addresses -> first load met four such trips one after the other.
+// With that, divisions by reciprocals from the host, tap masks without loops and the affines published by the loop's barriers: yolov3 f16 b1 746 -> 690 us
+// (75 convolutions), yolov5s f16 b3 609 -> 581, resnet50 f16 b32 897 -> 816 (on one box 870 -> 816 from the start of both steps), yolov3 f32 b1 1919 -> 1819.
+__device__ __forceinline__ void touchArgs(const IgemmArgs &a)
+{
+    static_assert(sizeof(IgemmArgs) > 6 * 64 && sizeof(IgemmArgs) <= 8 * 64, "lines to touch");
+    const int *q = reinterpret_cast<const int *>(&a);
+    asm volatile("" ::"s"(q[0]), "s"(q[16]), "s"(q[32]), "s"(q[48]), "s"(q[64]), "s"(q[80]), "s"(q[96]), "s"(q[(sizeof(IgemmArgs) - 4) / 4]));
 }
 
 // grid.x of a launch over a.mTiles x nTilesP tiles, and the XCD arrangement it runs under (see igemmTileOf).  a.xcdGm comes in as
 // the caller's wish (msnh_conv_desc::xcd_blocks): 1, 2, 4, 8 are taken as they are; 0 picks the arrangement that makes the eight
 // L2s fetch the fewest bytes, counted as (8 / g) x filters + g x input -- the default one stays unless another saves a quarter
-// of that without more workgroup slots per XCD.  Grouped and split-K launches (plainGrid false) keep the default.
+// of that without more workgroup slots per XCD.  Grouped and split-K launches (plainGrid false) keep the default.  Also fills in what igemmTileOf divides by.
 inline unsigned igemmGridX(IgemmArgs &a, int nTilesP, size_t es, bool plainGrid)
 {
     static const bool off = std::getenv("MSNH_NO_XCD_BLOCKS") != nullptr;      // (for A/B timing of whole networks)
     const int wish = a.xcdGm;
     const int tiles = a.mTiles * nTilesP;
     const unsigned plain = static_cast<unsigned>((tiles + 7) / 8 * 8);
-    a.xcdGm = 1; a.xcdMPer = a.mTiles; a.xcdPPer = nTilesP;
+    a.xcdGm = 1; a.xcdGmLog2 = 0; a.xcdMPer = a.mTiles; a.xcdPPer = nTilesP;
+    a.nTilesP = nTilesP; a.tiles = tiles; a.tilesPerXcd = static_cast<int>(plain / 8);
+    a.byMTiles = a.byXcdMPer = makeFastDiv(static_cast<unsigned>(a.mTiles));
     if (!plainGrid || wish == 1 || (wish == 0 && off)) return plain;
     const double wB = static_cast<double>(a.coutG) * a.taps * a.cinG * es;
     const double xB = static_cast<double>(a.batch) * a.H * a.W * a.cinG * es;
@@ -114,8 +131,9 @@ inline unsigned igemmGridX(IgemmArgs &a, int nTilesP, size_t es, bool plainGrid)
         const int gp = 8 / gm, mPer = (a.mTiles + gm - 1) / gm, pPer = (nTilesP + gp - 1) / gp;
         const double cost = gp * wB + gm * xB;
         const bool take = wish == gm || (wish == 0 && 8 * mPer * pPer <= static_cast<int>(plain) && cost < need && cost < best);
-        if (take) { best = cost; a.xcdGm = gm; a.xcdMPer = mPer; a.xcdPPer = pPer; grid = 8u * mPer * pPer; }
+        if (take) { best = cost; a.xcdGm = gm; a.xcdGmLog2 = gm == 2 ? 1 : gm == 4 ? 2 : 3; a.xcdMPer = mPer; a.xcdPPer = pPer; grid = 8u * mPer * pPer; }
     }
+    a.byXcdMPer = makeFastDiv(static_cast<unsigned>(a.xcdMPer));
     return grid;
 }
 
@@ -375,8 +393,8 @@ __device__ __forceinline__ bool splitKCombine(float *ws, int slices, f32x16 (&ac
     return true;
 }
 
-// ssReady / stageOwn (the K-split epilogue): the affines already stand at ssReady, published by a barrier the caller has passed, and this
-// wavefront stages in stageOwn (32 x (TM + 4) floats of its own) -- then the epilogue meets no workgroup barrier at all.
+// ssReady: the affines already stand there, published by a barrier the caller has passed -- then the epilogue meets no workgroup barrier at all.
+// stageOwn (the K-split epilogue): this wavefront stages there (32 x (TM + 4) floats of its own).
 template <typename T, typename TOut, int BM, int BN, int TM, int TN>
 __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[TM / 32][TN / 32], unsigned char *smemRaw, float chScale,
                                               float chShift, int m0, int p0, int wm, int wn, int wave, int lane, int g,
@@ -390,7 +408,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
     constexpr int PASSES = 32 / RPI;
     static_assert(BM <= 256 && VPR <= 32, "epilogue geometry");
     float *ss    = ssReady ? ssReady : reinterpret_cast<float *>(smemRaw);                 // [BM] scale, [BM] shift
-    float *stage = stageOwn ? stageOwn : ss + 2 * BM + wave * (32 * LDE);
+    float *stage = stageOwn ? stageOwn : (ssReady ? reinterpret_cast<float *>(smemRaw) : ss + 2 * BM) + wave * (32 * LDE);
     const int tid = wave * 64 + lane;
     if (!ssReady)
     {
@@ -548,12 +566,13 @@ template <int NW, int BM> constexpr size_t igemmSwapLds() { return (static_cast<
 
 template <typename T, typename TOut, int BM, int BN>
 __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&acc)[2][2], unsigned char *smemRaw, float chScale, float chShift,
-                                                  int m0, int p0, int wm, int wn, int kg, int wt, int wave, int lane, int g, int nWaves, int tileIdx = 0, int nTiles = 0)
+                                                  int m0, int p0, int wm, int wn, int kg, int wt, int wave, int lane, int g, int nWaves, int tileIdx = 0, int nTiles = 0,
+                                                  float *ssReady = nullptr)
 {
     float *xch = reinterpret_cast<float *>(smemRaw);
-    float *ss  = xch + nWaves * kSwapRegion;
+    float *ss  = ssReady ? ssReady : xch + nWaves * kSwapRegion;
     const int tid = wave * 64 + lane;
-    if (tid < BM) { ss[tid] = chScale; ss[BM + tid] = chShift; }
+    if (!ssReady && tid < BM) { ss[tid] = chScale; ss[BM + tid] = chShift; }
     f32x16 mine[2][1];
     float *stageOwn = nullptr;
     auto swap = [&](auto gTag) {
@@ -586,17 +605,29 @@ __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&a
 
 // Epilogue of the kernels whose four wavefronts multiplied different k-blocks of the one wave tile: wavefront 0 adds what the others park in LDS
 // and finishes alone (the tile is small: 1024 or 2048 results).
-template <int BM, int BN> constexpr size_t igemmGatherLds() { return (static_cast<size_t>(3) * BM * BN + 2 * BM) * sizeof(float); }       // (fusedK: a flag behind it)
+template <int BM, int BN> constexpr size_t igemmGatherLds() { return static_cast<size_t>(3) * BM * BN * sizeof(float); }
+
+// Where the implicit GEMM keeps its affines (and the flag of splitKCombine behind them): past the loop's stages and everything the epilogue stages, so that
+// they are written while the loop's first loads travel and the loop's own barriers publish them.
+template <int BM, int BN, int TM, int NW, int KG, size_t LOOP> constexpr size_t igemmAffineOff()
+{
+    const size_t stage = KG == 4 ? igemmGatherLds<BM, BN>() : KG == 2 ? static_cast<size_t>(NW) * kSwapRegion * sizeof(float) : static_cast<size_t>(NW) * 32 * (TM + 4) * sizeof(float);
+    return stage > LOOP ? stage : LOOP;
+}
+
+// (not where the room for them would cost a workgroup per CU; the tiles with a tail have their own)
+template <int BM, int BN, int TM, int NW, int KG, size_t LOOP, int TAIL> constexpr bool igemmAffineEarly()
+{
+    const size_t off = igemmAffineOff<BM, BN, TM, NW, KG, LOOP>(), with = off + 2 * BM * sizeof(float) + 16, cu = 160 * 1024;
+    return TAIL == 0 && (KG != 1 || cu / with == cu / off);
+}
 
 template <typename T, typename TOut, int BM, int BN>
 __device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (&acc)[BM / 32][BN / 32], unsigned char *smemRaw, float chScale, float chShift,
-                                                    int m0, int p0, int wave, int lane, int g, int tileIdx, int nTiles)
+                                                    int m0, int p0, int wave, int lane, int g, int tileIdx, int nTiles, float *ss)
 {
     constexpr int MB = BM / 32, NB = BN / 32;
     float *xch = reinterpret_cast<float *>(smemRaw);
-    float *ss  = xch + 3 * BM * BN;
-    const int tid = wave * 64 + lane;
-    if (tid < BM) { ss[tid] = chScale; ss[BM + tid] = chShift; }
     if (wave > 0)
         staticFor<0, MB * NB>([&](auto ijTag) {
             constexpr int ij = decltype(ijTag)::value;
@@ -985,9 +1016,14 @@ void convIgemmKernel(IgemmArgs a)
     static_assert(TM % 32 == 0 && TN % 32 == 0 && (NT == 256 || NT == 512 || NT == 768) && S % 2 == 0, "wave grid");
     static_assert(KG == 1 || (KG == 2 && TM == 64 && TN == 64) || (KG == 4 && NWT == 1), "the K-split variants work on 64 x 64 wave tiles or on one wave tile");
     static_assert(NS >= 2 && NS <= 8, "LDS stages");
+    constexpr bool SS_EARLY = igemmAffineEarly<BM, BN, TM, NT / 64, KG, NS * STAGE, TAIL>();
+    constexpr size_t SS_OFF = igemmAffineOff<BM, BN, TM, NT / 64, KG, NS * STAGE>();
+    constexpr size_t FLAG_OFF = SS_EARLY ? SS_OFF + 2 * BM * sizeof(float) : igemmEpilogueLds<BM, TM, NT / 64>();
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smemRaw[];
     const unsigned ldsBase = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char *)smemRaw));
+
+    [[maybe_unused]] float *ssEarly = reinterpret_cast<float *>(smemRaw + SS_OFF);
 
     const int tid  = threadIdx.x;
     const int lane = tid & 63;
@@ -996,8 +1032,9 @@ void convIgemmKernel(IgemmArgs a)
     const int wm   = (wave % NWT) / WN;
     const int wn   = (wave % NWT) % WN;
     const int g    = blockIdx.z;
+    touchArgs(a);
     int mTile, pTile;
-    if (!igemmTileOf(a, (a.P + BN - 1) / BN, mTile, pTile)) return;
+    if (!igemmTileOf(a, mTile, pTile)) return;
     const int m0   = mTile * BM;
     const int p0   = pTile * BN;
 
@@ -1032,12 +1069,18 @@ void convIgemmKernel(IgemmArgs a)
     }
 
     // split-K: this workgroup multiplies tile steps [itBegin, itBegin + nLocal) of the K loop
-    const int itBegin = a.splitK > 1 ? static_cast<int>(static_cast<long long>(blockIdx.y) * a.nIter / a.splitK) : 0;
-    const int nLocal  = a.splitK > 1 ? static_cast<int>(static_cast<long long>(blockIdx.y + 1) * a.nIter / a.splitK) - itBegin : a.nIter;
+    // (nIter x slices fits 32 bits: a filter row of nIter steps has at least 64 bytes each and the filters stay below 2 GiB)
+    int itBegin = 0, nLocal = a.nIter, tapFirst = 0, chunkFirst = 0;
+    if (a.splitK > 1)
+    {
+        itBegin = static_cast<int>(fastDiv(blockIdx.y * static_cast<unsigned>(a.nIter), a.bySplitK));
+        nLocal = static_cast<int>(fastDiv((blockIdx.y + 1) * static_cast<unsigned>(a.nIter), a.bySplitK)) - itBegin;
+        tapFirst = static_cast<int>(fastDiv(static_cast<unsigned>(itBegin), a.byChunks));
+        chunkFirst = itBegin - tapFirst * a.cChunks;
+    }
     const unsigned waveLds = ldsBase + wave * 1024;
     // The filters of the first tile step are asked for before the pixel rows are located: they come from far away (every launch reads
     // its own), and the address arithmetic below runs while they travel.
-    const int tapFirst = itBegin / a.cChunks, chunkFirst = itBegin - tapFirst * a.cChunks;
     {
         const unsigned sA = (static_cast<unsigned>(tapFirst) * a.cinG + chunkFirst * BK) * ES;
         const bool cut = a.ragged && (chunkFirst * BK + ldVec * VEC >= a.cinG);
@@ -1052,37 +1095,58 @@ void convIgemmKernel(IgemmArgs a)
     // the image for this output pixel.
     unsigned bOff[BROWS];
     unsigned long long bMask[BROWS];
-#pragma unroll
-    for (int i = 0; i < BROWS; ++i)
+    if (a.pointwise)
     {
-        const int p = p0 + ldRow + i * RPP;
-        const bool ok = p < a.P && ldRow + i * RPP < BN;
-        const int pp = ok ? p : 0;
-        const int t  = static_cast<int>(fastDiv(static_cast<unsigned>(pp), a.byOW));
-        const int ox = pp - t * a.OW;
-        const int b  = static_cast<int>(fastDiv(static_cast<unsigned>(t), a.byOH));
-        const int oy = t - b * a.OH;
-        const int iy0 = oy * a.stride - a.pad;
-        const int ix0 = ox * a.stride - a.pad;
-        const long long pix = (static_cast<long long>(b) * a.H + iy0) * a.W + ix0;
-        bOff[i] = static_cast<unsigned>((pix * a.inLd + ldVec * VEC) * static_cast<long long>(ES));
-        // a tap lies inside the image when its row does and its column does: ksize row tests and ksize column tests instead of ksize^2 of both
-        unsigned rowBits = 0, colBits = 0;
-        for (int k = 0; k < a.ksize; ++k)
+#pragma unroll
+        for (int i = 0; i < BROWS; ++i)
         {
-            const int iy = iy0 + k * a.dil, ix = ix0 + k * a.dil;
-            rowBits |= ((iy >= 0 && iy < a.H) ? 1u : 0u) << k;
-            colBits |= ((ix >= 0 && ix < a.W) ? 1u : 0u) << k;
+            const int p = p0 + ldRow + i * RPP;
+            bOff[i] = (static_cast<unsigned>(p) * static_cast<unsigned>(a.inLd) + ldVec * VEC) * ES;
+            bMask[i] = p < a.P && ldRow + i * RPP < BN ? 1ull : 0ull;
         }
-        unsigned long long mask = 0;
-        for (int ki = 0; ki < a.ksize; ++ki)
-            if ((rowBits >> ki) & 1u) mask |= static_cast<unsigned long long>(colBits) << (ki * a.ksize);
-        bMask[i] = ok ? mask : 0ull;
+    }
+    else
+    {
+#pragma unroll
+        for (int i = 0; i < BROWS; ++i)
+        {
+            const int p = p0 + ldRow + i * RPP;
+            const bool ok = p < a.P && ldRow + i * RPP < BN;
+            const int pp = ok ? p : 0;
+            const int t  = static_cast<int>(fastDiv(static_cast<unsigned>(pp), a.byOW));
+            const int ox = pp - t * a.OW;
+            const int b  = static_cast<int>(fastDiv(static_cast<unsigned>(t), a.byOH));
+            const int oy = t - b * a.OH;
+            const int iy0 = oy * a.stride - a.pad;
+            const int ix0 = ox * a.stride - a.pad;
+            // (modulo 2^32: the extent of the tensor is below 2 GiB)
+            bOff[i] = (static_cast<unsigned>((b * a.H + iy0) * a.W + ix0) * static_cast<unsigned>(a.inLd) + ldVec * VEC) * ES;
+            // a tap lies inside the image when its row and its column do: the filter rows and columns inside, each a run of taps (dilation 1) or tested
+            // one by one, and the product of the two as bits -- the column bits repeated at every filter row that is inside
+            unsigned colBits = 0;
+            unsigned long long rows = 0;
+            if (a.dil == 1)
+            {
+                const int x0 = max(-ix0, 0), x1 = min(a.W - ix0, a.ksize), y0 = max(-iy0, 0), y1 = min(a.H - iy0, a.ksize);
+                if (x1 > x0 && y1 > y0)
+                {
+                    colBits = (1u << x1) - (1u << x0);
+                    rows = a.tapRows & ((~0ull >> (64 - y1 * a.ksize)) & (~0ull << (y0 * a.ksize)));
+                }
+            }
+            else
+                for (int q = 0; q < a.ksize; ++q)
+                {
+                    const int iy = iy0 + q * a.dil, ix = ix0 + q * a.dil;
+                    colBits |= ((ix >= 0 && ix < a.W) ? 1u : 0u) << q;
+                    rows |= ((iy >= 0 && iy < a.H) ? 1ull : 0ull) << (q * a.ksize);
+                }
+            bMask[i] = ok ? colBits * rows : 0ull;
+        }
     }
     unsigned bVoff[BROWS];                       // B offsets of the tap being loaded
+    int ki = 0, kj = 0;                          // the tap's filter row and column
     auto setTap = [&](int tap) {
-        const int ki = tap / a.ksize;
-        const int kj = tap - ki * a.ksize;
         const unsigned tapOff = static_cast<unsigned>((ki * a.dil * a.W + kj * a.dil) * a.inLd) * ES;
 #pragma unroll
         for (int i = 0; i < BROWS; ++i) bVoff[i] = ((bMask[i] >> tap) & 1ull) ? bOff[i] + tapOff : kOobOffset;
@@ -1101,7 +1165,13 @@ void convIgemmKernel(IgemmArgs a)
     bool cutNext = false, pastEndNext = false;
     auto advance = [&](bool pastEnd) {
         pastEndNext = pastEnd;
-        if (++chunkNext == a.cChunks) { chunkNext = 0; ++tapNext; if (tapNext < a.taps) setTap(tapNext); }
+        if (++chunkNext == a.cChunks)
+        {
+            chunkNext = 0;
+            ++tapNext;
+            if (++kj == a.ksize) { kj = 0; ++ki; }
+            if (tapNext < a.taps) setTap(tapNext);
+        }
         sANext = (static_cast<unsigned>(tapNext) * a.cinG + chunkNext * BK) * ES;
         sBNext = static_cast<unsigned>(chunkNext * BK) * ES;
         cutNext = pastEnd || (a.ragged && (chunkNext * BK + ldVec * VEC >= a.cinG));
@@ -1159,6 +1229,8 @@ void convIgemmKernel(IgemmArgs a)
     auto fillStages = [&](auto skip) {
         tapNext = tapFirst;
         chunkNext = chunkFirst - 1;                           // advance() steps onto the first tile step
+        ki = static_cast<int>(fastDiv(static_cast<unsigned>(tapNext), a.byKsize));
+        kj = tapNext - ki * a.ksize;
         setTap(tapNext);
         staticFor<0, AHEAD>([&](auto stTag) {
             constexpr int st = decltype(stTag)::value;
@@ -1166,6 +1238,8 @@ void convIgemmKernel(IgemmArgs a)
             staticFor<st == 0 ? decltype(skip)::value : 0, NL>([&](auto lTag) { issueLoad(lTag, sANext, sBNext, cutNext, st * STAGE); });
         });
         dmaWait<(AHEAD - 1) * NL>();             // step 0 has landed
+        // (and with it the affines, which were asked for before it)
+        if (SS_EARLY && tid < BM) { ssEarly[tid] = chScale; ssEarly[BM + tid] = chShift; }
         __syncthreads();
     };
 
@@ -1306,12 +1380,12 @@ void convIgemmKernel(IgemmArgs a)
         igemmTailEpilogue<BM, BN, WM, WN, STAGE>(a, acc, smemRaw, ldsBase, chScale, chShift, sc2, sh2, p0, wm, wn, wave, lane, tailPrefetch, tailPrefetch ? (nLocal & 1) : 0);
         return;
     }
-    const int nTilesP = (a.P + BN - 1) / BN;
-    const int nTiles = a.mTiles * nTilesP * static_cast<int>(gridDim.z), tileIdx = (g * nTilesP + pTile) * a.mTiles + mTile;
-    if constexpr (KG == 4) igemmEpilogueGather<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wave, lane, g, tileIdx, nTiles);
-    else if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles);
-    else if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + igemmEpilogueLds<BM, TM, NT / 64>()))) return;
-    else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g);
+    const int nTiles = a.tiles * static_cast<int>(gridDim.z), tileIdx = (g * a.nTilesP + pTile) * a.mTiles + mTile;
+    float *ss = SS_EARLY ? ssEarly : nullptr;
+    if constexpr (KG == 4) igemmEpilogueGather<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wave, lane, g, tileIdx, nTiles, ss);
+    else if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles, ss);
+    else if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + FLAG_OFF))) return;
+    else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g, ss);
 }
 
 constexpr int kSplitKMax = 8;
@@ -1359,8 +1433,13 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         constexpr unsigned STAGE = static_cast<unsigned>(((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16);
         smemEpi = TailLds<BM, BN, STAGE>::bytes();
     }
-    else smemEpi = std::max(igemmEpilogueLds<BM, BM / WM, WM * WN * KG>(), KG == 4 ? igemmGatherLds<BM, BN>() : KG == 2 ? igemmSwapLds<WM * WN * KG, BM>() : size_t(0));
-    if (a.fusedK > 1) smemEpi += 16;                  // the flag of splitKCombine
+    else
+    {
+        constexpr size_t LOOP = static_cast<size_t>(NS) * ((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16;
+        // (16 bytes: the flag of splitKCombine)
+        if constexpr (igemmAffineEarly<BM, BN, BM / WM, WM * WN * KG, KG, LOOP, TAIL>()) smemEpi = igemmAffineOff<BM, BN, BM / WM, WM * WN * KG, KG, LOOP>() + 2 * BM * sizeof(float) + 16;
+        else smemEpi = igemmEpilogueLds<BM, BM / WM, WM * WN * KG>() + (a.fusedK > 1 ? 16 : 0);
+    }
     const size_t smem = smemLoop > smemEpi ? smemLoop : smemEpi;
     a.mTiles = (a.coutG + BM - 1) / BM;
     const int tiles = a.mTiles * ((a.P + BN - 1) / BN);
@@ -1396,6 +1475,8 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         a.splitK = a.fusedK;
     }
     dim3 grid(igemmGridX(a, (a.P + BN - 1) / BN, sizeof(T), a.splitK == 1 && groups == 1), a.splitK, groups);
+    a.bySplitK = makeFastDiv(static_cast<unsigned>(a.splitK));
+    a.byChunks = makeFastDiv(static_cast<unsigned>(a.cChunks));
     if (a.dryRun) return 0;
     auto kern = convIgemmKernel<T, TOut, BM, BN, KV, WM, WN, NS, KG, TAIL>;
     if (smem > 48 * 1024)

@@ -57,7 +57,8 @@ void convPatch3x3Kernel(IgemmArgs a)
     const int wm   = wave / WN;
     const int wn   = wave % WN;
     int mTile, pTile;
-    if (!igemmTileOf(a, (a.P + BN - 1) / BN, mTile, pTile)) return;
+    touchArgs(a);
+    if (!igemmTileOf(a, mTile, pTile)) return;
     const int m0 = mTile * BM;
     const int p0 = pTile * BN;
 

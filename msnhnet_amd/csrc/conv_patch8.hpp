@@ -75,7 +75,8 @@ void convPatch8Kernel(IgemmArgs a)
     const int wm   = (wave % NWT) / WN;
     const int wn   = (wave % NWT) % WN;
     int mTile, pTile;
-    if (!igemmTileOf(a, (a.P + BN - 1) / BN, mTile, pTile)) return;
+    touchArgs(a);
+    if (!igemmTileOf(a, mTile, pTile)) return;
     const int m0 = mTile * BM;
     const int p0 = pTile * BN;
 

@@ -428,6 +428,27 @@ def test_conv_f32_split_products_not_finite(slices, tile):
     assert gu.rel_err(y, ref) <= TOL[abi.F32]
 
 
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F16])
+@pytest.mark.parametrize("h,w,k,stride,pad,dil", [(9, 11, 8, 1, 7, 1), (8, 8, 8, 8, 0, 1), (2, 3, 5, 1, 4, 1), (1, 1, 3, 1, 1, 1), (13, 10, 7, 3, 3, 1), (12, 9, 3, 2, 3, 3),
+                                                  (5, 6, 1, 2, 0, 1), (4, 5, 1, 1, 1, 1), (7, 7, 1, 1, 0, 1)])
+def test_conv_tap_masks(h, w, k, stride, pad, dil, dtype):
+    """Which taps lie inside the image: filters larger than the image, paddings of a filter less one, 64 taps, dilation, and the 1x1 forms with and without
+    the shortcut for an input pixel that is the output pixel; sliced as well, where the slices start inside a filter."""
+    import gpuutil as gu
+    rng = np.random.default_rng(h * 100 + k)
+    x, wt = _case(rng, 2, 64, h, w, 48, k)
+    if dtype == abi.F16:
+        x, wt = gu.round_f16(x), gu.round_f16(wt)
+    ref = _ref(x, wt, stride, pad, dil, 1, None, None, "none", 0.1, None, "none", 1.0, 1.0)
+    for algo, tile in (("igemm", 6), ("igemm", 1), ("igemm", 59), ("igemm_splitk", 12)):
+        try:
+            y, _ = gu.conv2d(x, wt, dtype=dtype, stride=stride, pad=pad, dil=dil, algo=algo, tile=tile)
+        except abi.HipError as e:
+            assert algo == "igemm_splitk" and "split-K does not apply" in str(e)
+            continue
+        assert gu.rel_err(y, ref) <= TOL[dtype], (algo, tile)
+
+
 SPLITK_CASES = [
     # b, c, h, w, oc, k, stride, pad, groups
     (1, 512, 7, 7, 512, 3, 1, 1, 1),
