@@ -346,11 +346,10 @@ template <int BM, int TM, int NW = 4> constexpr size_t igemmEpilogueLds() { retu
 constexpr size_t kFusedKHead = 64 * 1024;          // counters at the start of the workspace, zero between launches
 constexpr int kCpolAgent = 16;                     // sc1
 
-// (waves past nWaves hold nothing and only keep the barriers)
-template <int A, int B>
-__device__ __forceinline__ bool splitKCombine(float *ws, int slices, f32x16 (&acc)[A][B], int tileIdx, int nTiles, int wave, int nWaves, int lane, int *flag)
+// vec(v) is the lane's vector v of V, a reference to four of its sums; waves past nWaves hold nothing and only keep the barriers.
+template <int V, typename F>
+__device__ __forceinline__ bool splitKCombineVectors(float *ws, int slices, F &&vec, int tileIdx, int nTiles, int wave, int nWaves, int lane, int *flag)
 {
-    constexpr int V = A * B * 4;                   // 16-byte vectors per lane
     const size_t slot = static_cast<size_t>(nWaves) * V * 1024;
     unsigned char *part = reinterpret_cast<unsigned char *>(ws) + kFusedKHead + static_cast<size_t>(tileIdx) * slot;
     const size_t step = static_cast<size_t>(nTiles) * slot;        // from a slice to the next one's partial sums of the same tile
@@ -360,9 +359,8 @@ __device__ __forceinline__ bool splitKCombine(float *ws, int slices, f32x16 (&ac
         const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + blockIdx.y * step, static_cast<unsigned>(slot));
         staticFor<0, V>([&](auto vTag) {
             constexpr int v = decltype(vTag)::value;
-            constexpr int ij = v / 4, q = v % 4;
-            const f32x16 &c = acc[ij / B][ij % B];
-            const f32x4 d = {c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
+            f32x4 d;
+            vec(vTag, [&](int e, float &x) { d[e] = x; });
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, d), rs, off + v * 1024, 0, kCpolAgent);
         });
     }
@@ -384,13 +382,26 @@ __device__ __forceinline__ bool splitKCombine(float *ws, int slices, f32x16 (&ac
             const __amdgpu_buffer_rsrc_t rs = makeRsrc(part + s * step, static_cast<unsigned>(slot));
             staticFor<0, V>([&](auto vTag) {
                 constexpr int v = decltype(vTag)::value;
-                constexpr int ij = v / 4, q = v % 4;
                 const f32x4 d = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + v * 1024, 0, kCpolAgent));
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[ij / B][ij % B][q * 4 + e] = s == 0 ? d[e] : acc[ij / B][ij % B][q * 4 + e] + d[e];
+                vec(vTag, [&](int e, float &x) { x = s == 0 ? d[e] : x + d[e]; });
             });
         }
     return true;
+}
+
+template <int A, int B>
+__device__ __forceinline__ bool splitKCombine(float *ws, int slices, f32x16 (&acc)[A][B], int tileIdx, int nTiles, int wave, int nWaves, int lane, int *flag)
+{
+    return splitKCombineVectors<A * B * 4>(ws, slices, [&](auto vTag, auto &&each) {
+        constexpr int ij = decltype(vTag)::value / 4, q = decltype(vTag)::value % 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+        {
+            float x = acc[ij / B][ij % B][q * 4 + e];
+            each(e, x);
+            acc[ij / B][ij % B][q * 4 + e] = x;
+        }
+    }, tileIdx, nTiles, wave, nWaves, lane, flag);
 }
 
 // ssReady: the affines already stand there, published by a barrier the caller has passed -- then the epilogue meets no workgroup barrier at all.
@@ -603,15 +614,123 @@ __device__ __forceinline__ void igemmEpilogueSwap(const IgemmArgs &a, f32x16 (&a
     igemmEpilogue<T, TOut, BM, BN, 64, 32>(a, mine, smemRaw, chScale, chShift, m0, p0, wm, wn * 2 + kg, wave, lane, g, ss, stageOwn);
 }
 
-// Epilogue of the kernels whose four wavefronts multiplied different k-blocks of the one wave tile: wavefront 0 adds what the others park in LDS
-// and finishes alone (the tile is small: 1024 or 2048 results).
-template <int BM, int BN> constexpr size_t igemmGatherLds() { return static_cast<size_t>(3) * BM * BN * sizeof(float); }
+// Epilogue of the kernels whose KG wavefronts multiplied different k-blocks of the one wave tile of 32 channels: everybody parks its sums in LDS, then wavefront
+// q adds up channels 8q .. 8q + 7, in the order of the k-groups, and finishes them: four channels per lane, straight from registers.  With eight
+// wavefronts and two pixel blocks the upper four take the second block.
+// Against one wavefront that adds and finishes alone: float32 3x3 64 -> 64 at 56 x 56 8.35 -> 7.94 us, 1x1 512 -> 256 at 38 x 38 9.47 -> 8.98.
+template <int BM, int BN, int KG> constexpr size_t igemmGatherLds() { return static_cast<size_t>(KG) * BM * BN * sizeof(float); }
+
+template <typename T, typename TOut, int BM, int BN, int KG>
+__device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (&acc)[1][BN / 32], unsigned char *smemRaw, int m0, int p0, int wave, int lane, int g,
+                                                    int tileIdx, int nTiles, const float *ss)
+{
+    static_assert(BM == 32 && (KG == 4 || KG == 8) && (KG == 4 || BN <= 64), "one block of channels");
+    constexpr int NBLK = BN / 32;
+    constexpr int NB = KG == 8 && NBLK == 2 ? 1 : NBLK;           // pixel blocks a wavefront finishes
+    constexpr int NW = KG == 8 && NBLK == 1 ? 4 : KG;             // wavefronts that finish anything
+    f32x4 *xch = reinterpret_cast<f32x4 *>(smemRaw) + lane;       // [k-group][pixel block][quarter][lane]
+    staticFor<0, NBLK * 4>([&](auto jqTag) {
+        constexpr int j = decltype(jqTag)::value / 4, q = decltype(jqTag)::value % 4;
+        xch[(wave * NBLK * 4 + decltype(jqTag)::value) * 64] = f32x4{acc[0][j][q * 4], acc[0][j][q * 4 + 1], acc[0][j][q * 4 + 2], acc[0][j][q * 4 + 3]};
+    });
+    const int q = wave & 3, j0 = wave / 4;
+    const int chBase = g * a.coutG;
+    const int ml = q * 8 + (lane >> 5) * 4;                       // first of this lane's channels inside the tile
+    const int mv = m0 + ml;
+    const bool full = a.vecOk && mv + 3 < a.coutG;
+    const unsigned ch = static_cast<unsigned>(chBase + mv);
+    const int npix = min(a.P - p0, BN);
+    TOut    *yBlock = static_cast<TOut *>(a.y) + blockIdx.y * a.slicePitch + static_cast<size_t>(p0) * a.outLd;
+    const T *rBlock = static_cast<const T *>(a.res) + static_cast<size_t>(p0) * a.resLd;
+    // the residual travels while the sums are parked and added
+    float r[NB][4];
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    typedef TOut TOut4 __attribute__((ext_vector_type(4)));
+    staticFor<0, NB>([&](auto jTag) {
+        constexpr int j = decltype(jTag)::value;
+        const int pl = (j0 + j) * 32 + (lane & 31);
+        const T *rp = rBlock + static_cast<size_t>(pl) * a.resLd + ch;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[j][e] = 0.f;
+        if (a.hasRes && wave < NW && pl < npix)
+        {
+            if (full)
+            {
+                const T4 v = *reinterpret_cast<const T4 *>(rp);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[j][e] = toF(v[e]);
+            }
+            else
+            {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (mv + e < a.coutG) r[j][e] = toF(rp[e]);
+            }
+        }
+    });
+    __syncthreads();
+    float v[NB][4];
+    staticFor<0, NB>([&](auto jTag) {
+        constexpr int j = decltype(jTag)::value;
+        f32x4 t = xch[((j0 + j) * 4 + q) * 64];
+#pragma unroll
+        for (int k = 1; k < KG; ++k) t += xch[((k * NBLK + j0 + j) * 4 + q) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = t[e];
+    });
+    if (a.fusedK > 1 && !splitKCombineVectors<NB>(a.ws, a.splitK, [&](auto jTag, auto &&each) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) each(e, v[decltype(jTag)::value][e]);
+        }, tileIdx, nTiles, wave, NW, lane, reinterpret_cast<int *>(const_cast<float *>(ss) + 2 * BM))) return;
+    if (wave >= NW || mv >= a.coutG) return;
+    const f32x4 sc = *reinterpret_cast<const f32x4 *>(ss + ml);
+    const f32x4 sh = *reinterpret_cast<const f32x4 *>(ss + BM + ml);
+    staticFor<0, NB>([&](auto jTag) {
+        constexpr int j = decltype(jTag)::value;
+        const int pl = (j0 + j) * 32 + (lane & 31);
+        if (pl >= npix) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = v[j][e] * sc[e] + sh[e];
+        activateArray<4>(v[j], a.act, a.actParam);
+        if (a.hasRes)
+        {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j][e] += a.resMul * r[j][e];
+            activateArray<4>(v[j], a.act2, a.act2Param);
+        }
+        TOut4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = fromF<TOut>(v[j][e] * a.outMul);
+        const auto put = [&](TOut *yp) {
+            if (full) *reinterpret_cast<TOut4 *>(yp) = o;
+            else
+            {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (mv + e < a.coutG) yp[e] = o[e];
+            }
+        };
+        if (a.up2)
+        {
+            const unsigned p = static_cast<unsigned>(p0) + pl;
+            const unsigned t1 = fastDiv(p, a.byOW), bImg = fastDiv(t1, a.byOH);
+            const unsigned ox = p - t1 * a.OW, oy = t1 - bImg * a.OH;
+            TOut *yq = static_cast<TOut *>(a.y) + (static_cast<size_t>(bImg * 2u * a.OH + 2u * oy) * 2u * a.OW + 2u * ox) * a.outLd + ch;
+            const size_t rowStep = static_cast<size_t>(2) * a.OW * a.outLd;
+            put(yq);
+            put(yq + a.outLd);
+            put(yq + rowStep);
+            put(yq + rowStep + a.outLd);
+        }
+        else put(yBlock + static_cast<size_t>(pl) * a.outLd + ch);
+    });
+}
 
 // Where the implicit GEMM keeps its affines (and the flag of splitKCombine behind them): past the loop's stages and everything the epilogue stages, so that
 // they are written while the loop's first loads travel and the loop's own barriers publish them.
 template <int BM, int BN, int TM, int NW, int KG, size_t LOOP> constexpr size_t igemmAffineOff()
 {
-    const size_t stage = KG == 4 ? igemmGatherLds<BM, BN>() : KG == 2 ? static_cast<size_t>(NW) * kSwapRegion * sizeof(float) : static_cast<size_t>(NW) * 32 * (TM + 4) * sizeof(float);
+    const size_t stage = KG >= 4 ? igemmGatherLds<BM, BN, KG>() : KG == 2 ? static_cast<size_t>(NW) * kSwapRegion * sizeof(float) : static_cast<size_t>(NW) * 32 * (TM + 4) * sizeof(float);
     return stage > LOOP ? stage : LOOP;
 }
 
@@ -683,7 +802,7 @@ template <typename T> constexpr int igemmWavesMin(int bm, int bn, int kv, int wm
 {
     const int nw = wm * wn * kg;
     if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg)) return (nw + 3) / 4;
-    return kg == 4 ? 1 : kg == 2 ? nw / 4 : igemmWavesPerSimd(bm, bn, kv, ns, nw);
+    return kg >= 4 ? kg / 4 : kg == 2 ? nw / 4 : igemmWavesPerSimd(bm, bn, kv, ns, nw);
 }
 
 template <typename T> constexpr int igemmWavesMax(int bm, int bn, int kv, int wm, int wn, int ns, int kg)
@@ -694,7 +813,7 @@ template <typename T> constexpr int igemmWavesMax(int bm, int bn, int kv, int wm
         const int fit = 512 / igemmSplitRegs(bm / wm / 32, bn / wn / 32);
         return fit > nw / 4 ? fit : nw / 4;
     }
-    return kg == 4 ? 4 : kg == 2 ? (nw == 4 ? 3 : nw / 4) : igemmWavesPerSimd(bm, bn, kv, ns, nw);
+    return kg >= 4 ? 4 : kg == 2 ? (nw == 4 ? 3 : nw / 4) : igemmWavesPerSimd(bm, bn, kv, ns, nw);
 }
 
 // 16-byte-per-lane load from a buffer resource straight into LDS: the 64 lanes of the wave fill 1 KiB starting at
@@ -985,7 +1104,7 @@ __device__ __forceinline__ void igemmTailEpilogue(const IgemmArgs &a, f32x16 (&a
 
 // KG = 2: two groups of wavefronts share the WM x WN grid of (then 64 x 64) wave tiles and split the k-blocks of every tile step
 // between them, which takes a third off the LDS fragment reads per MFMA against 32 x 64 wave tiles of the same workgroup tile.
-// KG = 4: the four wavefronts multiply one k-block each of every step for the workgroup's only wave tile.
+// KG = 4, 8: the wavefronts multiply a pair of k-blocks each of every step for the workgroup's only wave tile.
 // TAIL = 1: the epilogue also computes the 1x1 convolution that reads this one's result (igemmTailEpilogue); float16 only.
 template <typename T, typename TOut, int BM, int BN, int KV, int WM, int WN, int NS, int KG = 1, int TAIL = 0>
 __global__ __launch_bounds__(64 * WM * WN * KG)
@@ -1010,12 +1129,14 @@ void convIgemmKernel(IgemmArgs a)
     constexpr int S     = KV / 2 / KG;            // MFMA k-steps per tile step and wavefront (one k-block = two 16-byte chunks)
     constexpr unsigned ES = sizeof(T);
     constexpr int ROWB  = KV * 16;                // bytes per LDS row: unpadded
-    constexpr int SWDIV = 16 / KV;                // rows per 256 bytes of LDS
+    constexpr int SWDIV = KV > 16 ? 1 : 16 / KV;  // rows per 256 bytes of LDS
+    constexpr int SWMOD = KV > 16 ? 16 : KV;      // (rows a pass apart share the swizzle)
     constexpr int A_BYTES = BML * ROWB;
     constexpr unsigned STAGE = (BML + BNL) * ROWB; // one LDS stage: A rows, then B rows
     static_assert(TM % 32 == 0 && TN % 32 == 0 && (NT == 256 || NT == 512 || NT == 768) && S % 2 == 0, "wave grid");
-    static_assert(KG == 1 || (KG == 2 && TM == 64 && TN == 64) || (KG == 4 && NWT == 1), "the K-split variants work on 64 x 64 wave tiles or on one wave tile");
+    static_assert(KG == 1 || (KG == 2 && TM == 64 && TN == 64) || (KG >= 4 && NWT == 1), "the K-split variants work on 64 x 64 wave tiles or on one wave tile");
     static_assert(NS >= 2 && NS <= 8, "LDS stages");
+    static_assert((RPP / SWDIV) % SWMOD == 0, "rows a pass apart share the swizzle");
     constexpr bool SS_EARLY = igemmAffineEarly<BM, BN, TM, NT / 64, KG, NS * STAGE, TAIL>();
     constexpr size_t SS_OFF = igemmAffineOff<BM, BN, TM, NT / 64, KG, NS * STAGE>();
     constexpr size_t FLAG_OFF = SS_EARLY ? SS_OFF + 2 * BM * sizeof(float) : igemmEpilogueLds<BM, TM, NT / 64>();
@@ -1054,11 +1175,11 @@ void convIgemmKernel(IgemmArgs a)
         }
 
     // LDS layout of a stage: rows of KV 16-byte chunks without padding; chunk c of row r sits at chunk position
-    // c ^ ((r / SWDIV) % KV).  With that XOR the 16 lanes the LDS serves per cycle hit 16 different 16-byte bank
+    // c ^ ((r / SWDIV) % SWMOD).  With that XOR the 16 lanes the LDS serves per cycle hit 16 different 16-byte bank
     // groups when a wave reads one chunk column of 32 rows, while a wave's load fills 64 consecutive chunk
     // positions.  Thread tid owns chunk position tid % KV of row tid / KV (+ RPP rows per pass): byte tid * 16.
     const int ldRow = tid / KV;
-    const int ldVec = (tid % KV) ^ ((ldRow / SWDIV) % KV);   // the logical chunk this thread fetches
+    const int ldVec = (tid % KV) ^ ((ldRow / SWDIV) % SWMOD);   // the logical chunk this thread fetches
 
     unsigned aOff[AROWS];
 #pragma unroll
@@ -1179,7 +1300,7 @@ void convIgemmKernel(IgemmArgs a)
 
     // fragment addresses: lane l feeds MFMA row l % 32 with chunk 2 * kb + l / 32 of k-step kb
     const int fragRow = lane & 31;
-    const int fragSw  = (fragRow / SWDIV) % KV;
+    const int fragSw  = (fragRow / SWDIV) % SWMOD;
     unsigned aAddr[S], bAddr[S];
 #pragma unroll
     for (int kb = 0; kb < S; ++kb)
@@ -1382,7 +1503,7 @@ void convIgemmKernel(IgemmArgs a)
     }
     const int nTiles = a.tiles * static_cast<int>(gridDim.z), tileIdx = (g * a.nTilesP + pTile) * a.mTiles + mTile;
     float *ss = SS_EARLY ? ssEarly : nullptr;
-    if constexpr (KG == 4) igemmEpilogueGather<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wave, lane, g, tileIdx, nTiles, ss);
+    if constexpr (KG >= 4) igemmEpilogueGather<T, TOut, BM, BN, KG>(a, acc, smemRaw, m0, p0, wave, lane, g, tileIdx, nTiles, ss);
     else if constexpr (KG == 2) igemmEpilogueSwap<T, TOut, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, kg, wave % NWT, wave, lane, g, NT / 64, tileIdx, nTiles, ss);
     else if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, NT / 64, lane, reinterpret_cast<int *>(smemRaw + FLAG_OFF))) return;
     else igemmEpilogue<T, TOut, BM, BN, TM, TN>(a, acc, smemRaw, chScale, chShift, m0, p0, wm, wn, wave, lane, g, ss);
@@ -1420,7 +1541,7 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
     }
     // Below 1024 products per result a float16 tile has at most eight k-steps, so parking and adding the three partial tiles costs what the smaller tile
     // saves (level with 64 x 64), and float16 results keep one summation order over all tiles there.  float32 steps take half the channels: no line.
-    if (KG == 4 && sizeof(T) == 2 && a.taps * a.cinG < 1024)
+    if (KG >= 4 && sizeof(T) == 2 && a.taps * a.cinG < 1024)
     {
         setError("conv2d: this tile needs float32 tensors or a float16 convolution of at least 1024 products per result");
         return 3;
@@ -1500,14 +1621,14 @@ namespace msnh {
 // Tile configurations (BM x BN output tile, KV 16-byte vectors of K per step, WM x WN wavefront grid).
 // Index 0 is "choose for me"; the others can be forced through msnh_conv_desc::tile, which is how the host
 // library's per-layer search picks the fastest one at load time.
-constexpr int kIgemmTiles = 71;
-constexpr int kIgemmTailTileFirst = 70;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
+constexpr int kIgemmTiles = 76;
+constexpr int kIgemmTailTileFirst = 75;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
 
 // The configurations on which a sliced launch (MSNH_CONV_IGEMM_FUSEDK) is worth timing whatever they do unsliced: 32 x 32 to 128 x 64, which give a layer of
 // few output tiles the most workgroups before it is cut.  (Larger ones are tried where they are among a layer's fastest unsliced.)  Over the layers of 16
 // networks at batch 1 to 32 in both types the search took 67 83 times, 68 20, 12 19, 65 16, 6 twice, 64 and 66 once; 30 (64 x 64 with two stages of
 // 64-byte rows) and 69 (32 x 64) never, and timing them costs a load 1 to 3 %.
-constexpr int kIgemmSlicedTiles[] = {6, 12, 64, 65, 66, 67, 68};
+constexpr int kIgemmSlicedTiles[] = {6, 12, 64, 65, 66, 67, 68, 70, 71, 72, 73, 74};
 
 // One translation unit instantiates every third configuration of one type pair (tile % kIgemmParts == PART), so that they compile in parallel.
 constexpr int kIgemmParts = 3;
@@ -1622,10 +1743,19 @@ int igemmDispatch(IgemmArgs &a, int groups, int tile, hipStream_t st)
     MSNH_TILE(67, launchIgemm, 32, 32, 16, 1, 1, 3, 4)
     MSNH_TILE(68, launchIgemm, 32, 32, 16, 1, 1, 2, 4)
     MSNH_TILE(69, launchIgemm, 32, 64, 16, 1, 1, 2, 4)
+    // the same with eight wavefronts and 512-byte rows: twice the K per barrier.  A step of the small tiles is bound by its instructions (75 for two MFMAs
+    // per wavefront) and by LDS latency, about 550 cycles whatever the number of stages: sets of cold buffers, best of the tiles above -> of these,
+    // float16 1x1 1024 -> 512 at 13 x 13 6.2 -> 5.4 us, 3x3 512 -> 1024 there 12.0 -> 10.1, 3x3 256 -> 512 at 26 x 26 10.4 -> 9.7; float32, five pictures,
+    // 1x1 1024 -> 256 at 14 x 14 10.2 -> 9.2, 3x3 256 -> 256 17.2 -> 15.6; 64 x 64 with a fourth stage: 3x3 256 -> 256 at 34 x 34, three pictures, 12.2 -> 11.5
+    MSNH_TILE(70, launchIgemm, 32, 32, 32, 1, 1, 3, 8)
+    MSNH_TILE(71, launchIgemm, 32, 64, 32, 1, 1, 2, 8)
+    MSNH_TILE(72, launchIgemm, 32, 64, 32, 1, 1, 3, 8)
+    MSNH_TILE(73, launchIgemm, 32, 32, 32, 1, 1, 4, 8)
+    MSNH_TILE(74, launchIgemm, 64, 64, 16, 2, 2, 4)
     // tiles whose epilogue also computes the 1x1 convolution that follows (msnh_hip_conv2d_tail only; float16): the tile holds every
     // output channel of the first convolution (at most 256 / 128)
-    MSNH_TILE_TAIL(70, launchIgemm, 256, 192, 8, 4, 3, 2, 1, 1)
-    MSNH_TILE_TAIL(71, launchIgemm, 128, 192, 8, 4, 3, 2, 1, 1)
+    MSNH_TILE_TAIL(75, launchIgemm, 256, 192, 8, 4, 3, 2, 1, 1)
+    MSNH_TILE_TAIL(76, launchIgemm, 128, 192, 8, 4, 3, 2, 1, 1)
     default: break;
     }
 #undef MSNH_TILE

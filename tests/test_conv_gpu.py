@@ -376,7 +376,7 @@ def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
         res = gu.round_f16(res) if act2 else None
     ref = _ref(x, wt, 1, 1, 1, 1, scale, shift, act, 0.1, res, act2 or "none", 0.5, 2.0)
     ran = 0
-    for tile in (1, 5, 6, 9, 13, 14, 31, 32, 36, 37, 38, 46, 52, 55, 58, 61, 64, 66, 67, 69):
+    for tile in (1, 5, 6, 9, 13, 14, 31, 32, 36, 37, 38, 46, 52, 55, 58, 61, 64, 66, 67, 69, 70, 71):
         try:
             y, used = gu.conv2d(x, wt, dtype=dtype, stride=1, pad=1, scale=scale, shift=shift, act=act, residual=res, act2=act2 or "none", res_mul=0.5, out_mul=2.0,
                                 algo="igemm", tile=tile, out_ld=oc + pad_ld, res_ld=oc + pad_ld)
@@ -388,7 +388,7 @@ def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
     assert ran >= 15
 
 
-@pytest.mark.parametrize("tile", [1, 5, 9, 23, 32, 36, 38, 41, 58, 61, 69])
+@pytest.mark.parametrize("tile", [1, 5, 9, 23, 32, 36, 38, 41, 58, 61, 69, 71])
 @pytest.mark.parametrize("c,oc,k", [(256, 96, 3), (40, 72, 1), (64, 130, 3)])
 def test_conv_f32_split_products(c, oc, k, tile):
     """float32 tiles that multiply bfloat16 pieces: their error against 64-bit sums is that of one float32 rounding per 16 products.  With partial sums that grow
@@ -404,7 +404,7 @@ def test_conv_f32_split_products(c, oc, k, tile):
     assert err <= 2.0 ** -24 * (1.5 * np.sqrt(c * k * k / 16 / 6) + 1), err
 
 
-@pytest.mark.parametrize("tile", [2, 5, 23, 36, 38, 58, 61, 69])
+@pytest.mark.parametrize("tile", [2, 5, 23, 36, 38, 58, 61, 69, 71])
 @pytest.mark.parametrize("slices", [0, 2])
 def test_conv_f32_split_products_not_finite(slices, tile):
     """Infinities, NaN and the largest values, against filters with zero pieces: the same classes of results as float32 products give"""
@@ -528,7 +528,7 @@ def test_conv_fused_k(case, dtype):
     assert L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), 12) == 0          # a tile without slices is not this algorithm
     ws = torch.zeros(64 << 20, dtype=torch.uint8).cuda()
     tried = 0
-    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66, 67, 68, 69):
+    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66, 67, 68, 69, 70, 71, 72):
         for slices in (2, 3, 7, 16):
             d.tile = tile + 256 * slices
             need = L.msnh_hip_conv2d_workspace_bytes(ctypes.byref(d), algo)
