@@ -169,6 +169,19 @@ __device__ __forceinline__ unsigned fastDiv(unsigned n, const FastDiv &f)
     return (t + ((n - t) >> f.s1)) >> f.s2;
 }
 
+// One word of every 64-byte line of the arguments, so that all lines are in the scalar cache after one trip to memory.  The compiler loads a field where
+// it is used, and the cache is cold at the start of a launch: the chain tile -> addresses -> first load met four such trips one after the other.
+// With that, divisions by reciprocals from the host, tap masks without loops and the affines published by the loop's barriers: yolov3 f16 b1 746 -> 690 us
+// (75 convolutions), yolov5s f16 b3 609 -> 581, resnet50 f16 b32 897 -> 816 (on one box 870 -> 816 from the start of both steps), yolov3 f32 b1 1919 -> 1819.
+template <typename A> __device__ __forceinline__ void touchArgs(const A &a)
+{
+    constexpr int words = sizeof(A) / 4, last = words - 1;
+    static_assert(sizeof(A) % 4 == 0, "lines to touch: the first eight and the last");
+    constexpr auto line = [](int n) { return n * 16 < last ? n * 16 : last; };
+    const int *q = reinterpret_cast<const int *>(&a);
+    asm volatile("" ::"s"(q[0]), "s"(q[line(1)]), "s"(q[line(2)]), "s"(q[line(3)]), "s"(q[line(4)]), "s"(q[line(5)]), "s"(q[line(6)]), "s"(q[line(7)]), "s"(q[last]));
+}
+
 inline unsigned gridFor(long long n, int block)
 {
     long long g = (n + block - 1) / block;

@@ -151,6 +151,7 @@ __global__ __launch_bounds__(256) void convDepthwise3x3FastKernel(DwFastArgs g, 
     constexpr int COLS = 3 * STRIDE + 3;
     typedef f16 HV __attribute__((ext_vector_type(CPL)));
     const DwArgs &a = g.d;
+    touchArgs(g);
     const int perXcd = (blocks + 7) / 8;
     const int logical = static_cast<int>(blockIdx.x % 8) * perXcd + static_cast<int>(blockIdx.x / 8);
     if (logical >= blocks) return;
@@ -171,6 +172,14 @@ __global__ __launch_bounds__(256) void convDepthwise3x3FastKernel(DwFastArgs g, 
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<f16 *>(a.w), 0, static_cast<int>(g.wBytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(a.y, 0, static_cast<int>(g.yBytes), 0x00020000);
 
+    // (the affine with the other loads: behind the multiply-adds it cost a round trip more)
+    float sc[CPL], sh[CPL];
+#pragma unroll
+    for (int e = 0; e < CPL; ++e)
+    {
+        sc[e] = a.scale ? a.scale[c0 + e] : 1.f;
+        sh[e] = a.shift ? a.shift[c0 + e] : 0.f;
+    }
     HV wv[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k)
@@ -214,13 +223,6 @@ __global__ __launch_bounds__(256) void convDepthwise3x3FastKernel(DwFastArgs g, 
                 for (int e = 0; e < CPL; ++e)
                     acc[j][e] += static_cast<float>(xv[r][j * STRIDE + kx][e]) * static_cast<float>(wv[r * 3 + kx][e]);
 
-    float sc[CPL], sh[CPL];
-#pragma unroll
-    for (int e = 0; e < CPL; ++e)
-    {
-        sc[e] = a.scale ? a.scale[c0 + e] : 1.f;
-        sh[e] = a.shift ? a.shift[c0 + e] : 0.f;
-    }
     float v[4 * CPL];
 #pragma unroll
     for (int j = 0; j < 4; ++j)

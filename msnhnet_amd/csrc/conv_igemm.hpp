@@ -96,17 +96,6 @@ __device__ __forceinline__ bool igemmTileOf(const IgemmArgs &a, int &mTile, int 
     return lp < a.xcdPPer && mTile < a.mTiles && pTile < a.nTilesP;
 }
 
-// One word of every 64-byte line of the arguments, so that all lines are in the scalar cache after one trip to memory.  The compiler loads a field where
-// it is used, and the cache is cold at the start of a launch: the chain tile -> addresses -> first load met four such trips one after the other.
-// With that, divisions by reciprocals from the host, tap masks without loops and the affines published by the loop's barriers: yolov3 f16 b1 746 -> 690 us
-// (75 convolutions), yolov5s f16 b3 609 -> 581, resnet50 f16 b32 897 -> 816 (on one box 870 -> 816 from the start of both steps), yolov3 f32 b1 1919 -> 1819.
-__device__ __forceinline__ void touchArgs(const IgemmArgs &a)
-{
-    static_assert(sizeof(IgemmArgs) > 6 * 64 && sizeof(IgemmArgs) <= 8 * 64, "lines to touch");
-    const int *q = reinterpret_cast<const int *>(&a);
-    asm volatile("" ::"s"(q[0]), "s"(q[16]), "s"(q[32]), "s"(q[48]), "s"(q[64]), "s"(q[80]), "s"(q[96]), "s"(q[(sizeof(IgemmArgs) - 4) / 4]));
-}
-
 // grid.x of a launch over a.mTiles x nTilesP tiles, and the XCD arrangement it runs under (see igemmTileOf).  a.xcdGm comes in as
 // the caller's wish (msnh_conv_desc::xcd_blocks): 1, 2, 4, 8 are taken as they are; 0 picks the arrangement that makes the eight
 // L2s fetch the fewest bytes, counted as (8 / g) x filters + g x input -- the default one stays unless another saves a quarter

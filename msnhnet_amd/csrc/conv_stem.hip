@@ -68,6 +68,7 @@ template <int K> __device__ __forceinline__ f16x8 stemKeepTaps(f16x8 b, bool hi)
 template <int TAPS, int MBLK>
 __global__ __launch_bounds__(256) void convStemMfmaKernel(StemArgs a)
 {
+    touchArgs(a);
     constexpr int KB = (TAPS + 31) / 32;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     f16 *wl = reinterpret_cast<f16 *>(smem);                                  // [MBLK][KB*2][64][8]
@@ -252,6 +253,7 @@ struct StemRowsArgs
 template <int KS, int MBLK>
 __global__ __launch_bounds__(256) void convStemRowsKernel(StemRowsArgs a)
 {
+    touchArgs(a);
     constexpr int kRowChunks = stemRowChunks(KS);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     f16 *wl = reinterpret_cast<f16 *>(smem);                                        // [MBLK][kRowChunks][64][8]
@@ -410,6 +412,7 @@ constexpr int stemF32Steps(int ks, int cin) { return (cin * ks + 1) / 2 * ks; }
 template <int KS, int CIN, int MBLK>
 __global__ __launch_bounds__(256) void convStemMfmaF32Kernel(StemF32Args a)
 {
+    touchArgs(a);
     constexpr int ROWS = CIN * KS, CHUNKS = (ROWS + 1) / 2, QUADS = (stemF32Steps(KS, CIN) + 3) / 4;
     constexpr int GC = 4;                                                          // chunks per group; 4 KS steps are whole quads
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];

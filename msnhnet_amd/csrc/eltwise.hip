@@ -87,6 +87,41 @@ __global__ __launch_bounds__(256) void addActKernel(const T *__restrict__ a, int
     storeVec<T, VEC>(y + p * yLd + c0, va);
 }
 
+// Item -> (channel vector, output column, output row, image) by reciprocals from the host where the items can be counted in 31 bits.  With divisions of 64-bit
+// indices by run-time divisors the small launches spent more on finding their place, about 2000 cycles, than on their data.
+struct ItemDiv { FastDiv cv, ow, oh; long long total; };
+
+static ItemDiv makeItemDiv(int cv, int ow, int oh, long long total)
+{
+    return {makeFastDiv(static_cast<unsigned>(cv)), makeFastDiv(static_cast<unsigned>(ow)), makeFastDiv(static_cast<unsigned>(oh)), total};
+}
+
+struct Item { int c, ox, oy; long long p, b; };
+
+__device__ __forceinline__ Item itemOf(const ItemDiv &d, long long idx)
+{
+    Item i;
+    if (d.total <= 0x7fffffffll)
+    {
+        const unsigned n = static_cast<unsigned>(idx), p = fastDiv(n, d.cv), t = fastDiv(p, d.ow), b = fastDiv(t, d.oh);
+        i.c = static_cast<int>(n - p * d.cv.d);
+        i.ox = static_cast<int>(p - t * d.ow.d);
+        i.oy = static_cast<int>(t - b * d.oh.d);
+        i.p = p;
+        i.b = b;
+    }
+    else
+    {
+        i.p = idx / d.cv.d;
+        i.c = static_cast<int>(idx - i.p * d.cv.d);
+        const long long t = i.p / d.ow.d;
+        i.ox = static_cast<int>(i.p - t * d.ow.d);
+        i.b = t / d.oh.d;
+        i.oy = static_cast<int>(t - i.b * d.oh.d);
+    }
+    return i;
+}
+
 // ---- max pooling -----------------------------------------------------------------------------------
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void maxPoolKernel(const T *__restrict__ x, int xLd, int H, int W, int c, int ksize, int stride,
@@ -129,21 +164,15 @@ __global__ __launch_bounds__(256) void maxPoolKernel(const T *__restrict__ x, in
 // above waits for each load in turn -- 25 dependent round trips for a 5 x 5 window.  Workgroups are dealt to the 8 XCDs in
 // contiguous runs, so the rows that neighbouring output rows share are found in one L2.
 template <typename T, int VEC, int K>
-__global__ __launch_bounds__(256) void maxPoolUnrolledKernel(const T *__restrict__ x, int xLd, int H, int W, int c, int stride, int pad, int OH,
-                                                             int OW, T *__restrict__ y, int yLd, long long total, int blocks)
+__global__ __launch_bounds__(256) void maxPoolUnrolledKernel(const T *__restrict__ x, int xLd, int H, int W, int stride, int pad, T *__restrict__ y, int yLd,
+                                                             ItemDiv div, int perXcd)
 {
-    const int perXcd = (blocks + 7) / 8;
     const int logical = static_cast<int>(blockIdx.x % 8) * perXcd + static_cast<int>(blockIdx.x / 8);
-    if (logical >= blocks) return;
     const long long idx = static_cast<long long>(logical) * 256 + threadIdx.x;
-    if (idx >= total) return;
-    const int cv = c / VEC;
-    const int c0 = static_cast<int>(idx % cv) * VEC;
-    const long long p = idx / cv;
-    const int ox = static_cast<int>(p % OW);
-    const long long t = p / OW;
-    const int oy = static_cast<int>(t % OH);
-    const long long b = t / OH;
+    if (idx >= div.total) return;
+    const Item item = itemOf(div, idx);
+    const int c0 = item.c * VEC, ox = item.ox, oy = item.oy;
+    const long long b = item.b;
     const int y0 = oy * stride - pad, x0 = ox * stride - pad;
     float m[VEC];
 #pragma unroll
@@ -176,7 +205,7 @@ __global__ __launch_bounds__(256) void maxPoolUnrolledKernel(const T *__restrict
 #pragma unroll
         for (int i = 0; i < VEC; ++i) m[i] = m[i] < -65504.f ? -65504.f : m[i];
     }
-    storeVec<T, VEC>(y + p * yLd + c0, m);
+    storeVec<T, VEC>(y + item.p * yLd + c0, m);
 }
 
 // A chain of stride-1 "same" max-pools of one window size, each reading the result of the one before it (the SPP block of the YOLOv4 /
@@ -354,24 +383,17 @@ __global__ __launch_bounds__(256) void avgPoolGlobalKernel(const T *__restrict__
 
 // ---- nearest upsample / channel copy -------------------------------------------------------------------
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void upsampleKernel(const T *__restrict__ x, int xLd, int H, int W, int c, int stride, float scale,
-                                                      T *__restrict__ y, int yLd, long long total)
+__global__ __launch_bounds__(256) void upsampleKernel(const T *__restrict__ x, int xLd, int H, int W, FastDiv byStride, float scale, T *__restrict__ y, int yLd, ItemDiv div)
 {
-    long long idx = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= total) return;
-    const int cv = c / VEC;
-    const int c0 = static_cast<int>(idx % cv) * VEC;
-    const long long p = idx / cv;
-    const int OW = W * stride, OH = H * stride;
-    const int ox = static_cast<int>(p % OW);
-    const long long t = p / OW;
-    const int oy = static_cast<int>(t % OH);
-    const long long b = t / OH;
+    const long long idx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= div.total) return;
+    const Item item = itemOf(div, idx);
+    const int c0 = item.c * VEC;
     float v[VEC];
-    loadVec<T, VEC>(x + ((b * H + oy / stride) * W + ox / stride) * xLd + c0, v);
+    loadVec<T, VEC>(x + ((item.b * H + fastDiv(static_cast<unsigned>(item.oy), byStride)) * W + fastDiv(static_cast<unsigned>(item.ox), byStride)) * xLd + c0, v);
 #pragma unroll
     for (int i = 0; i < VEC; ++i) v[i] = scale * v[i];
-    storeVec<T, VEC>(y + p * yLd + c0, v);
+    storeVec<T, VEC>(y + item.p * yLd + c0, v);
 }
 
 template <typename T, int VEC>
@@ -392,23 +414,17 @@ __global__ __launch_bounds__(256) void copyChannelsKernel(const T *__restrict__ 
 
 // ---- constant padding / strided slice / bilinear resize ---------------------------------------------------------
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void padKernel(const T *__restrict__ x, int xLd, int H, int W, int c, int top, int left, int OH, int OW,
-                                                 float mul, float value, T *__restrict__ y, int yLd, long long total)
+__global__ __launch_bounds__(256) void padKernel(const T *__restrict__ x, int xLd, int H, int W, int top, int left, float mul, float value, T *__restrict__ y, int yLd, ItemDiv div)
 {
-    long long idx = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= total) return;
-    const int cv = c / VEC;
-    const int c0 = static_cast<int>(idx % cv) * VEC;
-    const long long p = idx / cv;
-    const int ox = static_cast<int>(p % OW);
-    const long long t = p / OW;
-    const int oy = static_cast<int>(t % OH);
-    const long long b = t / OH;
-    const int iy = oy - top, ix = ox - left;
+    const long long idx = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= div.total) return;
+    const Item item = itemOf(div, idx);
+    const int c0 = item.c * VEC;
+    const int iy = item.oy - top, ix = item.ox - left;
     float v[VEC];
     if (iy >= 0 && iy < H && ix >= 0 && ix < W)
     {
-        loadVec<T, VEC>(x + ((b * H + iy) * W + ix) * xLd + c0, v);
+        loadVec<T, VEC>(x + ((item.b * H + iy) * W + ix) * xLd + c0, v);
 #pragma unroll
         for (int i = 0; i < VEC; ++i) v[i] = mul * v[i];
     }
@@ -417,7 +433,7 @@ __global__ __launch_bounds__(256) void padKernel(const T *__restrict__ x, int xL
 #pragma unroll
         for (int i = 0; i < VEC; ++i) v[i] = value;
     }
-    storeVec<T, VEC>(y + p * yLd + c0, v);
+    storeVec<T, VEC>(y + item.p * yLd + c0, v);
 }
 
 template <typename T>
@@ -567,26 +583,48 @@ __global__ __launch_bounds__(256) void col2imKernel(const T *__restrict__ cols, 
 }
 
 // ---- fully connected: one wavefront per (batch row, output), wave-level reduction -------------------------
-template <typename T>
+// A wavefront per (image, output), VEC consecutive inputs per lane and load, eight loads in flight.  Bound by latency: with one input per lane and load
+// the 1280 inputs of MobileNetV2's classifier were 20 loads, a few at a time.
+template <typename T, int VEC>
 __global__ __launch_bounds__(256) void connectedKernel(const T *__restrict__ x, float xMul, const T *__restrict__ w,
                                                        const float *__restrict__ bias, int act, float actParam, float *__restrict__ y,
                                                        int batch, int inputs, int outputs)
 {
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const int lane = threadIdx.x & 63;
     if (wave >= batch * outputs) return;
-    const int b = wave / outputs, o = wave - b * outputs;
+    const int b = batch == 1 ? 0 : wave / outputs, o = wave - b * outputs;
     const T *xp = x + static_cast<size_t>(b) * inputs;
     const T *wp = w + static_cast<size_t>(o) * inputs;
-    float sum = 0.f;
-    for (int i = lane; i < inputs; i += 64) sum += toF(xp[i]) * toF(wp[i]);
+    const float shift = bias ? bias[o] : 0.f;
+    float part[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) part[e] = 0.f;
+    constexpr int AHEAD = 8;                          // loads of a round, all in flight together
+    for (int i0 = 0; i0 < inputs; i0 += AHEAD * 64 * VEC)
+    {
+        float xv[AHEAD][VEC], wv[AHEAD][VEC];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+        {
+            const int i = i0 + (k * 64 + lane) * VEC, at = i < inputs ? i : 0;      // (past the end: any value, not added)
+            loadVec<T, VEC>(xp + at, xv[k]);
+            loadVec<T, VEC>(wp + at, wv[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+            if (i0 + (k * 64 + lane) * VEC < inputs)
+            {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) part[e] += xv[k][e] * wv[k][e];
+            }
+    }
+    float sum = part[0];
+#pragma unroll
+    for (int e = 1; e < VEC; ++e) sum += part[e];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-    if (lane == 0)
-    {
-        float v = sum * xMul + (bias ? bias[o] : 0.f);
-        y[static_cast<size_t>(b) * outputs + o] = activate(v, act, actParam);
-    }
+    if (lane == 0) y[static_cast<size_t>(b) * outputs + o] = activate(sum * xMul + shift, act, actParam);
 }
 
 // ---- boundary layout conversions (tiled transposes through LDS) --------------------------------------------
@@ -738,11 +776,12 @@ int msnh_hip_maxpool(int dtype, int batch, int in_h, int in_w, int c, const void
     dim3 grid(gridFor(total, 256));
     if ((ksize == 2 || ksize == 3 || ksize == 5) && vec > 1)
     {
-        const int blocks = static_cast<int>(grid.x);
-        const dim3 xgrid((blocks + 7) / 8 * 8);
+        const int perXcd = (static_cast<int>(grid.x) + 7) / 8;
+        const dim3 xgrid(perXcd * 8);
+        const ItemDiv div = makeItemDiv(c / vec, out_w, out_h, total);
 #define MSNH_MPU(T, V, K)                                                                                               \
-        hipLaunchKernelGGL((maxPoolUnrolledKernel<T, V, K>), xgrid, dim3(256), 0, st, static_cast<const T *>(x), x_ld, in_h, in_w, c, stride, \
-                           pad, out_h, out_w, static_cast<T *>(y), y_ld, total, blocks)
+        hipLaunchKernelGGL((maxPoolUnrolledKernel<T, V, K>), xgrid, dim3(256), 0, st, static_cast<const T *>(x), x_ld, in_h, in_w, stride, pad, \
+                           static_cast<T *>(y), y_ld, div, perXcd)
 #define MSNH_MPUK(T, V) do { if (ksize == 2) MSNH_MPU(T, V, 2); else if (ksize == 3) MSNH_MPU(T, V, 3); else MSNH_MPU(T, V, 5); } while (0)
         if (dtype == MSNH_F16) MSNH_MPUK(f16, 8); else MSNH_MPUK(float, 4);
 #undef MSNH_MPUK
@@ -853,8 +892,8 @@ int msnh_hip_upsample_nearest(int dtype, int batch, int in_h, int in_w, int c, c
     const long long total = static_cast<long long>(batch) * in_h * stride * in_w * stride * (c / vec);
     dim3 grid(gridFor(total, 256));
 #define MSNH_UP(T, V)                                                                                                  \
-    hipLaunchKernelGGL((upsampleKernel<T, V>), grid, dim3(256), 0, st, static_cast<const T *>(x), x_ld, in_h, in_w, c, stride, scale, \
-                       static_cast<T *>(y), y_ld, total)
+    hipLaunchKernelGGL((upsampleKernel<T, V>), grid, dim3(256), 0, st, static_cast<const T *>(x), x_ld, in_h, in_w, makeFastDiv(static_cast<unsigned>(stride)), scale, \
+                       static_cast<T *>(y), y_ld, makeItemDiv(c / vec, in_w * stride, in_h * stride, total))
     if (dtype == MSNH_F16) { if (vec == 8) MSNH_UP(f16, 8); else MSNH_UP(f16, 1); }
     else { if (vec == 4) MSNH_UP(float, 4); else MSNH_UP(float, 1); }
 #undef MSNH_UP
@@ -873,8 +912,8 @@ int msnh_hip_pad(int dtype, int batch, int in_h, int in_w, int c, const void *x,
     const long long total = static_cast<long long>(batch) * out_h * out_w * (c / vec);
     dim3 grid(gridFor(total, 256));
 #define MSNH_PAD(T, V)                                                                                                 \
-    hipLaunchKernelGGL((padKernel<T, V>), grid, dim3(256), 0, st, static_cast<const T *>(x), x_ld, in_h, in_w, c, top, left, out_h, out_w, \
-                       mul, value, static_cast<T *>(y), y_ld, total)
+    hipLaunchKernelGGL((padKernel<T, V>), grid, dim3(256), 0, st, static_cast<const T *>(x), x_ld, in_h, in_w, top, left, mul, value, \
+                       static_cast<T *>(y), y_ld, makeItemDiv(c / vec, out_w, out_h, total))
     if (dtype == MSNH_F16) { if (vec == 8) MSNH_PAD(f16, 8); else MSNH_PAD(f16, 1); }
     else { if (vec == 4) MSNH_PAD(float, 4); else MSNH_PAD(float, 1); }
 #undef MSNH_PAD
@@ -989,12 +1028,13 @@ int msnh_hip_connected(int dtype, int batch, int inputs, int outputs, const void
     }
     const long long waves = static_cast<long long>(batch) * outputs;
     dim3 grid(gridFor(waves * 64, 256));
-    if (dtype == MSNH_F16)
-        hipLaunchKernelGGL((connectedKernel<f16>), grid, dim3(256), 0, st, static_cast<const f16 *>(x), x_mul, static_cast<const f16 *>(w),
-                           bias, act, act_param, y, batch, inputs, outputs);
-    else
-        hipLaunchKernelGGL((connectedKernel<float>), grid, dim3(256), 0, st, static_cast<const float *>(x), x_mul,
-                           static_cast<const float *>(w), bias, act, act_param, y, batch, inputs, outputs);
+    const bool wide = inputs % vec == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+#define MSNH_FC(T, V)                                                                                                  \
+    hipLaunchKernelGGL((connectedKernel<T, V>), grid, dim3(256), 0, st, static_cast<const T *>(x), x_mul, static_cast<const T *>(w), bias, act, act_param, y, batch, \
+                       inputs, outputs)
+    if (dtype == MSNH_F16) { if (wide) MSNH_FC(f16, 8); else MSNH_FC(f16, 1); }
+    else { if (wide) MSNH_FC(float, 4); else MSNH_FC(float, 1); }
+#undef MSNH_FC
     MSNH_LAUNCH_CHECK();
     return 0;
 }

@@ -327,6 +327,30 @@ def test_connected(dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("inputs,shifted", [(1, 0), (7, 0), (8, 0), (256, 0), (2048, 0), (2056, 0), (4096, 1), (4100, 0), (5003, 0)])
+def test_connected_rounds(inputs, shifted, dtype):
+    """row lengths around a round of vector loads (2048 / 4096 inputs), below a vector and unaligned: float32 sums in any order, so within
+    a rounding per product and addition of the sum of magnitudes"""
+    import gpuutil as gu
+    gu.init()
+    rng = np.random.default_rng(inputs)
+    x = _x(rng, (2, inputs + shifted), dtype)
+    w = rng.uniform(-0.05, 0.05, 11 * inputs + shifted).astype(np.float32)
+    w = gu.round_f16(w) if dtype == abi.F16 else w
+    xd, wd = gu.dev(x, dtype), gu.dev(w, dtype)
+    yd = torch.zeros((2, 11), dtype=torch.float32).cuda()
+    gu.sync()
+    es = 4 if dtype == abi.F32 else 2
+    at = lambda t: ctypes.c_void_p(t.data_ptr() + es * shifted)
+    abi.check(abi.lib().msnh_hip_connected(dtype, 2, inputs, 11, at(xd), 1.0, at(wd), None, abi.ACT["none"], 0.1, gu.ptr(yd), None))
+    gu.sync()
+    xs = np.lib.stride_tricks.as_strided(x.ravel()[shifted:], (2, inputs), (x.itemsize * inputs, x.itemsize)).astype(np.float64)
+    ws = w[shifted:].reshape(11, inputs).astype(np.float64)
+    bound = 2.0 ** -24 * (inputs + 1) * (np.abs(xs) @ np.abs(ws).T)
+    assert (np.abs(yd.cpu().numpy() - xs @ ws.T) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("batch,inputs,outputs,act", [(32, 2048, 1000, "none"), (64, 1280, 1000, "relu"), (9, 64, 24, "leaky")])
 def test_connected_batched(dtype, batch, inputs, outputs, act):
     """with a real batch the fully connected layer runs as the 1x1 case of the MFMA implicit GEMM"""
