@@ -821,10 +821,14 @@ int msnh_hip_maxpool_chain(int dtype, int batch, int in_h, int in_w, int c, int 
 {
     MSNH_REQUIRE(dtypeOk(dtype), "maxpool_chain: bad dtype");
     MSNH_REQUIRE(batch > 0 && in_h > 0 && in_w > 0 && c > 0 && x && y && y_ld && x_ld >= c, "maxpool_chain: bad argument");
-    const int cg = poolChainGroup(dtype, in_h, in_w, c, ksize, steps);
+    int cg = poolChainGroup(dtype, in_h, in_w, c, ksize, steps);
     MSNH_REQUIRE(cg > 0, "maxpool_chain: windows of 3 or 5, 2 or 3 pools, channels a multiple of the 16-byte vector, and an H x W tile that fits LDS "
                          "(msnh_hip_maxpool_chain_supported)");
     const int vec = dtype == MSNH_F16 ? 8 : 4;
+    // Few images leave most CUs without a workgroup, and one workgroup's chain of passes over LDS is then the launch's time: fewer channels
+    // each, down to one vector, for a workgroup per CU.  float16, 3 x 17x17x256: 12.5 -> 7.4 us, 1 x 19x19x512: 13.8 -> 7.5.  Not two per CU:
+    // 16 x 19x19x512 takes 16.1 us with 256 workgroups of 32 channels and 19.8 with 512 of 16 (half a cache line per pixel).
+    while (cg > vec && static_cast<long long>(batch) * ((c + cg - 1) / cg) < 256) cg /= 2;
     MSNH_REQUIRE(x_ld % vec == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0, "maxpool_chain: input must be 16-byte aligned with a row stride of whole vectors");
     for (int i = 0; i < steps; ++i)
         MSNH_REQUIRE(y[i] && y_ld[i] >= c && y_ld[i] % vec == 0 && reinterpret_cast<uintptr_t>(y[i]) % 16 == 0,

@@ -110,6 +110,32 @@ def test_maxpool_windows_compose(h, w, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,h,w,c", [(1, 17, 17, 40), (1, 13, 13, 264), (4, 9, 9, 512), (20, 13, 13, 136), (70, 5, 7, 256)])
+def test_maxpool_chain_groups(batch, h, w, c, dtype):
+    """the chain's channels per workgroup go from one 16-byte vector (few images) to 64 (many), with a last group that is not whole: each
+    pool's result equals the separate launch's bit for bit"""
+    import ctypes
+    import gpuutil as gu
+    gu.init()
+    L = abi.lib()
+    rng = np.random.default_rng(batch * 7 + c)
+    xd = gu.nhwc_dev(_x(rng, (batch, c, h, w), dtype), dtype)
+    out = [torch.zeros((batch, h, w, c), dtype=gu.TORCH_DT[dtype]).cuda() for _ in range(3)]
+    ys = (ctypes.c_void_p * 3)(*[o.data_ptr() for o in out])
+    gu.sync()
+    abi.check(L.msnh_hip_maxpool_chain(dtype, batch, h, w, c, 5, 3, gu.ptr(xd), c, ys, (ctypes.c_int * 3)(c, c, c), None))
+    gu.sync()
+    src = xd
+    for o in out:
+        sep = torch.zeros_like(o)
+        gu.sync()
+        abi.check(L.msnh_hip_maxpool(dtype, batch, h, w, c, gu.ptr(src), c, 5, 1, 2, h, w, gu.ptr(sep), c, None))
+        gu.sync()
+        assert torch.equal(o, sep)
+        src = sep
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("h,w,c,k,steps", [(19, 19, 512, 5, 3), (13, 13, 72, 5, 3), (7, 5, 24, 5, 2), (16, 16, 256, 3, 3), (2, 2, 8, 5, 3)])
 def test_maxpool_chain(h, w, c, k, steps, dtype):
     """the pools of an SPP block in one launch (msnh_hip_maxpool_chain): every pool's result equals the oracle's max-pool with the
