@@ -221,6 +221,24 @@ int msnh_hip_conv2d_tail_supported(const msnh_conv_desc *d, const msnh_conv_tail
 int msnh_hip_conv2d_tail(const msnh_conv_desc *d, const msnh_conv_tail_desc *t, const void *x, const void *w, const float *scale, const float *shift,
                          const void *residual, void *y, const void *w2, const float *scale2, const float *shift2, void *z, msnh_stream_t s);
 
+/* Two 1x1 stride-1 convolutions over one tensor as one launch: those that open a cross-stage block of CSPDarknet-53 and YOLOv5 (two
+ * ConvolutionalLayer::forwardGPU calls, src/layers/MsnhConvolutionalLayer.cpp:984-1169, over the same route).  d describes both together: out_c is the sum
+ * of their channels, w / scale / shift hold the first one's filters and then the second one's, packed as for MSNH_CONV_IGEMM (d->out_ld is only
+ * checked to be at least out_c; d->act, act_param and out_mul are the first one's); algo MSNH_CONV_IGEMM or MSNH_CONV_IGEMM_FUSEDK, no residual.  Channels
+ * below p->first_c (a multiple of 32) go to y, the others, with their own activation and factor, to y2.  _supported: pure host function; tile as for
+ * msnh_hip_conv2d_tile_supported; the workspace is msnh_hip_conv2d_workspace_bytes(d). */
+typedef struct msnh_conv_pair_desc
+{
+    int   first_c;          /* channels of y */
+    int   out_ld, out_ld2;  /* pixel strides of y and y2 */
+    int   act;              /* msnh_act of the second convolution */
+    float act_param;
+    float out_mul;
+} msnh_conv_pair_desc;
+int msnh_hip_conv2d_pair_supported(const msnh_conv_desc *d, const msnh_conv_pair_desc *p, int tile);
+int msnh_hip_conv2d_pair(const msnh_conv_desc *d, const msnh_conv_pair_desc *p, const void *x, const void *w, const float *scale, const float *shift, void *y, void *y2,
+                         void *workspace, size_t workspace_bytes, msnh_stream_t s);
+
 /* The first two convolutions of the Darknet-53 / CSPDarknet-53 trunks as one launch, float16: a 3x3 stride-1 pad-1 convolution with 32
  * filters over the 3-channel NCHW float32 network input, then a 3x3 stride-2 pad-1 convolution with c2 = 32 / 64 / 128 filters
  * (two ConvolutionalLayer::forwardGPU calls, src/layers/MsnhConvolutionalLayer.cpp:984-1169, with the full-resolution 32-channel tensor

@@ -13,6 +13,8 @@ int convIgemm(const msnh_conv_desc *d, const void *x, const void *w, const float
               const void *residual, void *y, hipStream_t st, bool dryRun);
 int convIgemmTail(const msnh_conv_desc *d, const msnh_conv_tail_desc *tail, const void *x, const void *w, const float *scale, const float *shift,
                   const void *residual, void *y, const void *w2, const float *scale2, const float *shift2, void *z, hipStream_t st, bool dryRun);
+int convIgemmPair(const msnh_conv_desc *d, const msnh_conv_pair_desc *pair, const void *x, const void *w, const float *scale, const float *shift, void *y, void *y2,
+                  hipStream_t st, bool dryRun, void *ws, size_t wsBytes);
 int igemmTailTileFirst();
 int convIgemmWs(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                 const void *residual, void *y, hipStream_t st, bool dryRun, void *splitWs, size_t splitWsBytes);
@@ -417,6 +419,34 @@ int msnh_hip_conv2d_tail(const msnh_conv_desc *d, const msnh_conv_tail_desc *t, 
     msnh_conv_desc c = *d;
     c.algo = MSNH_CONV_IGEMM;
     return convIgemmTail(&c, t, x, w, scale, shift, residual, y, w2, scale2, shift2, z, resolveStream(s), false);
+}
+
+static bool pairDescOk(const msnh_conv_desc *d, const msnh_conv_pair_desc *p)
+{
+    return d && p && !validate(d) && igemmOk(d) && d->groups == 1 && d->ksize == 1 && d->stride == 1 && d->pad == 0 && !d->has_residual && d->out_upsample != 2 &&
+           (d->algo == MSNH_CONV_IGEMM || d->algo == MSNH_CONV_IGEMM_FUSEDK) && d->tile >= 0 && d->out_c % 8 == 0 && p->first_c > 0 && p->first_c % 32 == 0 &&
+           p->first_c < d->out_c && p->out_ld >= p->first_c && p->out_ld2 >= d->out_c - p->first_c && actOk(p->act);
+}
+
+int msnh_hip_conv2d_pair_supported(const msnh_conv_desc *d, const msnh_conv_pair_desc *p, int tile)
+{
+    if (tile < 0 || (d && tile > igemmTileCount() && d->algo != MSNH_CONV_IGEMM_FUSEDK) || !pairDescOk(d, p)) return 0;
+    msnh_conv_desc c = *d;
+    c.out_ld = p->out_ld;
+    c.tile = tile;
+    return convIgemmPair(&c, p, d, d, nullptr, nullptr, &c, &c, nullptr, true, nullptr, 0) == 0 ? 1 : 0;      // pointers unused in a dry run
+}
+
+int msnh_hip_conv2d_pair(const msnh_conv_desc *d, const msnh_conv_pair_desc *p, const void *x, const void *w, const float *scale, const float *shift, void *y, void *y2,
+                         void *workspace, size_t workspace_bytes, msnh_stream_t s)
+{
+    MSNH_REQUIRE(pairDescOk(d, p), "conv2d_pair: an ungrouped 1x1 stride-1 IGEMM or IGEMM_FUSEDK convolution without residual, channel counts multiples of 8, the first tensor's of 32");
+    MSNH_REQUIRE(x && w && y && y2, "conv2d_pair: NULL tensor pointer");
+    MSNH_REQUIRE(d->in_ld >= d->in_c, "conv2d_pair: in_ld < in_c");
+    MSNH_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0, "conv2d_pair: 16-byte aligned x and w");
+    msnh_conv_desc c = *d;
+    c.out_ld = p->out_ld;
+    return convIgemmPair(&c, p, x, w, scale, shift, y, y2, resolveStream(s), false, workspace, workspace_bytes);
 }
 
 int msnh_hip_conv2d_select_algo(const msnh_conv_desc *d)

@@ -108,7 +108,8 @@ static int convIgemmSplitK(IgemmArgs &a, const msnh_conv_desc *d, int tile, hipS
 // tiles that carry a tail, 0 the first of them that takes the shape.
 static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,
                         const void *residual, void *y, hipStream_t st, bool dryRun, void *splitWs, size_t splitWsBytes,
-                        const msnh_conv_tail_desc *tail, const void *w2, const float *scale2, const float *shift2, void *z, size_t *wsNeed = nullptr)
+                        const msnh_conv_tail_desc *tail, const void *w2, const float *scale2, const float *shift2, void *z, size_t *wsNeed = nullptr,
+                        const msnh_conv_pair_desc *pair = nullptr)
 {
     IgemmArgs a;
     a.tailOn = tail ? 1 : 0;
@@ -116,6 +117,11 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
     a.cout2 = tail ? tail->out_c : 0; a.zLd = tail ? tail->out_ld : 0; a.act3 = tail ? tail->act : MSNH_ACT_NONE; a.writeY = tail ? (tail->write_y ? 1 : 0) : 1;
     a.act3Param = tail ? tail->act_param : 0.f; a.zMul = tail ? tail->out_mul : 1.f;
     a.w2Bytes = tail ? static_cast<unsigned>(tail->out_c) * static_cast<unsigned>(d->out_c) * 2u : 0u;
+    a.pairC = 0;
+    if (pair)
+    {
+        a.pairC = pair->first_c; a.z = z; a.zLd = pair->out_ld2; a.act3 = pair->act; a.act3Param = pair->act_param; a.zMul = pair->out_mul;
+    }
     a.x = x; a.w = w; a.scale = scale; a.shift = shift; a.res = residual; a.y = y;
     a.batch = d->batch; a.H = d->in_h; a.W = d->in_w; a.inLd = d->in_ld;
     a.OH = d->out_h; a.OW = d->out_w; a.outLd = d->out_ld; a.resLd = d->res_ld;
@@ -150,6 +156,7 @@ static int convIgemmAny(const msnh_conv_desc *d, const void *x, const void *w, c
     a.vecOk = (d->out_ld % 8 == 0) && ((d->out_c / d->groups) % 8 == 0 || d->groups == 1) &&
               (reinterpret_cast<uintptr_t>(y) % (8 * outEl) == 0) &&
               (!a.hasRes || (d->res_ld % 8 == 0 && reinterpret_cast<uintptr_t>(residual) % 16 == 0));
+    if (pair) a.vecOk = a.vecOk && pair->out_ld2 % 8 == 0 && reinterpret_cast<uintptr_t>(z) % (8 * outEl) == 0;
     a.splitMax = 0; a.splitK = 1; a.fusedK = 0; a.wsNeed = a.wsBytes = 0; a.ws = nullptr; a.wsLd = d->out_c; a.slicePitch = 0;
     if (a.up2) MSNH_REQUIRE(d->algo != MSNH_CONV_IGEMM_SPLITK && !tail, "conv2d: the upsampling epilogue goes with the plain implicit GEMM");
     if (d->algo == MSNH_CONV_IGEMM_SPLITK)
@@ -210,6 +217,18 @@ int convIgemmTail(const msnh_conv_desc *d, const msnh_conv_tail_desc *tail, cons
                   const void *residual, void *y, const void *w2, const float *scale2, const float *shift2, void *z, hipStream_t st, bool dryRun)
 {
     return convIgemmAny(d, x, w, scale, shift, residual, y, st, dryRun, nullptr, 0, tail, w2, scale2, shift2, z);
+}
+
+// d->out_ld: the first tensor's.  Tile 0: the one the shape's rule names or, where that one's wave tiles are cut by the border between the tensors, the first
+// that takes the pair.
+int convIgemmPair(const msnh_conv_desc *d, const msnh_conv_pair_desc *pair, const void *x, const void *w, const float *scale, const float *shift, void *y, void *y2,
+                  hipStream_t st, bool dryRun, void *ws, size_t wsBytes)
+{
+    msnh_conv_desc c = *d;
+    const auto run = [&](bool dry) { return convIgemmAny(&c, x, w, scale, shift, nullptr, y, st, dry, ws, wsBytes, nullptr, nullptr, nullptr, nullptr, y2, nullptr, pair); };
+    if (c.algo != MSNH_CONV_IGEMM_FUSEDK && c.tile == 0 && run(true) != 0)
+        for (c.tile = 1; c.tile < kIgemmTailTileFirst && run(true) != 0;) ++c.tile;
+    return run(dryRun);
 }
 
 int convIgemm(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,

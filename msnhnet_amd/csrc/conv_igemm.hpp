@@ -72,7 +72,13 @@ struct IgemmArgs
     int cout2, zLd, act3, writeY;
     float act3Param, zMul;
     unsigned w2Bytes;
+    // pair (msnh_hip_conv2d_pair): channels from pairC on belong to a second tensor z with pixel stride zLd, activation act3 and factor zMul; a multiple of
+    // the rows of a wave tile, so a wavefront's results go to one of the two.  0: no second tensor.
+    int pairC;
 };
+
+// whether channel m and those of its wave tile belong to the second tensor of a pair
+__device__ __forceinline__ bool igemmSecond(const IgemmArgs &a, int m) { return static_cast<unsigned>(m) > static_cast<unsigned>(a.pairC) - 1u; }
 
 // Workgroup -> tile.  Consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its own L2: id % 8 selects
 // the XCD, id / 8 the position inside it.  Default arrangement (xcdGm <= 1): an XCD takes a contiguous run of tiles with the
@@ -421,14 +427,17 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
     const int mv   = m0 + wm * TM + vcol;             // first channel of this lane's vector (within the group)
     const bool chOk = mv < a.coutG;
     const bool full = a.vecOk && (mv + 7 < a.coutG);
-    const unsigned ch = static_cast<unsigned>(chBase + mv);
+    const bool second = igemmSecond(a, __builtin_amdgcn_readfirstlane(m0 + wm * TM));
+    const int outLd = second ? a.zLd : a.outLd, act = second ? a.act3 : a.act;
+    const float actParam = second ? a.act3Param : a.actParam, outMul = second ? a.zMul : a.outMul;
+    const unsigned ch = static_cast<unsigned>(chBase + mv) - (second ? a.pairC : 0);
     const int npix = min(a.P - p0, BN);
-    TOut    *yBlock = static_cast<TOut *>(a.y) + blockIdx.y * a.slicePitch + static_cast<size_t>(p0) * a.outLd;
+    TOut    *yBlock = static_cast<TOut *>(second ? a.z : a.y) + blockIdx.y * a.slicePitch + static_cast<size_t>(p0) * outLd;
     const T *rBlock = static_cast<const T *>(a.res) + static_cast<size_t>(p0) * a.resLd;
-    const __amdgpu_buffer_rsrc_t ry = a.up2 ? makeRsrc(a.y, a.yBytes) : makeRsrc(yBlock, static_cast<unsigned>(npix) * a.outLd * sizeof(TOut));
+    const __amdgpu_buffer_rsrc_t ry = a.up2 ? makeRsrc(a.y, a.yBytes) : makeRsrc(yBlock, static_cast<unsigned>(npix) * outLd * sizeof(TOut));
     const __amdgpu_buffer_rsrc_t rr = makeRsrc(a.hasRes ? rBlock : nullptr, a.hasRes ? static_cast<unsigned>(npix) * a.resLd * sizeof(T) : 0u);
     float slope1, slope2;
-    const bool lin1 = actIsSlope(a.act, a.actParam, slope1);
+    const bool lin1 = actIsSlope(act, actParam, slope1);
     const bool lin2 = actIsSlope(a.act2, a.act2Param, slope2);
 
     staticFor<0, NB>([&](auto jTag) {
@@ -461,9 +470,9 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
             if (lin1)
             {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) v[e] = activateSel<true>(v[e], slope1, a.act, a.actParam);
+                for (int e = 0; e < 16; ++e) v[e] = activateSel<true>(v[e], slope1, act, actParam);
             }
-            else activateArray<16>(v, a.act, a.actParam);
+            else activateArray<16>(v, act, actParam);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<f32x4 *>(stage + (lane & 31) * LDE + i * 32 + q * 8 + (lane >> 5) * 4) = f32x4{v[q * 4], v[q * 4 + 1], v[q * 4 + 2], v[q * 4 + 3]};
@@ -499,7 +508,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
                     for (int e = 0; e < 8; ++e) v[e] = activateSel<true>(v[e] + a.resMul * r[e], slope2, a.act2, a.act2Param);
                 }
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] *= a.outMul;
+                for (int e = 0; e < 8; ++e) v[e] *= outMul;
                 Raw8<TOut> o;
                 o.fromFloat(v);
                 if (a.up2)
@@ -517,7 +526,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
                     bufferStore8<TOut>(o, ry, in ? (q + rowStep) * es : kOobOffset);
                     bufferStore8<TOut>(o, ry, in ? (q + rowStep + a.outLd) * es : kOobOffset);
                 }
-                else bufferStore8<TOut>(o, ry, (pl * a.outLd + ch) * static_cast<unsigned>(sizeof(TOut)));
+                else bufferStore8<TOut>(o, ry, (pl * outLd + ch) * static_cast<unsigned>(sizeof(TOut)));
             }
         }
         else if (chOk)
@@ -533,7 +542,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
                 float v[8];
                 readStaged(row, v);
                 const T *rp = rBlock + static_cast<size_t>(pl) * a.resLd + ch;
-                TOut *yp = yBlock + static_cast<size_t>(pl) * a.outLd + ch;
+                TOut *yp = yBlock + static_cast<size_t>(pl) * outLd + ch;
                 if (a.hasRes)
                 {
 #pragma unroll
@@ -543,7 +552,7 @@ __device__ __forceinline__ void igemmEpilogue(const IgemmArgs &a, f32x16 (&acc)[
                 }
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    if (mv + e < a.coutG) yp[e] = fromF<TOut>(a.outMul * v[e]);
+                    if (mv + e < a.coutG) yp[e] = fromF<TOut>(outMul * v[e]);
             }
         }
         if (j + 1 < NB)
@@ -627,9 +636,12 @@ __device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (
     const int ml = q * 8 + (lane >> 5) * 4;                       // first of this lane's channels inside the tile
     const int mv = m0 + ml;
     const bool full = a.vecOk && mv + 3 < a.coutG;
-    const unsigned ch = static_cast<unsigned>(chBase + mv);
+    const bool second = igemmSecond(a, m0);
+    const int outLd = second ? a.zLd : a.outLd, act = second ? a.act3 : a.act;
+    const float actParam = second ? a.act3Param : a.actParam, outMul = second ? a.zMul : a.outMul;
+    const unsigned ch = static_cast<unsigned>(chBase + mv) - (second ? a.pairC : 0);
     const int npix = min(a.P - p0, BN);
-    TOut    *yBlock = static_cast<TOut *>(a.y) + blockIdx.y * a.slicePitch + static_cast<size_t>(p0) * a.outLd;
+    TOut    *yBlock = static_cast<TOut *>(second ? a.z : a.y) + blockIdx.y * a.slicePitch + static_cast<size_t>(p0) * outLd;
     const T *rBlock = static_cast<const T *>(a.res) + static_cast<size_t>(p0) * a.resLd;
     // the residual travels while the sums are parked and added
     float r[NB][4];
@@ -680,7 +692,7 @@ __device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (
         if (pl >= npix) return;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[j][e] = v[j][e] * sc[e] + sh[e];
-        activateArray<4>(v[j], a.act, a.actParam);
+        activateArray<4>(v[j], act, actParam);
         if (a.hasRes)
         {
 #pragma unroll
@@ -689,7 +701,7 @@ __device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (
         }
         TOut4 o;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = fromF<TOut>(v[j][e] * a.outMul);
+        for (int e = 0; e < 4; ++e) o[e] = fromF<TOut>(v[j][e] * outMul);
         const auto put = [&](TOut *yp) {
             if (full) *reinterpret_cast<TOut4 *>(yp) = o;
             else
@@ -711,7 +723,7 @@ __device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (
             put(yq + rowStep);
             put(yq + rowStep + a.outLd);
         }
-        else put(yBlock + static_cast<size_t>(pl) * a.outLd + ch);
+        else put(yBlock + static_cast<size_t>(pl) * outLd + ch);
     });
 }
 
@@ -1518,6 +1530,11 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
     if (a.up2 && (TAIL != 0 || groups != 1 || a.hasRes || a.splitMax > 1 || (!a.vecOk && !a.dryRun) || a.coutG % 8 != 0))
     {
         setError("conv2d: the upsampling epilogue takes an ungrouped convolution without residual, channel counts multiples of 8");
+        return 3;
+    }
+    if (a.pairC > 0 && (TAIL != 0 || groups != 1 || a.hasRes || a.up2 || a.splitMax > 1 || a.pairC % (BM / WM) != 0))
+    {
+        setError("conv2d_pair: the first tensor's channels must be whole wave tiles of this tile");
         return 3;
     }
     a.cChunks = (a.cinG + BK - 1) / BK;

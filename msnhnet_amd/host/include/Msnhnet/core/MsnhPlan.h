@@ -89,6 +89,8 @@ struct PlanOp
     int  tail = -1;                         // CONV: the 1x1 convolution op that reads this one's result and that the same launch can compute
                                             // (Plan::fuse e); it does when the search set algo to MSNH_CONV_IGEMM_TAIL, and the 1x1 op is then dead
     int  tailOf = -1;                       // CONV 1x1: the op whose launch may compute it
+    int  pair = -1;                         // CONV 1x1: the (dead) 1x1 convolution over the same input whose result this launch writes as well
+                                            // (Plan::pairConvs, msnh_hip_conv2d_pair)
     double ownFlops = 0;                    // CONV with a tail: flops without the tail's
     bool tailSkipY = false;                 // CONV computing its tail: nothing but the tail reads this op's own result, which therefore is not written
 
@@ -169,6 +171,7 @@ public:
     void fuse();                            // passes 1
     void chainMaxPools();                   // stride-1 max-pools of one tensor (SPP): each larger window reads the next smaller one's result
     void aliasConcats();                    // pass 2
+    void pairConvs();                       // pass 2b: 1x1 convolutions over one tensor, two to a launch (not on the calibration twin)
     void applyCalibration(const std::vector<float> &amax);   // pass 3: amax per tensor, from an executed float32 twin (or from its record on disk)
     std::vector<float> amaxOfTensors() const;
     uint64_t structureHash() const;         // over ops and tensors as lowered and optimised (before placement): what a pack file must match

@@ -424,6 +424,7 @@ void NetBuilder::finalizePlan()
     plan->fuse();
     plan->chainMaxPools();
     plan->aliasConcats();
+    if (std::getenv("MSNH_NO_CONV_PAIR") == nullptr) plan->pairConvs();
     const float lowerMs = msSince(t0);
 
     // The packed kernels and the calibration of an earlier load of these weights into this graph, if asked for and still valid

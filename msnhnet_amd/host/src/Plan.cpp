@@ -503,6 +503,31 @@ void Plan::aliasConcats()
     }
 }
 
+// ---- pass 2b: two 1x1 convolutions over one tensor -------------------------------------------------------------------
+// The two convolutions that open a cross-stage block (CSPDarknet-53, YOLOv5) read one tensor: as one launch with both sets of filters they read it
+// once, and where they are small the launch that goes costs as much as the one that stays.  Each writes its own tensor with its own activation and scale.
+// Always taken: yolov5s float16 b3 544 (eight pairs of 64 .. 512 channels over at most 136 x 136 pixels, 4 - 5 us a launch) 570 -> 528 us; yolov4 float16
+// b16 608 (five, the first 64 -> 64 + 64 over 304 x 304) 3939 -> 3889.  Not a wider concatenation that holds both results, written by an ordinary launch:
+// its readers then walk longer pixel rows (yolov4 0.993x).
+void Plan::pairConvs()
+{
+    const auto eligible = [&](const PlanOp &op) {
+        if (op.dead || op.kind != PlanOp::CONV || op.ksize != 1 || op.stride != 1 || op.pad != 0 || op.groups != 1 || op.in1 >= 0 || op.stemOp >= 0 || op.mbExpand >= 0 ||
+            op.tail >= 0 || op.tailOf >= 0 || op.pair >= 0 || op.up2)
+            return false;
+        const PlanTensor &x = tensors[static_cast<size_t>(op.in0)], &y = tensors[static_cast<size_t>(op.out)];
+        return x.layout == PlanTensor::NHWC && y.layout == PlanTensor::NHWC && x.c % 8 == 0 && y.c % 8 == 0 && (x.dtype == MSNH_F16 || y.dtype == MSNH_F32);
+    };
+    for (size_t i = 0; i < ops.size(); ++i)
+        for (size_t k = i + 1; k < ops.size() && eligible(ops[i]) && tensors[static_cast<size_t>(ops[i].out)].c % 32 == 0; ++k)
+        {
+            PlanOp &a = ops[i], &b = ops[k];
+            if (a.in0 != b.in0 || !eligible(b) || tensors[static_cast<size_t>(a.out)].dtype != tensors[static_cast<size_t>(b.out)].dtype) continue;
+            a.pair = static_cast<int>(k);
+            b.dead = true;
+        }
+}
+
 // ---- pass 3: calibration -------------------------------------------------------------------------------------------
 // Runs the plan once and takes max|x| of every tensor right behind the launch that writes it.  (Measuring after the whole forward
 // would read arena space that later tensors have reused: a tensor of the first layers would then be given the magnitude of whatever
@@ -549,10 +574,14 @@ float Plan::fp16Headroom(msnh_stream_t s)
         if (op.dead) continue;
         launch(op, s);
         if (op.out < 0) continue;
-        const PlanTensor &pt = tensors[static_cast<size_t>(op.out)];
-        if (pt.layout != PlanTensor::NHWC || pt.dtype != MSNH_F16 || op.kind == PlanOp::COPY) continue;
-        MSNH_DEV(msnh_hip_absmax(pt.dtype, pt.pixels(), pt.c, ptr(op.out), ld(op.out), res.as<float>(), s));
-        MSNH_DEV(msnh_hip_count_nonfinite(pt.dtype, pt.pixels(), pt.c, ptr(op.out), ld(op.out), res.as<unsigned>() + 1, s));
+        for (int t : {op.out, op.pair >= 0 ? ops[static_cast<size_t>(op.pair)].out : -1})
+        {
+            if (t < 0) continue;
+            const PlanTensor &pt = tensors[static_cast<size_t>(t)];
+            if (pt.layout != PlanTensor::NHWC || pt.dtype != MSNH_F16 || op.kind == PlanOp::COPY) continue;
+            MSNH_DEV(msnh_hip_absmax(pt.dtype, pt.pixels(), pt.c, ptr(t), ld(t), res.as<float>(), s));
+            MSNH_DEV(msnh_hip_count_nonfinite(pt.dtype, pt.pixels(), pt.c, ptr(t), ld(t), res.as<unsigned>() + 1, s));
+        }
     }
     float host[2] = {0.f, 0.f};
     MSNH_DEV(msnh_hip_memcpy_d2h(host, res.ptr(), sizeof(host), s));
@@ -578,7 +607,7 @@ uint64_t Plan::structureHash() const
     for (const PlanOp &op : ops)
         os << static_cast<int>(op.kind) << ' ' << op.in0 << ' ' << op.in1 << ' ' << op.out << ' ' << (op.dead && op.tailOf < 0) << ' ' << op.layerIndex << ' ' << op.ksize << ' ' << op.stride << ' '
            << op.pad << ' ' << op.dilation << ' ' << op.groups << ' ' << static_cast<int>(op.act) << ' ' << static_cast<int>(op.act2) << ' ' << op.in1Sign << ' ' << (op.src2 != nullptr)
-           << ' ' << op.dstChanOffset << ' ' << op.stemOp << ' ' << op.chainHead << ' ' << op.mbExpand << ' ' << op.tail << ' ' << op.stemTail << ' ' << op.up2 << ' ' << op.src2Offset << ' ' << op.focusAt[0]
+           << ' ' << op.dstChanOffset << ' ' << op.pair << ' ' << op.stemOp << ' ' << op.chainHead << ' ' << op.mbExpand << ' ' << op.tail << ' ' << op.stemTail << ' ' << op.up2 << ' ' << op.src2Offset << ' ' << op.focusAt[0]
            << ';';
     const std::string text = os.str();
     return PackFile::hash(text.data(), text.size());
@@ -638,6 +667,12 @@ void Plan::place()
         touch(op.in0, i); touch(op.in1, i); touch(op.out, i);
         if (op.chainHead >= 0) touch(op.out, op.chainHead);      // written by the launch of the chain's first pool
         if (op.tail >= 0) touch(ops[static_cast<size_t>(op.tail)].out, i);   // may be written by this launch (msnh_hip_conv2d_tail)
+        if (op.pair >= 0)
+        {
+            // written by this launch, and kept as if it were written where its own op stands (a layer's output is fetched behind that layer)
+            touch(ops[static_cast<size_t>(op.pair)].out, i);
+            touch(ops[static_cast<size_t>(op.pair)].out, op.pair);
+        }
         if (op.stemTail >= 0) touch(ops[static_cast<size_t>(op.stemTail)].out, i);   // written by this launch (msnh_hip_conv_stem_down_tail)
     }
     {
@@ -717,7 +752,30 @@ static msnh_conv_desc convDesc(const Plan &plan, const PlanOp &op)
     d.algo = op.algo;
     d.tile = op.tile;
     if (op.up2) { d.out_h = out.h / 2; d.out_w = out.w / 2; d.out_upsample = 2; }
+    if (op.pair >= 0) d.out_c = d.out_ld = out.c + plan.tensors[static_cast<size_t>(plan.ops[static_cast<size_t>(op.pair)].out)].c;      // (the strides are in pairDesc)
     return d;
+}
+
+static msnh_conv_pair_desc pairDesc(const Plan &plan, const PlanOp &op)
+{
+    const PlanOp &b = plan.ops[static_cast<size_t>(op.pair)];
+    msnh_conv_pair_desc p;
+    std::memset(&p, 0, sizeof(p));
+    p.first_c = plan.tensors[static_cast<size_t>(op.out)].c;
+    p.out_ld = plan.ld(op.out);
+    p.out_ld2 = plan.ld(b.out);
+    p.act = static_cast<int>(b.act);
+    p.act_param = b.actParam;
+    p.out_mul = 1.f / plan.mulOf(b.out);
+    return p;
+}
+
+// whether the library takes the op as described by `d` on that tile
+static bool tileSupported(const Plan &plan, const PlanOp &op, const msnh_conv_desc &d, int tile)
+{
+    if (op.pair < 0) return msnh_hip_conv2d_tile_supported(&d, tile) != 0;
+    const msnh_conv_pair_desc p = pairDesc(plan, op);
+    return msnh_hip_conv2d_pair_supported(&d, &p, tile) != 0;
 }
 
 static msnh_mbconv_desc mbconvDesc(const Plan &plan, const PlanOp &op)
@@ -864,7 +922,10 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             }
             d.algo = op.algo;
             workspace = std::max(workspace, msnh_hip_conv2d_workspace_bytes(&d, op.algo));
-            const std::vector<float> &w0 = op.src->kernelWeights();
+            std::vector<float> both;
+            if (op.pair >= 0)
+                for (const PlanOp *o : {&op, &ops[static_cast<size_t>(op.pair)]}) both.insert(both.end(), o->src->kernelWeights().begin(), o->src->kernelWeights().end());
+            const std::vector<float> &w0 = op.pair >= 0 ? both : op.src->kernelWeights();
             const bool focus = op.focusAt[0] >= 0;
             const size_t expect = static_cast<size_t>(d.out_c) * (focus ? 4 * d.in_c * 9 : (d.in_c / d.groups) * d.ksize * d.ksize);
             if (w0.size() != expect) MSNH_THROW("conv weights are not loaded (" + op.name + ")");
@@ -894,7 +955,21 @@ void Plan::prepareWeights(PackFile *from, PackFile *to)
             }
 
             std::vector<float> scale, shift;
-            foldAffine(op, d.out_c, in.layout == PlanTensor::NCHW_INPUT ? 1.f : mulOf(op.in0), scale, shift);
+            const int ownC = tensors[static_cast<size_t>(op.out)].c;
+            foldAffine(op, ownC, in.layout == PlanTensor::NCHW_INPUT ? 1.f : mulOf(op.in0), scale, shift);
+            if (op.pair >= 0)
+            {
+                std::vector<float> scale2, shift2;
+                foldAffine(ops[static_cast<size_t>(op.pair)], d.out_c - ownC, mulOf(op.in0), scale2, shift2);
+                const auto join = [&](std::vector<float> &x, const std::vector<float> &y, float none) {
+                    if (x.empty() && y.empty()) return;
+                    x.resize(static_cast<size_t>(ownC), none);
+                    x.insert(x.end(), y.begin(), y.end());
+                    x.resize(static_cast<size_t>(d.out_c), none);
+                };
+                join(scale, scale2, 1.f);
+                join(shift, shift2, 0.f);
+            }
             if (!scale.empty()) op.scaleDev.upload(scale.data(), scale.size() * sizeof(float));
             if (!shift.empty()) op.shiftDev.upload(shift.data(), shift.size() * sizeof(float));
             op.flops = 2.0 * d.batch * d.out_h * d.out_w * static_cast<double>(w0.size());
@@ -982,6 +1057,7 @@ static std::string tuneSignature(const Plan &plan, const PlanOp &op)
        << plan.ld(op.out) << ' ' << op.ksize << ' ' << op.stride << ' ' << op.pad << ' ' << op.dilation << ' ' << op.groups << ' ' << (op.in1 >= 0) << ' '
        << in.dtype << ' ' << out.dtype;
     if (op.up2) os << " up2";
+    if (op.pair >= 0) os << " pair " << plan.tensors[static_cast<size_t>(plan.ops[static_cast<size_t>(op.pair)].out)].c << ' ' << plan.ld(plan.ops[static_cast<size_t>(op.pair)].out);
     if (op.tail >= 0) os << " tail " << plan.tensors[static_cast<size_t>(plan.ops[static_cast<size_t>(op.tail)].out)].c;
     return os.str();
 }
@@ -1096,7 +1172,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
                     if (before.back().first != MSNH_CONV_IGEMM || ops[static_cast<size_t>(op.tail)].algo == MSNH_CONV_WINOGRAD || !msnh_hip_conv2d_tail_supported(&c, &t, op.tile)) ok = false;
                     continue;
                 }
-                if (!msnh_hip_conv2d_tile_supported(&d, op.tile)) ok = false;
+                if (!tileSupported(*this, op, d, op.tile)) ok = false;
                 if (op.kind == PlanOp::CONV && op.wDev.bytes() != msnh_hip_conv2d_packed_weight_elems(&d, op.algo) * (d.dtype == MSNH_F16 ? 2u : 4u)) ok = false;
                 size_t &most = op.algo == MSNH_CONV_IGEMM_FUSEDK ? needSliced : need;
                 most = std::max(most, msnh_hip_conv2d_workspace_bytes(&d, op.algo));
@@ -1150,7 +1226,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
     msnh_event_t e0 = nullptr, e1 = nullptr;
     MSNH_DEV(msnh_hip_event_create(&e0));
     MSNH_DEV(msnh_hip_event_create(&e1));
-    struct Key { int kind, b, h, w, c, inLd, oc, outLd, k, st, pad, dil, g, res, odt, algo, up; bool operator==(const Key &o) const { return std::memcmp(this, &o, sizeof(Key)) == 0; } };
+    struct Key { int kind, b, h, w, c, inLd, oc, outLd, k, st, pad, dil, g, res, odt, algo, up, pairC, pairLd; bool operator==(const Key &o) const { return std::memcmp(this, &o, sizeof(Key)) == 0; } };
     std::vector<std::pair<Key, int>> memo;         // identical shapes share one search
     for (PlanOp &op : ops)
     {
@@ -1163,6 +1239,12 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
         key.b = in.n; key.h = in.h; key.w = in.w; key.c = in.c; key.inLd = ld(op.in0); key.oc = out.c; key.outLd = ld(op.out);
         key.k = op.ksize; key.st = op.stride; key.pad = op.pad; key.dil = op.dilation; key.g = op.groups;
         key.res = op.in1 >= 0; key.odt = out.dtype; key.algo = op.algo; key.up = op.up2 ? 1 : 0;
+        if (op.pair >= 0)
+        {
+            const int mate = ops[static_cast<size_t>(op.pair)].out;
+            key.pairC = tensors[static_cast<size_t>(mate)].c;
+            key.pairLd = ld(mate);
+        }
         bool found = false;
         for (const auto &m : memo)
         {
@@ -1171,7 +1253,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
             const int wasAlgo = op.algo, wasTile = op.tile;
             op.algo = m.second >> 16; op.tile = m.second & 0xffff;
             const msnh_conv_desc d = convDesc(*this, op);
-            if (msnh_hip_conv2d_tile_supported(&d, op.tile) &&
+            if (tileSupported(*this, op, d, op.tile) &&
                 msnh_hip_conv2d_workspace_bytes(&d, op.algo) <= (op.algo == MSNH_CONV_IGEMM_FUSEDK ? _sliceWorkspace : _convWorkspace).bytes())
                 found = true;
             else { op.algo = wasAlgo; op.tile = wasTile; }
@@ -1201,7 +1283,7 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
                 op.tile = tile;
                 {
                     const msnh_conv_desc probe = convDesc(*this, op);
-                    if (!msnh_hip_conv2d_tile_supported(&probe, tile)) continue;
+                    if (!tileSupported(*this, op, probe, tile)) continue;
                 }
                 cands.push_back({timeOne(algo, tile, 1, 3), algo, tile});
             }
@@ -1225,14 +1307,14 @@ void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
                 {
                     op.tile = tile + 256 * slices;
                     const msnh_conv_desc probe = convDesc(*this, op);
-                    if (!msnh_hip_conv2d_tile_supported(&probe, op.tile)) continue;
+                    if (!tileSupported(*this, op, probe, op.tile)) continue;
                     const size_t need = msnh_hip_conv2d_workspace_bytes(&probe, MSNH_CONV_IGEMM_FUSEDK);
                     if (need == 0 || need > (static_cast<size_t>(64) << 20)) continue;
                     reserveSliceWorkspace(need, s);
                     cands.push_back({timeOne(MSNH_CONV_IGEMM_FUSEDK, tile + 256 * slices, 1, 3), MSNH_CONV_IGEMM_FUSEDK, tile + 256 * slices});
                 }
         }
-        if (baseAlgo == MSNH_CONV_IGEMM && op.kind == PlanOp::CONV) search(MSNH_CONV_POINTWISE);      // (refused by the library unless the shape fits)
+        if (baseAlgo == MSNH_CONV_IGEMM && op.kind == PlanOp::CONV && op.pair < 0) search(MSNH_CONV_POINTWISE);      // (refused by the library unless the shape fits)
         int best = 0, bestAlgo = baseAlgo;
         if (!cands.empty())
         {
@@ -1402,6 +1484,13 @@ void Plan::launch(PlanOp &op, msnh_stream_t s)
         if (op.wDev.bytes() != msnh_hip_conv2d_packed_weight_elems(&d, op.algo) * (d.dtype == MSNH_F16 ? 2u : 4u))
             MSNH_THROW("conv weights on the device are not packed for the algorithm of this launch (" + op.name + ")");
         const DeviceBuffer &ws = op.algo == MSNH_CONV_IGEMM_FUSEDK ? _sliceWorkspace : _convWorkspace;
+        if (op.pair >= 0)
+        {
+            const msnh_conv_pair_desc p = pairDesc(*this, op);
+            MSNH_DEV(msnh_hip_conv2d_pair(&d, &p, ptr(op.in0), op.wDev.ptr(), op.scaleDev.as<float>(), op.shiftDev.as<float>(), ptr(op.out),
+                                          ptr(ops[static_cast<size_t>(op.pair)].out), ws.ptr(), ws.bytes(), s));
+            break;
+        }
         MSNH_DEV(msnh_hip_conv2d(&d, ptr(op.in0), op.wDev.ptr(), op.scaleDev.as<float>(), op.shiftDev.as<float>(),
                                  op.in1 >= 0 ? ptr(op.in1) : nullptr, ptr(op.out), ws.ptr(), ws.bytes(), s));
         break;
@@ -1610,7 +1699,7 @@ std::string Plan::describe() const
         const PlanTensor &out = tensors[static_cast<size_t>(op.out)];
         os << "  L" << op.layerIndex << " " << kinds[op.kind];
         if (op.kind == PlanOp::CONV)
-            os << "[" << algos[op.algo] << (op.stemTail >= 0 ? "+1x1" : "") << (op.tile ? " t" + std::to_string(op.tile) : std::string()) << " k" << op.ksize << " s" << op.stride << " g" << op.groups << (op.in1 >= 0 ? " +res" : "") << (op.src2 ? " +bn" : "") << (op.up2 ? " +up2" : "") << "]";
+            os << "[" << algos[op.algo] << (op.stemTail >= 0 ? "+1x1" : "") << (op.tile ? " t" + std::to_string(op.tile) : std::string()) << " k" << op.ksize << " s" << op.stride << " g" << op.groups << (op.in1 >= 0 ? " +res" : "") << (op.src2 ? " +bn" : "") << (op.up2 ? " +up2" : "") << (op.pair >= 0 ? " +pair" : "") << "]";
         if (op.kind == PlanOp::MAXPOOL || op.kind == PlanOp::AVGPOOL)
             os << "[k" << op.ksize << " s" << op.stride << " p" << op.pad << (op.chainHead >= 0 ? " in the launch of the pool before it" : "") << "]";
         os << " " << in.n << "x" << in.h << "x" << in.w << "x" << in.c << " -> " << out.h << "x" << out.w << "x" << out.c

@@ -113,6 +113,38 @@ def conv2d_tail(x, w_oihw, w2_oi, *, stride=1, pad=0, scale=None, shift=None, ac
     return (nchw_host(ydev, oc) if write_y else None), nchw_host(zdev, oc2)
 
 
+def conv2d_pair(x, w1, w2, *, dtype, out_dtype=None, scale=None, shift=None, acts=("none", "none"), muls=(1.0, 1.0), tile=0, slices=0, out_ld=None, out_ld2=None):
+    """msnh_hip_conv2d_pair: x NCHW float32 numpy, w1 / w2 [out_c][in_c] filters of the two 1x1 convolutions, scale / shift over both.  Returns (y, y2) as NCHW
+    float32 numpy, or None where the library does not take the tile."""
+    init()
+    L = abi.lib()
+    out_dtype = dtype if out_dtype is None else out_dtype
+    b, c, h, wd = x.shape
+    oc1, oc2 = w1.shape[0], w2.shape[0]
+    oc = oc1 + oc2
+    algo = "igemm_fusedk" if slices else "igemm"
+    d = abi.ConvDesc(dtype, out_dtype, b, h, wd, c, c, oc, h, wd, oc, 1, 1, 0, 1, 1, abi.ACT[acts[0]], 0.1, 0, oc, abi.ACT["none"], 0.1, 1.0, muls[0], abi.ALGO[algo],
+                     tile + 256 * slices)
+    p = abi.ConvPairDesc(oc1, out_ld or oc1, out_ld2 or oc2, abi.ACT[acts[1]], 0.2, muls[1])
+    if not L.msnh_hip_conv2d_pair_supported(ctypes.byref(d), ctypes.byref(p), d.tile):
+        return None
+    wf = np.ascontiguousarray(np.concatenate([w1, w2]).reshape(oc, c, 1, 1), np.float32)
+    packed = np.zeros(L.msnh_hip_conv2d_packed_weight_elems(ctypes.byref(d), abi.ALGO["igemm"]), np.float16 if dtype == abi.F16 else np.float32)
+    abi.check(L.msnh_hip_conv2d_pack_weights(ctypes.byref(d), abi.ALGO["igemm"], wf.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), packed.ctypes.data_as(ctypes.c_void_p)))
+    wdev, xdev = dev(packed), nhwc_dev(x, dtype)
+    mk = lambda v: dev(np.asarray(v, np.float32)) if v is not None else None
+    sdev, hdev = mk(scale), mk(shift)
+    ydev = torch.full((b, h, wd, p.out_ld), 3.0, dtype=TORCH_DT[out_dtype]).cuda()
+    zdev = torch.full((b, h, wd, p.out_ld2), 5.0, dtype=TORCH_DT[out_dtype]).cuda()
+    n = L.msnh_hip_conv2d_workspace_bytes(ctypes.byref(d), abi.ALGO[algo])
+    ws = torch.zeros(max(n, 16), dtype=torch.uint8).cuda()
+    sync()
+    abi.check(L.msnh_hip_conv2d_pair(ctypes.byref(d), ctypes.byref(p), ptr(xdev), ptr(wdev), ptr(sdev), ptr(hdev), ptr(ydev), ptr(zdev), ptr(ws), n, None))
+    sync()
+    assert (ydev[..., oc1:].float().cpu().numpy() == 3.0).all() and (zdev[..., oc2:].float().cpu().numpy() == 5.0).all(), "wrote outside a channel slice"
+    return nchw_host(ydev, oc1), nchw_host(zdev, oc2)
+
+
 def conv2d(x, w_oihw, *, dtype, out_dtype=None, stride=1, pad=0, dil=1, groups=1, scale=None, shift=None, act="none",
            act_param=0.1, residual=None, act2="none", act2_param=0.1, res_mul=1.0, out_mul=1.0, algo="auto",
            in_ld=None, out_ld=None, res_ld=None, tile=0, upsample=1, xcd_blocks=0):

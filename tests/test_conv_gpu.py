@@ -388,6 +388,57 @@ def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
     assert ran >= 15
 
 
+@pytest.mark.parametrize("dtype,out_dtype", [(abi.F32, abi.F32), (abi.F16, abi.F16), (abi.F16, abi.F32)])
+@pytest.mark.parametrize("c,oc1,oc2,pad1,pad2", [(64, 32, 32, 8, 0), (72, 64, 64, 0, 24), (40, 96, 40, 3, 5), (256, 128, 8, 0, 0), (1040, 160, 160, 0, 8)])
+def test_conv_pair(c, oc1, oc2, pad1, pad2, dtype, out_dtype):
+    """Two 1x1 convolutions of one tensor in one launch, on every tile that takes the pair and with the K loop sliced: each result with its own activation,
+    factor and pixel stride against the float32 reference of its convolution; a last pixel tile of 13 x 11 pixels, second tensors that end inside a wave
+    tile, rows that are no multiple of eight channels."""
+    import gpuutil as gu
+    b, h, w = 3, 13, 11
+    rng = np.random.default_rng(c + oc1 + oc2)
+    x, wt = _case(rng, b, c, h, w, oc1 + oc2, 1)
+    scale = rng.uniform(0.5, 1.5, oc1 + oc2).astype(np.float32)
+    shift = (rng.standard_normal(oc1 + oc2) * 0.1).astype(np.float32)
+    if dtype == abi.F16:
+        x, wt = gu.round_f16(x), gu.round_f16(wt)
+    ref1 = _ref(x, wt[:oc1], 1, 0, 1, 1, scale[:oc1], shift[:oc1], "leaky", 0.1, None, "none", 1.0, 2.0)
+    ref2 = _ref(x, wt[oc1:], 1, 0, 1, 1, scale[oc1:], shift[oc1:], "hardswish", 0.2, None, "none", 1.0, 0.5)
+    ran = 0
+    for tile in range(0, abi.lib().msnh_hip_conv2d_tile_count() + 1):
+        for slices in (0, 2):
+            if slices and tile == 0:
+                continue
+            got = gu.conv2d_pair(x, wt[:oc1, :, 0, 0], wt[oc1:, :, 0, 0], dtype=dtype, out_dtype=out_dtype, scale=scale, shift=shift, acts=("leaky", "hardswish"), muls=(2.0, 0.5),
+                                 tile=tile, slices=slices, out_ld=oc1 + pad1, out_ld2=oc2 + pad2)
+            if got is None:
+                assert tile != 0
+                continue
+            ran += 1
+            assert gu.rel_err(got[0], ref1) <= TOL[dtype] and gu.rel_err(got[1], ref2) <= TOL[dtype], (tile, slices, gu.rel_err(got[0], ref1), gu.rel_err(got[1], ref2))
+    assert ran >= 10
+
+
+def test_conv_pair_rejects():
+    """a border that cuts a wave tile, a first tensor of no whole 32 channels, a residual, a filter of more than one tap, strides below the channels"""
+    L = abi.lib()
+    d = abi.ConvDesc(abi.F16, abi.F16, 1, 8, 8, 64, 64, 96, 8, 8, 96, 1, 1, 0, 1, 1, 22, 0.1, 0, 96, 22, 0.1, 1.0, 1.0, abi.ALGO["igemm"], 0)
+    p = abi.ConvPairDesc(32, 32, 64, 22, 0.1, 1.0)
+    ok = lambda tile=0: L.msnh_hip_conv2d_pair_supported(ctypes.byref(d), ctypes.byref(p), tile)
+    assert ok() == 1 and ok(1) == 0 and ok(6) == 1 and ok(-1) == 0
+    for field, value in (("first_c", 40), ("first_c", 96), ("first_c", 0), ("out_ld", 24), ("out_ld2", 56), ("act", 99)):
+        keep = getattr(p, field)
+        setattr(p, field, value)
+        assert ok() == 0, field
+        setattr(p, field, keep)
+    for field, value in (("has_residual", 1), ("groups", 2), ("algo", abi.ALGO["pointwise"]), ("out_c", 92), ("in_ld", 68)):
+        keep = getattr(d, field)
+        setattr(d, field, value)
+        assert ok() == 0, field
+        setattr(d, field, keep)
+    assert ok() == 1
+
+
 @pytest.mark.parametrize("tile", [1, 5, 9, 23, 32, 36, 38, 41, 58, 61, 69, 71])
 @pytest.mark.parametrize("c,oc,k", [(256, 96, 3), (40, 72, 1), (64, 130, 3)])
 def test_conv_f32_split_products(c, oc, k, tile):

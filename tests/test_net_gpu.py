@@ -669,6 +669,35 @@ def test_conv_writes_the_upsampled_tensor(fp16):
         assert len(b) > 0 and abs(len(a) - len(b)) <= (max(2, len(b) // 100) if fp16 else 0)
 
 
+@pytest.mark.parametrize("arch,batch,size,fp16", [("yolov5s", 2, 96, True), ("yolov5s", 3, 160, False), ("yolov4", 1, 160, True), ("yolov4", 2, 96, False)])
+def test_sibling_convolutions_are_paired(arch, batch, size, fp16):
+    """The two 1x1 convolutions that open a cross-stage block run as one launch (Plan::pairConvs): the head logits equal those of the plan that keeps two
+    (MSNH_NO_CONV_PAIR) -- to 1e-5 in float32, to 5e-3 in float16 (two separately tuned plans may sum in different orders) -- and the oracle's."""
+    net, binp, g = nu.model(arch, batch, size, seed=7)
+    x = zoo.seeded_input(batch, 3, size, size, seed=8)
+    ref, _ = _oracle_layers(arch, size, binp, x)
+    m = netapi.Net(net, binp, fp16=fp16)
+    assert m.plan_detail().count("+pair") == {"yolov5s": 8, "yolov4": 5}[arch], m.plan_detail()
+    m.run_yolo(x)
+    os.environ["MSNH_NO_CONV_PAIR"] = "1"
+    try:
+        m0 = netapi.Net(net, binp, fp16=fp16)
+    finally:
+        del os.environ["MSNH_NO_CONV_PAIR"]
+    assert "+pair" not in m0.plan_detail()
+    m0.run_yolo(x)
+    yolo = [i for i in range(m.num_layers()) if m.layer_info(i)["type"] == "yolo"]
+    for h, i in enumerate(yolo):
+        got = m.yolo_head_logits(h).reshape(batch, -1)
+        e = nu.rel_err(got, m0.yolo_head_logits(h).reshape(batch, -1))
+        print(arch, "head", h, "fp16" if fp16 else "fp32", e, flush=True)
+        assert e <= (5e-3 if fp16 else 1e-5), h
+        for b in range(batch):
+            assert nu.rel_err(got[b], ref[b][i - 1]) <= (2e-2 if fp16 else 1e-4), (h, b)
+    h1, h0 = m.fp16_headroom(x), m0.fp16_headroom(x)
+    assert h1 == h0 if not fp16 else abs(h1 - h0) <= 1e-2 * h0
+
+
 @pytest.mark.parametrize("size,batch,fp16", [(32, 1, True), (96, 3, True), (160, 2, True), (96, 2, False)])
 def test_focus_and_concatenated_norms_are_fused(size, batch, fp16):
     """YOLOv5s: the focus opening (four slices, concatenation, 3x3 convolution) is one first-layer launch, and the batch norms behind
