@@ -59,13 +59,21 @@ struct MbArgs
 // multiplied into the stage's scale and shift at pack time -- exactly, it is a power of two -- and costs no instruction per element.
 __host__ __device__ inline bool mbFolds(int act) { return act == MSNH_ACT_NONE || act == MSNH_ACT_RELU || act == MSNH_ACT_LEAKY || act == MSNH_ACT_RELU6; }
 
-template <int N> __device__ __forceinline__ void mbActivate(float (&v)[N], int act, float param, float cap, float mul)
+// SIMPLE: one of the activations that fold.
+template <bool SIMPLE, int N> __device__ __forceinline__ void mbActivate(float (&v)[N], int act, float param, float cap, float mul)
 {
     if (act == MSNH_ACT_RELU6)
     {
         // one median instruction per element; a NaN gives 0 as in activate()
 #pragma unroll
         for (int e = 0; e < N; ++e) v[e] = __builtin_amdgcn_fmed3f(v[e], 0.f, cap);
+        return;
+    }
+    if constexpr (SIMPLE)
+    {
+        const float slope = act == MSNH_ACT_NONE ? 1.f : act == MSNH_ACT_RELU ? 0.f : param;
+#pragma unroll
+        for (int e = 0; e < N; ++e) v[e] = v[e] > 0.f ? v[e] : slope * v[e];
         return;
     }
     activateArray<N>(v, act, param);
@@ -84,11 +92,23 @@ __host__ __device__ inline unsigned mbWdOff(int ks, int mb) { return static_cast
 __host__ __device__ inline unsigned mbAffOff(int ks, int mb) { return mbWdOff(ks, mb) + 9u * MB_CH * 2u; }
 __host__ __device__ inline unsigned mbChunkBytes(int ks, int mb) { return static_cast<unsigned>(2 * ks + 4 * mb + 3) * 1024u; }
 
-template <int S>
-__global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
+// LDS: the input tile (whole 1 KiB deliveries), the widened chunk, the depthwise output, two chunk records.  The operand columns that round the pixel
+// counts up to whole column blocks have no rows of their own: their reads run into the region behind, their results are never stored.
+// (A row for each of them, and the registers of the transcendental activations, kept the 56 x 56 blocks of MobileNetV2 at one or two workgroups per CU:
+// 64 images, 24 -> 144 -> 24 at 56 x 56 64.3 -> 48.6 us, 24 -> 144 -> 32 to 28 x 28 33.9 -> 22.2, 32 -> 192 -> 32 at 28 x 28 19.5 -> 17.2, the whole
+// network 556 -> 514.  Not two pixels per thread in the depthwise step, which halves its LDS reads: 14 x 14 13.7 -> 17.4, where a workgroup has a CU.)
+__host__ __device__ constexpr int mbInputPixels(int stride) { return ((MB_TO - 1) * stride + 3) * ((MB_TO - 1) * stride + 3); }
+__host__ __device__ inline unsigned mbEOff(int stride, int ks) { return (static_cast<unsigned>(mbInputPixels(stride)) * (static_cast<unsigned>(ks) * 32u + 16u) + 1023u) & ~1023u; }
+__host__ __device__ inline unsigned mbYOff(int stride, int ks) { return mbEOff(stride, ks) + static_cast<unsigned>(mbInputPixels(stride)) * MB_ROW; }
+__host__ __device__ inline unsigned mbBOff(int stride, int ks) { return (mbYOff(stride, ks) + static_cast<unsigned>(MB_TO * MB_TO) * MB_ROW + 1023u) & ~1023u; }
+
+// SIMPLE: both widened tensors' activations fold (mbFolds).  Without the transcendental ones the kernel is 17 KB instead of 27 and 78 registers instead of
+// 84: six wavefronts per SIMD, three workgroups per CU where LDS has the room.  (A register bound of 80 by launch bounds spills; one of 128 does not.)
+template <int S, bool SIMPLE>
+__global__ __launch_bounds__(64 * MB_NW, 4) void mbconvKernel(MbArgs a)
 {
     constexpr int IT = (MB_TO - 1) * S + 3;           // input tile edge: 9 or 15
-    constexpr int IP = IT * IT;
+    constexpr int IP = mbInputPixels(S);
     constexpr int NE = (IP + 31) / 32;                // 32-pixel column blocks of the expand GEMM
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const unsigned ldsBase = static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char *)smem));
@@ -110,9 +130,7 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
 
     const unsigned xStr = static_cast<unsigned>(a.ks) * 32u + 16u;      // bytes of an input pixel's row in LDS
     const unsigned xOff = 0;
-    const unsigned eOff = (xOff + NE * 32u * xStr + 1023u) & ~1023u;    // (the input tile's region ends on a 1 KiB boundary: it is filled in 1 KiB deliveries)
-    const unsigned yOff = eOff + NE * 32u * MB_ROW;
-    const unsigned bOff = (yOff + 64u * MB_ROW + 1023u) & ~1023u;
+    const unsigned eOff = mbEOff(S, a.ks), yOff = mbYOff(S, a.ks), bOff = mbBOff(S, a.ks);
 
     const i32x4 rxw = makeRsrcWords(a.x, a.xBytes);
     const i32x4 rb = makeRsrcWords(a.blob, a.blobBytes);
@@ -141,9 +159,9 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
             const unsigned voff = ok ? (static_cast<unsigned>((img * a.H + gy) * a.W + gx) * a.inLd + v * 8) * 2u : kOobOffset;
             dmaLoad16(rxw, voff, 0u, ldsBase + xOff + static_cast<unsigned>(p) * 1024u);
         }
-        // the depthwise output starts as zeros: its pixel rows 49..63 are operand columns whose results nobody stores, and the channel
-        // vectors past exp_c of a last, partial chunk are never written (their filter values are zeros, but 0 * garbage may be a NaN)
-        for (int idx = tid; idx < 64 * MB_ROW / 16; idx += 64 * MB_NW)
+        // the depthwise output starts as zeros: the channel vectors past exp_c of a last, partial chunk are never written (their filter values
+        // are zeros, but 0 * garbage may be a NaN)
+        for (int idx = tid; idx < MB_TO * MB_TO * MB_ROW / 16; idx += 64 * MB_NW)
             *reinterpret_cast<f32x4 *>(smem + yOff + idx * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
@@ -197,7 +215,7 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[4 * q + e] = acc[4 * q + e] * sc[e] + sh[e];
             }
-            mbActivate<16>(v, a.act1, a.act1Param, a.cap1, a.mul1);
+            mbActivate<SIMPLE, 16>(v, a.act1, a.act1Param, a.cap1, a.mul1);
             // (a pixel outside the image is exactly zero, also where the activation of the shift is not: masked as bits)
             const unsigned keep = ((inImage >> j) & 1u) ? 0xffffffffu : 0u;
             f16x8 o0, o1;
@@ -213,8 +231,11 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
             o0 = __builtin_bit_cast(f16x8, b0);
             o1 = __builtin_bit_cast(f16x8, b1);
             unsigned char *ep = smem + eOff + (32 * j + n) * MB_ROW + c0 * 2;
-            *reinterpret_cast<f16x8 *>(ep) = o0;
-            *reinterpret_cast<f16x8 *>(ep + 16) = o1;
+            if (32 * j + n < IP)
+            {
+                *reinterpret_cast<f16x8 *>(ep) = o0;
+                *reinterpret_cast<f16x8 *>(ep + 16) = o1;
+            }
         }
     };
     expandChunk(cBegin);
@@ -256,7 +277,7 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
                     sum[e]     = sum[e] * s0[e] + h0[e];
                     sum[4 + e] = sum[4 + e] * s1[e] + h1[e];
                 }
-                mbActivate<8>(sum, a.act2, a.act2Param, a.cap2, a.mul2);
+                mbActivate<SIMPLE, 8>(sum, a.act2, a.act2Param, a.cap2, a.mul2);
                 f16x8 o;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[e] = static_cast<f16>(sum[e]);
@@ -325,11 +346,7 @@ __global__ __launch_bounds__(64 * MB_NW) void mbconvKernel(MbArgs a)
 size_t mbLdsBytes(const msnh_mbconv_desc *d)
 {
     const int ks = (d->in_c + 15) / 16, mb = (d->out_c + 31) / 32;
-    const int it = (MB_TO - 1) * d->stride + 3;
-    const size_t ne = static_cast<size_t>((it * it + 31) / 32);
-    const size_t xRegion = (ne * 32 * (static_cast<size_t>(ks) * 32 + 16) + 1023) & ~static_cast<size_t>(1023);
-    const size_t acts = xRegion + ne * 32 * MB_ROW + 64 * MB_ROW;
-    return ((acts + 1023) & ~static_cast<size_t>(1023)) + 2 * static_cast<size_t>(mbChunkBytes(ks, mb));
+    return mbBOff(d->stride, ks) + 2 * static_cast<size_t>(mbChunkBytes(ks, mb));
 }
 
 } // namespace
@@ -473,18 +490,10 @@ int msnh_hip_mbconv_sliced(const msnh_mbconv_desc *d, const void *x, const void 
     const size_t lds = mbLdsBytes(d);
     const unsigned blocks = static_cast<unsigned>((total + 7) / 8 * 8);
     hipStream_t st = resolveStream(s);
-    if (d->stride == 1)
-    {
-        static bool raised = false;
-        if (!raised) { MSNH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mbconvKernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); raised = true; }
-        hipLaunchKernelGGL((mbconvKernel<1>), dim3(blocks, static_cast<unsigned>(a.slices)), dim3(64 * MB_NW), lds, st, a);
-    }
-    else
-    {
-        static bool raised = false;
-        if (!raised) { MSNH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(mbconvKernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); raised = true; }
-        hipLaunchKernelGGL((mbconvKernel<2>), dim3(blocks, static_cast<unsigned>(a.slices)), dim3(64 * MB_NW), lds, st, a);
-    }
+    const bool simple = mbFolds(d->act1) && mbFolds(d->act2);
+    const auto kern = d->stride == 1 ? (simple ? mbconvKernel<1, true> : mbconvKernel<1, false>) : (simple ? mbconvKernel<2, true> : mbconvKernel<2, false>);
+    if (lds > 48 * 1024) MSNH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    hipLaunchKernelGGL(kern, dim3(blocks, static_cast<unsigned>(a.slices)), dim3(64 * MB_NW), lds, st, a);
     MSNH_LAUNCH_CHECK();
     return 0;
 }

@@ -155,6 +155,31 @@ def test_mbconv_activations_and_limits():
         assert L.msnh_hip_mbconv(ctypes.byref(d), None, None, None, None, None, None, None) != 0
 
 
+@pytest.mark.parametrize("stride", [1, 2])
+@pytest.mark.parametrize("acts", [("none", "leaky"), ("relu", "relu6"), ("leaky", "relu"), ("relu6", "none"), ("relu6", "swish"), ("mish", "relu6")])
+def test_mbconv_activation_kinds(acts, stride):
+    """the kernel for activations that fold (none, relu, leaky, relu6 in front of and behind the depthwise layer) and the one for the others, on both
+    strides, cut tiles and a partial last chunk; an image that holds an infinity and a NaN leaves the other images' results, bit for bit, what they are"""
+    import gpuutil as gu
+    rng = np.random.default_rng(17 + stride)
+    b, cin, h, w, cexp, cout = 3, 24, 17, 20, 144, 40
+    x = gu.round_f16(rng.standard_normal((b, cin, h, w), dtype=np.float32))
+    we = gu.round_f16(rng.standard_normal((cexp, cin), dtype=np.float32) * 0.3)
+    wd = gu.round_f16(rng.standard_normal((cexp, 9), dtype=np.float32) * 0.4)
+    wp = gu.round_f16(rng.standard_normal((cout, cexp), dtype=np.float32) * 0.1)
+    one, zero = np.ones(cexp, np.float32), np.zeros(cexp, np.float32)
+    s3, h3 = np.ones(cout, np.float32), (rng.standard_normal(cout) * 0.1).astype(np.float32)
+    args = (we, wd, wp, one, zero + 0.3, one * 2, zero - 0.1, s3, h3, stride, acts + ("none", "none"), 0.5, 0.5, 1.0, None, 1.0)
+    y = run_mbconv(x, *args)
+    e = gu.rel_err(y, _reference(x, *args))
+    print("mbconv", acts, stride, e, flush=True)
+    assert e <= 1e-3
+    bad = x.copy()
+    bad[1, 3, 8, 9], bad[1, 5, 0, 0] = np.inf, np.nan
+    z = run_mbconv(bad, *args)
+    assert np.array_equal(z[0], y[0]) and np.array_equal(z[2], y[2]) and not np.array_equal(z[1], y[1])
+
+
 @pytest.mark.parametrize("case,slices", [((1, 96, 14, 14, 576, 96, 1, True), 9), ((2, 64, 14, 14, 384, 64, 1, True), 4), ((1, 24, 21, 28, 144, 32, 2, False), 3),
                                          ((1, 8, 10, 13, 136, 8, 1, True), 2), ((3, 16, 7, 7, 64, 24, 1, False), 1)])
 def test_mbconv_sliced(case, slices):
