@@ -516,7 +516,8 @@ void Plan::pairConvs()
             op.tail >= 0 || op.tailOf >= 0 || op.pair >= 0 || op.up2)
             return false;
         const PlanTensor &x = tensors[static_cast<size_t>(op.in0)], &y = tensors[static_cast<size_t>(op.out)];
-        return x.layout == PlanTensor::NHWC && y.layout == PlanTensor::NHWC && x.c % 8 == 0 && y.c % 8 == 0 && (x.dtype == MSNH_F16 || y.dtype == MSNH_F32);
+        // (a pinned output belongs to a layer that runs, and is timed, by itself)
+        return !y.pinned && x.layout == PlanTensor::NHWC && y.layout == PlanTensor::NHWC && x.c % 8 == 0 && y.c % 8 == 0 && (x.dtype == MSNH_F16 || y.dtype == MSNH_F32);
     };
     for (size_t i = 0; i < ops.size(); ++i)
         for (size_t k = i + 1; k < ops.size() && eligible(ops[i]) && tensors[static_cast<size_t>(ops[i].out)].c % 32 == 0; ++k)

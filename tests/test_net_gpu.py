@@ -684,7 +684,7 @@ def test_sibling_convolutions_are_paired(arch, batch, size, fp16):
         m0 = netapi.Net(net, binp, fp16=fp16)
     finally:
         del os.environ["MSNH_NO_CONV_PAIR"]
-    assert "+pair" not in m0.plan_detail()
+    assert "+pair" not in m0.plan_detail() and "+pair" not in netapi.Net(net, binp, fp16=fp16, dump_layers=True).plan_detail()
     m0.run_yolo(x)
     yolo = [i for i in range(m.num_layers()) if m.layer_info(i)["type"] == "yolo"]
     for h, i in enumerate(yolo):
