@@ -159,21 +159,29 @@ __device__ __forceinline__ void mfmaBlock(const f32x4 &a, const f32x4 &b, f32x16
 // accumulator of their own: added to the large one they would be rounded at its magnitude five times per 16 k, apart from it they are not, and the
 // large one is rounded once per 16 k instead of eight times.  Against 64-bit sums, normal and rectified operands, K = 576 / 4608: 1.3e-7 / 4.2e-7 of
 // the results' rms, where the float32 MFMAs give 4.4e-7 / 1.2e-6 (one accumulator for all six: 3.7e-7 / 1.1e-6).
-// bfloat16 has float32's exponents, so nothing overflows that did not before, apart from values within a half of 2^-8 of the largest float32; an infinity
-// times a piece that is zero is NaN, however, where the float32 product is an infinity.  Every result that such an operand reaches is not finite
-// either way, so a workgroup that finds a result that is not finite multiplies its tile again with the float32 MFMAs.
+// A piece keeps its bits down to 2^-133 and the pieces of a float32 value reach down to 2^-149, so both operands are multiplied by 2^16 before they are split
+// and the sums by 2^-32 behind the loop: every float32 value, subnormal ones too, is then exactly the sum of its pieces (the matrix cores and the
+// conversions keep subnormal numbers).  Without it operands below 2^-110 lose their low pieces: 2^-118 times 2^60, K = 576, errs by 8.7e-6 of the
+// results' rms.  (It costs eight of 52 instructions: yolov3 f32 b1 1845 -> 1901 us, resnet50 f32 b5 794 -> 806.  Looking for such operands instead, to multiply
+// their tiles as float32, costs four, but swish and mish turn every strongly negative value into one.)
+// What the factors push out of range -- operands from 2^111, sums from 2^95 -- becomes an infinity or NaN, as do infinities themselves (an infinity
+// times a piece that is zero is NaN, where the float32 product is an infinity); every result that such an operand reaches is then not finite, so a workgroup
+// that finds a result that is not finite multiplies its tile again with the float32 MFMAs.
+// (The pieces and the choice of six products: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", ARITH 2019.)
+constexpr float kSplitScale = 65536.f, kSplitUnscale = 1.f / (65536.f * 65536.f);
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-// 8 values in 44 vector instructions: a conversion rounds two values, a shift and a mask widen them again.
+// 8 values in 52 vector instructions: a conversion rounds two values, a shift and a mask widen them again.
 __device__ __forceinline__ void splitF32(const f32x4 &a, const f32x4 &b, bf16x8 &hi, bf16x8 &mid, bf16x8 &lo)
 {
     u32x4 h, m, l;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
     {
-        const float v0 = e < 2 ? a[2 * e] : b[2 * e - 4], v1 = e < 2 ? a[2 * e + 1] : b[2 * e - 3];
+        const float v0 = kSplitScale * (e < 2 ? a[2 * e] : b[2 * e - 4]), v1 = kSplitScale * (e < 2 ? a[2 * e + 1] : b[2 * e - 3]);
         h[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
         const float r0 = v0 - __builtin_bit_cast(float, h[e] << 16), r1 = v1 - __builtin_bit_cast(float, h[e] & 0xffff0000u);
         m[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
@@ -789,7 +797,7 @@ constexpr int igemmWavesPerSimd(int bm, int bn, int kv = 8, int ns = 3, int nw =
 
 // float32 tiles whose wavefronts have the registers for the split product (splitF32): per 32 x 32 block two accumulators, per block row and column the
 // three pieces and the values they come from.  The others multiply with the float32 MFMAs, and so do those with one block per wavefront: there the split
-// of two operands (88 vector instructions) costs what the matrix cores save, 3x3 64 -> 64 at 56 x 56 8.66 -> 9.21 us, 256 -> 256 at 14 x 14 11.2 -> 11.9.
+// of two operands (88 vector instructions, 104 with the factors) costs what the matrix cores save, 3x3 64 -> 64 at 56 x 56 8.66 -> 9.21 us, 256 -> 256 at 14 x 14 11.2 -> 11.9.
 // The others, start -> now: 3x3 256 -> 512 at 38 x 38 eight images 214 -> 172 us, one image 38.2 -> 32.2; 128 -> 256 at 76 x 76 eight images 223 -> 173;
 // 1x1 512 -> 256 at 38 x 38 eight images 32.3 -> 28.0.  What binds then is the bfloat16 rate under load: 159 x 6 = 954 TFLOP/s where a large matrix product gets 1120.
 constexpr int igemmSplitRegs(int mb, int nb) { return 32 * mb * nb + 20 * (mb + nb) + 40; }
@@ -1468,7 +1476,7 @@ void convIgemmKernel(IgemmArgs a)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
             {
-                acc[i][j][r] += low[i][j][r];
+                acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * kSplitUnscale;
                 probe = __builtin_fmaf(acc[i][j][r], 0.f, probe);
             }
         });

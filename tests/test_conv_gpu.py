@@ -455,6 +455,24 @@ def test_conv_f32_split_products(c, oc, k, tile):
     assert err <= 2.0 ** -24 * (1.5 * np.sqrt(c * k * k / 16 / 6) + 1), err
 
 
+@pytest.mark.parametrize("tile", [1, 5, 9, 28, 36, 38, 58, 61, 69, 71])
+@pytest.mark.parametrize("ex,ew,redone", [(-118, 60, False), (60, -118, False), (-118, 0, False), (-142, 100, False), (-60, -40, False), (-118, 118, True), (120, -120, True)])
+def test_conv_f32_split_products_small_and_large(ex, ew, redone, tile):
+    """Operands of 2^ex and 2^ew, among them subnormal ones and those whose low bfloat16 pieces lie below what bfloat16 can hold: the error against 64-bit
+    sums is the one of operands of order one (test_conv_f32_split_products).  redone: an operand from 2^111 on is multiplied as float32, one rounding per
+    2 products -- the same bound with K / 2 roundings."""
+    import torch
+    import gpuutil as gu
+    c, oc, k = 64, 96, 3
+    rng = np.random.default_rng(ex * 1000 + ew + tile + 10 ** 6)
+    x, wt = _case(rng, 1, c, 13, 11, oc, k)
+    x, wt = np.ldexp(x, ex), np.ldexp(wt, ew)
+    y, _ = gu.conv2d(x, wt, dtype=abi.F32, stride=1, pad=k // 2, algo="igemm", tile=tile)
+    ref = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(wt).double(), padding=k // 2).numpy()
+    err = np.linalg.norm(np.ldexp(y.astype(np.float64) - ref, -ex - ew)) / np.linalg.norm(np.ldexp(ref, -ex - ew))
+    assert err <= 2.0 ** -24 * (1.5 * np.sqrt(c * k * k / (2 if redone else 16) / 6) + 1), err
+
+
 @pytest.mark.parametrize("tile", [2, 5, 23, 36, 38, 58, 61, 69, 71])
 @pytest.mark.parametrize("slices", [0, 2])
 def test_conv_f32_split_products_not_finite(slices, tile):
