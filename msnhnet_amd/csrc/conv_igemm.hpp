@@ -807,21 +807,30 @@ constexpr bool igemmSplits(int bm, int bn, int wm, int wn, int kg)
     return mb * nb >= 2 && mb * nb <= 4 && igemmSplitRegs(mb, nb) <= 512 / ((wm * wn * kg + 3) / 4);
 }
 
+// LDS of a workgroup without a tail
+template <int BM, int BN, int KV, int WM, int WN, int NS, int KG> constexpr size_t igemmLds()
+{
+    constexpr int NW = WM * WN * KG, RPP = 64 * NW / KV;
+    constexpr size_t LOOP = static_cast<size_t>(NS) * ((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16;
+    if (igemmAffineEarly<BM, BN, BM / WM, NW, KG, LOOP, 0>()) return igemmAffineOff<BM, BN, BM / WM, NW, KG, LOOP>() + 2 * BM * sizeof(float) + 16;
+    return std::max(LOOP, igemmEpilogueLds<BM, BM / WM, NW>() + 16);      // (16 bytes: the flag of splitKCombine)
+}
+
+// Wavefronts per SIMD the compiler is asked for.  At least two: with the registers of one it keeps the accumulators in the other half of the file, and values
+// that come and go between the halves wait for the loads they belong to.  Split products: as many as the rule's registers allow -- asked for one, it took 277
+// to 302 registers for 64 x 64 wave tiles, and the second workgroup that LDS has room for had none: float32 1x1 64 -> 32 at 304 x 304, 128 x 128 tiles with
+// 64-byte rows 27.9 -> 19.4 us; 1x1 512 -> 256 at 38 x 38, 32 x 64 tiles 9.8 -> 9.2; the layers bound by the matrix rate level.
 template <typename T> constexpr int igemmWavesMin(int bm, int bn, int kv, int wm, int wn, int ns, int kg)
 {
     const int nw = wm * wn * kg;
-    if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg)) return (nw + 3) / 4;
-    return kg >= 4 ? kg / 4 : kg == 2 ? nw / 4 : igemmWavesPerSimd(bm, bn, kv, ns, nw);
+    if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg)) return std::max(512 / igemmSplitRegs(bm / wm / 32, bn / wn / 32), nw / 4);
+    return kg > 1 ? std::max(nw / 4, 2) : igemmWavesPerSimd(bm, bn, kv, ns, nw);
 }
 
 template <typename T> constexpr int igemmWavesMax(int bm, int bn, int kv, int wm, int wn, int ns, int kg)
 {
     const int nw = wm * wn * kg;
-    if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg))
-    {
-        const int fit = 512 / igemmSplitRegs(bm / wm / 32, bn / wn / 32);
-        return fit > nw / 4 ? fit : nw / 4;
-    }
+    if (std::is_same<T, float>::value && igemmSplits(bm, bn, wm, wn, kg)) return igemmWavesMin<T>(bm, bn, kv, wm, wn, ns, kg);
     return kg >= 4 ? 4 : kg == 2 ? (nw == 4 ? 3 : nw / 4) : igemmWavesPerSimd(bm, bn, kv, ns, nw);
 }
 
@@ -1483,12 +1492,26 @@ void convIgemmKernel(IgemmArgs a)
         return probe != 0.f;
     };
 
-    fillStages(std::integral_constant<int, AROWS>());         // (step 0: the filters are on their way)
+    // (the first fill: step 0's filters are on their way)
     if constexpr (std::is_same<T, float>::value && igemmSplits(BM, BN, WM, WN, KG))
     {
+        // the word in which wavefronts report a result that is not finite: beside splitKCombine's flag or, where that costs a workgroup per CU, in the last
+        // stage, which is free behind a barrier and which the first loads below do not reach.  (__syncthreads_or has 256 bytes of its own.)
+        static_assert(SS_EARLY || (KG == 1 && AHEAD < NS && NS * STAGE >= igemmEpilogueLds<BM, TM, NT / 64>() + 32), "room for the word");
+        int *notFinite = reinterpret_cast<int *>(smemRaw + (SS_EARLY ? FLAG_OFF + 4 : NS * STAGE - 16));
+        if (SS_EARLY && tid == 0) *notFinite = 0;
+        fillStages(std::integral_constant<int, AROWS>());
         const bool odd = multiplySplit();
         dmaWait<0>();
-        if (__syncthreads_or(odd))
+        if (!SS_EARLY)
+        {
+            __syncthreads();
+            if (tid == 0) *notFinite = 0;
+            __syncthreads();
+        }
+        if (odd) *notFinite = 1;
+        __syncthreads();
+        if (*notFinite)
         {
             clearBlocks(acc);
             fillStages(std::integral_constant<int, 0>());
@@ -1499,6 +1522,7 @@ void convIgemmKernel(IgemmArgs a)
     }
     else
     {
+        fillStages(std::integral_constant<int, AROWS>());
         multiply();
         dmaWait<0>();
         __syncthreads();
@@ -1561,21 +1585,12 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
         return 3;
     }
     constexpr int RPP = 64 * WM * WN * KG / KV;
-    const size_t smemLoop = static_cast<size_t>(NS) * ((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16;
-    size_t smemEpi = 0;
+    size_t smem = igemmLds<BM, BN, KV, WM, WN, NS, KG>();
     if constexpr (TAIL != 0)
     {
         constexpr unsigned STAGE = static_cast<unsigned>(((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16);
-        smemEpi = TailLds<BM, BN, STAGE>::bytes();
+        smem = std::max(static_cast<size_t>(NS) * STAGE, static_cast<size_t>(TailLds<BM, BN, STAGE>::bytes()));
     }
-    else
-    {
-        constexpr size_t LOOP = static_cast<size_t>(NS) * ((BM + RPP - 1) / RPP * RPP + (BN + RPP - 1) / RPP * RPP) * KV * 16;
-        // (16 bytes: the flag of splitKCombine)
-        if constexpr (igemmAffineEarly<BM, BN, BM / WM, WM * WN * KG, KG, LOOP, TAIL>()) smemEpi = igemmAffineOff<BM, BN, BM / WM, WM * WN * KG, KG, LOOP>() + 2 * BM * sizeof(float) + 16;
-        else smemEpi = igemmEpilogueLds<BM, BM / WM, WM * WN * KG>() + (a.fusedK > 1 ? 16 : 0);
-    }
-    const size_t smem = smemLoop > smemEpi ? smemLoop : smemEpi;
     a.mTiles = (a.coutG + BM - 1) / BM;
     const int tiles = a.mTiles * ((a.P + BN - 1) / BN);
     a.splitK = 1;
