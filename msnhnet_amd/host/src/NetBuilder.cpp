@@ -970,6 +970,14 @@ void NetBuilder::setSaveLayerOutput(bool v)
     if (_planReady) finalizePlan();
 }
 
+// the second tensor of a launch that computes two convolutions (Plan::pairConvs)
+static double pairOutBytes(const Plan &plan, const PlanOp &op)
+{
+    if (op.pair < 0) return 0.0;
+    const PlanTensor &t = plan.tensors[static_cast<size_t>(plan.ops[static_cast<size_t>(op.pair)].out)];
+    return static_cast<double>(t.elems()) * (t.dtype == MSNH_F16 ? 2 : 4);
+}
+
 static double opBytes(const Plan &plan, const PlanOp &op)
 {
     // what the launch must move at least: its input, its output, a fused residual, its weights
@@ -977,6 +985,7 @@ static double opBytes(const Plan &plan, const PlanOp &op)
     const PlanTensor &out = plan.tensors[static_cast<size_t>(op.out)];
     double oe = static_cast<double>(out.elems()) * (out.dtype == MSNH_F16 ? 2 : 4);
     for (int nx = op.chainNext; nx >= 0; nx = plan.ops[static_cast<size_t>(nx)].chainNext) oe += static_cast<double>(out.elems()) * (out.dtype == MSNH_F16 ? 2 : 4);   // one launch, every pool's result
+    oe += pairOutBytes(plan, op);
     if (op.stemTail >= 0)
     {
         const PlanOp &b = plan.ops[static_cast<size_t>(op.stemTail)];
@@ -1069,11 +1078,12 @@ std::string NetBuilder::profileEachOp(int reps, std::vector<double> *values)
         const PlanTensor &in = plan.tensors[static_cast<size_t>(op.in0)];
         const PlanTensor &out = plan.tensors[static_cast<size_t>(op.out)];
         const double bytes = static_cast<double>(in.elems()) * (in.dtype == MSNH_F16 ? 2 : 4) + static_cast<double>(out.elems()) * (out.dtype == MSNH_F16 ? 2 : 4) +
-                             (op.in1 >= 0 ? static_cast<double>(out.elems()) * (out.dtype == MSNH_F16 ? 2 : 4) : 0.0);
+                             (op.in1 >= 0 ? static_cast<double>(out.elems()) * (out.dtype == MSNH_F16 ? 2 : 4) : 0.0) + pairOutBytes(plan, op);
+        const std::string second = op.pair >= 0 ? "+" + std::to_string(plan.tensors[static_cast<size_t>(plan.ops[static_cast<size_t>(op.pair)].out)].c) : std::string();
         char line[320];
-        snprintf(line, sizeof(line), "L%-3d %-11s %-9s t%-2d k%d s%d g%-4d %4dx%4dx%4dx%4d -> %4dx%4dx%4d %s%s %9.2f us %8.2f TF/s %8.1f GB/s\n", op.layerIndex,
+        snprintf(line, sizeof(line), "L%-3d %-11s %-9s t%-2d k%d s%d g%-4d %4dx%4dx%4dx%4d -> %4dx%4dx%4d%s %s%s %9.2f us %8.2f TF/s %8.1f GB/s\n", op.layerIndex,
                  kinds[op.kind], (op.kind == PlanOp::CONV || op.algo != MSNH_CONV_AUTO) ? algos[op.algo] : "-", op.tile, op.ksize, op.stride, op.groups, in.n, in.h, in.w, in.c, out.h, out.w,
-                 out.c, out.dtype == MSNH_F16 ? "f16" : "f32", op.in1 >= 0 ? "+res" : "    ", us, op.flops / us * 1e-6, bytes / us * 1e-3);
+                 out.c, second.c_str(), out.dtype == MSNH_F16 ? "f16" : "f32", op.in1 >= 0 ? "+res" : "    ", us, op.flops / us * 1e-6, bytes / us * 1e-3);
         os << line;
     }
     os << "total " << totalUs << " us over " << plan.liveOps() << " launches\n";

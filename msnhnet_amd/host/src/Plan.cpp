@@ -1704,7 +1704,7 @@ std::string Plan::describe() const
         if (op.kind == PlanOp::MAXPOOL || op.kind == PlanOp::AVGPOOL)
             os << "[k" << op.ksize << " s" << op.stride << " p" << op.pad << (op.chainHead >= 0 ? " in the launch of the pool before it" : "") << "]";
         os << " " << in.n << "x" << in.h << "x" << in.w << "x" << in.c << " -> " << out.h << "x" << out.w << "x" << out.c
-           << (out.dtype == MSNH_F16 ? " f16" : " f32") << " e" << out.scaleExp;
+           << (op.pair >= 0 ? "+" + std::to_string(tensors[static_cast<size_t>(ops[static_cast<size_t>(op.pair)].out)].c) : std::string()) << (out.dtype == MSNH_F16 ? " f16" : " f32") << " e" << out.scaleExp;
         if (out.parent >= 0) os << " (slice@" << chanOffsetInRoot(op.out) << " of " << tensors[static_cast<size_t>(root(op.out))].c << ")";
         os << "\n";
     }

@@ -179,6 +179,7 @@ def test_fp16_headroom_and_hot_input(arch, size, batch):
 
 
 import os
+import re
 GOLD = np.load(os.path.join(os.path.dirname(__file__), "golden", "ref_golden.npz"))
 MICRO = bytes(GOLD["micro/names"]).decode().split("\n")
 
@@ -696,6 +697,26 @@ def test_sibling_convolutions_are_paired(arch, batch, size, fp16):
             assert nu.rel_err(got[b], ref[b][i - 1]) <= (2e-2 if fp16 else 1e-4), (h, b)
     h1, h0 = m.fp16_headroom(x), m0.fp16_headroom(x)
     assert h1 == h0 if not fp16 else abs(h1 - h0) <= 1e-2 * h0
+
+
+@pytest.mark.parametrize("arch,fp16", [("yolov5s", True), ("yolov4", False)])
+def test_paired_convolutions_are_counted(arch, fp16):
+    """The profile of a plan with paired convolutions: the work of the plan without, its least bytes but for the input that a pair reads once, and both
+    tensors named in the plan and in the per-launch lines"""
+    net, binp, g = nu.model(arch, 1, 96, seed=7)
+    m = netapi.Net(net, binp, fp16=fp16)
+    os.environ["MSNH_NO_CONV_PAIR"] = "1"
+    try:
+        m0 = netapi.Net(net, binp, fp16=fp16)
+    finally:
+        del os.environ["MSNH_NO_CONV_PAIR"]
+    pairs = [re.search(r" (\d+)x(\d+)x(\d+)x(\d+) -> (\d+)x(\d+)x(\d+)\+(\d+) f", l) for l in m.plan_detail().splitlines() if "+pair" in l]
+    assert pairs and all(pairs)
+    shared = sum(int(p[1]) * int(p[2]) * int(p[3]) * int(p[4]) * (2 if fp16 else 4) for p in pairs)
+    (_, n1, f1, b1), (_, n0, f0, b0) = m.profile_ops_bytes(0, 1), m0.profile_ops_bytes(0, 1)
+    assert n0 - n1 == len(pairs) and f1 == f0 and b1 == b0 - shared
+    lines = m.profile_each_op(1)
+    assert all(f"{p[7]}+{p[8]}" in lines for p in pairs)
 
 
 @pytest.mark.parametrize("size,batch,fp16", [(32, 1, True), (96, 3, True), (160, 2, True), (96, 2, False)])
