@@ -182,6 +182,16 @@ template <typename A> __device__ __forceinline__ void touchArgs(const A &a)
     asm volatile("" ::"s"(q[0]), "s"(q[line(1)]), "s"(q[line(2)]), "s"(q[line(3)]), "s"(q[line(4)]), "s"(q[line(5)]), "s"(q[line(6)]), "s"(q[line(7)]), "s"(q[last]));
 }
 
+// Lets a kernel be launched with any LDS size that a workgroup can have (beyond the first 48 KiB it has to be asked for).  Always the whole of it: the limit
+// belongs to the kernel, not to the launch, and a smaller launch of another thread must not take it back between this call and the launch behind it.
+inline int allowLds(const void *kernel, size_t bytes)
+{
+    if (bytes <= 48 * 1024) return 0;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
+    return 0;
+}
+
 inline unsigned gridFor(long long n, int block)
 {
     long long g = (n + block - 1) / block;

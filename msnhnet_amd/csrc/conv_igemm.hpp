@@ -1659,12 +1659,7 @@ inline int launchIgemm(IgemmArgs &a, int groups, hipStream_t st)
     a.byChunks = makeFastDiv(static_cast<unsigned>(a.cChunks));
     if (a.dryRun) return 0;
     auto kern = convIgemmKernel<T, TOut, BM, BN, KV, WM, WN, NS, KG, TAIL>;
-    if (smem > 48 * 1024)
-    {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           static_cast<int>(smem));
-        if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
-    }
+    if (const int rc = allowLds(reinterpret_cast<const void *>(kern), smem)) return rc;
     hipLaunchKernelGGL(kern, grid, dim3(64 * WM * WN * KG), smem, st, a);
     MSNH_LAUNCH_CHECK();
     return 0;

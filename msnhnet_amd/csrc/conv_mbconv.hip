@@ -492,7 +492,7 @@ int msnh_hip_mbconv_sliced(const msnh_mbconv_desc *d, const void *x, const void 
     hipStream_t st = resolveStream(s);
     const bool simple = mbFolds(d->act1) && mbFolds(d->act2);
     const auto kern = d->stride == 1 ? (simple ? mbconvKernel<1, true> : mbconvKernel<1, false>) : (simple ? mbconvKernel<2, true> : mbconvKernel<2, false>);
-    if (lds > 48 * 1024) MSNH_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+    if (const int rc = allowLds(reinterpret_cast<const void *>(kern), lds)) return rc;
     hipLaunchKernelGGL(kern, dim3(blocks, static_cast<unsigned>(a.slices)), dim3(64 * MB_NW), lds, st, a);
     MSNH_LAUNCH_CHECK();
     return 0;

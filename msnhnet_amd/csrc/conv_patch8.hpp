@@ -381,11 +381,7 @@ inline int launchPatch8(IgemmArgs &a, int groups, hipStream_t st)
     a.splitK  = 1;
     dim3 grid(igemmGridX(a, (a.P + BN - 1) / BN, sizeof(T), true), 1, 1);
     auto kern = convPatch8Kernel<T, TOut, BM, BN, WM, WN, NSA, PS, DBG, KG>;
-    if (smem > 48 * 1024)
-    {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
-        if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
-    }
+    if (const int rc = allowLds(reinterpret_cast<const void *>(kern), smem)) return rc;
     hipLaunchKernelGGL(kern, grid, dim3(64 * WM * WN * KG), smem, st, a);
     MSNH_LAUNCH_CHECK();
     return 0;

@@ -199,11 +199,7 @@ int launchStem(const StemArgs &a, unsigned blocks, hipStream_t st)
     constexpr int KB = (TAPS + 31) / 32;
     const size_t smem = static_cast<size_t>(MBLK) * KB * 2 * 1024 + 2 * MBLK * 32 * sizeof(float);
     auto kern = convStemMfmaKernel<TAPS, MBLK>;
-    if (smem > 48 * 1024)
-    {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
-        if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
-    }
+    if (const int rc = allowLds(reinterpret_cast<const void *>(kern), smem)) return rc;
     hipLaunchKernelGGL(kern, dim3((blocks + 7) / 8 * 8), dim3(256), smem, st, a);      // a multiple of 8: the XCD regrouping is a bijection then
     MSNH_LAUNCH_CHECK();
     return 0;
@@ -372,11 +368,7 @@ int launchStemRows(const StemRowsArgs &a, unsigned blocks, hipStream_t st)
 {
     const size_t smem = static_cast<size_t>(MBLK) * stemRowChunks(KS) * 1024 + 2 * MBLK * 32 * sizeof(float);
     auto kern = convStemRowsKernel<KS, MBLK>;
-    if (smem > 48 * 1024)
-    {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
-        if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
-    }
+    if (const int rc = allowLds(reinterpret_cast<const void *>(kern), smem)) return rc;
     hipLaunchKernelGGL(kern, dim3((blocks + 7) / 8 * 8), dim3(256), smem, st, a);      // a multiple of 8: the XCD regrouping is a bijection then
     MSNH_LAUNCH_CHECK();
     return 0;
@@ -542,11 +534,7 @@ int launchStemF32(const StemF32Args &a, unsigned blocks, hipStream_t st)
 {
     const size_t smem = static_cast<size_t>(MBLK) * ((stemF32Steps(KS, CIN) + 3) / 4) * 1024 + 2 * MBLK * 32 * sizeof(float);
     auto kern = convStemMfmaF32Kernel<KS, CIN, MBLK>;
-    if (smem > 48 * 1024)
-    {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
-        if (e != hipSuccess) { setError("hipFuncSetAttribute: %s", hipGetErrorString(e)); return 1; }
-    }
+    if (const int rc = allowLds(reinterpret_cast<const void *>(kern), smem)) return rc;
     hipLaunchKernelGGL(kern, dim3((blocks + 7) / 8 * 8, static_cast<unsigned>((a.outC + 31) / (32 * MBLK))), dim3(256), smem, st, a);
     MSNH_LAUNCH_CHECK();
     return 0;

@@ -220,3 +220,36 @@ def test_mbconv_sliced(case, slices):
     if slices > 1:
         assert L.msnh_hip_mbconv_sliced(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), None, gu.ptr(shift), None, gu.ptr(xd), slices, gu.ptr(ws), need - 1, None) != 0
     assert L.msnh_hip_mbconv_sliced(ctypes.byref(d), gu.ptr(xd), gu.ptr(pd), None, gu.ptr(shift), None, gu.ptr(xd), (cexp + 63) // 64 + 1, gu.ptr(ws), need, None) != 0
+
+
+def test_mbconv_sizes_from_two_threads():
+    """Blocks of one kernel with different LDS sizes (68 and 139 KiB) launched by two threads at once: the larger one's limit is not taken back by the
+    smaller one's launch, and each has the result it has alone"""
+    import threading
+    import gpuutil as gu
+    gu.init()
+    runs = []
+    for case in ((1, 8, 13, 15, 72, 8, 2, False), (1, 96, 14, 14, 576, 96, 2, False)):
+        b, cin, h, w, cexp, cout, stride, _ = case
+        rng = np.random.default_rng(cin)
+        f = lambda *shape, k=1.0: gu.round_f16(rng.standard_normal(shape, dtype=np.float32) * np.float32(k))
+        one, zero = np.ones(cexp, np.float32), np.zeros(cexp, np.float32)
+        args = (f(b, cin, h, w), f(cexp, cin, k=0.3), f(cexp, 9, k=0.4), f(cout, cexp, k=0.1), one, zero, one, zero, np.ones(cout, np.float32), np.zeros(cout, np.float32), stride,
+                ("relu6", "relu6", "none", "none"), 1.0, 1.0, 1.0, None, 1.0)
+        runs.append((args, run_mbconv(*args)))
+    wrong = []
+
+    def loop(args, alone):
+        try:
+            for _ in range(25):
+                if not np.array_equal(run_mbconv(*args), alone):
+                    wrong.append("other result")
+        except Exception as e:              # (abi.HipError of a launch that was refused)
+            wrong.append(repr(e))
+
+    threads = [threading.Thread(target=loop, args=r) for r in runs for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:3]
