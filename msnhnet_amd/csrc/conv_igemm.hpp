@@ -774,37 +774,6 @@ template <int BM, int BN, int TM, int NW, int KG, size_t LOOP, int TAIL> constex
     return TAIL == 0 && (KG != 1 || cu / with == cu / off);
 }
 
-template <typename T, typename TOut, int BM, int BN>
-__device__ __forceinline__ void igemmEpilogueGather(const IgemmArgs &a, f32x16 (&acc)[BM / 32][BN / 32], unsigned char *smemRaw, float chScale, float chShift,
-                                                    int m0, int p0, int wave, int lane, int g, int tileIdx, int nTiles, float *ss)
-{
-    constexpr int MB = BM / 32, NB = BN / 32;
-    float *xch = reinterpret_cast<float *>(smemRaw);
-    if (wave > 0)
-        staticFor<0, MB * NB>([&](auto ijTag) {
-            constexpr int ij = decltype(ijTag)::value;
-            float *put = xch + (wave - 1) * BM * BN + ij * 1024 + lane;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) put[r * 64] = acc[ij / NB][ij % NB][r];
-        });
-    __syncthreads();
-    if (wave == 0)
-        for (int k = 0; k < 3; ++k)
-            staticFor<0, MB * NB>([&](auto ijTag) {
-                constexpr int ij = decltype(ijTag)::value;
-                const float *get = xch + k * BM * BN + ij * 1024 + lane;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[ij / NB][ij % NB][r] += get[r * 64];
-            });
-    if (a.fusedK > 1 && !splitKCombine(a.ws, a.splitK, acc, tileIdx, nTiles, wave, 1, lane, reinterpret_cast<int *>(ss + 2 * BM))) return;
-    if (wave > 0) return;
-    // (the parked sums are in registers before the staging writes reach their region: one wavefront's LDS accesses are served in order)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    igemmEpilogue<T, TOut, BM, BN, BM, BN>(a, acc, smemRaw, chScale, chShift, m0, p0, 0, 0, 0, lane, g, ss, xch);
-}
-
 // Register budget: two workgroups per CU (one wave of each per SIMD) so that one workgroup's barrier and epilogue
 // are covered by the other's MFMAs; smaller tiles, which serve the short-K bandwidth-bound layers, get three to six.
 constexpr int igemmWavesPerSimd(int bm, int bn, int kv = 8, int ns = 3, int nw = 4)

@@ -1116,8 +1116,8 @@ static std::string tuneHeader(int nTiles, bool preferWinograd)
 }
 
 // Per-layer search over the implicit-GEMM tile configurations: each candidate runs the real launch (same buffers,
-// same epilogue) a few times between two device events; the fastest wins.  Tiles change the result by nothing but the
-// float32 summation order, and so does the split-K variant tried for layers with few output tiles.
+// same epilogue) a few times between two device events; the fastest wins.  Tiles and slices change the result by the order of the
+// float32 sums, and a float32 layer's by how its products are formed (float32 or split into bfloat16 pieces), within float32's rounding either way.
 // With a cache file: a file written by an earlier search over the same launches on the same device replaces the search.
 void Plan::tuneConvs(msnh_stream_t s, const std::string &cacheFile)
 {

@@ -362,7 +362,8 @@ def test_conv_winograd_fused(b, c, h, w, oc, with_res):
 @pytest.mark.parametrize("act,act2", [("mish", "none"), ("swish", "mish"), ("leaky", "swish"), ("relu6", "relu"), ("logistic", None)])
 @pytest.mark.parametrize("oc,pad_ld", [(200, 0), (93, 3)])
 def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
-    """The epilogue's paths on tiles of every wavefront grid: transcendental activations in front of and behind the residual, channel vectors cut off by
+    """The epilogue's paths on tiles of every wavefront grid (those that deal a step's k-blocks to four or eight wavefronts in float32 only: they take float16 from 1024
+    products on, test_conv_epilogue_forms_gathered): transcendental activations in front of and behind the residual, channel vectors cut off by
     out_c, rows that are no multiple of eight channels, a last pixel tile of 13 x 11 pixels."""
     import gpuutil as gu
     b, c, h, w = 3, 72, 13, 11
@@ -386,6 +387,29 @@ def test_conv_epilogue_forms(oc, pad_ld, act, act2, dtype):
         ran += 1
         assert gu.rel_err(y, ref) <= TOL[dtype], (tile, gu.rel_err(y, ref))
     assert ran >= 15
+
+
+@pytest.mark.parametrize("dtype,out_dtype", [(abi.F32, abi.F32), (abi.F16, abi.F16), (abi.F16, abi.F32)])
+@pytest.mark.parametrize("act,act2", [("mish", "none"), ("swish", "mish"), ("leaky", "swish"), ("relu6", "relu"), ("logistic", None)])
+@pytest.mark.parametrize("oc,pad_ld", [(96, 0), (93, 3), (90, 0)])
+def test_conv_epilogue_forms_gathered(oc, pad_ld, act, act2, dtype, out_dtype):
+    """The same for the tiles that add up the k-blocks of four or eight wavefronts, at a depth that they take in either type: whole four-channel vectors, vectors cut off by
+    out_c and unaligned rows, with the residual read and added element by element"""
+    import gpuutil as gu
+    b, c, h, w = 3, 136, 13, 11
+    rng = np.random.default_rng(oc + len(act) + 1)
+    x, wt = _case(rng, b, c, h, w, oc, 3)
+    res = rng.standard_normal((b, oc, h, w), dtype=np.float32) if act2 else None
+    scale = rng.uniform(0.5, 1.5, oc).astype(np.float32)
+    shift = (rng.standard_normal(oc) * 0.1).astype(np.float32)
+    if dtype == abi.F16:
+        x, wt = gu.round_f16(x), gu.round_f16(wt)
+        res = gu.round_f16(res) if act2 else None
+    ref = _ref(x, wt, 1, 1, 1, 1, scale, shift, act, 0.1, res, act2 or "none", 0.5, 2.0)
+    for tile in (67, 68, 69, 70, 71, 72, 73):
+        y, _ = gu.conv2d(x, wt, dtype=dtype, out_dtype=out_dtype, stride=1, pad=1, scale=scale, shift=shift, act=act, residual=res, act2=act2 or "none", res_mul=0.5, out_mul=2.0,
+                         algo="igemm", tile=tile, out_ld=oc + pad_ld, res_ld=oc + pad_ld)
+        assert gu.rel_err(y, ref) <= TOL[dtype], (tile, gu.rel_err(y, ref))
 
 
 @pytest.mark.parametrize("dtype,out_dtype", [(abi.F32, abi.F32), (abi.F16, abi.F16), (abi.F16, abi.F32)])
@@ -495,6 +519,8 @@ def test_conv_f32_split_products_not_finite(slices, tile):
     else:
         y, _ = gu.conv2d(x, wt, algo="igemm", tile=tile, **kw)
     assert gu.rel_err(y, ref) <= TOL[abi.F32]
+    ordinary = np.isfinite(ref) & (np.abs(np.where(np.isfinite(ref), ref, 0)) < 1e6)       # (beside results of 1e38 any of them would pass)
+    assert ordinary.sum() > 1000 and gu.rel_err(y[ordinary], ref[ordinary]) <= TOL[abi.F32]
 
 
 @pytest.mark.parametrize("dtype", [abi.F32, abi.F16])
@@ -597,7 +623,7 @@ def test_conv_fused_k(case, dtype):
     assert L.msnh_hip_conv2d_tile_supported(ctypes.byref(d), 12) == 0          # a tile without slices is not this algorithm
     ws = torch.zeros(64 << 20, dtype=torch.uint8).cuda()
     tried = 0
-    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66, 67, 68, 69, 70, 71, 72):
+    for tile in (1, 6, 9, 12, 30, 36, 38, 57, 58, 59, 60, 64, 65, 66, 67, 68, 69, 70, 71, 72, 73, 74):
         for slices in (2, 3, 7, 16):
             d.tile = tile + 256 * slices
             need = L.msnh_hip_conv2d_workspace_bytes(ctypes.byref(d), algo)
