@@ -219,16 +219,15 @@ int convIgemmTail(const msnh_conv_desc *d, const msnh_conv_tail_desc *tail, cons
     return convIgemmAny(d, x, w, scale, shift, residual, y, st, dryRun, nullptr, 0, tail, w2, scale2, shift2, z);
 }
 
-// d->out_ld: the first tensor's.  Tile 0: the one the shape's rule names or, where that one's wave tiles are cut by the border between the tensors, the first
-// that takes the pair.
+// d->out_ld: the first tensor's.  Tile 0: the one that the shape's rule names, whose wave tiles have 64 channels, or, where the border between the tensors cuts
+// those, a 64 x 64 tile, whose wave tiles have 32.  (Of the tiles with 32, float32 1x1 512 -> 256 at 38 x 38, one / eight images: 64 x 64 13.3 / 30.5 us, 64 x 128
+// 20.4 / 41.4, 32 x 256 21.1 / 42.8, 128 x 192 39.7 / 44.8; float16 256 -> 256 at 38 x 38, eight images, 64 x 64 7.0, 128 x 192 7.9.)
 int convIgemmPair(const msnh_conv_desc *d, const msnh_conv_pair_desc *pair, const void *x, const void *w, const float *scale, const float *shift, void *y, void *y2,
                   hipStream_t st, bool dryRun, void *ws, size_t wsBytes)
 {
     msnh_conv_desc c = *d;
-    const auto run = [&](bool dry) { return convIgemmAny(&c, x, w, scale, shift, nullptr, y, st, dry, ws, wsBytes, nullptr, nullptr, nullptr, nullptr, y2, nullptr, pair); };
-    if (c.algo != MSNH_CONV_IGEMM_FUSEDK && c.tile == 0 && run(true) != 0)
-        for (c.tile = 1; c.tile < kIgemmTailTileFirst && run(true) != 0;) ++c.tile;
-    return run(dryRun);
+    if (c.algo != MSNH_CONV_IGEMM_FUSEDK && c.tile == 0 && pair->first_c % 64 != 0) c.tile = c.in_c >= (c.dtype == MSNH_F16 ? 64 : 32) ? 12 : 6;
+    return convIgemmAny(&c, x, w, scale, shift, nullptr, y, st, dryRun, ws, wsBytes, nullptr, nullptr, nullptr, nullptr, y2, nullptr, pair);
 }
 
 int convIgemm(const msnh_conv_desc *d, const void *x, const void *w, const float *scale, const float *shift,

@@ -1647,11 +1647,11 @@ namespace msnh {
 constexpr int kIgemmTiles = 76;
 constexpr int kIgemmTailTileFirst = 75;         // tiles from here on carry a tail (msnh_hip_conv2d_tail)
 
-// The configurations on which a sliced launch (MSNH_CONV_IGEMM_FUSEDK) is worth timing whatever they do unsliced: 32 x 32 to 128 x 64, which give a layer of
-// few output tiles the most workgroups before it is cut.  (Larger ones are tried where they are among a layer's fastest unsliced.)  Over the layers of 16
-// networks at batch 1 to 32 in both types the search took 67 83 times, 68 20, 12 19, 65 16, 6 twice, 64 and 66 once; 30 (64 x 64 with two stages of
-// 64-byte rows) and 69 (32 x 64) never, and timing them costs a load 1 to 3 %.
-constexpr int kIgemmSlicedTiles[] = {6, 12, 64, 65, 66, 67, 68, 70, 71, 72, 73, 74};
+// The configurations on which a sliced launch (MSNH_CONV_IGEMM_FUSEDK) is worth timing whatever they do unsliced: 32 x 32 to 64 x 64, which give a layer of
+// few output tiles the most workgroups before it is cut.  (Larger ones are tried where they are among a layer's six fastest unsliced.)  Over the layers of
+// seven networks at batch 1 to 64 in both types (97 loads) the search took 69 164 times, 67 87, 70 83, 68 59, 73 25, 71 21, 72 15, 6 13, 12 9, 64 3 and, as one of the
+// fastest unsliced, 8 19 times; 66 (eight wavefronts over 128 x 64) once, 65 (over 64 x 128) and 74 (64 x 64 with a fourth stage) never.
+constexpr int kIgemmSlicedTiles[] = {6, 12, 64, 67, 68, 69, 70, 71, 72, 73};
 
 // One translation unit instantiates every third configuration of one type pair (tile % kIgemmParts == PART), so that they compile in parallel.
 constexpr int kIgemmParts = 3;
