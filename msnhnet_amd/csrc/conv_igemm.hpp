@@ -159,34 +159,59 @@ __device__ __forceinline__ void mfmaBlock(const f32x4 &a, const f32x4 &b, f32x16
 // accumulator of their own: added to the large one they would be rounded at its magnitude five times per 16 k, apart from it they are not, and the
 // large one is rounded once per 16 k instead of eight times.  Against 64-bit sums, normal and rectified operands, K = 576 / 4608: 1.3e-7 / 4.2e-7 of
 // the results' rms, where the float32 MFMAs give 4.4e-7 / 1.2e-6 (one accumulator for all six: 3.7e-7 / 1.1e-6).
-// A piece keeps its bits down to 2^-133 and the pieces of a float32 value reach down to 2^-149, so both operands are multiplied by 2^16 before they are split
-// and the sums by 2^-32 behind the loop: every float32 value, subnormal ones too, is then exactly the sum of its pieces (the matrix cores and the
-// conversions keep subnormal numbers).  Without it operands below 2^-110 lose their low pieces: 2^-118 times 2^60, K = 576, errs by 8.7e-6 of the
-// results' rms.  (It costs eight of 52 instructions: yolov3 f32 b1 1845 -> 1901 us, resnet50 f32 b5 794 -> 806.  Looking for such operands instead, to multiply
-// their tiles as float32, costs four, but swish and mish turn every strongly negative value into one.)
-// What the factors push out of range -- operands from 2^111, sums from 2^95 -- becomes an infinity or NaN, as do infinities themselves (an infinity
+// A piece keeps its bits down to 2^-133 and the pieces of a float32 value reach down to 2^-149, so both operands are multiplied by 2^24 before they are split
+// and the sums by 2^-48 behind the loop: every float32 value, subnormal ones too, is then exactly the sum of its pieces, none of them subnormal.
+// Without it operands below 2^-110 lose their low pieces: 2^-118 times 2^60, K = 576, errs by 8.7e-6 of the results' rms.  (Looking for such operands instead,
+// to multiply their tiles as float32, does not do: swish and mish turn every strongly negative value into one.)
+// What the factors push out of range -- operands from 2^103, sums from 2^79 -- becomes an infinity or NaN, as do infinities themselves (an infinity
 // times a piece that is zero is NaN, where the float32 product is an infinity); every result that such an operand reaches is then not finite, so a workgroup
 // that finds a result that is not finite multiplies its tile again with the float32 MFMAs.
 // (The pieces and the choice of six products: Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
 // Computations", ARITH 2019.)
-constexpr float kSplitScale = 65536.f, kSplitUnscale = 1.f / (65536.f * 65536.f);
+constexpr float kSplitScale = 16777216.f, kSplitUnscale = 1.f / (16777216.f * 16777216.f);
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-// 8 values in 52 vector instructions: a conversion rounds two values, a shift and a mask widen them again.
-__device__ __forceinline__ void splitF32(const f32x4 &a, const f32x4 &b, bf16x8 &hi, bf16x8 &mid, bf16x8 &lo)
+// Both halves of a packed pair taken off the float32 values they were rounded from; exact, the remainders have 16 significant bits at most.  Widening a half and
+// subtracting it are two instructions, a dot product of the pair with {-1, 0} or {0, -1} is one (2^30 pairs of random bits agree), but those go where the
+// MFMAs go.  So the tiles take them that deal a step's k-blocks to two or eight groups of wavefronts, which leave the matrix cores waiting at one or two wavefronts
+// per SIMD.  float32 3x3 256 -> 512 at 38 x 38, eight images, two instructions -> one: 128 x 64 in two groups 196 -> 185 us, 128 x 128 in two 203 -> 198, 32 x 64 in
+// eight 254 -> 242; in four, three workgroups per CU, 209 -> 210; undivided 128 x 128 194 -> 204, 256 x 128 177 -> 186, 64 x 128 201 -> 207; resnet50 f32 b5
+// 799 -> 788.
+// (The selectors are kept from the compiler, which would put the constants into the instruction, where one half stands for both.)
+template <bool DOT> struct SplitRest
+{
+    unsigned takeLo = 0x0000bf80u, takeHi = 0xbf800000u;
+    __device__ __forceinline__ SplitRest() { asm("" : "+s"(takeLo), "+s"(takeHi)); }
+    __device__ __forceinline__ void operator()(float &v0, float &v1, unsigned pair) const
+    {
+        if constexpr (DOT)
+        {
+            v0 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, takeLo), v0, false);
+            v1 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pair), __builtin_bit_cast(bf16x2, takeHi), v1, false);
+        }
+        else
+        {
+            v0 -= __builtin_bit_cast(float, pair << 16);
+            v1 -= __builtin_bit_cast(float, pair & 0xffff0000u);
+        }
+    }
+};
+
+// 8 values in 52 vector instructions, 36 with dot products: a factor each, a conversion rounds two values.
+template <bool DOT> __device__ __forceinline__ void splitF32(const f32x4 &a, const f32x4 &b, const SplitRest<DOT> &rest, bf16x8 &hi, bf16x8 &mid, bf16x8 &lo)
 {
     u32x4 h, m, l;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
     {
-        const float v0 = kSplitScale * (e < 2 ? a[2 * e] : b[2 * e - 4]), v1 = kSplitScale * (e < 2 ? a[2 * e + 1] : b[2 * e - 3]);
+        float v0 = kSplitScale * (e < 2 ? a[2 * e] : b[2 * e - 4]), v1 = kSplitScale * (e < 2 ? a[2 * e + 1] : b[2 * e - 3]);
         h[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
-        const float r0 = v0 - __builtin_bit_cast(float, h[e] << 16), r1 = v1 - __builtin_bit_cast(float, h[e] & 0xffff0000u);
-        m[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{r0, r1}, bf16x2));
-        const float s0 = r0 - __builtin_bit_cast(float, m[e] << 16), s1 = r1 - __builtin_bit_cast(float, m[e] & 0xffff0000u);
-        l[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{s0, s1}, bf16x2));
+        rest(v0, v1, h[e]);
+        m[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
+        rest(v0, v1, m[e]);
+        l[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
     }
     hi = __builtin_bit_cast(bf16x8, h);
     mid = __builtin_bit_cast(bf16x8, m);
@@ -790,9 +815,10 @@ constexpr int igemmWavesPerSimd(int bm, int bn, int kv = 8, int ns = 3, int nw =
 
 // float32 tiles whose wavefronts have the registers for the split product (splitF32): per 32 x 32 block two accumulators, per block row and column the
 // three pieces and the values they come from.  The others multiply with the float32 MFMAs, and so do those with one block per wavefront: there the split
-// of two operands (88 vector instructions, 104 with the factors) costs what the matrix cores save, 3x3 64 -> 64 at 56 x 56 8.66 -> 9.21 us, 256 -> 256 at 14 x 14 11.2 -> 11.9.
-// The others, start -> now: 3x3 256 -> 512 at 38 x 38 eight images 214 -> 172 us, one image 38.2 -> 32.2; 128 -> 256 at 76 x 76 eight images 223 -> 173;
-// 1x1 512 -> 256 at 38 x 38 eight images 32.3 -> 28.0.  What binds then is the bfloat16 rate under load: 159 x 6 = 954 TFLOP/s where a large matrix product gets 1120.
+// of two operands costs what the matrix cores save, 3x3 64 -> 64 at 56 x 56 8.66 -> 9.21 us, 256 -> 256 at 14 x 14 11.2 -> 11.9 (at 88 vector instructions; 104 now).
+// float32 MFMAs -> split, best tile: 3x3 256 -> 512 at 38 x 38 eight images 212 -> 177 us, one image 35.9 -> 33.0; 128 -> 256 at 76 x 76 eight images 218 -> 168;
+// 1x1 512 -> 256 at 38 x 38 eight images 31.2 -> 29.4.  What binds then is the SIMD, which has the split and the MFMAs one after the other: 32 x 64 tiles spend
+// 764 cycles of vector instructions per 16 k, 624 of them on the split, and 384 of MFMAs (counted), 64 x 64 wave tiles 832 and 768.
 constexpr int igemmSplitRegs(int mb, int nb) { return 32 * mb * nb + 20 * (mb + nb) + 40; }
 constexpr bool igemmSplits(int bm, int bn, int wm, int wn, int kg)
 {
@@ -1436,6 +1462,7 @@ void convIgemmKernel(IgemmArgs a)
         constexpr int S2     = S / 2;            // pairs of k-blocks per tile step and wavefront
         constexpr int NPRE2  = NS >= 3 ? (S2 - 1) * NL / S2 : 0;              // loads of a step in front of its barrier
         constexpr int INFL2  = NS >= 3 ? (NS - 3) * NL + NPRE2 : 0;
+        const SplitRest<(KG == 2 || KG == 8)> rest;
         f32x16 low[MB][NB];
         clearBlocks(low);
         unsigned cur = 0, nxt = STAGE, nn = NS >= 3 ? (NS - 1) * STAGE : 0;
@@ -1450,9 +1477,9 @@ void convIgemmKernel(IgemmArgs a)
                 if constexpr (std::is_same<T, float>::value)
                 {
 #pragma unroll
-                    for (int i = 0; i < MB; ++i) splitF32(fa[0][i], fa[1][i], sa[0][i], sa[1][i], sa[2][i]);
+                    for (int i = 0; i < MB; ++i) splitF32(fa[0][i], fa[1][i], rest, sa[0][i], sa[1][i], sa[2][i]);
 #pragma unroll
-                    for (int j = 0; j < NB; ++j) splitF32(fb[0][j], fb[1][j], sb[0][j], sb[1][j], sb[2][j]);
+                    for (int j = 0; j < NB; ++j) splitF32(fb[0][j], fb[1][j], rest, sb[0][j], sb[1][j], sb[2][j]);
                 }
                 if constexpr (p < S2 - 1)
                 {
