@@ -171,8 +171,7 @@ __device__ __forceinline__ unsigned fastDiv(unsigned n, const FastDiv &f)
 
 // One word of every 64-byte line of the arguments, so that all lines are in the scalar cache after one trip to memory.  The compiler loads a field where
 // it is used, and the cache is cold at the start of a launch: the chain tile -> addresses -> first load met four such trips one after the other.
-// With that, divisions by reciprocals from the host, tap masks without loops and the affines published by the loop's barriers: yolov3 f16 b1 746 -> 690 us
-// (75 convolutions), yolov5s f16 b3 609 -> 581, resnet50 f16 b32 870 -> 816 (with the epilogue kept out of scratch memory), yolov3 f32 b1 1919 -> 1819.
+// Alone, 12 networks 1.017x: yolov3 f16 b1 (75 convolutions) 682 -> 643 us, b8 1970 -> 1918, resnet50 f16 b32 852 -> 837, yolov5s f16 b3 531 -> 521.
 template <typename A> __device__ __forceinline__ void touchArgs(const A &a)
 {
     constexpr int words = sizeof(A) / 4, last = words - 1;

@@ -248,6 +248,7 @@ template <typename V> __device__ __forceinline__ V bufferLoad16(__amdgpu_buffer_
 // memory with a wait behind every residual load.  So there is one instance of it per kernel, a transcendental activation meets 16 values at a time, and the
 // rare paths are rolled loops.  (Raw partial sums as a second instance, 32 values per activation and the rare paths unrolled: 128 x 128 tile 27.8k instead
 // of 5.9k instructions and 218 instead of 0 values in scratch; yolov4 f16 b16 4396 -> 4204 us, yolov3 f16 b8 2076 -> 2011, resnet50 f16 b32 926 -> 897.)
+// (What is left in scratch: two to four values of the 64 x 128 and 128 x 64 wave tiles, and 28 of the 256 x 192 tile with a tail, whose epilogue is its own.)
 template <typename T> struct Raw8;               // 8 consecutive elements as loaded / stored
 template <> struct Raw8<f16>
 {

@@ -36,10 +36,15 @@ def _kernels():
 
 
 @pytest.fixture(scope="module")
-def igemm():
+def kernels():
+    return _kernels()
+
+
+@pytest.fixture(scope="module")
+def igemm(kernels):
     """(types, BM, BN, KV, WM, WN, NS, KG, tail) -> metadata of the implicit-GEMM kernels"""
     out = {}
-    for n, k in _kernels().items():
+    for n, k in kernels.items():
         m = re.match(r"_ZN4msnh15convIgemmKernelI(\w+?)((?:Li\d+E)+)E", n)
         if m:
             out[(m.group(1),) + tuple(int(v) for v in re.findall(r"Li(\d+)E", m.group(2)))] = k
@@ -65,3 +70,15 @@ def test_split_product_tiles_reach_their_occupancy(igemm):
         seen += 1
         assert k[".vgpr_count"] <= (256 if blocks == 4 else 168) and k[".vgpr_spill_count"] == 0, (bm, bn, kv, wm, wn, ns, kg)
     assert seen == 29
+
+
+def test_scratch_memory_stays_where_it_is_known(kernels, igemm):
+    """Values that kernels keep in scratch memory: a few of the 64 x 128 and 128 x 64 wave tiles, the tile with a tail, one LDS-patch tile and the widest pointwise
+    kernel; no other"""
+    for (types, bm, bn, kv, wm, wn, ns, kg, tail), k in igemm.items():
+        most = 28 if tail and bm == 256 else 4 if (bm // wm) * (bn // wn) == 64 * 128 else 0
+        assert k[".vgpr_spill_count"] <= most, (types, bm, bn, kv, wm, wn, ns, kg, tail)
+    for n, k in kernels.items():
+        if "convIgemmKernel" not in n:
+            most = 1 if "convPatch8KernelI" in n and "Li256ELi192E" in n else 14 if "convPointwiseKernelILi4ELi4EE" in n else 0
+            assert k[".vgpr_spill_count"] <= most, n
