@@ -817,8 +817,8 @@ constexpr int igemmWavesPerSimd(int bm, int bn, int kv = 8, int ns = 3, int nw =
 // float32 tiles whose wavefronts have the registers for the split product (splitF32): per 32 x 32 block two accumulators, per block row and column the
 // three pieces and the values they come from.  The others multiply with the float32 MFMAs, and so do those with one block per wavefront: there the split
 // of two operands costs what the matrix cores save, 3x3 64 -> 64 at 56 x 56 8.66 -> 9.21 us, 256 -> 256 at 14 x 14 11.2 -> 11.9 (at 88 vector instructions; 104 now).
-// float32 MFMAs -> split, best tile: 3x3 256 -> 512 at 38 x 38 eight images 212 -> 177 us, one image 35.9 -> 33.0; 128 -> 256 at 76 x 76 eight images 218 -> 168;
-// 1x1 512 -> 256 at 38 x 38 eight images 31.2 -> 29.4.  What binds then is the SIMD, which has the split and the MFMAs one after the other: 32 x 64 tiles spend
+// float32 MFMAs -> split, best unsliced tile, eight images: 3x3 256 -> 512 at 38 x 38 211 -> 179 us, 128 -> 256 at 76 x 76 217 -> 169, 512 -> 1024 at 19 x 19
+// 228 -> 190, 1x1 512 -> 256 at 38 x 38 33.0 -> 30.1.  What binds then is the SIMD, which has the split and the MFMAs one after the other: 32 x 64 tiles spend
 // 764 cycles of vector instructions per 16 k, 624 of them on the split, and 384 of MFMAs (counted), 64 x 64 wave tiles 832 and 768.
 constexpr int igemmSplitRegs(int mb, int nb) { return 32 * mb * nb + 20 * (mb + nb) + 40; }
 constexpr bool igemmSplits(int bm, int bn, int wm, int wn, int kg)

@@ -483,7 +483,7 @@ def test_conv_f32_split_products(c, oc, k, tile):
 @pytest.mark.parametrize("ex,ew,redone", [(-118, 60, False), (60, -118, False), (-118, 0, False), (-142, 100, False), (-60, -40, False), (-118, 118, True), (120, -120, True)])
 def test_conv_f32_split_products_small_and_large(ex, ew, redone, tile):
     """Operands of 2^ex and 2^ew, among them subnormal ones and those whose low bfloat16 pieces lie below what bfloat16 can hold: the error against 64-bit
-    sums is the one of operands of order one (test_conv_f32_split_products).  redone: an operand from 2^111 on is multiplied as float32, one rounding per
+    sums is the one of operands of order one (test_conv_f32_split_products).  redone: an operand from 2^103 on is multiplied as float32, one rounding per
     2 products -- the same bound with K / 2 roundings."""
     import torch
     import gpuutil as gu
